@@ -9,6 +9,7 @@ import os
 import shutil
 import subprocess
 import sys
+from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 PKG = os.path.dirname(HERE)
@@ -19,7 +20,11 @@ LIB = os.path.join(PKG, "libsdmd.so")
 ARCH = os.environ.get("SDMD_OFFLOAD_ARCH", "gfx950")
 
 HOST_SOURCES = ["host/sdmd_host.c", "host/sdmd_remd.c", "host/sdmd_io.c"]
-HIP_SOURCES = ["sdmd_gpu.hip", "sdmd_fast.hip"]
+# (source, extra flags, object): the fast engine's kernels are one unit per
+# workgroup size (SDMD_FAST_WAVES wavefronts), compiled side by side
+FAST_WAVES = (8, 4, 16, 12, 1)
+HIP_UNITS = [("sdmd_fast.hip", ["-DSDMD_FAST_WAVES=%d" % w], "sdmd_fast_w%d.o" % w) for w in FAST_WAVES]
+HIP_UNITS += [("sdmd_gpu.hip", [], "sdmd_gpu.hip.o"), ("sdmd_fast.hip", [], "sdmd_fast.hip.o")]
 
 
 def _hipcc():
@@ -43,12 +48,17 @@ def build(verbose=True):
               "-Wall", "-Wno-format-truncation", "-I" + INC, "-c", os.path.join(HERE, src), "-o", obj])
         objs.append(obj)
     hipcc = _hipcc()
-    for src in HIP_SOURCES:
-        obj = os.path.join(BUILD, os.path.basename(src) + ".o")
+
+    def compile_unit(unit):
+        src, flags, name = unit
+        obj = os.path.join(BUILD, name)
         _run([hipcc, "--offload-arch=" + ARCH, "-O3", "-std=c++17", "-fPIC", "-ffp-contract=off",
-              "-fno-fast-math", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
-              "-I" + INC, "-c", os.path.join(HERE, src), "-o", obj])
-        objs.append(obj)
+              "-fno-fast-math", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"] + flags +
+             ["-I" + INC, "-c", os.path.join(HERE, src), "-o", obj])
+        return obj
+
+    with ThreadPoolExecutor(max_workers=max(1, min(8, os.cpu_count() or 1))) as ex:
+        objs += list(ex.map(compile_unit, HIP_UNITS))
     tmp = LIB + ".tmp"
     _run([hipcc, "--offload-arch=" + ARCH, "-shared", "-fPIC", "-o", tmp] + objs + ["-lm"])
     os.replace(tmp, LIB)

@@ -1772,19 +1772,6 @@ __device__ __forceinline__ void job_done(FJobs *J) {
     __hip_atomic_fetch_add(&J->done, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// reset every system's job word before a launch (a kernel, not a memset, so
-// it can sit in a captured graph)
-__global__ void k_fast_jobs_reset(FJobs *jobs, int nsys) {
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s < nsys) {
-        jobs[s].word = 0;
-        jobs[s].done = 0;
-        jobs[s].stop = 0;
-        jobs[s].err = 0;
-        jobs[s].xcc = -1;
-    }
-}
-
 // ---------------------------------------------------------------- shared memory
 struct FShared {
     long long run_clock_end, run_count_end;   // the launch's bounds (thread 0)
@@ -2345,9 +2332,123 @@ __global__ __launch_bounds__(64 * W) void k_fast_run(FSys *systems, FJobs *jobs,
     fsys_store<W>(&systems[sys], Fl);
 }
 
+// CalKinetE + CalPotenE (ToolFunctions.c:626-752) of every system at its
+// snapshot time T (the earliest pending event, the time a download reports):
+// positions are x + v (T - t0), one thread per atom i scanning the 27 cells'
+// arrays for partners j > i
+template <int W>
+__global__ __launch_bounds__(64 * W) void k_fast_energy(FSys *systems, double *out) {
+    __shared__ FSys Fl;
+    __shared__ double tw[W];
+    fsys_load<W>(Fl, &systems[blockIdx.x]);
+    const FSys &F = Fl;
+    const Sys &S = F.s;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    double tm = __builtin_inf();
+    for (int b = tid; b < F.nblk; b += 64 * W) tm = fmin(tm, G(F.b1)[b]);
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) tm = fmin(tm, __shfl_xor(tm, off, 64));
+    if (lane == 0) tw[wave] = tm;
+    __syncthreads();
+    double T = tw[0];
+    for (int w = 1; w < W; w++) T = fmin(T, tw[w]);
+    if (!(T < INFINIT)) T = F.tlast;
+    const int N = S.N;
+    const double cut2 = S.cutoffr * S.cutoffr;
+    double ke = 0, pe = 0;
+    int err = 0;
+    for (int i = 1 + tid; i <= N; i += 64 * W) {
+        const double dti = T - G(F.t0)[i];
+        const double vi[3] = {G(S.vx)[i], G(S.vy)[i], G(S.vz)[i]};
+        const double xi = G(S.x)[i] + vi[0] * dti, yi = G(S.y)[i] + vi[1] * dti, zi = G(S.z)[i] + vi[2] * dti;
+        ke += 0.5 * G(S.mass)[i] * (vi[0] * vi[0] + vi[1] * vi[1] + vi[2] * vi[2]);
+        const int ci[3] = {G(S.cx)[i], G(S.cy)[i], G(S.cz)[i]};
+        for (int n = 0; n < 27; n++) {
+            int cc[3] = {ci[0] + c_OX[n], ci[1] + c_OY[n], ci[2] + c_OZ[n]};
+            double sh[3] = {0, 0, 0};
+            for (int k = 0; k < 3; k++) {
+                if (cc[k] < 0) { cc[k] = S.cellnum[k + 1] - 1; sh[k] = -1 * S.box[k + 1]; }
+                else if (cc[k] >= S.cellnum[k + 1]) { cc[k] = 0; sh[k] = S.box[k + 1]; }
+            }
+            const int cell = cell_id(S, cc[0], cc[1], cc[2]);
+            const int cnt = min(G(F.ccnt)[cell], F.cap);
+            for (int q = 0; q < cnt; q++) {
+                const int j = G(F.cmem)[(size_t)cell * F.cap + q];
+                if (j <= i || j > N) continue;
+                const double dtj = T - G(F.t0)[j];
+                const double vj[3] = {G(S.vx)[j], G(S.vy)[j], G(S.vz)[j]};
+                const double xj = G(S.x)[j] + vj[0] * dtj, yj = G(S.y)[j] + vj[1] * dtj, zj = G(S.z)[j] + vj[2] * dtj;
+                const double r1 = xi - (xj + sh[0]), r2 = yi - (yj + sh[1]), r3 = zi - (zj + sh[2]);
+                const double rr = r1 * r1 + r2 * r2 + r3 * r3;
+                if (rr > cut2) continue;
+                pe += pair_energy(S, i, j, r1, r2, r3, rr, vi, vj, &err);
+            }
+        }
+    }
+    block_sum3<64 * W>(ke, pe, err || S.error, out);
+}
+
+// The event loop, the bulk prediction and the energies for workgroups of W
+// wavefronts.  This file is compiled once per W with SDMD_FAST_WAVES = W
+// (the units build in parallel; each holds the kernels of its W) and once
+// without it for the host side.
+struct FastRun {
+    hipStream_t stream;
+    FSys *sys;
+    FJobs *jobs;
+    FHelp *help;
+    int nsys, helpers, depth;
+    long long npops, budget;
+    double t_end;
+};
+template <int W> void fast_launch_run(const FastRun &r);
+template <int W> void fast_launch_prepare(hipStream_t stream, FSys *sys, int nsys);
+template <int W> void fast_launch_energy(hipStream_t stream, FSys *sys, int nsys, double *out);
+
+#ifdef SDMD_FAST_WAVES
+// one workgroup per system and role, 8 * ceil(nsys / 8) * (1 + helpers) in all
+template <int W>
+void fast_launch_run(const FastRun &r) {
+    const dim3 g(8 * ((r.nsys + 7) / 8) * (1 + r.helpers)), b(64 * W);
+    if (r.depth == 2)
+        hipLaunchKernelGGL((k_fast_run<W, 2>), g, b, 0, r.stream, r.sys, r.jobs, r.help, r.nsys, r.helpers, r.npops,
+                           r.budget, r.t_end);
+    else
+        hipLaunchKernelGGL((k_fast_run<W, 4>), g, b, 0, r.stream, r.sys, r.jobs, r.help, r.nsys, r.helpers, r.npops,
+                           r.budget, r.t_end);
+}
+template <int W>
+void fast_launch_prepare(hipStream_t stream, FSys *sys, int nsys) {
+    hipLaunchKernelGGL((k_fast_prepare<W>), dim3(nsys), dim3(64 * W), 0, stream, sys);
+}
+template <int W>
+void fast_launch_energy(hipStream_t stream, FSys *sys, int nsys, double *out) {
+    hipLaunchKernelGGL((k_fast_energy<W>), dim3(nsys), dim3(64 * W), 0, stream, sys, out);
+}
+template void fast_launch_run<SDMD_FAST_WAVES>(const FastRun &);
+template void fast_launch_prepare<SDMD_FAST_WAVES>(hipStream_t, FSys *, int);
+template void fast_launch_energy<SDMD_FAST_WAVES>(hipStream_t, FSys *, int, double *);
+#endif
+
 }  // namespace sdmd
 
+#ifndef SDMD_FAST_WAVES
 // ==================================================================== host side
+namespace sdmd {
+// reset every system's job word before a launch (a kernel, not a memset, so
+// it can sit in a captured graph)
+__global__ void k_fast_jobs_reset(FJobs *jobs, int nsys) {
+    const int s = blockIdx.x * blockDim.x + threadIdx.x;
+    if (s < nsys) {
+        jobs[s].word = 0;
+        jobs[s].done = 0;
+        jobs[s].stop = 0;
+        jobs[s].err = 0;
+        jobs[s].xcc = -1;
+    }
+}
+}  // namespace sdmd
+
 using namespace sdmd;
 
 struct sdmd::FastState {
@@ -2592,41 +2693,20 @@ static int fast_sync_from(sdmd_gpu_ctx *c) {
 
 int sdmd_fast_sync(sdmd_gpu_ctx *c) { return fast_sync_from(c); }
 
-#define FDISPATCH(kern, ...) do { switch (fs->waves) { \
-    case 4: hipLaunchKernelGGL(kern<4>, dim3(c->nsys), dim3(256), 0, c->stream, __VA_ARGS__); break; \
-    case 8: hipLaunchKernelGGL(kern<8>, dim3(c->nsys), dim3(512), 0, c->stream, __VA_ARGS__); break; \
-    case 12: hipLaunchKernelGGL(kern<12>, dim3(c->nsys), dim3(768), 0, c->stream, __VA_ARGS__); break; \
-    case 16: hipLaunchKernelGGL(kern<16>, dim3(c->nsys), dim3(1024), 0, c->stream, __VA_ARGS__); break; \
-    default: hipLaunchKernelGGL(kern<1>, dim3(c->nsys), dim3(64), 0, c->stream, __VA_ARGS__); break; } } while (0)
+#define FDISPATCH(fn, ...) do { switch (fs->waves) { \
+    case 4: fn<4>(__VA_ARGS__); break; \
+    case 8: fn<8>(__VA_ARGS__); break; \
+    case 12: fn<12>(__VA_ARGS__); break; \
+    case 16: fn<16>(__VA_ARGS__); break; \
+    default: fn<1>(__VA_ARGS__); break; } } while (0)
 
 // the event loop for the context's shape (wavefronts x staging depth x
-// helper workgroups): the job words are reset, then one workgroup per
-// system and role, 8 * ceil(nsys / 8) * (1 + helpers) in all
+// helper workgroups), after a reset of the job words
 static void launch_run(sdmd_gpu_ctx *c, long long pops, long long budget, double t_end) {
     FastState *fs = c->fast;
-    const int H = fs->helpers;
     hipLaunchKernelGGL(k_fast_jobs_reset, dim3((c->nsys + 255) / 256), dim3(256), 0, c->stream, fs->jobs, c->nsys);
-    const dim3 g(8 * ((c->nsys + 7) / 8) * (1 + H));
-#define FRUN(Wv, Qv) hipLaunchKernelGGL((k_fast_run<Wv, Qv>), g, dim3(64 * Wv), 0, c->stream, fs->dev, fs->jobs, \
-                                        fs->help, c->nsys, H, pops, budget, t_end)
-    if (fs->depth == 2) {
-        switch (fs->waves) {
-        case 4: FRUN(4, 2); break;
-        case 8: FRUN(8, 2); break;
-        case 12: FRUN(12, 2); break;
-        case 16: FRUN(16, 2); break;
-        default: FRUN(1, 2); break;
-        }
-    } else {
-        switch (fs->waves) {
-        case 4: FRUN(4, 4); break;
-        case 8: FRUN(8, 4); break;
-        case 12: FRUN(12, 4); break;
-        case 16: FRUN(16, 4); break;
-        default: FRUN(1, 4); break;
-        }
-    }
-#undef FRUN
+    const FastRun r = {c->stream, fs->dev, fs->jobs, fs->help, c->nsys, fs->helpers, fs->depth, pops, budget, t_end};
+    FDISPATCH(fast_launch_run, r);
 }
 
 static int budget_ticks(double max_ms, long long *out) {
@@ -2661,7 +2741,7 @@ double *sdmd_fast_temperature_addr(sdmd_gpu_ctx *c, int s) { return &c->fast->de
 int sdmd_fast_prepare(sdmd_gpu_ctx *c) {
     FastState *fs = c->fast;
     HIPV(hipEventRecord(c->ev0, c->stream));
-    FDISPATCH(k_fast_prepare, fs->dev);
+    FDISPATCH(fast_launch_prepare, c->stream, fs->dev, c->nsys);
     if (hipGetLastError() != hipSuccess) return SDMD_EDEVICE;   // launch rejected (shape, resources)
     HIPV(hipEventRecord(c->ev1, c->stream));
     if (hipStreamSynchronize(c->stream) != hipSuccess) return SDMD_EDEVICE;
@@ -2747,67 +2827,11 @@ int sdmd_fast_download(sdmd_gpu_ctx *c, int s, sdmd_system_desc *out) {
     return rc;
 }
 
-// CalKinetE + CalPotenE (ToolFunctions.c:626-752) of every system at its
-// snapshot time T (the earliest pending event, the time a download reports):
-// positions are x + v (T - t0), one thread per atom i scanning the 27 cells'
-// arrays for partners j > i
-template <int W>
-__global__ __launch_bounds__(64 * W) void k_fast_energy(FSys *systems, double *out) {
-    __shared__ FSys Fl;
-    __shared__ double tw[W];
-    fsys_load<W>(Fl, &systems[blockIdx.x]);
-    const FSys &F = Fl;
-    const Sys &S = F.s;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    double tm = __builtin_inf();
-    for (int b = tid; b < F.nblk; b += 64 * W) tm = fmin(tm, G(F.b1)[b]);
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) tm = fmin(tm, __shfl_xor(tm, off, 64));
-    if (lane == 0) tw[wave] = tm;
-    __syncthreads();
-    double T = tw[0];
-    for (int w = 1; w < W; w++) T = fmin(T, tw[w]);
-    if (!(T < INFINIT)) T = F.tlast;
-    const int N = S.N;
-    const double cut2 = S.cutoffr * S.cutoffr;
-    double ke = 0, pe = 0;
-    int err = 0;
-    for (int i = 1 + tid; i <= N; i += 64 * W) {
-        const double dti = T - G(F.t0)[i];
-        const double vi[3] = {G(S.vx)[i], G(S.vy)[i], G(S.vz)[i]};
-        const double xi = G(S.x)[i] + vi[0] * dti, yi = G(S.y)[i] + vi[1] * dti, zi = G(S.z)[i] + vi[2] * dti;
-        ke += 0.5 * G(S.mass)[i] * (vi[0] * vi[0] + vi[1] * vi[1] + vi[2] * vi[2]);
-        const int ci[3] = {G(S.cx)[i], G(S.cy)[i], G(S.cz)[i]};
-        for (int n = 0; n < 27; n++) {
-            int cc[3] = {ci[0] + c_OX[n], ci[1] + c_OY[n], ci[2] + c_OZ[n]};
-            double sh[3] = {0, 0, 0};
-            for (int k = 0; k < 3; k++) {
-                if (cc[k] < 0) { cc[k] = S.cellnum[k + 1] - 1; sh[k] = -1 * S.box[k + 1]; }
-                else if (cc[k] >= S.cellnum[k + 1]) { cc[k] = 0; sh[k] = S.box[k + 1]; }
-            }
-            const int cell = cell_id(S, cc[0], cc[1], cc[2]);
-            const int cnt = min(G(F.ccnt)[cell], F.cap);
-            for (int q = 0; q < cnt; q++) {
-                const int j = G(F.cmem)[(size_t)cell * F.cap + q];
-                if (j <= i || j > N) continue;
-                const double dtj = T - G(F.t0)[j];
-                const double vj[3] = {G(S.vx)[j], G(S.vy)[j], G(S.vz)[j]};
-                const double xj = G(S.x)[j] + vj[0] * dtj, yj = G(S.y)[j] + vj[1] * dtj, zj = G(S.z)[j] + vj[2] * dtj;
-                const double r1 = xi - (xj + sh[0]), r2 = yi - (yj + sh[1]), r3 = zi - (zj + sh[2]);
-                const double rr = r1 * r1 + r2 * r2 + r3 * r3;
-                if (rr > cut2) continue;
-                pe += pair_energy(S, i, j, r1, r2, r3, rr, vi, vj, &err);
-            }
-        }
-    }
-    block_sum3<64 * W>(ke, pe, err || S.error, out);
-}
-
 // energies of every system into out's three planes (kinetic, potential,
 // error flag; energy_planes_to_host reads them back)
 int sdmd_fast_energy_launch(sdmd_gpu_ctx *c, double *out) {
     FastState *fs = c->fast;
-    FDISPATCH(k_fast_energy, fs->dev, out);
+    FDISPATCH(fast_launch_energy, c->stream, fs->dev, c->nsys, out);
     return hipGetLastError() == hipSuccess ? SDMD_OK : SDMD_EDEVICE;
 }
 
@@ -2940,3 +2964,4 @@ void sdmd_fast_close(sdmd_gpu_ctx *c) {
     free(c->fast);
     c->fast = nullptr;
 }
+#endif  // SDMD_FAST_WAVES
