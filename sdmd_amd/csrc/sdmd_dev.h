@@ -763,33 +763,59 @@ static __device__ void hb_event(Sys &S, int i, int j, int nbi, int nbj, int *err
 }
 
 
-// Sum of two per-thread values over a workgroup of B threads, in a fixed
-// order (each wave by butterfly, then the waves in index order); thread 0
-// writes the two sums to out[0], out[1].
-// Workgroup sums of a and b and the OR of a per-thread error flag, written
-// to out[blockIdx.x], out[gridDim.x + blockIdx.x] and
-// out[2 * gridDim.x + blockIdx.x] (three planes: kinetic, potential, error).
-template <int B>
-static __device__ void block_sum3(double a, double b, int err, double *out) {
-    __shared__ double red[2 * (B / 64)];
-    __shared__ int any_err;
-    if (threadIdx.x == 0) any_err = 0;
-    __syncthreads();
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-        a += __shfl_xor(a, off, 64);
-        b += __shfl_xor(b, off, 64);
-    }
-    if (err) atomicOr(&any_err, 1);
+// Energy sums: workgroup (x, y) of EWAVES wavefronts leaves the sums of its
+// threads' a and b and the OR of their error flags for system x in
+// part[3 * (x * gridDim.y + y) ..]; k_energy_reduce adds a system's
+// workgroups.  Both run in a fixed order (butterfly within a wavefront, then
+// by index), so the energies of a state are the same on every call.
+constexpr int EWAVES = 4;
+template <int S>
+static __device__ __forceinline__ void dsum_step(double &v) {
+    unsigned long long a, b;
+    xpair64<S>((unsigned long long)__double_as_longlong(v), a, b);
+    v = __longlong_as_double((long long)a) + __longlong_as_double((long long)b);
+}
+static __device__ __forceinline__ double wave_sum_d(double v) {
+    dsum_step<0>(v); dsum_step<1>(v); dsum_step<2>(v); dsum_step<3>(v); dsum_step<4>(v); dsum_step<5>(v);
+    return lane_get(v, 0);
+}
+static __device__ __forceinline__ void energy_partial(double a, double b, int err, double *part) {
+    __shared__ double red[2 * EWAVES];
+    __shared__ int any_err[EWAVES];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    if (lane == 0) { red[2 * wave] = a; red[2 * wave + 1] = b; }
+    a = wave_sum_d(a);
+    b = wave_sum_d(b);
+    const bool bad = __ballot(err != 0) != 0;
+    if (lane == 0) { red[2 * wave] = a; red[2 * wave + 1] = b; any_err[wave] = bad; }
     __syncthreads();
     if (threadIdx.x == 0) {
         double sa = 0, sb = 0;
-        for (int w = 0; w < B / 64; w++) { sa += red[2 * w]; sb += red[2 * w + 1]; }
-        G(out)[blockIdx.x] = sa;
-        G(out)[gridDim.x + blockIdx.x] = sb;
-        G(out)[2 * gridDim.x + blockIdx.x] = any_err ? 1.0 : 0.0;
+        int se = 0;
+        for (int w = 0; w < EWAVES; w++) { sa += red[2 * w]; sb += red[2 * w + 1]; se |= any_err[w]; }
+        double *p = part + 3 * ((size_t)blockIdx.x * gridDim.y + blockIdx.y);
+        G(p)[0] = sa;
+        G(p)[1] = sb;
+        G(p)[2] = se ? 1.0 : 0.0;
+    }
+}
+
+// one wavefront per system: out's three planes (kinetic, potential, error)
+static __global__ __launch_bounds__(64) void k_energy_reduce(const double *part, int chunks, double *out) {
+    const int s = blockIdx.x, n = gridDim.x, lane = threadIdx.x;
+    double a = 0, b = 0, e = 0;
+    for (int k = lane; k < chunks; k += 64) {
+        const double *p = part + 3 * ((size_t)s * chunks + k);
+        a += G(p)[0];
+        b += G(p)[1];
+        e += G(p)[2];
+    }
+    a = wave_sum_d(a);
+    b = wave_sum_d(b);
+    e = wave_sum_d(e);
+    if (lane == 0) {
+        G(out)[s] = a;
+        G(out)[n + s] = b;
+        G(out)[2 * n + s] = e != 0 ? 1.0 : 0.0;
     }
 }
 
@@ -812,6 +838,8 @@ struct sdmd_gpu_ctx {
     int nalloc, capalloc;
     int *dev_renew;
     double *dev_energy;        // 3 planes of nsys doubles (kinetic, potential, error flag)
+    double *epart;             // partial energy sums: 3 doubles per system and workgroup
+    int echunks;               // energy workgroups per system
     double *scratch;           // device address of the allocation-free energy planes on this GPU
     double last_ms;
 };

@@ -1846,46 +1846,123 @@ __device__ __forceinline__ void tab_load(ScrTab &dst, const void *src) {
     __syncthreads();
 }
 
+#ifndef SDMD_FAST_WAVES
+// mirror records of every atom, before the bulk prediction reads them
+__global__ __launch_bounds__(256) void k_fast_records(FSys *systems) {
+    FSys &F = systems[blockIdx.x];
+    for (int a = 1 + blockIdx.y * 256 + threadIdx.x; a <= F.s.N; a += 256 * gridDim.y) put_record(F, a);
+}
+
+// Bulk Predict(1..N): a prediction reads positions, velocities and counters
+// but no other atom's event record, so the atoms are spread over gridDim.y
+// workgroups per system (one wavefront per atom at a time).  Bound by the
+// instruction latency of a prediction (about 16 us on one wavefront); with
+// one workgroup per system a 26 080-atom system took 58 ms on one CU.
 template <int W>
-__global__ __launch_bounds__(64 * W) void k_fast_prepare(FSys *systems) {
+__global__ __launch_bounds__(64 * W) void k_fast_predict(FSys *systems) {
     __shared__ FSys Fl;
-    __shared__ FShared sh;
+    __shared__ FWave w[W];
     __shared__ ScrTab tab;
-    fsys_load<W>(Fl, &systems[blockIdx.x]);
+    FSys &Fg = systems[blockIdx.x];
+    fsys_load<W>(Fl, &Fg);
     tab_load<W>(tab, Fl.scrtab);
     FSys &F = Fl;
     Sys &S = F.s;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    if (tid == 0) sh.err = 0;
+    if (tid == 0) {                         // statistics of this workgroup only
+        F.validated = F.agree = F.causal = 0;
+        F.max_screen_err = F.max_time_err = 0;
+        S.prof = nullptr;
+    }
     __syncthreads();
-    for (int a = tid + 1; a <= S.N; a += 64 * W) put_record(F, a);
-    __syncthreads();
-    WStats &ws = sh.w[wave].st;             // in LDS: no registers held across the loop
+    WStats &ws = w[wave].st;                // in LDS: no registers held across the loop
     ws.screen = ws.conf = ws.fp64 = ws.cand = 0;
     __builtin_amdgcn_wave_barrier();
     int err = 0;
-    for (int i = wave + 1; i <= S.N; i += W) {
-        predict_fast<4>(F, tab, sh.w[wave], i, G(F.t0)[i], ws, &err);
+    for (int i = 1 + blockIdx.y * W + wave; i <= S.N; i += W * gridDim.y) {
+        predict_fast<4>(F, tab, w[wave], i, G(F.t0)[i], ws, &err);
         if (__ballot(err != 0)) break;              // uniform across the wave
     }
-    if (err) atomicCAS(&sh.err, 0, err);
+    if (err) atomicCAS(&Fg.s.error, 0, err);
+    if (lane == 0) {
+        cnt_add(Fg.screens, ws.screen);
+        cnt_add(Fg.confirms, ws.conf);
+        cnt_add(Fg.s.pair_evals, ws.fp64 + ws.conf);
+        cnt_add(Fg.s.candidates, ws.cand);
+    }
     __syncthreads();
-    for (int b = wave; b < F.nblk; b += W) {
+    if (tid == 0) {
+        if (F.validated) cnt_add(Fg.validated, F.validated);
+        if (F.agree) cnt_add(Fg.agree, F.agree);
+        if (F.causal) cnt_add(Fg.causal, F.causal);
+        cnt_max(Fg.max_screen_err, F.max_screen_err);
+        cnt_max(Fg.max_time_err, F.max_time_err);
+    }
+}
+
+// the block minima of every system, one wavefront per 64-atom block
+__global__ __launch_bounds__(256) void k_fast_blocks(FSys *systems) {
+    FSys &F = systems[blockIdx.x];
+    for (int b = blockIdx.y * 4 + (threadIdx.x >> 6); b < F.nblk; b += 4 * gridDim.y) {
         double t1, t2, t3;
         int a1, a2;
         block_scan(F, b, t1, a1, t2, a2, t3);
-        if (lane == 0) { G(F.b1)[b] = t1; G(F.ba)[b] = a1; G(F.b2)[b] = t2; G(F.bb)[b] = a2; G(F.b3)[b] = t3; }
+        if ((threadIdx.x & 63) == 0) {
+            G(F.b1)[b] = t1; G(F.ba)[b] = a1; G(F.b2)[b] = t2; G(F.bb)[b] = a2; G(F.b3)[b] = t3;
+        }
     }
-    if (lane == 0) {
-        atomicAdd((unsigned long long *)&F.screens, (unsigned long long)ws.screen);
-        atomicAdd((unsigned long long *)&F.confirms, (unsigned long long)ws.conf);
-        atomicAdd((unsigned long long *)&S.pair_evals, (unsigned long long)(ws.fp64 + ws.conf));
-        atomicAdd((unsigned long long *)&S.candidates, (unsigned long long)ws.cand);
-    }
-    __syncthreads();
-    if (tid == 0 && sh.err) S.error = sh.err;
-    fsys_store<W>(&systems[blockIdx.x], Fl);
 }
+
+// CalKinetE + CalPotenE (ToolFunctions.c:626-752) of every system at its
+// snapshot time T (the earliest pending event, the time a download reports):
+// positions are x + v (T - t0); one wavefront per atom i, two lanes per
+// neighbour cell, for partners j > i.  A chain of dependent loads per pair
+// bounds it, so the atoms are spread over the GPU: gridDim.y workgroups per
+// system, each leaving its sums in `part` (energy_reduce adds them in a fixed
+// order).  One workgroup per system with one thread per atom took 4.0 ms for
+// 64 systems of 1 536 atoms.
+__global__ __launch_bounds__(64 * EWAVES) void k_fast_energy(FSys *systems, double *part) {
+    const FSys &F = systems[blockIdx.x];
+    const Sys &S = F.s;
+    const int tid = threadIdx.x, lane = tid & 63;
+    double tm = __builtin_inf();
+    for (int b = lane; b < F.nblk; b += 64) tm = fmin(tm, G(F.b1)[b]);
+    double T = wave_min_d(tm);
+    if (!(T < INFINIT)) T = F.tlast;
+    const int N = S.N;
+    const double cut2 = S.cutoffr * S.cutoffr;
+    const int c = min(lane >> 1, 26);
+    double ke = 0, pe = 0;
+    int err = 0;
+    for (int i = 1 + blockIdx.y * EWAVES + (tid >> 6); i <= N; i += EWAVES * gridDim.y) {
+        const double dti = T - G(F.t0)[i];
+        const double vi[3] = {G(S.vx)[i], G(S.vy)[i], G(S.vz)[i]};
+        const double xi = G(S.x)[i] + vi[0] * dti, yi = G(S.y)[i] + vi[1] * dti, zi = G(S.z)[i] + vi[2] * dti;
+        if (lane == 0) ke += 0.5 * G(S.mass)[i] * (vi[0] * vi[0] + vi[1] * vi[1] + vi[2] * vi[2]);
+        int cc[3] = {G(S.cx)[i] + c_OX[c], G(S.cy)[i] + c_OY[c], G(S.cz)[i] + c_OZ[c]};
+        double sh[3] = {0, 0, 0};
+        for (int k = 0; k < 3; k++) {
+            if (cc[k] < 0) { cc[k] = S.cellnum[k + 1] - 1; sh[k] = -1 * S.box[k + 1]; }
+            else if (cc[k] >= S.cellnum[k + 1]) { cc[k] = 0; sh[k] = S.box[k + 1]; }
+        }
+        const int cell = cell_id(S, cc[0], cc[1], cc[2]);
+        const int cnt = lane < 54 ? min(G(F.ccnt)[cell], F.cap) : 0;
+        for (int q = lane & 1; q < cnt; q += 2) {
+            const int j = G(F.cmem)[(size_t)cell * F.cap + q];
+            if (j <= i || j > N) continue;
+            const double dtj = T - G(F.t0)[j];
+            const double vj[3] = {G(S.vx)[j], G(S.vy)[j], G(S.vz)[j]};
+            const double xj = G(S.x)[j] + vj[0] * dtj, yj = G(S.y)[j] + vj[1] * dtj, zj = G(S.z)[j] + vj[2] * dtj;
+            const double r1 = xi - (xj + sh[0]), r2 = yi - (yj + sh[1]), r3 = zi - (zj + sh[2]);
+            const double rr = r1 * r1 + r2 * r2 + r3 * r3;
+            if (rr > cut2) continue;
+            pe += pair_energy(S, i, j, r1, r2, r3, rr, vi, vj, &err);
+        }
+    }
+    energy_partial(ke, pe, err || S.error, part);
+}
+
+#endif  // SDMD_FAST_WAVES
 
 // A helper workgroup: its wavefronts claim the owner's published jobs
 // (re-predictions) until the owner stops, then add their statistics to hp.
@@ -2332,66 +2409,10 @@ __global__ __launch_bounds__(64 * W) void k_fast_run(FSys *systems, FJobs *jobs,
     fsys_store<W>(&systems[sys], Fl);
 }
 
-// CalKinetE + CalPotenE (ToolFunctions.c:626-752) of every system at its
-// snapshot time T (the earliest pending event, the time a download reports):
-// positions are x + v (T - t0), one thread per atom i scanning the 27 cells'
-// arrays for partners j > i
-template <int W>
-__global__ __launch_bounds__(64 * W) void k_fast_energy(FSys *systems, double *out) {
-    __shared__ FSys Fl;
-    __shared__ double tw[W];
-    fsys_load<W>(Fl, &systems[blockIdx.x]);
-    const FSys &F = Fl;
-    const Sys &S = F.s;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    double tm = __builtin_inf();
-    for (int b = tid; b < F.nblk; b += 64 * W) tm = fmin(tm, G(F.b1)[b]);
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) tm = fmin(tm, __shfl_xor(tm, off, 64));
-    if (lane == 0) tw[wave] = tm;
-    __syncthreads();
-    double T = tw[0];
-    for (int w = 1; w < W; w++) T = fmin(T, tw[w]);
-    if (!(T < INFINIT)) T = F.tlast;
-    const int N = S.N;
-    const double cut2 = S.cutoffr * S.cutoffr;
-    double ke = 0, pe = 0;
-    int err = 0;
-    for (int i = 1 + tid; i <= N; i += 64 * W) {
-        const double dti = T - G(F.t0)[i];
-        const double vi[3] = {G(S.vx)[i], G(S.vy)[i], G(S.vz)[i]};
-        const double xi = G(S.x)[i] + vi[0] * dti, yi = G(S.y)[i] + vi[1] * dti, zi = G(S.z)[i] + vi[2] * dti;
-        ke += 0.5 * G(S.mass)[i] * (vi[0] * vi[0] + vi[1] * vi[1] + vi[2] * vi[2]);
-        const int ci[3] = {G(S.cx)[i], G(S.cy)[i], G(S.cz)[i]};
-        for (int n = 0; n < 27; n++) {
-            int cc[3] = {ci[0] + c_OX[n], ci[1] + c_OY[n], ci[2] + c_OZ[n]};
-            double sh[3] = {0, 0, 0};
-            for (int k = 0; k < 3; k++) {
-                if (cc[k] < 0) { cc[k] = S.cellnum[k + 1] - 1; sh[k] = -1 * S.box[k + 1]; }
-                else if (cc[k] >= S.cellnum[k + 1]) { cc[k] = 0; sh[k] = S.box[k + 1]; }
-            }
-            const int cell = cell_id(S, cc[0], cc[1], cc[2]);
-            const int cnt = min(G(F.ccnt)[cell], F.cap);
-            for (int q = 0; q < cnt; q++) {
-                const int j = G(F.cmem)[(size_t)cell * F.cap + q];
-                if (j <= i || j > N) continue;
-                const double dtj = T - G(F.t0)[j];
-                const double vj[3] = {G(S.vx)[j], G(S.vy)[j], G(S.vz)[j]};
-                const double xj = G(S.x)[j] + vj[0] * dtj, yj = G(S.y)[j] + vj[1] * dtj, zj = G(S.z)[j] + vj[2] * dtj;
-                const double r1 = xi - (xj + sh[0]), r2 = yi - (yj + sh[1]), r3 = zi - (zj + sh[2]);
-                const double rr = r1 * r1 + r2 * r2 + r3 * r3;
-                if (rr > cut2) continue;
-                pe += pair_energy(S, i, j, r1, r2, r3, rr, vi, vj, &err);
-            }
-        }
-    }
-    block_sum3<64 * W>(ke, pe, err || S.error, out);
-}
-
-// The event loop, the bulk prediction and the energies for workgroups of W
-// wavefronts.  This file is compiled once per W with SDMD_FAST_WAVES = W
-// (the units build in parallel; each holds the kernels of its W) and once
-// without it for the host side.
+// The event loop for workgroups of W wavefronts.  This file is compiled once
+// per W with SDMD_FAST_WAVES = W (the units build in parallel; each holds the
+// event loop of its W) and once without it for the host side and the bulk
+// prediction.
 struct FastRun {
     hipStream_t stream;
     FSys *sys;
@@ -2402,8 +2423,6 @@ struct FastRun {
     double t_end;
 };
 template <int W> void fast_launch_run(const FastRun &r);
-template <int W> void fast_launch_prepare(hipStream_t stream, FSys *sys, int nsys);
-template <int W> void fast_launch_energy(hipStream_t stream, FSys *sys, int nsys, double *out);
 
 #ifdef SDMD_FAST_WAVES
 // one workgroup per system and role, 8 * ceil(nsys / 8) * (1 + helpers) in all
@@ -2417,17 +2436,7 @@ void fast_launch_run(const FastRun &r) {
         hipLaunchKernelGGL((k_fast_run<W, 4>), g, b, 0, r.stream, r.sys, r.jobs, r.help, r.nsys, r.helpers, r.npops,
                            r.budget, r.t_end);
 }
-template <int W>
-void fast_launch_prepare(hipStream_t stream, FSys *sys, int nsys) {
-    hipLaunchKernelGGL((k_fast_prepare<W>), dim3(nsys), dim3(64 * W), 0, stream, sys);
-}
-template <int W>
-void fast_launch_energy(hipStream_t stream, FSys *sys, int nsys, double *out) {
-    hipLaunchKernelGGL((k_fast_energy<W>), dim3(nsys), dim3(64 * W), 0, stream, sys, out);
-}
 template void fast_launch_run<SDMD_FAST_WAVES>(const FastRun &);
-template void fast_launch_prepare<SDMD_FAST_WAVES>(hipStream_t, FSys *, int);
-template void fast_launch_energy<SDMD_FAST_WAVES>(hipStream_t, FSys *, int, double *);
 #endif
 
 }  // namespace sdmd
@@ -2741,7 +2750,16 @@ double *sdmd_fast_temperature_addr(sdmd_gpu_ctx *c, int s) { return &c->fast->de
 int sdmd_fast_prepare(sdmd_gpu_ctx *c) {
     FastState *fs = c->fast;
     HIPV(hipEventRecord(c->ev0, c->stream));
-    FDISPATCH(fast_launch_prepare, c->stream, fs->dev, c->nsys);
+    // predictions: enough workgroups of 8 wavefronts to fill the GPU, at
+    // least one atom per wavefront; a workgroup's set-up (50 KB of tables
+    // into LDS) costs about one prediction
+    int maxn = 1;
+    for (int s = 0; s < c->nsys; s++) maxn = fs->host[s].s.N > maxn ? fs->host[s].s.N : maxn;
+    const int want = (maxn + 7) / 8, fit = (1024 + c->nsys - 1) / c->nsys;
+    const dim3 gp(c->nsys, want < fit ? want : fit), ga(c->nsys, gp.y < 64 ? gp.y : 64);
+    hipLaunchKernelGGL(k_fast_records, ga, dim3(256), 0, c->stream, fs->dev);
+    hipLaunchKernelGGL((k_fast_predict<8>), gp, dim3(512), 0, c->stream, fs->dev);
+    hipLaunchKernelGGL(k_fast_blocks, ga, dim3(256), 0, c->stream, fs->dev);
     if (hipGetLastError() != hipSuccess) return SDMD_EDEVICE;   // launch rejected (shape, resources)
     HIPV(hipEventRecord(c->ev1, c->stream));
     if (hipStreamSynchronize(c->stream) != hipSuccess) return SDMD_EDEVICE;
@@ -2830,8 +2848,9 @@ int sdmd_fast_download(sdmd_gpu_ctx *c, int s, sdmd_system_desc *out) {
 // energies of every system into out's three planes (kinetic, potential,
 // error flag; energy_planes_to_host reads them back)
 int sdmd_fast_energy_launch(sdmd_gpu_ctx *c, double *out) {
-    FastState *fs = c->fast;
-    FDISPATCH(fast_launch_energy, c->stream, fs->dev, c->nsys, out);
+    hipLaunchKernelGGL(k_fast_energy, dim3(c->nsys, c->echunks), dim3(64 * EWAVES), 0, c->stream, c->fast->dev,
+                       c->epart);
+    hipLaunchKernelGGL(k_energy_reduce, dim3(c->nsys), dim3(64), 0, c->stream, c->epart, c->echunks, out);
     return hipGetLastError() == hipSuccess ? SDMD_OK : SDMD_EDEVICE;
 }
 

@@ -912,40 +912,40 @@ __global__ __launch_bounds__(B) void k_run(Sys *systems, long long npops, long l
 enum { OP_PREDICT, OP_CREATE_TREE, OP_UPDATE_TREE, OP_ADVANCE, OP_DO_EVENT, OP_CELL_MOVE };
 
 // CalKinetE + CalPotenE (ToolFunctions.c:626-752) of every system at its
-// current time, one workgroup per system, one thread per atom i scanning the
-// 27 cells (periodic wrap with position shift) for partners j > i
-template <int B>
-__global__ __launch_bounds__(B) void k_energy(Sys *systems, double *out) {
+// current time: one wavefront per atom i, one lane per neighbour cell
+// (periodic wrap with position shift) walking its list for partners j > i.
+// Bound by the lists' dependent loads, so the atoms are spread over the GPU:
+// gridDim.y workgroups per system leave their sums in `part`
+// (k_energy_reduce).
+__global__ __launch_bounds__(64 * EWAVES) void k_energy(Sys *systems, double *part) {
     const Sys &S = systems[blockIdx.x];
-    const int N = S.N;
+    const int N = S.N, tid = threadIdx.x, lane = tid & 63;
     const double cut2 = S.cutoffr * S.cutoffr;
+    const int c = min(lane, 26);
     double ke = 0, pe = 0;
     int err = 0;
-    for (int i = 1 + threadIdx.x; i <= N; i += B) {
+    for (int i = 1 + blockIdx.y * EWAVES + (tid >> 6); i <= N; i += EWAVES * gridDim.y) {
         const double xi = G(S.x)[i], yi = G(S.y)[i], zi = G(S.z)[i];
         const double vi[3] = {G(S.vx)[i], G(S.vy)[i], G(S.vz)[i]};
-        ke += 0.5 * G(S.mass)[i] * (vi[0] * vi[0] + vi[1] * vi[1] + vi[2] * vi[2]);
-        const int ci[3] = {G(S.cx)[i], G(S.cy)[i], G(S.cz)[i]};
-        for (int n = 0; n < 27; n++) {
-            int cc[3] = {ci[0] + c_OX[n], ci[1] + c_OY[n], ci[2] + c_OZ[n]};
-            double sh[3] = {0, 0, 0};
-            for (int k = 0; k < 3; k++) {
-                if (cc[k] < 0) { cc[k] = S.cellnum[k + 1] - 1; sh[k] = -1 * S.box[k + 1]; }
-                else if (cc[k] >= S.cellnum[k + 1]) { cc[k] = 0; sh[k] = S.box[k + 1]; }
-            }
-            const int cell = cc[2] * S.cellnum[1] * S.cellnum[2] + cc[1] * S.cellnum[1] + cc[0] + 1;
-            int guard = 0;
-            for (int j = G(S.celllist)[N + cell]; j && ++guard <= N; j = G(S.celllist)[j]) {
-                if (j <= i) continue;
-                const double r1 = xi - (G(S.x)[j] + sh[0]), r2 = yi - (G(S.y)[j] + sh[1]), r3 = zi - (G(S.z)[j] + sh[2]);
-                const double rr = r1 * r1 + r2 * r2 + r3 * r3;
-                if (rr > cut2) continue;
-                const double vj[3] = {G(S.vx)[j], G(S.vy)[j], G(S.vz)[j]};
-                pe += pair_energy(S, i, j, r1, r2, r3, rr, vi, vj, &err);
-            }
+        if (lane == 0) ke += 0.5 * G(S.mass)[i] * (vi[0] * vi[0] + vi[1] * vi[1] + vi[2] * vi[2]);
+        int cc[3] = {G(S.cx)[i] + c_OX[c], G(S.cy)[i] + c_OY[c], G(S.cz)[i] + c_OZ[c]};
+        double sh[3] = {0, 0, 0};
+        for (int k = 0; k < 3; k++) {
+            if (cc[k] < 0) { cc[k] = S.cellnum[k + 1] - 1; sh[k] = -1 * S.box[k + 1]; }
+            else if (cc[k] >= S.cellnum[k + 1]) { cc[k] = 0; sh[k] = S.box[k + 1]; }
+        }
+        const int cell = cc[2] * S.cellnum[1] * S.cellnum[2] + cc[1] * S.cellnum[1] + cc[0] + 1;
+        int guard = 0;
+        for (int j = lane < 27 ? G(S.celllist)[N + cell] : 0; j && ++guard <= N; j = G(S.celllist)[j]) {
+            if (j <= i) continue;
+            const double r1 = xi - (G(S.x)[j] + sh[0]), r2 = yi - (G(S.y)[j] + sh[1]), r3 = zi - (G(S.z)[j] + sh[2]);
+            const double rr = r1 * r1 + r2 * r2 + r3 * r3;
+            if (rr > cut2) continue;
+            const double vj[3] = {G(S.vx)[j], G(S.vy)[j], G(S.vz)[j]};
+            pe += pair_energy(S, i, j, r1, r2, r3, rr, vi, vj, &err);
         }
     }
-    block_sum3<B>(ke, pe, err || S.error, out);
+    energy_partial(ke, pe, err || S.error, part);
 }
 
 template <int B>
@@ -1121,6 +1121,15 @@ extern "C" int sdmd_gpu_open(const sdmd_system_desc *const *systems, int32_t nsy
     }
     if (rc == SDMD_OK) rc = dev_upload(c, &c->dev_sys, (const Sys *)nullptr, (size_t)nsys);
     if (rc == SDMD_OK) rc = dev_upload(c, &c->dev_renew, (const int *)nullptr, 8);
+    if (rc == SDMD_OK) {
+        // energy workgroups per system: about 2048 in all (8 per CU), each
+        // with an atom per wavefront at least
+        int maxn = 1;
+        for (int s = 0; s < nsys; s++) maxn = systems[s]->natom > maxn ? systems[s]->natom : maxn;
+        const int want = (maxn + EWAVES - 1) / EWAVES, fit = (2048 + nsys - 1) / nsys;
+        c->echunks = want < fit ? want : fit;
+        rc = dev_upload(c, &c->epart, (const double *)nullptr, (size_t)3 * nsys * c->echunks);
+    }
     if (rc == SDMD_OK) rc = sync_to_device(c);
     if (rc == SDMD_OK) rc = hip_ok(hipStreamSynchronize(c->stream));
     if (rc == SDMD_OK && mode == SDMD_MODE_FAST) rc = sdmd_fast_open(c, opts);
@@ -1165,10 +1174,6 @@ static void launch_prepare(sdmd_gpu_ctx *c) {
 template <int B>
 static void launch_run(sdmd_gpu_ctx *c, long long n, long long budget, double t_end, double t_out) {
     hipLaunchKernelGGL((k_run<B>), dim3(c->nsys), dim3(B), 0, c->stream, c->dev_sys, n, budget, t_end, t_out);
-}
-template <int B>
-static void launch_energy(sdmd_gpu_ctx *c, double *planes) {
-    hipLaunchKernelGGL((k_energy<B>), dim3(c->nsys), dim3(B), 0, c->stream, c->dev_sys, planes);
 }
 template <int B>
 static void launch_op(sdmd_gpu_ctx *c, int s, int op, double dt, int a, int b) {
@@ -1435,7 +1440,8 @@ extern "C" int sdmd_gpu_last_kernel_ms(sdmd_gpu_ctx *c, double *ms) {
 // No allocation: the error plane is read back through a stack buffer.
 static int energy_launch(sdmd_gpu_ctx *c, double *planes) {
     if (c->mode == SDMD_MODE_FAST) return sdmd_fast_energy_launch(c, planes);
-    DISPATCH(launch_energy, c, planes);
+    hipLaunchKernelGGL(k_energy, dim3(c->nsys, c->echunks), dim3(64 * EWAVES), 0, c->stream, c->dev_sys, c->epart);
+    hipLaunchKernelGGL(k_energy_reduce, dim3(c->nsys), dim3(64), 0, c->stream, c->epart, c->echunks, planes);
     return hip_ok(hipGetLastError());
 }
 
