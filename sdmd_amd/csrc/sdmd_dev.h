@@ -25,7 +25,7 @@ constexpr int NT = SDMD_NTYPE;
 constexpr int CELL_CAP = 64;               // atoms gathered per neighbour cell
 constexpr int MAXC = 27 * CELL_CAP;        // candidates per predicted atom
 constexpr int MAXBOND = 16;                // BondTime's connect[16], TimePrediction.c:188
-constexpr int ROWCAP = 96;                 // connection-map row staged in LDS
+constexpr int LPOOL = 2048;                // step pool entries of the collision table in LDS
 
 enum { K_COLLISION, K_CONSTRAINT, K_HB, K_NEIGHBOR };
 enum { ERR_NONE = 0, ERR_TABLE = 1, ERR_HBMODEL = 2, ERR_SUBTYPE = 3, ERR_PHI_NAN = 4,
@@ -89,6 +89,15 @@ struct Sys {
     unsigned long long *prof;   // per-phase wall-clock ticks, or null
     int steps_sorted;           // every step list strictly increasing and non-zero
     int last_exec;              // the last pop executed its event
+    // plain engine: cell arrays (a cell's list back to front, CELL_CAP slots;
+    // a fuller cell is read through its list), pops each atom's position and
+    // event time lack of the run's log, and tables derived at upload
+    int *ccnt, *cmem, *cmap_con;
+    unsigned char *lag;
+    sdmd_pair *rpair;
+    int ltab, logk;             // step pool entries held in LDS (0: none); pops between sweeps
+    const int *gbase[48];       // gather table of a staged atom
+    int gstride[48];
 };
 
 // phases timed when a context is opened with profiling on

@@ -3,23 +3,28 @@
 // Plain FP64 path: bit-exact with the reference event loop.  One workgroup
 // owns one system and runs SingleThreadRun (SGThread.c:67-156) on the
 // device:
-//   pop          lane 0 reads the CBT root (AssignJob, SGThread.c:237-259)
-//   sweep        all lanes: x += v*dt, t -= dt for every atom
-//                (UpdateData/TimeForward, ToolFunctions.c:23-36)
-//   event        lane 0 (DoEvent, Events.c:25-114)
-//   predict      per renewed atom (Predict, SGThread.c:158-211):
-//                27 lanes walk the 27 neighbour-cell lists in the
-//                reference's order into LDS, every lane evaluates
-//                candidates (shell lookup + contact-time quadratic), and
-//                wave 0 runs an ordered min-with-first-index selection that
-//                reproduces JobAssign's strict '<' and CheckDuplication's
-//                inheritance (TimePrediction.c:1101-1158)
-//   tree         lane 0 updates the complete binary tree (CBT.c:56-83)
+//   event        wave 0 takes the CBT root (AssignJob, SGThread.c:237-259)
+//                and executes it (DoEvent, Events.c:25-114)
+//   sweep        x += v*dt, t -= dt of every atom (UpdateData/TimeForward,
+//                ToolFunctions.c:23-36): the event's atoms at once, the
+//                others when they are read, or every few pops (same steps,
+//                same bits)
+//   predict      the renewed atoms (Predict, SGThread.c:158-211), two side
+//                by side: the 27 neighbour cells' atoms in the reference's
+//                order into LDS, every lane evaluates a candidate (shell
+//                lookup + contact-time quadratic), and one wave runs an
+//                ordered min-with-first-index selection that reproduces
+//                JobAssign's strict '<' and CheckDuplication's inheritance
+//                (TimePrediction.c:1101-1158)
+//   tree         wave 0 updates the complete binary tree (CBT.c:56-83)
+// A pop is a chain of dependent loads, LDS exchanges and FP64 sequences on
+// one CU; what bounds it is the length of that chain.
 // Arithmetic follows the reference's operation order; the file is compiled
 // with -ffp-contract=off, so every product and sum rounds separately as on
 // the x86-64 reference build, and double sqrt/div are correctly rounded.
 
 
+#include <cstddef>
 #include <mutex>
 
 #include "sdmd_dev.h"
@@ -28,63 +33,146 @@
 namespace sdmd {
 
 // ---------------------------------------------------------------- shared state
-struct Atom {          // the atom being predicted, staged once per Predict
+constexpr int PWIN = 768;          // candidates of one pass (a predicted atom has 60 to 400)
+constexpr int LOGK = 32;           // pops between two sweeps at most
+constexpr int PCON = 16;           // constraint partners staged per predicted atom
+constexpr int PCONSTEP = 8;        // steps per staged constraint
+constexpr int NGATHER = 46;        // words of Atom loaded through Sys.gbase
+
+// The atom being predicted, staged once per Predict.  The first NGATHER
+// words are loaded by one wavefront, one word per lane, through the gather
+// table of Sys (filled by atom_gather_table in the same order).
+struct Atom {
     double x, y, z, vx, vy, vz;
     long long counter;
-    int i, cx, cy, cz, type, hbbond, hbnb, protein, aanum, nbstat, nrow;
-    signed char role;
-    int nbp[SDMD_NBSLOTS];
-    int nbnum;
-    // current event record (JobAssign target)
-    double t, pot;
+    double t, pot;                 // current event record (JobAssign target)
     long long pc;
-    int partner, evtype, sub;
+    int cx, cy, cz, type, hbbond, hbnb, protein, aanum, nbstat, nbnum;
+    int nbp[SDMD_NBSLOTS];
+    int partner, evtype, sub, hbitype;
+    int ro, ro1, bo, bo1, co, co1; // cmap_off, bond_off, con_off at i and i + 1
+    int leaf;
+    // not gathered
+    int i, role, nb, spanok, rowlo, over, ncand, cnt_eval, exclude, hbscan;
+    double zn;                     // its thermostat draw
+    double pot0;                   // the record before the prediction (a repeated selection restarts from it)
+    long long pc0;
+    int sub0, nbnum0;
+};
+static_assert(offsetof(Atom, leaf) == 4 * (NGATHER - 1), "gathered words come first");
+
+// one atom's candidates in program order, and its bonds, constraints and
+// connection row
+struct Cand {
+    int j[PWIN];
+    unsigned char cell[PWIN], fl[PWIN], hfl[PWIN];
+    signed char sub[PWIN];
+    double t[PWIN], pot[PWIN], ht[PWIN], hpot[PWIN];
+    int cellcnt[27], celloff[28];
+    double shift[27][3];           // periodic image of neighbour cell c (PBCShift)
+    double pcc[3];                 // cell-crossing time along each axis
+    int bj[MAXBOND];
+    double bt[MAXBOND], bjt[MAXBOND];
+    signed char bsub[MAXBOND];
+    unsigned char bfl[MAXBOND];
+    double con_dmin[PCON], con_dmax[PCON];
+    int con_step0[PCON], con_nstep[PCON];
+    double con_d[PCON][PCONSTEP], con_e[PCON][PCONSTEP];
+    // connection row by offset from its first column: bits 0-1 BOND and
+    // CONSTRAINT, bits 2-6 the constraint's slot + 1 (0: not staged)
+    unsigned char conn[128];
 };
 
 struct Smem {
-    Atom A;
-    int cand_j[MAXC];
-    double cand_t[MAXC];
-    double cand_pot[MAXC];
-    signed char cand_sub[MAXC];
-    unsigned char cand_fl[MAXC];
-    int cellbuf[27 * CELL_CAP];
-    int cellcnt[27];
-    int celloff[28];
-    int ncand, over;
-    int row_j[ROWCAP];
-    int row_b[ROWCAP];
-    int dyn_j[SDMD_DYNSLOTS];
-    int dyn_b[SDMD_DYNSLOTS];
-    // bond entries
-    int bj[MAXBOND];
-    double bt[MAXBOND], bpot[MAXBOND];
-    signed char bsub[MAXBOND];
-    unsigned char bfl[MAXBOND];
-    int nb;
+    Atom A[2];
+    Cand c[2];
     // loop scalars
-    int target, partner, stale, renew[4], err, hbscan;
-    int cnt_cand, cnt_eval;
+    int target, partner, stale, renew[4], err, root, flush;
     double dt;
     long long zpos;
+    // pops whose time step the atoms have not taken yet (see sweep)
+    int nlog;
+    double log[LOGK];
 };
 
-__device__ __forceinline__ int row_bits(const Smem &sm, const Sys &S, int j) {
-    const Atom &A = sm.A;
-    int bits = 0;
-    if (A.nrow <= ROWCAP) {
-        int lo = 0, hi = A.nrow - 1;
-        while (lo <= hi) {
-            int m = (lo + hi) >> 1;
-            int v = sm.row_j[m];
-            if (v == j) { bits = sm.row_b[m]; break; }
-            if (v < j) lo = m + 1; else hi = m - 1;
-        }
-        for (int k = 0; k < SDMD_DYNSLOTS; k++)
-            if (sm.dyn_j[k] == j) { bits |= sm.dyn_b[k]; break; }
-        return bits;
+// The collision table (RightPair resolved per type pair) and the step pool
+// of the tables, in LDS: a candidate's shell is found without leaving the CU
+struct PairTab {
+    double dmin[NT * NT], dmax[NT * NT];
+    int step0[NT * NT], nstep[NT * NT];
+    double d[LPOOL], e[LPOOL];
+};
+
+// ---------------------------------------------------------------- lazy sweep
+// UpdateData + TimeForward (ToolFunctions.c:23-36) advance every atom by
+// every pop's dt: x += v dt, t -= dt, each step rounded.  The result of an
+// atom depends only on its own steps, so they are taken when the atom is
+// next read, or by a sweep of all atoms every few pops: sm.log holds the dt
+// of the last sm.nlog pops and S.lag[i] how many of them atom i has taken.
+// The same operations in the same order give the same bits; the sweep's
+// memory traffic is paid once per LOGK pops (a sweep per pop cost 33 us of a
+// 73 us pop at 26 080 atoms).
+__device__ __forceinline__ int lag_of(const Sys &S, int n, int j) { return n ? (int)G(S.lag)[j] : 0; }
+
+__device__ __forceinline__ void steps_pos(const double *log, int l, int n, double &x, double &y, double &z, double vx,
+                                          double vy, double vz) {
+    for (; l < n; l++) {
+        const double dt = log[l];
+        x = x + vx * dt;
+        y = y + vy * dt;
+        z = z + vz * dt;
     }
-    return cmap_get(S, A.i, j);
+}
+__device__ __forceinline__ double evt_now(const Sys &S, const Smem &sm, int j) {
+    double t = G(S.evt)[j];
+    const int n = sm.nlog;
+    for (int l = lag_of(S, n, j); l < n; l++) t = t - sm.log[l];
+    return t;
+}
+__device__ __forceinline__ void pos_now(const Sys &S, const Smem &sm, int j, double *p) {
+    const int n = sm.nlog, l = lag_of(S, n, j);
+    double x = G(S.x)[j], y = G(S.y)[j], z = G(S.z)[j];
+    if (l < n) steps_pos(sm.log, l, n, x, y, z, G(S.vx)[j], G(S.vy)[j], G(S.vz)[j]);
+    p[0] = x; p[1] = y; p[2] = z;
+}
+
+struct PosLazy {      // PosStored with the steps an atom has not taken yet
+    const Sys &S;
+    const Smem &sm;
+    __device__ void pos(int j, double *p) const { pos_now(S, sm, j, p); }
+    __device__ int first(int cell) const { return G(S.celllist)[S.N + cell]; }
+    __device__ int next(int, int j) const { return G(S.celllist)[j]; }
+};
+
+// pair kinematics of the staged atom and j's current state
+__device__ __forceinline__ void calc_params_now(const Sys &S, const Smem &sm, const Atom &A, int j, Kin &k) {
+    double p[3];
+    pos_now(S, sm, j, p);
+    calc_params_at(S, A.x, A.y, A.z, A.vx, A.vy, A.vz, A.cx, A.cy, A.cz, j, p[0], p[1], p[2], G(S.vx)[j], G(S.vy)[j],
+                   G(S.vz)[j], k);
+}
+
+// UpdateData + TimeForward over all atoms: each takes the steps it still lacks
+template <int B>
+__device__ __forceinline__ void sweep(const Sys &S, Smem &sm) {
+    const int n = sm.nlog, N = S.N;
+    for (int i = threadIdx.x + 1; i <= N; i += B) {
+        int l = G(S.lag)[i];
+        const double vx = G(S.vx)[i], vy = G(S.vy)[i], vz = G(S.vz)[i];
+        double x = G(S.x)[i], y = G(S.y)[i], z = G(S.z)[i], t = G(S.evt)[i];
+        for (; l < n; l++) {
+            const double dt = sm.log[l];
+            x = x + vx * dt;
+            y = y + vy * dt;
+            z = z + vz * dt;
+            t = t - dt;
+        }
+        G(S.x)[i] = x; G(S.y)[i] = y; G(S.z)[i] = z; G(S.evt)[i] = t;
+        G(S.lag)[i] = 0;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) sm.nlog = 0;
+    __syncthreads();
 }
 
 __device__ __forceinline__ int in_nb_list(const Atom &A, int j, int *err) {   // FindElemInList(neighborPartner, j, -1, -1, 0)
@@ -101,32 +189,64 @@ __device__ __forceinline__ int in_nb_list(const Atom &A, int j, int *err) {   //
 }
 
 // ---------------------------------------------------------------- wave helpers
+// LDS written by some lanes of a wave, read next by others of the same wave:
+// the wave's LDS operations run in order, so only the compiler is held
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// lane of the wave's smallest t, the lowest one on equal t; every t is
+// positive or +inf (no NaN, no -0).  The order of such doubles is that of
+// their bits, so the high words are reduced first (six DPP minima) and the
+// low words only where several lanes share the smallest high word.
+__device__ __forceinline__ unsigned wave_umin(unsigned v) {
+    v = min(v, (unsigned)__builtin_amdgcn_update_dpp(-1, (int)v, 0x111, 0xF, 0xF, false));   // row_shr:1
+    v = min(v, (unsigned)__builtin_amdgcn_update_dpp(-1, (int)v, 0x112, 0xF, 0xF, false));   // row_shr:2
+    v = min(v, (unsigned)__builtin_amdgcn_update_dpp(-1, (int)v, 0x114, 0xF, 0xF, false));   // row_shr:4
+    v = min(v, (unsigned)__builtin_amdgcn_update_dpp(-1, (int)v, 0x118, 0xF, 0xF, false));   // row_shr:8
+    v = min(v, (unsigned)__builtin_amdgcn_update_dpp(-1, (int)v, 0x142, 0xA, 0xF, false));   // row_bcast:15
+    v = min(v, (unsigned)__builtin_amdgcn_update_dpp(-1, (int)v, 0x143, 0xC, 0xF, false));   // row_bcast:31
+    return (unsigned)__builtin_amdgcn_readlane((int)v, 63);
+}
+__device__ __forceinline__ int wave_first_min(double t) {
+    const unsigned long long b = (unsigned long long)__double_as_longlong(t);
+    const unsigned hi = (unsigned)(b >> 32), lo = (unsigned)b;
+    unsigned long long m = __ballot(hi == wave_umin(hi));
+    if (m & (m - 1)) {
+        const unsigned l = ((m >> (threadIdx.x & 63)) & 1) ? lo : 0xffffffffu;
+        m &= __ballot(l == wave_umin(l));
+    }
+    return __ffsll((long long)m) - 1;
+}
 
 // Ordered selection over n entries in program order, run by one full wave.
 // Entry k offers its computed time ct[k] (+inf when it would not reach
 // JobAssign or fails `t > 0`); flagged entries (bit 0) first offer j's
-// current event (CheckDuplication) when strictly earlier than the running
-// minimum.  Returns the winning entry and whether it was inherited.
-__device__ void wave_select(int n, const double *ct, const unsigned char *fl, const int *cj,
-                            const double *evt, double &m, int &win, int &inh) {
+// current event (CheckDuplication; jt(k) its time) when strictly earlier
+// than the running minimum.  Returns the winning entry and whether it was
+// inherited.
+template <class JT>
+__device__ __forceinline__ void wave_select(int n, const double *ct, const unsigned char *fl, const JT &jt, double &m,
+                                            int &win, int &inh) {
     const int lane = threadIdx.x & 63;
     for (int base = 0; base < n; base += 64) {
         const int k = base + lane;
         const bool in = k < n;
-        const bool dup = in && (fl[k] & 1);
-        unsigned long long mask = __ballot(dup);
+        const double tk = in ? ct[k] : __builtin_inf();
+        unsigned long long mask = __ballot(in && (fl[in ? k : 0] & 1));
         const int end = min(base + 64, n);
         int start = base;
         while (true) {
             const int d = mask ? base + __ffsll((long long)mask) - 1 : end;
-            double t = (in && k >= start && k < d) ? ct[k] : __builtin_inf();
-            int kk = k;
-            wave_argmin(t, kk);
-            if (t < m) { m = t; win = kk; inh = 0; }
+            const double t = (k >= start && k < d) ? tk : __builtin_inf();
+            const int src = wave_first_min(t);
+            const double tm = lane_get(t, src);
+            if (tm < m) { m = tm; win = base + src; inh = 0; }
             if (d >= end) break;
-            const double jt = evt[cj[d]];
-            if (m > jt) { m = jt; win = d; inh = 1; }
-            else if (ct[d] < m) { m = ct[d]; win = d; inh = 0; }
+            const double tj = jt(d), td = lane_get(tk, d - base);
+            if (m > tj) { m = tj; win = d; inh = 1; }
+            else if (td < m) { m = td; win = d; inh = 0; }
             start = d + 1;
             mask &= mask - 1;
         }
@@ -140,25 +260,29 @@ __device__ __forceinline__ void take_computed(Atom &A, const Sys &S, double t, d
     else A.partner = INVALID;
 }
 
-__device__ __forceinline__ void take_inherited(Atom &A, const Sys &S, int j, int type) {
-    A.partner = j; A.pot = G(S.evpot)[j]; A.sub = G(S.evsub)[j]; A.t = G(S.evt)[j]; A.evtype = type; A.pc = G(S.evc)[j];
+__device__ __forceinline__ void take_inherited(Atom &A, const Sys &S, const Smem &sm, int j, int type) {
+    A.partner = j; A.pot = G(S.evpot)[j]; A.sub = G(S.evsub)[j]; A.t = evt_now(S, sm, j); A.evtype = type;
+    A.pc = G(S.evc)[j];
 }
 
-__device__ __forceinline__ bool dupable(const Sys &S, int i, long long ci, int j, int type) {
-    return G(S.evp)[j] == i && G(S.evtype)[j] == type && G(S.evpc)[j] == ci;
+// CheckDuplication's condition; A.exclude is an atom whose record is being
+// written by another wavefront (it held none when A's prediction began)
+__device__ __forceinline__ bool dupable(const Sys &S, const Atom &A, int j, int type) {
+    return j != A.exclude && G(S.evp)[j] == A.i && G(S.evtype)[j] == type && G(S.evpc)[j] == A.counter;
 }
 
 // ---------------------------------------------------------------- candidate evaluation
 // one BondTime entry, TimePrediction.c:219-293
-__device__ void eval_bond(const Sys &S, Smem &sm, int q, int *err) {
-    const Atom &A = sm.A;
-    const int e = G(S.bond_off)[A.i] + q;
+__device__ __forceinline__ void eval_bond(const Sys &S, const Smem &sm, const Atom &A, Cand &C, int q) {
+    const int e = A.bo + q;
     const int j = G(S.bond_j)[e];
-    sm.bj[q] = j;
-    sm.bfl[q] = dupable(S, A.i, A.counter, j, SDMD_BOND) ? 1 : 0;
     const double lo = G(S.bond_dmin)[e], hi = G(S.bond_dmax)[e];
+    C.bj[q] = j;
+    const bool dup = dupable(S, A, j, SDMD_BOND);
+    C.bfl[q] = dup ? 1 : 0;
+    C.bjt[q] = dup ? evt_now(S, sm, j) : 0;
     Kin k;
-    calc_params(S, A.x, A.y, A.z, A.vx, A.vy, A.vz, A.cx, A.cy, A.cz, j, k);
+    calc_params_now(S, sm, A, j, k);
     double t;
     int sub;
     if (k.rr - hi > ZERO && k.b >= 0) {
@@ -175,99 +299,166 @@ __device__ void eval_bond(const Sys &S, Smem &sm, int q, int *err) {
         t = calc_time(k, s, d2);
         if (t < 0) t = INFINIT;
     }
-    sm.bt[q] = (t > 0) ? t : __builtin_inf();
-    sm.bpot[q] = 0;
-    sm.bsub[q] = (signed char)sub;
+    C.bt[q] = (t > 0) ? t : __builtin_inf();
+    C.bsub[q] = (signed char)sub;
 }
 
-// one CollisionTime candidate, TimePrediction.c:79-179
-__device__ void eval_collision(const Sys &S, Smem &sm, int kidx, double calib, int *err) {
-    const Atom &A = sm.A;
-    const int j = sm.cand_j[kidx];
-    double tout = __builtin_inf();
-    double pot = 0;
+// FindPair's shell search (shell_lookup) for a collision or constraint pair
+// on radii d(k) and energies e(k): strictly increasing, non-zero, nstep <= 16
+template <class D, class E>
+__device__ __forceinline__ int shell_fast(double dmin, double dmax, int nstep, const D &d, const E &e, double direction,
+                                          double d2, double &flo, double &fhi, double &lopot, double &hipot, int *err) {
+    const double dir = (direction < 0) ? 1 : -1;
+    const double tol = dir * ZERO;
+    flo = fhi = INFINIT;
+    lopot = hipot = 0;
+    if (dmin == 0) { *err = ERR_TABLE; return -1; }
+    if (d2 < dmin - ZERO) return -1;
+    int ks = 0;
+#pragma unroll
+    for (int k0 = 0; k0 < 16; k0 += 4) {
+        if (k0 < nstep) {
+            double r[4];
+#pragma unroll
+            for (int u = 0; u < 4; u++) r[u] = d(k0 + u < nstep ? k0 + u : nstep - 1);
+#pragma unroll
+            for (int u = 0; u < 4; u++)
+                if (k0 + u < nstep) ks += (d2 >= r[u] + tol) ? 1 : 0;
+        }
+    }
+    flo = dmin;
+    if (ks > 0) {
+        flo = d(ks - 1);
+        lopot = e(ks - 1);
+    }
+    if (ks < nstep) {
+        fhi = d(ks);
+        hipot = -1 * e(ks);
+        return ks == 0 ? 0 : -1;
+    }
+    if (dmax > 0) {
+        if (d2 < dmax + ZERO) {
+            fhi = dmax; hipot = 0;
+            return (nstep == 0 && dir == 1) ? 0 : 1;
+        }
+        flo = INFINIT; fhi = INFINIT; lopot = 0; hipot = 0;
+        return -1;
+    }
+    fhi = INFINIT; hipot = INFINIT;
+    return 1;
+}
+
+// candidate k of the staged atom: CollisionTime (TimePrediction.c:79-179)
+// and, for a free H-bond atom, HBTime's scan (TimePrediction.c:414-478).
+// Every field of j that either may need is loaded at once (one round trip);
+// shells come from LDS.
+template <bool TAB>
+__device__ __forceinline__ void eval_candidate(const Sys &S, const Smem &sm, const PairTab *T, const Atom &A, Cand &C,
+                                               int kidx, double calib, int *err) {
+    const int j = C.j[kidx], i = A.i;
+    double tout = __builtin_inf(), pot = 0, ht = __builtin_inf(), hpot = 0;
     int sub = SDMD_INVALID_INTER;
-    unsigned char fl = 0;
-    if (j != A.i) {
-        if (dupable(S, A.i, A.counter, j, SDMD_COLI)) fl = 1;
-        const int bits = row_bits(sm, S, j);
-        if (!((bits & SDMD_BOND_CONNECT) || A.hbbond == j || in_nb_list(A, j, err))) {
-            Kin k;
-            calc_params(S, A.x, A.y, A.z, A.vx, A.vy, A.vz, A.cx, A.cy, A.cz, j, k);
-            if (k.rr <= calib) {
-                FP f;
-                int cs;
-                const int con = bits & SDMD_CONSTRAINT_CONNECT;
-                bool skip = false;
-                if (con) {
-                    cs = find_pair(S, A.i, j, K_CONSTRAINT, k.b, k.rr, f, 0, 0, err);
+    unsigned char fl = 0, hfl = 0;
+    if (j != i) {
+        const int n = sm.nlog;
+        const int l = lag_of(S, n, j);
+        const int evp = G(S.evp)[j], evtype = G(S.evtype)[j], tj = G(S.type)[j];
+        const long long evpc = G(S.evpc)[j];
+        double x = G(S.x)[j], y = G(S.y)[j], z = G(S.z)[j];
+        const double vx = G(S.vx)[j], vy = G(S.vy)[j], vz = G(S.vz)[j];
+        const bool hb = A.role == 'A' || A.role == 'D' || A.role == 'S';
+        int rj = 0, hj = 0, aj = 0, pj = 0;
+        if (hb) { rj = G(S.role)[j]; hj = G(S.hbbond)[j]; aj = G(S.aanum)[j]; pj = G(S.protein)[j]; }
+        steps_pos(sm.log, l, n, x, y, z, vx, vy, vz);
+        const bool mine = j != A.exclude && evp == i && evpc == A.counter;
+        if (mine && evtype == SDMD_COLI) fl = 1;
+        // PBCShift + CalculateParameters
+        const double *sh = C.shift[C.cell[kidx]];
+        Kin k;
+        k.r1 = A.x - (x + sh[0]);
+        k.r2 = A.y - (y + sh[1]);
+        k.r3 = A.z - (z + sh[2]);
+        const double v1 = A.vx - vx, v2 = A.vy - vy, v3 = A.vz - vz;
+        k.rr = k.r1 * k.r1 + k.r2 * k.r2 + k.r3 * k.r3;
+        k.b = k.r1 * v1 + k.r2 * v2 + k.r3 * v3;
+        k.v2 = v1 * v1 + v2 * v2 + v3 * v3;
+        int cb = 0;
+        if (A.spanok) {
+            const unsigned off = (unsigned)(j - A.rowlo);
+            if (off < 128u) cb = C.conn[off];
+        } else {
+            cb = cmap_get(S, i, j) & (SDMD_BOND_CONNECT | SDMD_CONSTRAINT_CONNECT);
+        }
+        if (!((cb & SDMD_BOND_CONNECT) || A.hbbond == j || in_nb_list(A, j, err)) && k.rr <= calib) {
+            double lo, hi, lopot, hipot;
+            int cs;
+            const int con = cb & SDMD_CONSTRAINT_CONNECT, slot = (cb >> 2) - 1;
+            bool skip = false;
+            if (con && slot >= 0 && S.steps_sorted) {
+                const double *d = C.con_d[slot], *e = C.con_e[slot];
+                cs = shell_fast(C.con_dmin[slot], C.con_dmax[slot], C.con_nstep[slot], [&](int q) { return d[q]; },
+                                [&](int q) { return e[q]; }, k.b, k.rr, lo, hi, lopot, hipot, err);
+            } else {
+                const int t12 = A.type * NT + tj;
+                if (TAB && !con && S.ltab) {
+                    const double *d = T->d + T->step0[t12], *e = T->e + T->step0[t12];
+                    cs = shell_fast(T->dmin[t12], T->dmax[t12], T->nstep[t12], [&](int q) { return d[q]; },
+                                    [&](int q) { return e[q]; }, k.b, k.rr, lo, hi, lopot, hipot, err);
                 } else {
-                    cs = find_pair(S, A.i, j, K_COLLISION, k.b, k.rr, f, 0, 0, err);
-                    if (f.lopot == 0 && f.hipot == 0) skip = true;
+                    FP f;
+                    cs = find_pair(S, i, j, con ? K_CONSTRAINT : K_COLLISION, k.b, k.rr, f, 0, 0, err);
+                    lo = f.lo; hi = f.hi; lopot = f.lopot; hipot = f.hipot;
+                }
+                if (!con && lopot == 0 && hipot == 0) skip = true;
+            }
+            if (!skip) {
+                int s;
+                double d2;
+                if (k.b < 0 && calc_disc(k, lo) > 0) {
+                    s = -1; d2 = lo; pot = lopot;
+                    sub = (cs == 0) ? SDMD_CORECOLLI : SDMD_TBDCAPTR;
+                } else {
+                    s = 1; d2 = hi; pot = hipot;
+                    if (con) sub = (cs == 1) ? SDMD_WELLBOUNC : SDMD_TBDESCAP;
+                    else if (cs == 1) skip = true;
+                    else sub = SDMD_TBDESCAP;
                 }
                 if (!skip) {
-                    int s;
-                    double d2;
-                    if (k.b < 0 && calc_disc(k, f.lo) > 0) {
-                        s = -1; d2 = f.lo; pot = f.lopot;
-                        sub = (cs == 0) ? SDMD_CORECOLLI : SDMD_TBDCAPTR;
-                    } else {
-                        s = 1; d2 = f.hi; pot = f.hipot;
-                        if (con) sub = (cs == 1) ? SDMD_WELLBOUNC : SDMD_TBDESCAP;
-                        else if (cs == 1) skip = true;
-                        else sub = SDMD_TBDESCAP;
-                    }
-                    if (!skip) {
-                        const double t = calc_time(k, s, d2);
-                        tout = (t > 0) ? t : __builtin_inf();
-                        fl |= 2;   // reached the quadratic
+                    const double t = calc_time(k, s, d2);
+                    tout = (t > 0) ? t : __builtin_inf();
+                    fl |= 2;   // reached the quadratic
+                }
+            }
+        }
+        if (hb) {
+            const int ri = A.role;
+            const bool pairok = (ri == 'A' && rj == 'D') || (ri == 'D' && rj == 'A') || (ri == 'S' && tj == 2) ||
+                                (rj == 'S' && A.type == 2) || (ri == 'S' && rj == 'S');
+            int sep = A.aanum - aj;
+            if (sep < 0) sep = -sep;
+            if (pairok && hj == 0 && ((A.protein == pj && sep >= 4) || A.protein != pj)) {
+                hfl = 4 | ((mine && evtype == SDMD_HB) ? 1 : 0);    // bit 2: an H-bond candidate
+                if (A.hbscan && k.rr <= calib && check_pair_match(S, i, j, err) >= 0) {
+                    FP f;
+                    const int cs = find_pair(S, i, j, K_HB, k.b, k.rr, f, 0, 0, err);
+                    if (k.b < 0 && cs == 1 && calc_disc(k, f.lo) > 0) {
+                        hpot = f.lopot;
+                        double t = calc_time(k, -1, f.lo);
+                        if (t < 0) t = INFINIT;
+                        ht = (t > 0) ? t : __builtin_inf();
+                        hfl |= 2;
                     }
                 }
             }
         }
     }
-    sm.cand_t[kidx] = tout;
-    sm.cand_pot[kidx] = pot;
-    sm.cand_sub[kidx] = (signed char)sub;
-    sm.cand_fl[kidx] = fl;
-}
-
-
-// one free-atom HBTime candidate, TimePrediction.c:414-478
-__device__ void eval_hb(const Sys &S, Smem &sm, int kidx, double calib, int *err) {
-    const Atom &A = sm.A;
-    const int j = sm.cand_j[kidx];
-    double tout = __builtin_inf();
-    double pot = 0;
-    unsigned char fl = 0;
-    const signed char ri = A.role, rj = G(S.role)[j];
-    const bool pairok = (ri == 'A' && rj == 'D') || (ri == 'D' && rj == 'A') ||
-                        (ri == 'S' && G(S.type)[j] == 2) || (rj == 'S' && A.type == 2) || (ri == 'S' && rj == 'S');
-    int sep = A.aanum - G(S.aanum)[j];
-    if (sep < 0) sep = -sep;
-    const int pj = G(S.protein)[j];
-    if (j != A.i && pairok && G(S.hbbond)[j] == 0 && ((A.protein == pj && sep >= 4) || A.protein != pj)) {
-        if (dupable(S, A.i, A.counter, j, SDMD_HB)) fl = 1;
-        Kin k;
-        calc_params(S, A.x, A.y, A.z, A.vx, A.vy, A.vz, A.cx, A.cy, A.cz, j, k);
-        if (k.rr <= calib && check_pair_match(S, A.i, j, err) >= 0) {
-            FP f;
-            int cs = find_pair(S, A.i, j, K_HB, k.b, k.rr, f, 0, 0, err);
-            if (k.b < 0 && cs == 1 && calc_disc(k, f.lo) > 0) {
-                pot = f.lopot;
-                double t = calc_time(k, -1, f.lo);
-                if (t < 0) t = INFINIT;
-                tout = (t > 0) ? t : __builtin_inf();
-                fl |= 2;
-            }
-        }
-    } else {
-        fl = 4;   // not an HB candidate: skipped before CheckDuplication
-    }
-    sm.cand_t[kidx] = tout;
-    sm.cand_pot[kidx] = pot;
-    sm.cand_sub[kidx] = (signed char)SDMD_TBDHBFORM;
-    sm.cand_fl[kidx] = fl & 3;
+    C.t[kidx] = tout;
+    C.pot[kidx] = pot;
+    C.sub[kidx] = (signed char)sub;
+    C.fl[kidx] = fl;
+    C.ht[kidx] = ht;
+    C.hpot[kidx] = hpot;
+    C.hfl[kidx] = hfl;
 }
 
 // ---------------------------------------------------------------- lane-0 pieces
@@ -280,35 +471,21 @@ __device__ double next_normal(Sys &S, Smem &sm) {
     return G(S.zn)[sm.zpos++];
 }
 
-// PBCandCrossCellTime, TimePrediction.c:598-632
-__device__ void pcc_time(const Sys &S, Atom &A) {
-    double t_ev = INFINIT;
-    const double pos[3] = {A.x, A.y, A.z}, v[3] = {A.vx, A.vy, A.vz};
-    const int ci[3] = {A.cx, A.cy, A.cz};
-    double lo[3], hi[3];
-    for (int n = 0; n < 3; n++) {
-        lo[n] = ci[n] * S.cellsize[n + 1];
-        hi[n] = (ci[n] + 1) * S.cellsize[n + 1];
-    }
-    for (int n = 0; n < 3; n++) {
-        double t;
-        if (v[n] > 0) {
-            t = (hi[n] - pos[n] + ZERO) / v[n];
-            if (t_ev > t && t > 0) t_ev = t;
-        } else if (v[n] < 0) {
-            t = (lo[n] - pos[n] - ZERO) / v[n];
-            if (t_ev > t && t > 0) t_ev = t;
-        }
-    }
-    job_assign_atom(A, S, t_ev, 0, SDMD_INVALID_INTER, SDMD_PCC, 0);
+// PBCandCrossCellTime along axis n, TimePrediction.c:598-632 (INFINIT: none)
+__device__ __forceinline__ double pcc_axis(const Sys &S, double pos, double v, int ci, int n) {
+    double t = -1;
+    const double lo = ci * S.cellsize[n + 1], hi = (ci + 1) * S.cellsize[n + 1];
+    if (v > 0) t = (hi - pos + ZERO) / v;
+    else if (v < 0) t = (lo - pos - ZERO) / v;
+    return (t > 0 && INFINIT > t) ? t : INFINIT;
 }
 
 // HBTime for a bonded HB atom, TimePrediction.c:330-383
-__device__ void hb_time_bonded(const Sys &S, Atom &A, int *err) {
+__device__ void hb_time_bonded(const Sys &S, const Smem &sm, Atom &A, int *err) {
     const int j = A.hbbond;
-    if (dupable(S, A.i, A.counter, j, SDMD_HB) && A.t > G(S.evt)[j]) { take_inherited(A, S, j, SDMD_HB); return; }
+    if (dupable(S, A, j, SDMD_HB) && A.t > evt_now(S, sm, j)) { take_inherited(A, S, sm, j, SDMD_HB); return; }
     Kin k;
-    calc_params(S, A.x, A.y, A.z, A.vx, A.vy, A.vz, A.cx, A.cy, A.cz, j, k);
+    calc_params_now(S, sm, A, j, k);
     FP f;
     int cs = find_pair(S, A.i, j, K_HB, k.b, k.rr, f, 0, 0, err);
     int s, sub;
@@ -326,19 +503,19 @@ __device__ void hb_time_bonded(const Sys &S, Atom &A, int *err) {
 }
 
 // HBNeighborTime, TimePrediction.c:486-579
-__device__ void hb_neighbor_time(const Sys &S, Atom &A, int *err) {
+__device__ void hb_neighbor_time(const Sys &S, const Smem &sm, Atom &A, int *err) {
     int flag = 0;
     for (int n = 1; n <= A.nbstat; n++) {
         const int j = A.nbp[n];
         if (flag == 0) A.nbnum = n;
-        if (dupable(S, A.i, A.counter, j, SDMD_HBNE) && A.t > G(S.evt)[j]) {
-            take_inherited(A, S, j, SDMD_HBNE);
+        if (dupable(S, A, j, SDMD_HBNE) && A.t > evt_now(S, sm, j)) {
+            take_inherited(A, S, sm, j, SDMD_HBNE);
             A.nbnum = n;
             flag = 1;
             continue;
         }
         Kin k;
-        calc_params(S, A.x, A.y, A.z, A.vx, A.vy, A.vz, A.cx, A.cy, A.cz, j, k);
+        calc_params_now(S, sm, A, j, k);
         int host, nb, partner;
         const bool ads = (A.role == 'A' || A.role == 'D' || A.role == 'S');
         if (ads && A.hbbond && G(S.hbnb)[A.hbbond] == j) { host = A.i; nb = j; partner = A.hbbond; }
@@ -364,242 +541,393 @@ __device__ void hb_neighbor_time(const Sys &S, Atom &A, int *err) {
     }
 }
 
-// ---------------------------------------------------------------- Predict (one atom)
-__device__ void stage_atom(Sys &S, Smem &sm, int i) {
-    Atom &A = sm.A;
-    A.i = i;
-    A.x = G(S.x)[i]; A.y = G(S.y)[i]; A.z = G(S.z)[i];
-    A.vx = G(S.vx)[i]; A.vy = G(S.vy)[i]; A.vz = G(S.vz)[i];
-    A.counter = G(S.evc)[i];
-    A.cx = G(S.cx)[i]; A.cy = G(S.cy)[i]; A.cz = G(S.cz)[i];
-    A.type = G(S.type)[i]; A.hbbond = G(S.hbbond)[i]; A.hbnb = G(S.hbnb)[i];
-    A.protein = G(S.protein)[i]; A.aanum = G(S.aanum)[i]; A.role = G(S.role)[i];
-    A.nbstat = G(S.nbstat)[i]; A.nbnum = G(S.nbnum)[i];
-    for (int k = 0; k < SDMD_NBSLOTS; k++) A.nbp[k] = G(S.nbp)[(size_t)i * SDMD_NBSLOTS + k];
-    A.t = G(S.evt)[i]; A.pot = G(S.evpot)[i]; A.pc = G(S.evpc)[i];
-    A.partner = G(S.evp)[i]; A.evtype = G(S.evtype)[i]; A.sub = G(S.evsub)[i];
-    const int o = G(S.cmap_off)[i], n = G(S.cmap_off)[i + 1] - o;
-    A.nrow = n;
-    sm.nb = G(S.bond_off)[i + 1] - G(S.bond_off)[i];
+// ---------------------------------------------------------------- Predict
+// Stage atom i (one wave): the gathered words, one per lane.
+__device__ __forceinline__ void stage_atom(const Sys &S, Atom &A, int i, int exclude) {
+    const int lane = threadIdx.x & 63;
+    if (lane < NGATHER) ((int *)&A)[lane] = G(S.gbase[lane])[(size_t)i * S.gstride[lane]];
+    if (lane == NGATHER) {
+        const int role = G(S.role)[i];
+        A.i = i;
+        A.role = role;
+        A.exclude = exclude;
+        A.cnt_eval = 0;
+    }
 }
 
-__device__ void unstage_atom(Sys &S, const Atom &A) {
+// Second level (the waves of a team; rank r of nw): bonds, connection row,
+// constraint shells and cell-crossing times on one wave each where the team
+// has several, and the candidates of the 27 cells (DMD.c:117-121 order, each
+// in list order: the cell arrays hold a list back to front) on all of them.
+template <bool CELLS>
+__device__ __forceinline__ void stage_neighbours(const Sys &S, const Smem &sm, Atom &A, Cand &C, int r, int nw, int *err) {
+    const int lane = threadIdx.x & 63;
+    // occupancy of the 27 cells, by every wave for itself
+    const int cl = min(lane, 26);
+    int n1 = A.cx + c_OX[cl], n2 = A.cy + c_OY[cl], n3 = A.cz + c_OZ[cl];
+    if (n1 < 0) n1 = S.cellnum[1] - 1; else if (n1 >= S.cellnum[1]) n1 = 0;
+    if (n2 < 0) n2 = S.cellnum[2] - 1; else if (n2 >= S.cellnum[2]) n2 = 0;
+    if (n3 < 0) n3 = S.cellnum[3] - 1; else if (n3 >= S.cellnum[3]) n3 = 0;
+    const int cell = n3 * S.cellnum[1] * S.cellnum[2] + n2 * S.cellnum[1] + n1 + 1;
+    int cnt = G(S.ccnt)[cell];
+    if (lane >= 27) cnt = 0;
+    if (r == 0) {
+        // connection row and constraints
+        const int nrow = A.ro1 - A.ro, ncon = A.co1 - A.co;
+        if (lane < 32) ((int *)C.conn)[lane] = 0;
+        int rj = 0, rb = 0, rc = 0;
+        if (lane < nrow) { rj = G(S.cmap_j)[A.ro + lane]; rb = G(S.cmap_bits)[A.ro + lane]; rc = G(S.cmap_con)[A.ro + lane]; }
+        double dmin = 0, dmax = 0;
+        int step0 = 0, nstep = 0;
+        if (lane < ncon && lane < PCON) {
+            const sdmd_pair *p = &S.con[A.co + lane];
+            dmin = G(p)->dmin; dmax = G(p)->dmax; step0 = G(p)->step0; nstep = G(p)->nstep;
+            C.con_dmin[lane] = dmin; C.con_dmax[lane] = dmax; C.con_nstep[lane] = nstep;
+        }
+        const int lo = lane_get(rj, 0), hi = nrow > 0 ? lane_get(rj, min(nrow, 64) - 1) : lo;
+        const bool spanok = nrow <= 64 && hi - lo < 128;
+        const int slot = rc - A.co;                       // rc < 0: no constraint
+        const int ns = __shfl(nstep, slot & 15, 64);
+        if (lane < nrow && spanok) {
+            const bool staged = rc >= 0 && slot >= 0 && slot < PCON && ns <= PCONSTEP;
+            C.conn[rj - lo] = (unsigned char)((rb & (SDMD_BOND_CONNECT | SDMD_CONSTRAINT_CONNECT)) | (staged ? (slot + 1) << 2 : 0));
+        }
+        if (lane == 0) { A.spanok = spanok; A.rowlo = lo; }
+#pragma unroll
+        for (int u = 0; u < PCON * PCONSTEP / 64; u++) {
+            const int q = (lane + 64 * u) / PCONSTEP, k = lane % PCONSTEP;
+            const int s0 = __shfl(step0, q, 64), sn = __shfl(nstep, q, 64);
+            if (q < ncon && k < sn) { C.con_d[q][k] = G(S.sd)[s0 + k]; C.con_e[q][k] = G(S.se)[s0 + k]; }
+        }
+    }
+    if (r == nw - 1) {
+        const int nb = A.bo1 - A.bo;
+        if (lane < min(nb, MAXBOND)) eval_bond(S, sm, A, C, lane);
+        else if (lane >= 32 && lane < 35) {
+            const int n = lane - 32;
+            C.pcc[n] = pcc_axis(S, n == 0 ? A.x : n == 1 ? A.y : A.z, n == 0 ? A.vx : n == 1 ? A.vy : A.vz,
+                                n == 0 ? A.cx : n == 1 ? A.cy : A.cz, n);
+        }
+        if (lane == 0) A.nb = nb;
+        if (nb > MAXBOND) *err = ERR_CELLCAP;
+    }
+    const int incl = scan32_incl(cnt);
+    const int off = incl - cnt;
+    const bool over = __ballot(cnt > CELL_CAP) != 0, broken = __ballot(cnt > S.N) != 0;
+    const int ntot = lane_get(incl, 26);
+    if (r == 0) {
+        if (lane < 27) {
+            C.cellcnt[lane] = cnt;
+            C.celloff[lane] = off;
+            // PBCShift, ToolFunctions.c:801-817, for the cell's atoms
+            const int ci[3] = {A.cx, A.cy, A.cz}, cj[3] = {n1, n2, n3};
+            for (int n = 0; n < 3; n++) {
+                double s = 0;
+                if (ci[n] != cj[n]) {
+                    if (ci[n] == 0 && cj[n] == S.cellnum[n + 1] - 1) s = -1 * S.box[n + 1];
+                    else if (ci[n] == S.cellnum[n + 1] - 1 && cj[n] == 0) s = S.box[n + 1];
+                }
+                C.shift[lane][n] = s;
+            }
+            if (broken) *err = ERR_LINKLIST;
+        }
+        if (lane == 27) C.celloff[27] = incl;             // lanes 27.. repeat the total
+        if (lane == 0) {
+            A.over = over && !broken;
+            A.ncand = broken ? 0 : ntot;             // a broken list: no scan (the error ends the run)
+        }
+    }
+    if (CELLS && !over && ntot <= PWIN) {
+        // four cells at a time, 16 atoms of each per load
+        int v[7];
+#pragma unroll
+        for (int u = 0; u < 7; u++) {
+            const int c = (u * nw + r) * 4 + (lane >> 4), q = lane & 15;
+            const int cc = __shfl(cnt, min(c, 31), 64), id = __shfl(cell, min(c, 26), 64);
+            v[u] = (c < 27 && q < cc) ? G(S.cmem)[(size_t)id * CELL_CAP + q] : 0;
+        }
+#pragma unroll
+        for (int u = 0; u < 7; u++) {
+            const int c = (u * nw + r) * 4 + (lane >> 4);
+            const int cc = __shfl(cnt, min(c, 31), 64), o = __shfl(off, min(c, 31), 64), id = __shfl(cell, min(c, 26), 64);
+            if (c < 27) {
+                int q = lane & 15;
+                if (q < cc) { C.j[o + cc - 1 - q] = v[u]; C.cell[o + cc - 1 - q] = (unsigned char)c; }
+                for (q += 16; q < cc; q += 16) {
+                    C.j[o + cc - 1 - q] = G(S.cmem)[(size_t)id * CELL_CAP + q];
+                    C.cell[o + cc - 1 - q] = (unsigned char)c;
+                }
+            }
+        }
+    }
+}
+
+// The predicted atom's record from the evaluated entries, in the reference's
+// order (one wave): bonds and collisions ...
+__device__ __forceinline__ void select_bonds(const Sys &S, const Smem &sm, Atom &A, Cand &C) {
+    double m = A.t;
+    int win = -1, inh = 0;
+    wave_select(min(A.nb, MAXBOND), C.bt, C.bfl, [&](int d) { return C.bjt[d]; }, m, win, inh);
+    if ((threadIdx.x & 63) == 0 && win >= 0) {
+        if (inh) take_inherited(A, S, sm, C.bj[win], SDMD_BOND);
+        else take_computed(A, S, C.bt[win], 0, C.bsub[win], SDMD_BOND, C.bj[win]);
+    }
+}
+__device__ __forceinline__ void select_collisions(const Sys &S, const Smem &sm, Atom &A, Cand &C, int n) {
+    double m = A.t;
+    int win = -1, inh = 0;
+    wave_select(n, C.t, C.fl, [&](int d) { return evt_now(S, sm, C.j[d]); }, m, win, inh);
+    if ((threadIdx.x & 63) == 0 && win >= 0) {
+        if (inh) take_inherited(A, S, sm, C.j[win], SDMD_COLI);
+        else take_computed(A, S, C.t[win], C.pot[win], C.sub[win], SDMD_COLI, C.j[win]);
+    }
+}
+// ... cell crossing, thermostat, the bonded H-bond partner (lane 0) ...
+__device__ __forceinline__ void assign_onebody(const Sys &S, const Smem &sm, Atom &A, const Cand &C, int *err) {
+    double t_ev = INFINIT;
+    for (int n = 0; n < 3; n++)
+        if (t_ev > C.pcc[n]) t_ev = C.pcc[n];
+    job_assign_atom(A, S, t_ev, 0, SDMD_INVALID_INTER, SDMD_PCC, 0);
+    if (S.thermostat) {
+        const double z = A.zn;
+        job_assign_atom(A, S, S.thermoF * ((z < 0) ? (-z) : (z)), 0, SDMD_INVALID_INTER, SDMD_THER, 0);
+    }
+    // HBTime head, TimePrediction.c:309-330
+    if (A.hbitype != SDMD_HBSKIP && A.hbbond > 0) hb_time_bonded(S, sm, A, err);
+}
+// ... the free H-bond scan ...
+__device__ __forceinline__ void select_hbonds(const Sys &S, const Smem &sm, Atom &A, Cand &C, int n) {
+    double m = A.t;
+    int win = -1, inh = 0;
+    wave_select(n, C.ht, C.hfl, [&](int d) { return evt_now(S, sm, C.j[d]); }, m, win, inh);
+    if ((threadIdx.x & 63) == 0 && win >= 0) {
+        if (inh) take_inherited(A, S, sm, C.j[win], SDMD_HB);
+        else take_computed(A, S, C.ht[win], C.hpot[win], SDMD_TBDHBFORM, SDMD_HB, C.j[win]);
+    }
+}
+// ... H-bond neighbours and the wall, and the record stored (lane 0)
+__device__ __forceinline__ void assign_tail(Sys &S, const Smem &sm, Atom &A, int *err) {
+    hb_neighbor_time(S, sm, A, err);
+    if (S.wall) {
+        WallEv w;
+        if (wall_time(S, A.y, A.z, A.vy, A.vz, A.type, w, err)) job_assign_atom(A, S, w.t, w.pot, w.sub, SDMD_WALL, 0);
+    }
     const int i = A.i;
     G(S.evt)[i] = A.t; G(S.evpot)[i] = A.pot; G(S.evpc)[i] = A.pc;
     G(S.evp)[i] = A.partner; G(S.evtype)[i] = A.evtype; G(S.evsub)[i] = A.sub;
     G(S.nbnum)[i] = A.nbnum;
+    G(S.hbitype)[i] = SDMD_NOEVENT;
 }
 
-// Predict for one atom whose record was already reset (ResetTarget).
-// All threads of the block call this.
+__device__ __forceinline__ void finish_atom(Sys &S, const Smem &sm, Atom &A, Cand &C, int *err) {
+    const int lane = threadIdx.x & 63, n = A.ncand;
+    select_bonds(S, sm, A, C);
+    wave_sync();
+    select_collisions(S, sm, A, C, n);
+    wave_sync();
+    if (lane == 0) assign_onebody(S, sm, A, C, err);
+    wave_sync();
+    if (A.hbscan) select_hbonds(S, sm, A, C, n);
+    wave_sync();
+    if (lane == 0) assign_tail(S, sm, A, err);
+}
+
+// The free H-bond scan runs unless the last event of the atom was a skipped
+// H-bond (HBTime head, TimePrediction.c:309-330)
+__device__ __forceinline__ int wants_hbscan(const Atom &A) {
+    return A.hbitype != SDMD_HBSKIP && A.hbbond <= 0 && (A.role == 'A' || A.role == 'D' || A.role == 'S');
+}
+
+// candidates [w0, w0 + n) of the staged atom's ordered list (all threads)
 template <int B>
-__device__ void predict_atom(Sys &S, Smem &sm, int i) {
-    const int tid = threadIdx.x;
-    const int wave = tid >> 6, lane = tid & 63;
-    unsigned long long pt = S.prof ? wall_clock64() : 0;
-    if (tid == 0) {
-        stage_atom(S, sm, i);
-        sm.cnt_cand = 0;
-        sm.cnt_eval = 0;
-    }
-    __syncthreads();
-    const int nrow = sm.A.nrow;
-    if (nrow <= ROWCAP)
-        for (int k = tid; k < nrow; k += B) {
-            sm.row_j[k] = G(S.cmap_j)[G(S.cmap_off)[i] + k];
-            sm.row_b[k] = G(S.cmap_bits)[G(S.cmap_off)[i] + k];
-        }
-    if (tid >= B - SDMD_DYNSLOTS) {
-        const int k = tid - (B - SDMD_DYNSLOTS);
-        sm.dyn_j[k] = G(S.dynj)[(size_t)i * SDMD_DYNSLOTS + k];
-        sm.dyn_b[k] = G(S.dynb)[(size_t)i * SDMD_DYNSLOTS + k];
-    }
-    int err = 0;
-    const int nb = sm.nb;
-    if (nb > MAXBOND && tid == 0) sm.err = ERR_CELLCAP;
-    PROF_MARK(S, PH_STAGE, pt);
-    // bonds (wave 0) and the 27-cell gather (wave 1, or wave 0 lanes 32.. when B == 64)
-    if (tid < min(nb, MAXBOND)) eval_bond(S, sm, tid, &err);
-    const int gwave = (B >= 128) ? 1 : 0;
-    const int glane = (B >= 128) ? lane : lane - 32;
-    const bool gatherer = wave == gwave && glane >= 0 && glane < 27;
-    if (gatherer) {
-        const int c = glane;
-        int j = G(S.celllist)[S.N + cell_index(S, sm.A.cx, sm.A.cy, sm.A.cz, c)];
-        int cnt = 0;
-        while (j && cnt <= CELL_CAP) {      // bounded walk: a fuller cell takes the windowed gather
-            if (cnt < CELL_CAP) sm.cellbuf[c * CELL_CAP + cnt] = j;
-            cnt++;
-            j = G(S.celllist)[j];
-        }
-        sm.cellcnt[c] = cnt;
-    }
-    if (tid == 0) sm.over = 0;
-    __syncthreads();
-    if (gatherer && sm.cellcnt[glane] > CELL_CAP) {
-        // a cell holds more atoms than the staging area: count every cell's
-        // list in full (the lists are the reference's, Events.c:158-200)
-        sm.over = 1;
-    }
-    __syncthreads();
-    const bool over = sm.over;
-    if (over && gatherer) {
-        const int c = glane;
-        int j = G(S.celllist)[S.N + cell_index(S, sm.A.cx, sm.A.cy, sm.A.cz, c)];
-        int cnt = 0;
-        while (j && cnt <= S.N) { cnt++; j = G(S.celllist)[j]; }
-        sm.cellcnt[c] = cnt;
-    }
-    __syncthreads();
-    PROF_MARK(S, PH_GATHER, pt);
-    if (wave == 0) {
-        // bond selection
-        double m = sm.A.t;
-        int win = -1, inh = 0;
-        wave_select(min(nb, MAXBOND), sm.bt, sm.bfl, sm.bj, S.evt, m, win, inh);
-        if (lane == 0 && win >= 0) {
-            if (inh) take_inherited(sm.A, S, sm.bj[win], SDMD_BOND);
-            else take_computed(sm.A, S, sm.bt[win], sm.bpot[win], sm.bsub[win], SDMD_BOND, sm.bj[win]);
-        }
-        // prefix sum of the cell counts (the candidates' order: cells in
-        // DMD.c:117-121 order, each in list order)
-        int c = lane < 27 ? sm.cellcnt[lane] : 0;
-        int incl = c;
-#pragma unroll
-        for (int off = 1; off < 32; off <<= 1) {
-            int v = __shfl_up(incl, off, 64);
-            if (lane >= off) incl += v;
-        }
-        if (lane < 27) sm.celloff[lane + 1] = incl;
-        if (lane == 0) sm.celloff[0] = 0;
-        if (lane == 26) sm.ncand = incl;
-        if (lane < 27 && sm.cellcnt[lane] > S.N) sm.err = ERR_LINKLIST;
-    }
-    __syncthreads();
-    const int ntot = sm.err ? 0 : sm.ncand;         // a broken list: no scan (the error ends the run)
-    const int wsz = S.win;                            // candidates per pass, <= MAXC
-    // the staged cells serve a single pass; a fuller cell or a longer list
-    // re-walks the lists for each window
-    const bool rewalk = over || ntot > wsz;
-    // the candidates of [w0, w0 + wsz) of the ordered list into cand_j
-    auto gather_window = [&](int w0) {
-        if (!rewalk) {
-            for (int k = tid; k < 27 * CELL_CAP; k += B) {
-                const int c = k / CELL_CAP, q = k % CELL_CAP;
-                if (q < sm.cellcnt[c]) sm.cand_j[sm.celloff[c] + q] = sm.cellbuf[k];
-            }
-        } else if (gatherer) {
-            const int c = glane;
-            const int w1 = w0 + wsz;
-            int g = sm.celloff[c];
-            if (g < w1 && sm.celloff[c + 1] > w0) {
-                int j = G(S.celllist)[S.N + cell_index(S, sm.A.cx, sm.A.cy, sm.A.cz, c)];
-                for (; j && g < w1; g++, j = G(S.celllist)[j])
-                    if (g >= w0) sm.cand_j[g - w0] = j;
+__device__ __forceinline__ void gather_window(const Sys &S, const Atom &A, Cand &C, int w0, int n) {
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    if (!A.over) {
+        for (int c = wave; c < 27; c += B / 64) {
+            const int cnt = C.cellcnt[c], g = C.celloff[c] + cnt - 1 - lane - w0;
+            if (lane < cnt && g >= 0 && g < n) {
+                C.j[g] = G(S.cmem)[(size_t)cell_index(S, A.cx, A.cy, A.cz, c) * CELL_CAP + lane];
+                C.cell[g] = (unsigned char)c;
             }
         }
-        __syncthreads();
-    };
-    PROF_MARK(S, PH_BONDSEL, pt);
-    double calib = S.cutoffr * SDMD_EXTEND_RATIO;
-    calib *= calib;
-    int my_cand = 0, my_eval = 0;
-    if (tid < min(nb, MAXBOND)) my_eval++;
-    // CollisionTime over the ordered candidates, window by window: the
-    // running minimum (and CheckDuplication against it) carries over, so the
-    // result is that of one sequential pass
-    for (int w0 = 0; w0 < ntot || w0 == 0; w0 += wsz) {
-        const int ncand = min(ntot - w0, wsz);
-        gather_window(w0);
-        for (int k = tid; k < ncand; k += B) {
-            eval_collision(S, sm, k, calib, &err);
-            my_cand += (sm.cand_j[k] != i);
-            my_eval += (sm.cand_fl[k] >> 1) & 1;
-        }
-        __syncthreads();
-        if (wave == 0) {
-            double m = sm.A.t;
-            int win = -1, inh = 0;
-            wave_select(ncand, sm.cand_t, sm.cand_fl, sm.cand_j, S.evt, m, win, inh);
-            if (lane == 0 && win >= 0) {
-                if (inh) take_inherited(sm.A, S, sm.cand_j[win], SDMD_COLI);
-                else take_computed(sm.A, S, sm.cand_t[win], sm.cand_pot[win], sm.cand_sub[win], SDMD_COLI, sm.cand_j[win]);
-            }
-        }
-        __syncthreads();
-    }
-    if (my_cand) atomicAdd(&sm.cnt_cand, my_cand);
-    if (my_eval) atomicAdd(&sm.cnt_eval, my_eval);
-    PROF_MARK(S, PH_EVAL, pt);
-    if (tid == 0) {
-        // PBCandCrossCellTime, ThermostatTime
-        pcc_time(S, sm.A);
-        if (S.thermostat) {
-            double z = next_normal(S, sm);
-            double t = S.thermoF * ((z < 0) ? (-z) : (z));
-            job_assign_atom(sm.A, S, t, 0, SDMD_INVALID_INTER, SDMD_THER, 0);
-        }
-        // HBTime head, TimePrediction.c:309-330
-        sm.hbscan = 0;
-        const int i0 = sm.A.i;
-        if (G(S.hbitype)[i0] == SDMD_HBSKIP) {
-            G(S.hbitype)[i0] = SDMD_NOEVENT;
-        } else {
-            G(S.hbitype)[i0] = SDMD_NOEVENT;
-            if (sm.A.hbbond > 0) hb_time_bonded(S, sm.A, &err);
-            else if (sm.A.role == 'A' || sm.A.role == 'D' || sm.A.role == 'S') sm.hbscan = 1;
+    } else if (wave == 0 && lane < 27) {
+        // a cell holds more atoms than its array: walk the lists (the
+        // reference's, Events.c:158-200)
+        int g = C.celloff[lane] - w0;
+        if (g < n && C.celloff[lane + 1] > w0) {
+            int j = G(S.celllist)[S.N + cell_index(S, A.cx, A.cy, A.cz, lane)];
+            for (; j && g < n; g++, j = G(S.celllist)[j])
+                if (g >= 0) { C.j[g] = j; C.cell[g] = (unsigned char)lane; }
         }
     }
     __syncthreads();
-    PROF_MARK(S, PH_SELECT, pt);
-    if (sm.hbscan) {
-        // the free-atom H-bond scan over the same ordered candidates
-        int my_hb = 0;
+}
+
+// The staged atom's prediction over windows of candidates: the running
+// minimum (and CheckDuplication against it) carries over, so the result is
+// that of one sequential pass.  All threads.
+template <int B, bool TAB>
+__device__ __forceinline__ void predict_windows(Sys &S, Smem &sm, const PairTab *T, Atom &A, Cand &C, double calib, int *err) {
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int ntot = A.ncand;
+    const int wsz = min(S.win, PWIN);
+    if (wave == 0) select_bonds(S, sm, A, C);
+    for (int pass = 0; pass < 2; pass++) {
+        if (pass == 1) {
+            if (tid == 0) assign_onebody(S, sm, A, C, err);
+            __syncthreads();
+            if (!A.hbscan) break;
+        }
         for (int w0 = 0; w0 < ntot; w0 += wsz) {
-            const int ncand = min(ntot - w0, wsz);
-            if (rewalk) gather_window(w0);
-            for (int k = tid; k < ncand; k += B) {
-                eval_hb(S, sm, k, calib, &err);
-                my_hb += (sm.cand_fl[k] >> 1) & 1;
+            const int n = min(ntot - w0, wsz);
+            gather_window<B>(S, A, C, w0, n);
+            int ev = 0;
+            for (int k = tid; k < n; k += B) {
+                eval_candidate<TAB>(S, sm, T, A, C, k, calib, err);
+                ev += ((pass ? C.hfl[k] : C.fl[k]) >> 1) & 1;
             }
+            if (ev) atomicAdd(&A.cnt_eval, ev);
             __syncthreads();
             if (wave == 0) {
-                double m = sm.A.t;
-                int win = -1, inh = 0;
-                wave_select(ncand, sm.cand_t, sm.cand_fl, sm.cand_j, S.evt, m, win, inh);
-                if (lane == 0 && win >= 0) {
-                    if (inh) take_inherited(sm.A, S, sm.cand_j[win], SDMD_HB);
-                    else take_computed(sm.A, S, sm.cand_t[win], sm.cand_pot[win], SDMD_TBDHBFORM, SDMD_HB, sm.cand_j[win]);
-                }
+                if (pass == 0) select_collisions(S, sm, A, C, n);
+                else select_hbonds(S, sm, A, C, n);
             }
             __syncthreads();
         }
-        if (my_hb) atomicAdd(&sm.cnt_eval, my_hb);
-    }
-    PROF_MARK(S, PH_HB, pt);
-    if (tid == 0) {
-        hb_neighbor_time(S, sm.A, &err);
-        if (S.wall) {
-            WallEv w;
-            if (wall_time(S, sm.A.y, sm.A.z, sm.A.vy, sm.A.vz, sm.A.type, w, &err))
-                job_assign_atom(sm.A, S, w.t, w.pot, w.sub, SDMD_WALL, 0);
-        }
-        unstage_atom(S, sm.A);
     }
     __syncthreads();
-    if (tid == 0) {
-        S.candidates += sm.cnt_cand;
-        S.pair_evals += sm.cnt_eval + sm.A.nbstat + (sm.A.hbbond > 0 ? 1 : 0);
-    }
-    PROF_MARK(S, PH_TAIL, pt);
-    // statistics: candidates scanned, quadratic evaluations
+    if (tid == 0) assign_tail(S, sm, A, err);
+    (void)lane;
+    __syncthreads();
+}
+
+// Predict of up to two atoms whose records were already reset (ResetTarget),
+// SGThread.c:158-211.  All threads call this.  Two atoms are predicted side
+// by side, each by half of the workgroup's waves: their predictions read
+// each other's record only through CheckDuplication, and the second atom's
+// selection is repeated when the first one's new event names it (its
+// evaluated candidates stay as they are).  Bound by the latency of one
+// candidate's evaluation, not by throughput: 205 candidates occupy four
+// wavefronts.
+template <int B, bool TAB>
+__device__ __forceinline__ void predict_atoms(Sys &S, Smem &sm, const PairTab *T, int n, int i0, int i1) {
+    constexpr int W = B / 64;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int nw = (W > 1 && n == 2) ? W / 2 : W;      // waves per team
+    const int team = wave / nw, r = wave % nw;
+    unsigned long long pt = S.prof ? wall_clock64() : 0;
+    double calib = S.cutoffr * SDMD_EXTEND_RATIO;
+    calib *= calib;
+    int err = 0;
+    for (int s = 0; s < n; s++)
+        if ((s == team || (nw == W && team == 0)) && r == 0) {
+            Atom &A = sm.A[s];
+            stage_atom(S, A, s ? i1 : i0, n == 2 ? (s ? i0 : i1) : 0);
+            const long long zp = sm.zpos + s;
+            if (lane == 0 && S.thermostat) A.zn = zp < S.nz ? G(S.zn)[zp] : 1.0;
+        }
+    __syncthreads();
+    PROF_MARK(S, PH_STAGE, pt);
+    for (int s = 0; s < n; s++)
+        if (s == team || (nw == W && team == 0)) {
+            Atom &A = sm.A[s];
+            if (r == 0 && lane == 0) {
+                A.hbscan = wants_hbscan(A);
+                A.pot0 = A.pot; A.pc0 = A.pc; A.sub0 = A.sub; A.nbnum0 = A.nbnum;
+            }
+            stage_neighbours<true>(S, sm, A, sm.c[s], r, nw, &err);
+        }
     if (err) atomicCAS(&sm.err, 0, err);
     __syncthreads();
+    PROF_MARK(S, PH_GATHER, pt);
+    const int wsz = min(S.win, PWIN);
+    bool whole = true;
+    for (int s = 0; s < n; s++) whole = whole && !sm.A[s].over && sm.A[s].ncand <= wsz;
+    err = 0;
+    if (whole) {
+        for (int s = 0; s < n; s++)
+            if (s == team || (nw == W && team == 0)) {
+                Atom &A = sm.A[s];
+                Cand &C = sm.c[s];
+                int ev = 0;
+                for (int k = r * 64 + lane; k < A.ncand; k += nw * 64) {
+                    eval_candidate<TAB>(S, sm, T, A, C, k, calib, &err);
+                    ev += ((C.fl[k] >> 1) & 1) + ((C.hfl[k] >> 1) & 1);
+                }
+                if (ev) atomicAdd(&A.cnt_eval, ev);
+            }
+        if (err) atomicCAS(&sm.err, 0, err);
+        __syncthreads();
+        PROF_MARK(S, PH_EVAL, pt);
+        err = 0;
+        for (int s = 0; s < n; s++)
+            if ((s == team || (nw == W && team == 0)) && r == 0) finish_atom(S, sm, sm.A[s], sm.c[s], &err);
+        __syncthreads();
+        PROF_MARK(S, PH_SELECT, pt);
+        if (n == 2) {
+            const Atom &P = sm.A[0];
+            Atom &A = sm.A[1];
+            if (P.partner == i1) {                     // uniform: the record in LDS is final
+                if (wave == 0) {
+                    // CheckDuplication against the first atom's new record
+                    Cand &C = sm.c[1];
+                    const bool same = P.pc == A.counter;
+                    if (same && P.evtype == SDMD_BOND && lane < min(A.nb, MAXBOND) && C.bj[lane] == i0) {
+                        C.bfl[lane] = 1;
+                        C.bjt[lane] = P.t;
+                    }
+                    if (same && (P.evtype == SDMD_COLI || P.evtype == SDMD_HB))
+                        for (int k = lane; k < A.ncand; k += 64)
+                            if (C.j[k] == i0) {
+                                if (P.evtype == SDMD_COLI) C.fl[k] |= 1;
+                                else C.hfl[k] |= (C.hfl[k] >> 2) & 1;
+                            }
+                    if (lane == 0) {
+                        A.t = INFINIT; A.evtype = SDMD_INVD; A.partner = INVALID;
+                        A.pot = A.pot0; A.pc = A.pc0; A.sub = A.sub0; A.nbnum = A.nbnum0;
+                        A.exclude = 0;
+                    }
+                    wave_sync();
+                    finish_atom(S, sm, A, C, &err);
+                }
+                __syncthreads();
+            }
+        }
+    } else {
+        for (int s = 0; s < n; s++) {
+            Atom &A = sm.A[s];
+            Cand &C = sm.c[s];
+            if (s == 1) {
+                // the second atom's bonds again, now against the first
+                // atom's new record
+                if (threadIdx.x == 0) A.exclude = 0;
+                __syncthreads();
+                if (threadIdx.x < min(A.nb, MAXBOND)) eval_bond(S, sm, A, C, threadIdx.x);
+                __syncthreads();
+            }
+            predict_windows<B, TAB>(S, sm, T, A, C, calib, &err);
+        }
+    }
+    if (err) atomicCAS(&sm.err, 0, err);
+    if (threadIdx.x == 0 && S.thermostat)              // one draw per predicted atom, in order
+        for (int s = 0; s < n; s++) {
+            if (sm.zpos < S.nz) sm.zpos++;
+            else sm.err = ERR_NORMALS;
+        }
+    if (threadIdx.x == 0)
+        // statistics: candidates scanned, quadratic evaluations
+        for (int s = 0; s < n; s++) {
+            const Atom &A = sm.A[s];
+            S.candidates += A.ncand > 0 ? A.ncand - 1 : 0;
+            S.pair_evals += A.cnt_eval + min(A.nb, MAXBOND) + A.nbstat + (A.hbbond > 0 ? 1 : 0);
+        }
+    __syncthreads();
+    PROF_MARK(S, PH_TAIL, pt);
 }
 
 // Predict(renewList) with ResetTarget, SGThread.c:158-211
-template <int B>
-__device__ void predict_list(Sys &S, Smem &sm, const int *renew) {
+template <int B, bool TAB>
+__device__ void predict_list(Sys &S, Smem &sm, const PairTab *T, const int *renew) {
     if (threadIdx.x == 0) {
         for (int n = 1; renew[n]; n++) {
             const int i = renew[n];
@@ -609,10 +937,65 @@ __device__ void predict_list(Sys &S, Smem &sm, const int *renew) {
         }
     }
     __syncthreads();
-    for (int n = 1; renew[n]; n++) predict_atom<B>(S, sm, renew[n]);
+    const bool two = renew[1] && renew[2] && renew[1] != renew[2];
+    for (int n = 1; renew[n]; n += two ? 2 : 1)
+        predict_atoms<B, TAB>(S, sm, T, two ? 2 : 1, renew[n], two ? renew[2] : 0);
 }
 
-// ---------------------------------------------------------------- CBT (lane 0), CBT.c
+// ---------------------------------------------------------------- CBT, CBT.c
+// UpdateCBT (CBT.c:33-39, 56-83) for one or two renewed atoms, by one wave.
+// A path's nodes follow from the leaf's index alone, so each lane holds one
+// level (lanes 0..31 the first atom's path, 32..63 the second's): the path's
+// node, the sibling on the way up and its current event time, read at once
+// instead of level by level; the walk itself runs on registers.  Where the
+// second path meets nodes the first has just written, it takes their new
+// values.
+__device__ __forceinline__ void cbt_update(Sys &S, Smem &sm, int n, int a0, int l0, double t0, int a1, int l1, double t1) {
+    const int lane = threadIdx.x & 63, half = lane >> 5, k = lane & 31;
+    const int L = half ? l1 : l0;
+    const bool on = half < n && k < 31 - __clz(L);
+    const int f = on ? L >> (k + 1) : 1, sib = on ? (L >> k) ^ 1 : 1;
+    int of = G(S.node)[f], sv = G(S.node)[sib];
+    double st = evt_now(S, sm, on ? sv : a0);
+    int nv = of;               // the node's new value and its time
+    double nt = 0;
+    bool done = false;         // the walk reached this lane's level
+    for (int h = 0; h < n; h++) {
+        if (h == 1) {
+            // nodes of the first path among this path's nodes and siblings
+            const int d0 = 31 - __clz(l0);
+            const int ms = d0 - (31 - __clz(sib)), mf = d0 - (31 - __clz(f));
+            const int qs = (half && ms >= 1 && (l0 >> ms) == sib) ? ms - 1 : -1;
+            const int qf = (half && mf >= 1 && (l0 >> mf) == f) ? mf - 1 : -1;
+            const int sn = __shfl(nv, max(qs, 0), 64), fn = __shfl(nv, max(qf, 0), 64);
+            const double tn = __shfl(nt, max(qs, 0), 64);
+            const int ds = __shfl((int)done, max(qs, 0), 64), df = __shfl((int)done, max(qf, 0), 64);
+            if (qs >= 0 && ds) { sv = sn; st = tn; }
+            if (qf >= 0 && df) { of = fn; nv = fn; }
+        }
+        const int a = h ? a1 : a0, Lh = h ? l1 : l0, d = 31 - __clz(Lh);
+        int cur = a;
+        double tc = h ? t1 : t0;
+        bool own = true;       // still on nodes that held the atom itself
+        for (int q = 0; q < d; q++) {
+            const int src = 32 * h + q;
+            const int o = lane_get(of, src), s = lane_get(sv, src);
+            const double ts = lane_get(st, src);
+            const bool left = !((Lh >> q) & 1);
+            own = own && o == a;
+            // node = (evt[left] < evt[right]) ? left : right
+            const bool keep = left ? tc < ts : !(ts < tc);
+            if (!keep) { cur = s; tc = ts; }
+            if (lane == src) { nv = cur; nt = tc; done = true; }
+            if (!own && cur == o) break;
+        }
+        if (half == h && on && done && nv != of) G(S.node)[f] = nv;
+        if (lane == 32 * h + d - 1) sm.root = nv;      // the top level: node 1
+        wave_sync();
+    }
+}
+
+// one atom's path (lane 0), for single operations
 __device__ void cbt_update_run(Sys &S, int a) {
     int father, left, right, old;
     for (father = G(S.leaf)[a] / 2; father > 0; father /= 2) {
@@ -630,19 +1013,30 @@ __device__ void cbt_update_run(Sys &S, int a) {
     }
 }
 
+// CreateCBT (CBT.c:16-30).  Inserting atom a splits leaf a - 1: its atom
+// moves to node 2 (a - 1), a takes node 2 (a - 1) + 1.  So the atom of a
+// leaf depends on the leaf's number alone (the right child 2c + 1 holds c +
+// 1, a left child what its parent held), and since no event time changes
+// meanwhile every inner node is the winner of its two children.
+template <int B>
 __device__ void cbt_create(Sys &S) {
-    for (int k = 0; k < 2 * S.N; k++) G(S.node)[k] = 0;
-    for (int k = 0; k <= S.N; k++) G(S.leaf)[k] = 0;
-    S.count = 0;
-    for (int a = 1; a <= S.N; a++) {
-        if (S.count == 0) { G(S.node)[1] = a; S.count++; continue; }
-        const int i = G(S.node)[S.count];
-        G(S.node)[S.count * 2] = i;
-        G(S.node)[S.count * 2 + 1] = a;
-        G(S.leaf)[i] = S.count * 2;
-        G(S.leaf)[a] = S.count * 2 + 1;
-        S.count++;
-        cbt_update_run(S, i);
+    const int N = S.N, tid = threadIdx.x;
+    if (tid == 0) { G(S.node)[0] = 0; G(S.leaf)[0] = 0; S.count = N; }
+    for (int m = N + tid; m < 2 * N; m += B) {
+        const int c = m >> __builtin_ctz(m);           // up the left edge to a right child (or node 1)
+        const int a = c == 1 ? 1 : (c >> 1) + 1;
+        G(S.node)[m] = a;
+        G(S.leaf)[a] = m;
+    }
+    __syncthreads();
+    for (int hi = N - 1; hi >= 1;) {                   // level by level, the deepest first
+        const int lo = 1 << (31 - __clz(hi));
+        for (int m = lo + tid; m <= hi; m += B) {
+            const int l = G(S.node)[2 * m], r = G(S.node)[2 * m + 1];
+            G(S.node)[m] = (G(S.evt)[l] < G(S.evt)[r]) ? l : r;
+        }
+        __syncthreads();
+        hi = lo - 1;
     }
 }
 
@@ -682,26 +1076,48 @@ __device__ void pcc_event(Sys &S, int i, int *err) {
         ci[n][i] = v;
     }
     const int newc = G(S.cz)[i] * S.cellnum[1] * S.cellnum[2] + G(S.cy)[i] * S.cellnum[1] + G(S.cx)[i] + 1;
-    int nx = oldc + N, guard = 0;
-    while (G(S.celllist)[nx] != i) {
-        nx = G(S.celllist)[nx];
-        if (nx == 0 || ++guard > N) { *err = ERR_LINKLIST; return; }
+    // out of the old cell: its array holds the list back to front, so the
+    // atom before i in the list is the next array entry (or the list's head)
+    int *m = S.cmem + (size_t)oldc * CELL_CAP;
+    const int cnt = G(S.ccnt)[oldc];
+    int nx = oldc + N;
+    if (cnt <= CELL_CAP) {
+        int q = 0;
+        while (q < cnt && G(m)[q] != i) q++;
+        if (q >= cnt) { *err = ERR_LINKLIST; return; }
+        if (q < cnt - 1) nx = G(m)[q + 1];
+        for (; q < cnt - 1; q++) G(m)[q] = G(m)[q + 1];
+    } else {
+        int guard = 0;
+        while (G(S.celllist)[nx] != i) {
+            nx = G(S.celllist)[nx];
+            if (nx == 0 || ++guard > N) { *err = ERR_LINKLIST; return; }
+        }
     }
     G(S.celllist)[nx] = G(S.celllist)[i];
-    nx = newc + N;
-    G(S.celllist)[i] = G(S.celllist)[nx];
-    G(S.celllist)[nx] = i;
+    G(S.ccnt)[oldc] = cnt - 1;
+    if (cnt == CELL_CAP + 1) {                          // the list fits its array again
+        int j = G(S.celllist)[oldc + N];
+        for (int q = CELL_CAP - 1; q >= 0 && j; q--, j = G(S.celllist)[j]) G(m)[q] = j;
+    }
+    // into the new one, at the head
+    const int cn = G(S.ccnt)[newc];
+    G(S.celllist)[i] = G(S.celllist)[newc + N];
+    G(S.celllist)[newc + N] = i;
+    if (cn < CELL_CAP) G(S.cmem)[(size_t)newc * CELL_CAP + cn] = i;
+    G(S.ccnt)[newc] = cn + 1;
 }
 
 __device__ void do_event(Sys &S, Smem &sm, int t, int p, int *err) {   // DoEvent, Events.c:25-114
     const int ty = G(S.evtype)[t];
+    const PosLazy pos{S, sm};
     switch (ty) {
     case SDMD_COLI: case SDMD_BOND: case SDMD_HBNE:
-        interaction_event(S, PosStored{S}, t, p, 0, 0, err);
+        interaction_event(S, pos, t, p, 0, 0, err);
         break;
     case SDMD_HB: {
         const int nbi = G(S.hbnb)[t], nbj = G(S.hbnb)[p];
-        interaction_event(S, PosStored{S}, t, p, nbi, nbj, err);
+        interaction_event(S, pos, t, p, nbi, nbj, err);
         hb_event(S, t, p, nbi, nbj, err);
         break;
     }
@@ -716,6 +1132,128 @@ __device__ void do_event(Sys &S, Smem &sm, int t, int p, int *err) {   // DoEven
     default: *err = ERR_EVENTTYPE; return;
     }
     if (ty >= 0 && ty < 16) S.per_type[ty]++;
+}
+
+// One pop up to its re-predictions (wave 0): AssignJob, UpdateData and
+// TimeForward of the event's atoms, HazardCheck, DoEvent, the event counters
+// and ResetTarget.  Lane 0 holds the target, lane 1 the partner: their state
+// is loaded side by side, and a collision, bond or H-bond-neighbour event
+// (InteractionEvent without its H-bond branch, Events.c:770-1025) runs on
+// registers.
+__device__ __forceinline__ void pop_event(Sys &S, Smem &sm) {
+    const int lane = threadIdx.x & 63;
+    const int target = sm.root, n0 = sm.nlog;
+    const int p0 = G(S.evp)[target], ty = G(S.evtype)[target], sub = G(S.evsub)[target];
+    const double pot0 = G(S.evpot)[target];
+    const long long pc = G(S.evpc)[target];
+    const int partner = p0 > 0 ? p0 : 0;
+    const int a = (lane == 1 && partner) ? partner : target;
+    double x = G(S.x)[a], y = G(S.y)[a], z = G(S.z)[a], t = G(S.evt)[a];
+    double vx = G(S.vx)[a], vy = G(S.vy)[a], vz = G(S.vz)[a];
+    const double mass = G(S.mass)[a];
+    const long long counter = G(S.evc)[a];
+    const int cx = G(S.cx)[a], cy = G(S.cy)[a], cz = G(S.cz)[a];
+    for (int l = lag_of(S, n0, a); l < n0; l++) {
+        const double h = sm.log[l];
+        x = x + vx * h; y = y + vy * h; z = z + vz * h; t = t - h;
+    }
+    const double dt = lane_get(t, 0);
+    if (S.trace) {
+        if (S.trace_n < S.trace_cap) {
+            if (lane == 0) {
+                sdmd_gpu_pop_rec &r = S.trace[S.trace_n];
+                r.target = target; r.partner = p0; r.type = ty; r.sub = sub; r.dt = dt; r.pot = pot0;
+            }
+        } else {
+            if (lane == 0) sm.err = ERR_TRACE;
+            return;
+        }
+    }
+    x = x + vx * dt; y = y + vy * dt; z = z + vz * dt; t = t - dt;
+    const bool mine = lane == 0 || (lane == 1 && partner);
+    if (mine) {
+        G(S.x)[a] = x; G(S.y)[a] = y; G(S.z)[a] = z; G(S.evt)[a] = t;
+        G(S.lag)[a] = (unsigned char)(n0 + 1);
+    }
+    const bool stale = partner && pc < lane_get(counter, 1);       // HazardCheck, SGThread.c:215-235
+    const bool pair = partner && (ty == SDMD_COLI || ty == SDMD_BOND || ty == SDMD_HBNE);
+    int err = 0;
+    if (lane == 0) {
+        sm.log[n0] = dt;
+        sm.nlog = n0 + 1;
+        sm.dt = dt;
+        sm.target = target;
+        sm.partner = partner;
+        sm.stale = stale;
+        S.currenttime += dt;
+        sm.renew[0] = (partner && !stale) ? 2 : 1;
+        sm.renew[1] = target;
+        sm.renew[2] = (partner && !stale) ? partner : 0;
+        sm.renew[3] = 0;
+        if (stale) S.recal++;
+        else S.frame++;
+        sm.flush = n0 + 1 >= S.logk || (S.hash_every > 0 && (S.pops + 1) % S.hash_every == 0);
+    }
+    if (!stale && pair) {
+        // InteractionEvent, Events.c:798-1024, from the two lanes' state
+        const int ci[3] = {lane_get(cx, 0), lane_get(cy, 0), lane_get(cz, 0)};
+        const int cj[3] = {lane_get(cx, 1), lane_get(cy, 1), lane_get(cz, 1)};
+        double pj[3] = {lane_get(x, 1), lane_get(y, 1), lane_get(z, 1)};
+        const double pi[3] = {lane_get(x, 0), lane_get(y, 0), lane_get(z, 0)};
+        const double vi[3] = {lane_get(vx, 0), lane_get(vy, 0), lane_get(vz, 0)};
+        const double vj[3] = {lane_get(vx, 1), lane_get(vy, 1), lane_get(vz, 1)};
+        const double mi = lane_get(mass, 0), mj = lane_get(mass, 1);
+        for (int n = 0; n < 3; n++) {
+            if (ci[n] != cj[n]) {
+                if (ci[n] == 0 && cj[n] == S.cellnum[n + 1] - 1) pj[n] -= S.box[n + 1];
+                else if (ci[n] == S.cellnum[n + 1] - 1 && cj[n] == 0) pj[n] += S.box[n + 1];
+            }
+        }
+        const double r1 = pi[0] - pj[0], r2 = pi[1] - pj[1], r3 = pi[2] - pj[2];
+        const double v1 = vi[0] - vj[0], v2 = vi[1] - vj[1], v3 = vi[2] - vj[2];
+        const double d2 = r1 * r1 + r2 * r2 + r3 * r3;
+        const double b = r1 * v1 + r2 * v2 + r3 * v3;
+        const double mu = mi * mj / (mi + mj);
+        double pot = pot0;
+        int s = 0;
+        bool ok = true;
+        switch (sub) {
+        case SDMD_CORECOLLI: s = 1; pot = 0; break;
+        case SDMD_WELLBOUNC: s = (b < 0) ? 1 : -1; pot = 0; break;
+        case SDMD_WELLCAPTR: s = -1; break;
+        case SDMD_WELLESCAP: s = (b < 0) ? -1 : 1; break;
+        case SDMD_TBDCAPTR:
+            if (b * b - 2 * d2 * pot / mu <= 0) { pot = 0; s = 1; } else s = -1;
+            break;
+        case SDMD_TBDESCAP:
+            if (b * b - 2 * d2 * pot / mu <= 0) { pot = 0; s = (b < 0) ? 1 : -1; }
+            else s = (b < 0) ? -1 : 1;
+            break;
+        default: err = ERR_SUBTYPE; ok = false; break;
+        }
+        if (ok) {
+            const double phi = (-1 * b + s * sqrt((b * b - 2 * d2 * pot / mu))) / ((mi + mj) * d2);
+            if (isnan(phi)) {
+                err = ERR_PHI_NAN;
+            } else {
+                const double fi = mj * phi, fj = mi * phi;
+                if (lane == 0) { vx = vx + fi * r1; vy = vy + fi * r2; vz = vz + fi * r3; }
+                else { vx = vx - fj * r1; vy = vy - fj * r2; vz = vz - fj * r3; }
+                if (mine) { G(S.vx)[a] = vx; G(S.vy)[a] = vy; G(S.vz)[a] = vz; }
+            }
+        }
+        if (lane == 0) S.per_type[ty]++;
+    } else if (!stale && lane == 0) {
+        do_event(S, sm, target, partner, &err);
+    }
+    if (err && lane == 0) sm.err = err;
+    // SGThread.c:100-104, then ResetTarget of the renewed atoms
+    if (mine && !stale) G(S.evc)[a] = counter + 1;
+    if (lane == 0 || (lane == 1 && partner && !stale)) {
+        G(S.evtype)[a] = SDMD_INVD;
+        G(S.evt)[a] = INFINIT;
+        G(S.evp)[a] = INVALID;
+    }
 }
 
 __device__ unsigned long long fnv(unsigned long long h, const void *p, int n) {
@@ -737,28 +1275,6 @@ __device__ unsigned long long state_hash(const Sys &S) {
     return h;
 }
 
-// UpdateData + TimeForward over all atoms, ToolFunctions.c:23-36
-template <int B>
-__device__ __forceinline__ void sweep(const Sys &S, const double dt) {
-    double *__restrict__ X = S.x;
-    double *__restrict__ Y = S.y;
-    double *__restrict__ Z = S.z;
-    double *__restrict__ T = S.evt;
-    const double *__restrict__ VX = S.vx;
-    const double *__restrict__ VY = S.vy;
-    const double *__restrict__ VZ = S.vz;
-    const int N = S.N;
-#pragma unroll 4
-    for (int i = threadIdx.x + 1; i <= N; i += B) {
-        const double vx = VX[i], vy = VY[i], vz = VZ[i];
-        const double x = X[i], y = Y[i], z = Z[i], t = T[i];
-        X[i] = x + vx * dt;
-        Y[i] = y + vy * dt;
-        Z[i] = z + vz * dt;
-        T[i] = t - dt;
-    }
-}
-
 // ---------------------------------------------------------------- kernels
 // The system struct is copied into LDS for the kernel's lifetime: its
 // pointers and constants are then LDS reads instead of dependent global
@@ -777,14 +1293,28 @@ __device__ __forceinline__ void sys_store(Sys *dst, const Sys &src) {
     for (int k = threadIdx.x; k < n; k += B) ((int *)dst)[k] = ((const int *)&src)[k];
 }
 
+// the collision table and the tables' step pool into LDS
+template <int B>
+__device__ __forceinline__ void tab_load(PairTab &T, const Sys &S) {
+    for (int k = threadIdx.x; k < NT * NT; k += B) {
+        const sdmd_pair *p = S.rpair + k;
+        T.dmin[k] = G(p)->dmin; T.dmax[k] = G(p)->dmax; T.step0[k] = G(p)->step0; T.nstep[k] = G(p)->nstep;
+    }
+    if (S.ltab)
+        for (int k = threadIdx.x; k < S.ltab; k += B) { T.d[k] = G(S.sd)[k]; T.e[k] = G(S.se)[k]; }
+    __syncthreads();
+}
+
 template <int B>
 __global__ __launch_bounds__(B) void k_prepare(Sys *systems) {
     __shared__ Smem sm;
     __shared__ Sys Sl;
+    __shared__ PairTab tab;
     sys_load<B>(Sl, &systems[blockIdx.x]);
     Sys &S = Sl;
+    tab_load<B>(tab, S);
     const int tid = threadIdx.x;
-    if (tid == 0) { sm.err = 0; sm.zpos = S.zpos; }
+    if (tid == 0) { sm.err = 0; sm.zpos = S.zpos; sm.nlog = 0; }
     __syncthreads();
     // ResetTarget for 1..N, then Predict(1..N) in order
     for (int i = tid + 1; i <= S.N; i += B) {
@@ -793,119 +1323,106 @@ __global__ __launch_bounds__(B) void k_prepare(Sys *systems) {
         G(S.evp)[i] = INVALID;
     }
     __syncthreads();
-    for (int i = 1; i <= S.N && sm.err == 0; i++) predict_atom<B>(S, sm, i);
+    for (int i = 1; i <= S.N && sm.err == 0; i++) predict_atoms<B, true>(S, sm, &tab, 1, i, 0);
+    __syncthreads();
+    if (sm.err == 0) cbt_create<B>(S);
     if (tid == 0) {
-        if (sm.err == 0) cbt_create(S);
         S.zpos = sm.zpos;
         if (sm.err) S.error = sm.err;
     }
     sys_store<B>(&systems[blockIdx.x], Sl);
 }
 
-template <int B>
 // t_out: stop after the first executed event that leaves the clock at or
 // past t_out -- where SingleThreadRun writes its output (SGThread.c:130-139)
+template <int B>
 __global__ __launch_bounds__(B) void k_run(Sys *systems, long long npops, long long budget, double t_end,
                                            double t_out) {
     __shared__ Smem sm;
     __shared__ Sys Sl;
+    __shared__ PairTab tab;
     __shared__ int stop;
     sys_load<B>(Sl, &systems[blockIdx.x]);
     Sys &S = Sl;
-    const int tid = threadIdx.x;
-    if (tid == 0) { sm.err = S.error; sm.zpos = S.zpos; stop = 0; }
-    __syncthreads();
-    const int N = S.N;
-    unsigned long long pt = S.prof ? wall_clock64() : 0;
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const unsigned long long t_start = wall_clock64();
     // npops < 0 asks for -npops executed events instead of pops
     const long long maxpops = npops < 0 ? LLONG_MAX : npops, evgoal = npops < 0 ? -npops : LLONG_MAX;
     const long long frame0 = S.frame;
-    for (long long pop = 0; pop < maxpops; pop++) {
-        if (sm.err) break;
-        if (tid == 0) {
+    if (S.error || maxpops == 0) return;
+    tab_load<B>(tab, S);
+    if (tid == 0) { sm.err = 0; sm.zpos = S.zpos; stop = 0; sm.nlog = 0; sm.root = G(S.node)[1]; }
+    __syncthreads();
+    unsigned long long pt = S.prof ? wall_clock64() : 0;
+    for (long long pop = 0;; pop++) {
+        if (wave == 0) {
             // device-time budget of a bounded run
-            if ((long long)(wall_clock64() - t_start) > budget || S.currenttime > t_end || S.frame - frame0 >= evgoal)
-                stop = 1;
-            // AssignJob, SGThread.c:237-259
-            const int target = G(S.node)[1];
-            sm.target = target;
-            sm.dt = G(S.evt)[target];
-            sm.renew[0] = 1; sm.renew[1] = target; sm.renew[2] = 0; sm.renew[3] = 0;
-            sm.partner = 0;
-            if (G(S.evp)[target] > 0) { sm.partner = G(S.evp)[target]; sm.renew[++sm.renew[0]] = sm.partner; }
-            if (S.trace) {
-                if (S.trace_n < S.trace_cap) {
-                    sdmd_gpu_pop_rec &r = S.trace[S.trace_n];
-                    r.target = target; r.partner = G(S.evp)[target]; r.type = G(S.evtype)[target];
-                    r.sub = G(S.evsub)[target]; r.dt = sm.dt; r.pot = G(S.evpot)[target];
-                } else {
-                    sm.err = ERR_TRACE;
-                }
+            if (pop >= maxpops || (long long)(wall_clock64() - t_start) > budget || S.currenttime > t_end ||
+                S.frame - frame0 >= evgoal || stop) {
+                if (lane == 0) stop = 1;
+            } else {
+                pop_event(S, sm);
             }
         }
         __syncthreads();
         if (sm.err || stop) break;
-        PROF_MARK(S, PH_POP, pt);
-        // UpdateData + TimeForward, ToolFunctions.c:23-36
-        sweep<B>(S, sm.dt);
-        __syncthreads();
-        PROF_MARK(S, PH_SWEEP, pt);
-        if (tid == 0) {
-            S.currenttime += sm.dt;
-            const int target = sm.target, partner = sm.partner;
-            // HazardCheck, SGThread.c:215-235
-            sm.stale = (partner > 0 && G(S.evpc)[target] < G(S.evc)[partner]);
-            if (!sm.stale) {
-                int err = 0;
-                S.frame++;
-                do_event(S, sm, target, partner, &err);
-                G(S.evc)[target]++;
-                if (sm.renew[0] == 2) G(S.evc)[partner]++;
-                if (err) sm.err = err;
-            } else {
-                sm.renew[0] = 1; sm.renew[2] = 0; sm.renew[3] = 0;
-                S.recal++;
-            }
-        }
-        __syncthreads();
-        if (sm.err) break;
+        const int flush = sm.flush;        // wave 0 runs ahead into the next pop's event
         PROF_MARK(S, PH_EVENT, pt);
-        predict_list<B>(S, sm, sm.renew);
+        predict_atoms<B, true>(S, sm, &tab, sm.renew[0], sm.renew[1], sm.renew[2]);
         if (S.prof) pt = wall_clock64();
-        if (tid == 0) {
-            for (int k = 1; sm.renew[k]; k++) cbt_update_run(S, sm.renew[k]);
+        if (flush) sweep<B>(S, sm);
+        PROF_MARK(S, PH_SWEEP, pt);
+        if (wave == 0) {
+            cbt_update(S, sm, sm.renew[0], sm.renew[1], sm.A[0].leaf, sm.A[0].t, sm.renew[2], sm.A[1].leaf, sm.A[1].t);
             PROF_MARK(S, PH_TREE, pt);
-            S.pops++;
-            S.last_exec = !sm.stale;
-            if (!sm.stale && S.currenttime >= t_out) stop = 1;
-            if (S.trace && S.trace_n < S.trace_cap) {
-                sdmd_gpu_pop_rec &r = S.trace[S.trace_n];
-                r.exec = !sm.stale;
-                r.rand_calls = sm.zpos;
-                int n = 0;
-                for (int k = 1; sm.renew[k] && n < 2; k++, n++) {
-                    const int a = sm.renew[k];
-                    r.r[n].atom = a; r.r[n].partner = G(S.evp)[a]; r.r[n].type = G(S.evtype)[a];
-                    r.r[n].sub = G(S.evsub)[a]; r.r[n].counter = G(S.evc)[a]; r.r[n].pcounter = G(S.evpc)[a];
-                    r.r[n].time = G(S.evt)[a]; r.r[n].pot = G(S.evpot)[a];
+            if (lane == 0) {
+                S.pops++;
+                S.last_exec = !sm.stale;
+                if (!sm.stale && S.currenttime >= t_out) stop = 1;
+                if (S.trace && S.trace_n < S.trace_cap) {
+                    sdmd_gpu_pop_rec &r = S.trace[S.trace_n];
+                    r.exec = !sm.stale;
+                    r.rand_calls = sm.zpos;
+                    int n = 0;
+                    for (int k = 1; sm.renew[k] && n < 2; k++, n++) {
+                        const int a = sm.renew[k];
+                        r.r[n].atom = a; r.r[n].partner = G(S.evp)[a]; r.r[n].type = G(S.evtype)[a];
+                        r.r[n].sub = G(S.evsub)[a]; r.r[n].counter = G(S.evc)[a]; r.r[n].pcounter = G(S.evpc)[a];
+                        r.r[n].time = G(S.evt)[a]; r.r[n].pot = G(S.evpot)[a];
+                    }
+                    r.nrenew = n;
+                    S.trace_n++;
                 }
-                r.nrenew = n;
-                S.trace_n++;
+                if (S.hash_every > 0 && S.pops % S.hash_every == 0 && S.hash_n < S.hash_cap) {
+                    G(S.hashes)[2 * S.hash_n] = S.pops;
+                    G(S.hashes)[2 * S.hash_n + 1] = (long long)state_hash(S);
+                    S.hash_n++;
+                }
             }
-            if (S.hash_every > 0 && S.pops % S.hash_every == 0 && S.hash_n < S.hash_cap) {
-                G(S.hashes)[2 * S.hash_n] = S.pops;
-                G(S.hashes)[2 * S.hash_n + 1] = (long long)state_hash(S);
-                S.hash_n++;
-            }
+            wave_sync();
         }
-        __syncthreads();
     }
+    __syncthreads();
+    if (sm.nlog) sweep<B>(S, sm);
     if (tid == 0) {
         S.zpos = sm.zpos;
         if (sm.err) S.error = sm.err;
     }
     sys_store<B>(&systems[blockIdx.x], Sl);
+}
+
+// cell arrays from the lists, for every cell of every system
+__global__ __launch_bounds__(256) void k_cells(const Sys *systems) {
+    const Sys &S = systems[blockIdx.x];
+    const int N = S.N, ncell = S.cellnum[1] * S.cellnum[2] * S.cellnum[3];
+    for (int c = 1 + blockIdx.y * 256 + threadIdx.x; c <= ncell; c += 256 * gridDim.y) {
+        int cnt = 0;
+        for (int j = G(S.celllist)[N + c]; j && cnt <= N; j = G(S.celllist)[j]) cnt++;
+        G(S.ccnt)[c] = cnt;
+        if (cnt > CELL_CAP) continue;
+        int q = cnt - 1;
+        for (int j = G(S.celllist)[N + c]; j && q >= 0; j = G(S.celllist)[j]) G(S.cmem)[(size_t)c * CELL_CAP + q--] = j;
+    }
 }
 
 // single operations behind the fine-grained entry points
@@ -955,10 +1472,11 @@ __global__ __launch_bounds__(B) void k_op(Sys *systems, int sys, int op, const i
     sys_load<B>(Sl, &systems[sys]);
     Sys &S = Sl;
     const int tid = threadIdx.x;
-    if (tid == 0) { sm.err = 0; sm.zpos = S.zpos; }
+    if (tid == 0) { sm.err = 0; sm.zpos = S.zpos; sm.nlog = 0; }
     __syncthreads();
+    if (op == OP_CREATE_TREE) cbt_create<B>(S);
     if (op == OP_PREDICT) {
-        predict_list<B>(S, sm, renew);
+        predict_list<B, false>(S, sm, nullptr, renew);
     } else if (op == OP_ADVANCE) {
         for (int i = tid + 1; i <= S.N; i += B) {
             G(S.x)[i] += G(S.vx)[i] * dt;
@@ -970,8 +1488,7 @@ __global__ __launch_bounds__(B) void k_op(Sys *systems, int sys, int op, const i
         if (tid == 0) S.currenttime += dt;
     } else if (tid == 0) {
         int err = 0;
-        if (op == OP_CREATE_TREE) cbt_create(S);
-        else if (op == OP_UPDATE_TREE) { for (int k = 1; renew[k]; k++) cbt_update_run(S, renew[k]); }
+        if (op == OP_UPDATE_TREE) { for (int k = 1; renew[k]; k++) cbt_update_run(S, renew[k]); }
         else if (op == OP_DO_EVENT) {
             // SingleThreadRun, SGThread.c:100-104
             S.frame++;
@@ -994,6 +1511,22 @@ __global__ __launch_bounds__(B) void k_op(Sys *systems, int sys, int op, const i
 using namespace sdmd;
 
 // ==================================================================== host side
+// The words of a staged Atom in the order of its first NGATHER members:
+// device address of the word for atom 0 and its stride from atom to atom.
+static void atom_gather_table(Sys *S) {
+    int w = 0;
+    auto word = [&](const int *p, int stride) { S->gbase[w] = p; S->gstride[w] = stride; w++; };
+    auto wide = [&](const void *p) { word((const int *)p, 2); word((const int *)p + 1, 2); };
+    for (const double *p : {S->x, S->y, S->z, S->vx, S->vy, S->vz}) wide(p);
+    wide(S->evc); wide(S->evt); wide(S->evpot); wide(S->evpc);
+    for (const int *p : {S->cx, S->cy, S->cz, S->type, S->hbbond, S->hbnb, S->protein, S->aanum, S->nbstat, S->nbnum})
+        word(p, 1);
+    for (int k = 0; k < SDMD_NBSLOTS; k++) word(S->nbp + k, SDMD_NBSLOTS);
+    for (const int *p : {S->evp, S->evtype, S->evsub, S->hbitype}) word(p, 1);
+    for (const int *p : {S->cmap_off, S->bond_off, S->con_off}) { word(p, 1); word(p + 1, 1); }
+    word(S->leaf, 1);
+}
+
 static int upload_system(sdmd_gpu_ctx *c, Sys *S, const sdmd_system_desc *d, const sdmd_gpu_opts *o) {
     memset(S, 0, sizeof *S);
     const int N = d->natom;
@@ -1052,6 +1585,49 @@ static int upload_system(sdmd_gpu_ctx *c, Sys *S, const sdmd_system_desc *d, con
     UP(node, (const int *)nullptr, 2 * N1);
     UP(leaf, (const int *)nullptr, N1 + 1);
     S->win = (o && o->window > 0) ? o->window : MAXC;
+    if (!o || o->mode == SDMD_MODE_PLAIN) {
+        // the plain engine's derived tables: cell arrays (filled by k_cells),
+        // pops each atom has taken, the constraint entry of each connection
+        // row entry (the first of its partner, as FindPair finds it), the
+        // collision table with RightPair resolved (ToolFunctions.c:278-292)
+        const size_t ncell = (size_t)d->cellnum[0] * d->cellnum[1] * d->cellnum[2];
+        UP(ccnt, (const int *)nullptr, ncell + 1);
+        UP(cmem, (const int *)nullptr, (ncell + 1) * CELL_CAP);
+        UP(lag, (const unsigned char *)nullptr, N1);
+        int *cc = (int *)malloc(sizeof(int) * (size_t)(ncm > 0 ? ncm : 1));
+        if (!cc) return SDMD_ENOMEM;
+        for (int a = 1; a <= N; a++)
+            for (int k = d->cmap_off[a]; k < d->cmap_off[a + 1]; k++) {
+                cc[k] = -1;
+                if (!(d->cmap_bits[k] & SDMD_CONSTRAINT_CONNECT)) continue;
+                for (int q = d->con_off[a]; q < d->con_off[a + 1]; q++)
+                    if (d->con_j[q] == d->cmap_j[k]) { cc[k] = q; break; }
+            }
+        rc = dev_upload(c, &S->cmap_con, cc, (size_t)ncm);
+        free(cc);
+        if (rc) return rc;
+        sdmd_pair rp[NT * NT];
+        auto back = [](int t) { return t == 3 ? 1 : t == 4 ? 2 : t == 27 ? 26 : t; };
+        int pool = 0, most = 0;
+        for (int t1 = 0; t1 < NT; t1++)
+            for (int t2 = 0; t2 < NT; t2++) {
+                const int a = back(t1), b = back(t2);
+                const int cand[4] = {t1 * NT + t2, a * NT + t2, t1 * NT + b, a * NT + b};
+                sdmd_pair p = {0, 0, 0, 0};
+                for (int q = 3; q >= 0; q--)
+                    if (d->pair[cand[q]].dmin > 0) p = d->pair[cand[q]];
+                rp[t1 * NT + t2] = p;
+                pool = p.step0 + p.nstep > pool ? p.step0 + p.nstep : pool;
+                most = p.nstep > most ? p.nstep : most;
+            }
+        UP(rpair, (const sdmd_pair *)rp, (size_t)NT * NT);
+        S->ltab = (S->steps_sorted && pool > 0 && pool <= LPOOL && most <= 16) ? pool : 0;
+        // a sweep of all atoms every logk pops: rare for large systems (its
+        // memory traffic), frequent for small ones (an atom read late takes
+        // the steps it lacks one by one, about 20 ns each)
+        S->logk = N / 64 < 8 ? 8 : (N / 64 > LOGK ? LOGK : N / 64);
+        atom_gather_table(S);
+    }
     if (o && o->trace) {
         S->trace_cap = o->trace_capacity > 0 ? o->trace_capacity : 100000;
         UP(trace, (const sdmd_gpu_pop_rec *)nullptr, (size_t)S->trace_cap);
@@ -1131,6 +1707,10 @@ extern "C" int sdmd_gpu_open(const sdmd_system_desc *const *systems, int32_t nsy
         rc = dev_upload(c, &c->epart, (const double *)nullptr, (size_t)3 * nsys * c->echunks);
     }
     if (rc == SDMD_OK) rc = sync_to_device(c);
+    if (rc == SDMD_OK && mode == SDMD_MODE_PLAIN) {
+        hipLaunchKernelGGL(k_cells, dim3(nsys, 64), dim3(256), 0, c->stream, c->dev_sys);
+        rc = hip_ok(hipGetLastError());
+    }
     if (rc == SDMD_OK) rc = hip_ok(hipStreamSynchronize(c->stream));
     if (rc == SDMD_OK && mode == SDMD_MODE_FAST) rc = sdmd_fast_open(c, opts);
     if (rc != SDMD_OK) { sdmd_gpu_close(c); return rc; }
