@@ -528,34 +528,56 @@ static __device__ __forceinline__ float lane_get(float v, int L) {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), L));
 }
 
-template <int S>
-static __device__ __forceinline__ void argmin_step(double &t, int &k) {
-    unsigned long long ta, tb;
-    unsigned ka, kb;
-    xpair64<S>((unsigned long long)__double_as_longlong(t), ta, tb);
-    xpair<S>((unsigned)k, ka, kb);
-    const double t1 = __longlong_as_double((long long)ta), t2 = __longlong_as_double((long long)tb);
-    const int k1 = (int)ka, k2 = (int)kb;
-    const bool two = t2 < t1 || (t2 == t1 && k2 < k1);
-    t = two ? t2 : t1;
-    k = two ? k2 : k1;
+// the wave's smallest unsigned word: six DPP minima (row shifts, then the
+// rows' last lanes into the following rows), the result in lane 63
+static __device__ __forceinline__ unsigned wave_umin(unsigned v) {
+    v = min(v, (unsigned)__builtin_amdgcn_update_dpp(-1, (int)v, 0x111, 0xF, 0xF, false));   // row_shr:1
+    v = min(v, (unsigned)__builtin_amdgcn_update_dpp(-1, (int)v, 0x112, 0xF, 0xF, false));   // row_shr:2
+    v = min(v, (unsigned)__builtin_amdgcn_update_dpp(-1, (int)v, 0x114, 0xF, 0xF, false));   // row_shr:4
+    v = min(v, (unsigned)__builtin_amdgcn_update_dpp(-1, (int)v, 0x118, 0xF, 0xF, false));   // row_shr:8
+    v = min(v, (unsigned)__builtin_amdgcn_update_dpp(-1, (int)v, 0x142, 0xA, 0xF, false));   // row_bcast:15
+    v = min(v, (unsigned)__builtin_amdgcn_update_dpp(-1, (int)v, 0x143, 0xC, 0xF, false));   // row_bcast:31
+    return (unsigned)__builtin_amdgcn_readlane((int)v, 63);
 }
-// the wave's smallest (t, k), smallest k on equal t, in every lane
+// A double's order as two unsigned words (no NaN): the high words alone
+// decide unless several lanes share the smallest one, so a reduction costs
+// about 15 instructions instead of 80 for a butterfly on pairs.
+static __device__ __forceinline__ void order_words(double t, unsigned &hi, unsigned &lo) {
+    const unsigned long long b = (unsigned long long)__double_as_longlong(t);
+    const unsigned s = (unsigned)((int)(b >> 32) >> 31);
+    hi = (unsigned)(b >> 32) ^ (s | 0x80000000u);
+    lo = (unsigned)b ^ s;
+}
+// lanes that hold the wave's smallest t
+static __device__ __forceinline__ unsigned long long wave_min_lanes(double t) {
+    unsigned hi, lo;
+    order_words(t, hi, lo);
+    unsigned long long m = __ballot(hi == wave_umin(hi));
+    if (m & (m - 1)) {
+        const bool in = (m >> (threadIdx.x & 63)) & 1;
+        m &= __ballot(lo == wave_umin(in ? lo : 0xffffffffu));
+    }
+    return m;
+}
+// lane of the wave's smallest t, the lowest one on equal t
+static __device__ __forceinline__ int wave_first_min(double t) { return __ffsll((long long)wave_min_lanes(t)) - 1; }
+// the wave's smallest (t, k), smallest k >= 0 on equal t, in every lane
 static __device__ __forceinline__ void wave_argmin(double &t, int &k) {
-    argmin_step<0>(t, k); argmin_step<1>(t, k); argmin_step<2>(t, k);
-    argmin_step<3>(t, k); argmin_step<4>(t, k); argmin_step<5>(t, k);
-    t = lane_get(t, 0);
-    k = lane_get(k, 0);
+    unsigned long long m = wave_min_lanes(t);
+    if (m & (m - 1)) {
+        const bool in = (m >> (threadIdx.x & 63)) & 1;
+        m &= __ballot((unsigned)k == wave_umin(in ? (unsigned)k : 0xffffffffu));
+    }
+    const int src = __ffsll((long long)m) - 1;
+    t = lane_get(t, src);
+    k = lane_get(k, src);
 }
-template <int S>
-static __device__ __forceinline__ void dmin_step(double &t) {
-    unsigned long long a, b;
-    xpair64<S>((unsigned long long)__double_as_longlong(t), a, b);
-    t = fmin(__longlong_as_double((long long)a), __longlong_as_double((long long)b));
-}
-static __device__ __forceinline__ double wave_min_d(double t) {
-    dmin_step<0>(t); dmin_step<1>(t); dmin_step<2>(t); dmin_step<3>(t); dmin_step<4>(t); dmin_step<5>(t);
-    return lane_get(t, 0);
+static __device__ __forceinline__ double wave_min_d(double t) { return lane_get(t, wave_first_min(t)); }
+// LDS written by some lanes of a wave, read next by others of the same wave:
+// the wave's LDS operations run in order, so only the compiler is held
+static __device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
 }
 template <int S>
 static __device__ __forceinline__ void or_step(unsigned long long &m) {

@@ -42,6 +42,8 @@
 // FP64 is kept for the clock, the confirmed pair times, the grazing cases
 // and the velocity updates (InteractionEvent, Events.c:798-1024).
 
+#include <cstddef>
+
 #include "sdmd_dev.h"
 
 namespace sdmd {
@@ -52,8 +54,7 @@ constexpr int FCAP_MIN = 64;      // slots per cell at least (a system's capacit
 constexpr int FCAP_MAX = 1024;    // ... at most
 constexpr int FMAXBLK = 1024;     // 64-atom blocks per system (N <= 65535)
 constexpr int FSEL = 64;          // events considered per round
-constexpr int FROW = 96;          // connection-map row staged per wave
-constexpr int FMAXW = 16;         // wavefronts per workgroup
+constexpr int FMAXW = 16;         // wavefronts per workgroup at most
 constexpr long long FDRAIN = 1 << 20;   // bound on the pops of a closing drain
 constexpr float FINF = 3.0e38f;
 
@@ -72,6 +73,8 @@ enum { FPH_SELECT, FPH_EXEC, FPH_STAGE, FPH_SCREEN, FPH_CONFIRM, FPH_OTHER, FPH_
 
 // step radii (squared, FP32) of one constraint entry and bit k set when
 // step k carries no energy
+constexpr int PROW = 16;          // steps per collision pair at most
+
 struct __attribute__((aligned(16))) ConRad {
     float rad[8];
     unsigned int ez;
@@ -93,6 +96,10 @@ struct FSys {
     int *bj16;
     double *blo16, *bhi16;
     struct ConRad *crad;
+    // FP64 shells at a fixed stride, read at a known shell without a
+    // dependent load: dmin, dmax, the radii, the energies
+    double *prow;               // [NT*NT][2 + 2 * PROW] by resolved collision pair
+    double *crow;               // [constraint entry][2 + 2 * FCONSTEP]
     int ncell, nblk;
     float L32[3];
     double Te, rebase_dt;
@@ -119,19 +126,39 @@ __device__ __forceinline__ void philox10(unsigned int c[4], unsigned int k0, uns
     }
 }
 
-// draw number `ctr` of atom a (the caller holds the atom's counter)
-__device__ double fast_normal_at(FSys &F, int a, unsigned int ctr) {
-    unsigned int c[4] = {(unsigned int)a, ctr, 0x5344u, 0x4d44u};
-    G(F.rctr)[a] = ctr + 1;
+// the four words of draw number `ctr` of atom a
+__device__ __forceinline__ void normal_words(const FSys &F, int a, unsigned int ctr, unsigned int c[4]) {
+    c[0] = (unsigned int)a; c[1] = ctr; c[2] = 0x5344u; c[3] = 0x4d44u;
     philox10(c, F.key0, F.key1);
-    const unsigned long long w1 = ((unsigned long long)c[0] << 32) | c[1];
-    const unsigned long long w2 = ((unsigned long long)c[2] << 32) | c[3];
+}
+// the standard normal of those words
+__device__ double normal_of(unsigned int c0, unsigned int c1, unsigned int c2, unsigned int c3) {
+    const unsigned long long w1 = ((unsigned long long)c0 << 32) | c1;
+    const unsigned long long w2 = ((unsigned long long)c2 << 32) | c3;
     const double u1 = ((double)(w1 >> 11) + 0.5) * 0x1.0p-53;
     const double u2 = ((double)(w2 >> 11) + 0.5) * 0x1.0p-53;
     return sqrt(-2.0 * log(u1)) * cos(6.283185307179586 * u2);
 }
+// A lower bound of the normal's absolute value in FP32: u1 is rounded up
+// (the logarithm's magnitude down), the logarithm and the cosine give up
+// 1e-5 (their hardware errors and that of u2's rounding are below 2e-6).
+// The FP64 normal takes about 400 dependent instructions on one lane; a
+// thermostat time beyond the earliest event is dismissed without it (all but
+// about 1 % of the predictions).
+__device__ __forceinline__ float normal_floor(unsigned int c0, unsigned int c2) {
+    const float u1 = fmaf((float)c0, 1.000001f, 1.f) * 0x1.0p-32f;
+    const float l = -1.3862944f * __builtin_amdgcn_logf(u1) - 1e-5f;        // -2 ln u1
+    const float c = fabsf(__builtin_amdgcn_cosf((float)c2 * 0x1.0p-32f)) - 1e-5f;
+    return (l > 0 && c > 0) ? 0.99999f * __builtin_amdgcn_sqrtf(l) * c : 0.f;
+}
 
-__device__ double fast_normal(FSys &F, int a) { return fast_normal_at(F, a, G(F.rctr)[a]); }
+__device__ double fast_normal(FSys &F, int a) {
+    const unsigned int ctr = G(F.rctr)[a];
+    unsigned int c[4];
+    normal_words(F, a, ctr, c);
+    G(F.rctr)[a] = ctr + 1;
+    return normal_of(c[0], c[1], c[2], c[3]);
+}
 
 // ---------------------------------------------------------------- shared counters
 // Several wavefronts update the system's counters (held in LDS) at once.
@@ -211,18 +238,21 @@ __device__ void put_record(FSys &F, int a) {
 }
 
 // ---------------------------------------------------------------- predicted atom
+// The first members are loaded by one wavefront, one per lane: lanes 0..6
+// eight bytes each, lanes 7..31 four (ScrTab's gather map).
 struct FAtom {
-    double x, y, z, vx, vy, vz, t;
+    double x, y, z, vx, vy, vz;
     long long counter;
-    int i, cx, cy, cz, type, hbbond, hbnb, protein, aanum, nbstat, nbnum, nrow, rowlo, rowhi;
-    int spanok;                  // the static row spans < 128 atom ids: bitmask lookup
-    int ncon, constaged;         // constraint partners; all staged in LDS
-    unsigned long long mb[2], mc[2];   // BOND / CONSTRAINT bits over rowlo .. rowlo+127
     unsigned int rctr;           // its thermostat draw counter
-    signed char role;
+    int cx, cy, cz, type, hbbond, hbnb, protein, aanum, nbstat, nbnum;
     int nbp[SDMD_NBSLOTS];
-    fvec4 s0, s1;            // the atom's own mirror record (position at t, velocity)
+    int pad23, ro, ro1, bo, bo1, co, co1, hbit, pad31;   // cmap_off, bond_off, con_off at i and i + 1
+    double t;
+    int i, role, rowlo, ncon;
+    int spanok;                  // the static row spans < 128 atom ids: byte lookup
+    float s0[3], s1[3];          // the atom's own mirror record (position at t, velocity)
 };
+static_assert(offsetof(FAtom, rctr) == 56 && offsetof(FAtom, pad31) == 56 + 4 * 24, "lane map of the gather");
 
 // statistics accumulated per wave, added to the system at the end
 struct WStats { long long screen, conf, fp64, cand; };
@@ -245,64 +275,58 @@ __device__ __forceinline__ void take(Best &B, const Sys &S, double t, double pot
 constexpr int FCON = 16;          // constraint partners staged per predicted atom
 constexpr int FCONSTEP = 8;       // steps per staged constraint
 
+// Per-wavefront LDS.  NL: candidates inside the scan radius listed for the
+// screen (25 to 60 at most sizes; a longer list takes the unlisted path).
+template <int NL>
 struct FWave {
+    static constexpr int LIST = NL;
     FAtom a;                     // the atom being predicted (uniform across the wave)
     union {
         // its bonded partners' states (lanes 32..47 stage bond q = lane - 32)
         struct {
             double bxj[16], byj[16], bzj[16], bvx[16], bvy[16], bvz[16], bt0[16], blo[16], bhi[16];
         };
-        // after the bond phase: the free H-bond scan's candidates that pass
-        // its cheap conditions (atom id and candidate index), 128 at a time
+        // after the bond phase: the candidates inside the scan radius, in
+        // candidate order; first their kinematics, then the screen's result
         struct {
-            int hbl_j[128], hbl_k[128];
+            float l_rr[NL], l_b[NL], l_v2[NL];
+        };
+        struct {
+            float l_t[NL], l_e[NL];              // time, error bound (negative: FP64 decides)
+            int l_sh[NL];                        // shell (low byte), constraint slot + 1
         };
     };
+    int l_id[NL];                // atom id << 8 | type, as in the mirror record
+    int l_k[NL];                 // candidate index; bit 31: its local time is later than the reader's
     long long bcj[16];
     int bjj[16];
-    int row_j[FROW], row_b[FROW];
-    int dyn_j[SDMD_DYNSLOTS], dyn_b[SDMD_DYNSLOTS];
     int coff[28];
     int cell[27];
     fvec4 cof[27];               // neighbour cell c's offset times the cell size (x, y, z)
     // the predicted atom's constraint shells (FP32), CONSTRn lists
-    int con_j[FCON], con_nstep[FCON];
+    int con_nstep[FCON];
     unsigned int con_ez[FCON];
     float con_dmin[FCON], con_dmax[FCON];
     float con_rad[FCON][FCONSTEP];
-    int hbl_n;                   // candidates in hbl_j / hbl_k from the screen, -1: none listed
-    unsigned char conidx[128];   // constraint slot + 1 of the partner at row offset j - rowlo (0: none)
+    int hbl_n;                   // entries of l_id / l_k left by the screen, -1: none listed
+    // connection row by offset from its first column: bits 0-1 BOND and
+    // CONSTRAINT, bits 2-6 the constraint's slot + 1 (0: not staged)
+    unsigned char conn[128];
     WStats st;                   // the wavefront's statistics (wave-uniform updates)
 };
-
-__device__ __forceinline__ int frow_bits(const FWave &wm, const Sys &S, const FAtom &A, int j) {
-    int bits = 0;
-    if (A.nrow <= FROW) {
-        int lo = 0, hi = (j < A.rowlo || j > A.rowhi) ? -1 : A.nrow - 1;   // outside the row's span: absent
-        while (lo <= hi) {
-            const int m = (lo + hi) >> 1;
-            const int v = wm.row_j[m];
-            if (v == j) { bits = wm.row_b[m]; break; }
-            if (v < j) lo = m + 1; else hi = m - 1;
-        }
-        for (int k = 0; k < SDMD_DYNSLOTS; k++)
-            if (wm.dyn_j[k] == j) { bits |= wm.dyn_b[k]; break; }
-        return bits;
-    }
-    return cmap_get(S, A.i, j);
-}
+// the list's length by workgroup size (the LDS of a CU holds it all)
+constexpr int flist(int W) { return W <= 8 ? 256 : 128; }
 
 // BOND / CONSTRAINT bits of (A, j), the only connection bits CollisionTime
-// tests (TimePrediction.c:96-118); the dynamic slots carry H-bond bits only
-__device__ __forceinline__ int coli_bits(const FWave &wm, const Sys &S, const FAtom &A, int j) {
+// tests (TimePrediction.c:96-118), with the staged constraint's slot; the
+// dynamic slots carry H-bond bits only
+template <class FW>
+__device__ __forceinline__ int coli_bits(const FW &wm, const Sys &S, const FAtom &A, int j) {
     if (A.spanok) {
         const unsigned off = (unsigned)(j - A.rowlo);
-        if (off >= 128u) return 0;
-        const int w = off >> 6, sh = off & 63;
-        const unsigned long long mb = w ? A.mb[1] : A.mb[0], mc = w ? A.mc[1] : A.mc[0];
-        return (int)((mb >> sh) & 1) * SDMD_BOND_CONNECT | (int)((mc >> sh) & 1) * SDMD_CONSTRAINT_CONNECT;
+        return off < 128u ? wm.conn[off] : 0;
     }
-    return frow_bits(wm, S, A, j) & (SDMD_BOND_CONNECT | SDMD_CONSTRAINT_CONNECT);
+    return cmap_get(S, A.i, j) & (SDMD_BOND_CONNECT | SDMD_CONSTRAINT_CONNECT);
 }
 
 __device__ __forceinline__ int fin_nb_list(const FAtom &A, int j) {
@@ -368,7 +392,7 @@ __device__ double coli64(const FSys &F, const FAtom &A, int j, int bits, int rp,
 
 // FP32 screen of one collision candidate: time t with absolute error bound e,
 // or flag when a decision lies inside the error band (FP64 decides then)
-struct Scr { float t, e; bool flag; };
+struct Scr { float t, e; bool flag; int ks; };    // ks: radii passed (the shell), valid unless flagged
 
 // One shell description for the screen: hard core, step radii, outer
 // limit (all squared), and bit k set when step k carries no energy.
@@ -388,7 +412,7 @@ __device__ __forceinline__ float frcp(float x) { return __builtin_amdgcn_rcpf(x)
 template <class R>
 __device__ __forceinline__ Scr screen_shell(const Shell &c, const R &rad, bool con, float rr, float b, float v2) {
     Scr o;
-    o.t = FINF; o.e = 0; o.flag = false;
+    o.t = FINF; o.e = 0; o.flag = false; o.ks = 0;
     const float band = 2e-5f * rr + 1e-5f;
     if (rr < c.dmin + band) { o.flag = true; return o; }   // core boundary or inside the core
     // count the radii passed (no early exit; four radii read at a time with
@@ -415,6 +439,7 @@ __device__ __forceinline__ Scr screen_shell(const Shell &c, const R &rad, bool c
         }
     }
     if (near) { o.flag = true; return o; }
+    o.ks = ks;
     const bool lopot0 = ks ? ((c.ezero >> (ks - 1)) & 1) : true;
     bool hipot0;
     int cs;
@@ -464,7 +489,8 @@ __device__ __forceinline__ Scr screen_shell(const Shell &c, const R &rad, bool c
 }
 
 // compact FP32 copy of the collision table (RightPair resolved), held in LDS
-constexpr int FRAD = 8192;
+constexpr int FRAD = 8192;        // steps of the defined pairs' lists in all at most
+constexpr int FRADL = 2048;       // ... in the pool (equal lists stored once); the other pairs go to FP64
 // indexed by (type_i, type_j) directly: the entry of the resolved pair,
 // with that pair's index (one LDS read per candidate)
 struct ScrPair {
@@ -477,7 +503,7 @@ struct ScrPair {
 static_assert(sizeof(ScrPair) == 16, "one 16-byte LDS read per screen table entry");
 struct ScrTab {
     ScrPair pr[NT * NT];
-    float rad[FRAD];
+    float rad[FRADL];
     // per-lane gather map of a predicted atom's fields: lane L loads the
     // 4-byte words gbase[L] + i*gstride[L] + goff[L] (+ gtwo[L]) of atom i
     unsigned long long gbase[64];
@@ -485,26 +511,20 @@ struct ScrTab {
 };
 
 // ---------------------------------------------------------------- wave helpers
-template <int S>
-__device__ __forceinline__ void fmin_step(float &t) {
-    unsigned a, b;
-    xpair<S>(__float_as_uint(t), a, b);
-    t = fminf(__uint_as_float(a), __uint_as_float(b));
-}
-__device__ __forceinline__ float wave_min_f(float t) {
-    fmin_step<0>(t); fmin_step<1>(t); fmin_step<2>(t); fmin_step<3>(t); fmin_step<4>(t); fmin_step<5>(t);
-    return lane_get(t, 0);
+__device__ __forceinline__ float wave_min_f(float t) {     // no NaN
+    const unsigned b = __float_as_uint(t), s = (unsigned)((int)b >> 31);
+    const unsigned m = wave_umin(b ^ (s | 0x80000000u));
+    return __uint_as_float(m ^ ((m >> 31) ? 0x80000000u : 0xffffffffu));
 }
 
-template <int S>
-__device__ __forceinline__ void isum_step(int &v) {
-    unsigned a, b;
-    xpair<S>((unsigned)v, a, b);
-    v = (int)(a + b);
-}
 __device__ __forceinline__ int wave_sum_i(int v) {
-    isum_step<0>(v); isum_step<1>(v); isum_step<2>(v); isum_step<3>(v); isum_step<4>(v); isum_step<5>(v);
-    return lane_get(v, 0);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, false);     // row_shr:1
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, false);     // row_shr:2
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, false);     // row_shr:4
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, false);     // row_shr:8
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false);     // row_bcast:15
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false);     // row_bcast:31
+    return lane_get(v, 63);
 }
 
 // broadcast a Best from lane src (uniform) to the wave
@@ -562,59 +582,40 @@ __device__ __forceinline__ int rl32(int v, int L) { return __builtin_amdgcn_read
 // radii, and the 27 cells' occupancy.  Every load of a level is issued by
 // all lanes (indices clamped into range, results masked afterwards), so a
 // level costs one memory latency.
-__device__ __forceinline__ void fstage(FSys &F, const ScrTab &T, FWave &wm, FAtom &A, int i, double t, int &nb) {
+template <class FW>
+__device__ __forceinline__ void fstage(FSys &F, const ScrTab &T, FW &wm, FAtom &A, int i, double t, int &nb) {
     const Sys &S = F.s;
     const int lane = threadIdx.x & 63;
     i = uni(i);
     t = uni(t);
-    // ---- level 1 (lane map of the host's gather table): 0-5 x y z vx vy
-    // vz, 6 event counter (two words), 7 thermostat draw counter; 8-16 cx cy cz type hbbond hbnb
-    // protein aanum nbstat, 17 nbnum, 18-22 neighbour slots, 24-29
-    // cmap/bond/con offsets at i and i+1, 32-39 dynamic slot atoms, 40-47
-    // their bits, 48-63 bonded partners; the role byte is loaded by every lane
-    static_assert(SDMD_NBSLOTS == 5 && SDMD_DYNSLOTS == 8 && FCONSTEP == 8, "lane map of the level-1 gather");
+    // ---- level 1 (lane map of the host's gather table): the members of
+    // FAtom, lanes 48-63 the bonded partners; the role byte is loaded by
+    // every lane
+    static_assert(SDMD_NBSLOTS == 5 && FCONSTEP == 8, "lane map of the level-1 gather");
     const int *gp = (const int *)T.gbase[lane] + (size_t)i * T.gstride[lane] + T.goff[lane];
     const int lo = G(gp)[0], hi = G(gp)[T.gtwo[lane]];
-    const int role = uni((int)G(S.role)[i]);
+    const int role = G(S.role)[i];
     const long long w = (long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo);
-    const double ax = __longlong_as_double(rl64(w, 0)), ay = __longlong_as_double(rl64(w, 1));
-    const double az = __longlong_as_double(rl64(w, 2)), avx = __longlong_as_double(rl64(w, 3));
-    const double avy = __longlong_as_double(rl64(w, 4)), avz = __longlong_as_double(rl64(w, 5));
     const int cx = rl32(lo, 8), cy = rl32(lo, 9), cz = rl32(lo, 10);
     const int o = rl32(lo, 24), nrow = rl32(lo, 25) - o;
-    const int bo = rl32(lo, 26);
-    nb = rl32(lo, 27) - bo;
+    nb = rl32(lo, 27) - rl32(lo, 26);
     const int co = rl32(lo, 28), ncon = rl32(lo, 29) - co;
-    if (lane == 0) {
-        A.i = i; A.t = t;
-        A.x = ax; A.y = ay; A.z = az; A.vx = avx; A.vy = avy; A.vz = avz;
-        A.counter = rl64(w, 6);
-        A.cx = cx; A.cy = cy; A.cz = cz;
-        A.type = rl32(lo, 11); A.hbbond = rl32(lo, 12); A.hbnb = rl32(lo, 13);
-        A.protein = rl32(lo, 14); A.aanum = rl32(lo, 15); A.nbstat = rl32(lo, 16); A.nbnum = rl32(lo, 17);
-        A.role = (signed char)role;
-        A.rctr = (unsigned int)rl32(lo, 7);
-        A.nrow = nrow;
-        A.ncon = ncon;
-    }
-    for (int k = 0; k < SDMD_NBSLOTS; k++) {
-        const int v = rl32(lo, 18 + k);
-        if (lane == 0) A.nbp[k] = v;
-    }
-    {
-        // lanes 0..7 take lanes 32..39 (half-wave swap) and 40..47 (then 8
-        // lanes down the row)
-        const auto sw = __builtin_amdgcn_permlane32_swap((unsigned)lo, (unsigned)lo, false, false);
-        const int dj = (int)sw[1];
-        const int db = __builtin_amdgcn_update_dpp(0, dj, 0x108, 0xF, 0xF, false);     // row_shl:8
-        if (lane < SDMD_DYNSLOTS) { wm.dyn_j[lane] = dj; wm.dyn_b[lane] = db; }
+    if (lane < 7) ((long long *)&A)[lane] = w;
+    else if (lane < 32) ((int *)&A.rctr)[lane - 7] = lo;
+    if (lane < 3) {
+        // own mirror record, as put_record writes it for a state at time t
+        const int c = lane == 0 ? cx : lane == 1 ? cy : cz;
+        A.s0[lane] = (float)(__longlong_as_double(w) - c * S.cellsize[lane + 1]);
+    } else if (lane < 6) {
+        A.s1[lane - 3] = (float)__longlong_as_double(w);
+    } else if (lane == 6) {
+        A.i = i; A.t = t; A.role = role; A.ncon = ncon;
     }
     // ---- level 2
-    int rj0 = 0, rb0 = 0, rj1 = 0, rb1 = 0;
+    int rj = 0, rb = 0, rc = 0;
     if (nrow > 0) {
-        const int k0 = o + min(lane, nrow - 1), k1 = o + min(lane + 64, nrow - 1);
-        rj0 = G(S.cmap_j)[k0]; rb0 = G(S.cmap_bits)[k0];
-        rj1 = G(S.cmap_j)[k1]; rb1 = G(S.cmap_bits)[k1];
+        const int k0 = o + min(lane, nrow - 1);
+        rj = G(S.cmap_j)[k0]; rb = G(S.cmap_bits)[k0]; rc = G(S.cmap_con)[k0];
     }
     // bond q on lane 32 + q: its partner id came with level 1 (lane 48 + q)
     const int q = lane - 32;
@@ -629,7 +630,7 @@ __device__ __forceinline__ void fstage(FSys &F, const ScrTab &T, FWave &wm, FAto
         bhi = G(F.bhi16)[qq];
     }
     double cdmin = 0, cdmax = 0;
-    int cnstep = 0, cj = 0;
+    int cnstep = 0;
     float rad[FCONSTEP];
     unsigned int ez = 0;
 #pragma unroll
@@ -639,7 +640,6 @@ __device__ __forceinline__ void fstage(FSys &F, const ScrTab &T, FWave &wm, FAto
         cdmin = G(S.con)[cc].dmin;
         cdmax = G(S.con)[cc].dmax;
         cnstep = G(S.con)[cc].nstep;
-        cj = G(S.con_j)[cc];
         const fvec4 *cv = (const fvec4 *)(F.crad + cc);
         const fvec4 r03 = G(cv)[0], r47 = G(cv)[1];
         rad[0] = r03.x; rad[1] = r03.y; rad[2] = r03.z; rad[3] = r03.w;
@@ -673,86 +673,44 @@ __device__ __forceinline__ void fstage(FSys &F, const ScrTab &T, FWave &wm, FAto
             wm.blo[q] = blo; wm.bhi[q] = bhi;
         }
     }
-    // ---- connection row: bitmasks over its span, or staged in LDS for a
-    // binary search when it spans 128 ids or more
-    const int rowlo = nrow > 0 ? rl32(rj0, 0) : 0x7fffffff;
-    const int rowhi = nrow <= 0 ? -1 : (nrow <= 64 ? rl32(rj0, (nrow - 1) & 63)
-                                         : nrow <= 128 ? rl32(rj1, (nrow - 65) & 63)
-                                                       : uni(G(S.cmap_j)[o + nrow - 1]));
-    const int spanok = (nrow == 0) || (rowhi - rowlo < 128);
+    // ---- connection row as bytes over its span (row and span small enough;
+    // otherwise it is searched in memory), with the slots of the staged
+    // constraint shells (one lane each)
     {
-        unsigned long long mb0 = 0, mb1 = 0, mc0 = 0, mc1 = 0;
-        for (int k = lane; k < nrow; k += 64) {
-            int j, b;
-            if (k < 64) { j = rj0; b = rb0; }
-            else if (k < 128) { j = rj1; b = rb1; }
-            else { j = G(S.cmap_j)[o + k]; b = G(S.cmap_bits)[o + k]; }
-            if (spanok) {
-                const int off = j - rowlo;
-                const unsigned long long bit = 1ull << (off & 63);
-                if (b & SDMD_BOND_CONNECT) { if (off >> 6) mb1 |= bit; else mb0 |= bit; }
-                if (b & SDMD_CONSTRAINT_CONNECT) { if (off >> 6) mc1 |= bit; else mc0 |= bit; }
-            } else if (nrow <= FROW) {
-                wm.row_j[k] = j;
-                wm.row_b[k] = b;
-            }
+        if (lane < 32) ((int *)wm.conn)[lane] = 0;
+        const int rowlo = nrow > 0 ? rl32(rj, 0) : 0, rowhi = nrow > 0 ? rl32(rj, min(nrow, 64) - 1) : 0;
+        const bool spanok = nrow <= 64 && rowhi - rowlo < 128;
+        const unsigned long long fits = __ballot(own_con && cnstep <= FCONSTEP);
+        wave_sync();
+        if (lane < nrow && spanok) {
+            const int slot = rc - co;                       // rc < 0: no constraint
+            const bool staged = rc >= 0 && slot >= 0 && slot < FCON && ((fits >> slot) & 1);
+            wm.conn[rj - rowlo] = (unsigned char)((rb & (SDMD_BOND_CONNECT | SDMD_CONSTRAINT_CONNECT)) |
+                                                  (staged ? (slot + 1) << 2 : 0));
         }
-        mb0 = wave_or64(mb0); mb1 = wave_or64(mb1);
-        mc0 = wave_or64(mc0); mc1 = wave_or64(mc1);
-        if (lane == 0) {
-            A.rowlo = rowlo; A.rowhi = rowhi; A.spanok = spanok;
-            A.mb[0] = mb0; A.mb[1] = mb1; A.mc[0] = mc0; A.mc[1] = mc1;
-        }
-    }
-    // ---- constraint shells (one lane each), and their slots by row offset
-    // when the row spans fewer than 128 ids
-    {
-        int ok = 1;
-        wm.conidx[lane] = 0;
-        wm.conidx[lane + 64] = 0;
-        if (own_con && spanok && cj >= rowlo && cj - rowlo < 128) wm.conidx[cj - rowlo] = (unsigned char)(lane + 1);
+        if (lane == 0) { A.rowlo = rowlo; A.spanok = spanok; }
         if (own_con) {
-            wm.con_j[lane] = cj;
             wm.con_dmin[lane] = (float)cdmin;
             wm.con_dmax[lane] = (float)cdmax;
             wm.con_nstep[lane] = cnstep;
-            if (cnstep <= FCONSTEP) {
-#pragma unroll
-                for (int k = 0; k < FCONSTEP; k++)
-                    if (k < cnstep) wm.con_rad[lane][k] = rad[k];
-            } else {
-                ok = 0;
-                ez = 0;
-            }
             wm.con_ez[lane] = ez;
+#pragma unroll
+            for (int k = 0; k < FCONSTEP; k++) wm.con_rad[lane][k] = rad[k];
         }
-        const int staged = (ncon <= FCON) && !__ballot(!ok);
-        if (lane == 0) A.constaged = staged;
     }
     if (lane < 27) {
         wm.cell[lane] = cell;
-        fvec4 co;
-        co.x = c_OX[lane] * F.L32[0];
-        co.y = c_OY[lane] * F.L32[1];
-        co.z = c_OZ[lane] * F.L32[2];
-        co.w = 0.f;
-        wm.cof[lane] = co;
-    }
-    // own mirror record, as put_record writes it for a state at time t
-    if (lane == 0) {
-        fvec4 s0, s1;
-        s0.x = (float)(ax - cx * S.cellsize[1]);
-        s0.y = (float)(ay - cy * S.cellsize[2]);
-        s0.z = (float)(az - cz * S.cellsize[3]);
-        s0.w = (float)(t - F.Te);
-        s1.x = (float)avx; s1.y = (float)avy; s1.z = (float)avz; s1.w = 0.f;
-        A.s0 = s0;
-        A.s1 = s1;
+        fvec4 co4;
+        co4.x = c_OX[lane] * F.L32[0];
+        co4.y = c_OY[lane] * F.L32[1];
+        co4.z = c_OZ[lane] * F.L32[2];
+        co4.w = 0.f;
+        wm.cof[lane] = co4;
     }
     const int incl = scan32_incl(cnt);
     if (lane < 27) wm.coff[lane + 1] = incl;
     if (lane == 0) wm.coff[0] = 0;
-    __builtin_amdgcn_wave_barrier();
+    wave_sync();
 }
 
 // BondTime entry (TimePrediction.c:219-293) from the staged partner state
@@ -782,7 +740,8 @@ __device__ __forceinline__ double bond64_pre(const FSys &F, const FAtom &A, cons
     return (t > 0) ? t : __builtin_inf();
 }
 
-__device__ __forceinline__ int cand_cell(const FWave &wm, int k) {
+template <class FW>
+__device__ __forceinline__ int cand_cell(const FW &wm, int k) {
     int lo = 0, hi = 26;                 // largest c with coff[c] <= k
     while (lo < hi) {
         const int m = (lo + hi + 1) >> 1;
@@ -791,110 +750,134 @@ __device__ __forceinline__ int cand_cell(const FWave &wm, int k) {
     return lo;
 }
 
-// FP32 screen of candidate k of the staged neighbourhood, from its mirror
-// record (r0, r1) in neighbour cell c
+// kinematics of a candidate from its mirror record (r0, r1) in neighbour
+// cell c, in FP32
+struct Near { float rr, b, v2, dt; };
+template <class FW>
+__device__ __forceinline__ Near near_at(const FW &wm, const FAtom &A, int c, const fvec4 &r0, const fvec4 &r1, float tA) {
+    Near o;
+    o.dt = tA - r0.w;
+    const fvec4 co = wm.cof[c];
+    const float rx = A.s0[0] - (r0.x + r1.x * o.dt) - co.x;
+    const float ry = A.s0[1] - (r0.y + r1.y * o.dt) - co.y;
+    const float rz = A.s0[2] - (r0.z + r1.z * o.dt) - co.z;
+    o.rr = rx * rx + ry * ry + rz * rz;
+    const float vx = A.s1[0] - r1.x, vy = A.s1[1] - r1.y, vz = A.s1[2] - r1.z;
+    o.b = rx * vx + ry * vy + rz * vz;
+    o.v2 = vx * vx + vy * vy + vz * vz;
+    return o;
+}
+
+// FP32 screen of one candidate inside the scan radius
 struct CandS {
     float t, e;       // screened time and its absolute error bound (t = FINF: no event)
     int j, bits;
     int rp;           // resolved collision pair (-1: none or a constraint pair)
+    int ks, slot;     // shell; staged constraint slot (-1: a collision pair)
     bool flag;        // a decision lies in the error band: FP64 decides
-    bool live;        // passed the exclusions and the scan radius
+    bool live;        // passed the exclusions
 };
 
-__device__ __forceinline__ void screen_at(const FSys &F, const ScrTab &T, const FWave &wm, const FAtom &A, int c,
-                                          const fvec4 &r0,
-                                          const fvec4 &r1, const fvec4 &s0, const fvec4 &s1, float tA,
-                                          float calib, float cband, CandS &o, int &causal) {
+template <class FW>
+__device__ __forceinline__ void screen_near(const FSys &F, const ScrTab &T, const FW &wm, const FAtom &A, int id, float rr,
+                                            float b, float v2, float rsafe, CandS &o) {
     const Sys &S = F.s;
-    o.t = FINF; o.e = 0; o.flag = false; o.live = false; o.rp = -1;
-    const int id = __float_as_int(r1.w);
+    o.t = FINF; o.e = 0; o.flag = false; o.live = false; o.rp = -1; o.ks = 0; o.slot = -1;
     const int j = id >> 8, tj = id & 255;
     o.j = j;
-    o.bits = 0;
-    if (j == A.i || j < 1 || j > S.N || tj >= NT) return;
-    const int bits = coli_bits(wm, S, A, j);
-    o.bits = bits;
-    if ((bits & SDMD_BOND_CONNECT) || A.hbbond == j || fin_nb_list(A, j)) return;
-    const float dtj = tA - r0.w;
-    const fvec4 co = wm.cof[c];
-    const float rx = s0.x - (r0.x + r1.x * dtj) - co.x;
-    const float ry = s0.y - (r0.y + r1.y * dtj) - co.y;
-    const float rz = s0.z - (r0.z + r1.z * dtj) - co.z;
-    const float rr = rx * rx + ry * ry + rz * rz;
-    if (rr > calib + cband) return;
+    const int cb = coli_bits(wm, S, A, j);
+    o.bits = cb & (SDMD_BOND_CONNECT | SDMD_CONSTRAINT_CONNECT);
+    if ((cb & SDMD_BOND_CONNECT) || A.hbbond == j || fin_nb_list(A, j)) return;
     o.live = true;
-    causal += (dtj < 0.f) ? 1 : 0;
-    const float vx = s1.x - r1.x, vy = s1.y - r1.y, vz = s1.z - r1.z;
-    const float b = rx * vx + ry * vy + rz * vz, v2 = vx * vx + vy * vy + vz * vz;
-    const bool con = bits & SDMD_CONSTRAINT_CONNECT;
-    Scr sc;
-    if (con && A.constaged) {
-        int q = -1;
-        const int off = j - A.rowlo;
-        if (A.spanok && off >= 0 && off < 128) {
-            q = (int)wm.conidx[off] - 1;
-        } else {
-            for (int k = 0; k < A.ncon; k++)
-                if (wm.con_j[k] == j) { q = k; break; }
-        }
-        if (q < 0) {
-            sc.flag = true; sc.t = FINF; sc.e = 0;
-        } else {
-            Shell c;
-            c.dmin = wm.con_dmin[q]; c.dmax = wm.con_dmax[q]; c.nstep = wm.con_nstep[q]; c.ezero = wm.con_ez[q];
-            const float *rad = wm.con_rad[q];
-            sc = screen_shell(c, [&](int k) { return rad[k]; }, true, rr, b, v2);
-        }
-    } else if (con) {
-        const sdmd_pair *pc = nullptr;
-        for (int q = G(S.con_off)[A.i]; q < G(S.con_off)[A.i + 1]; q++)
-            if (G(S.con_j)[q] == j) { pc = &S.con[q]; break; }
-        if (!pc || pc->nstep > 16) {
-            sc.flag = true; sc.t = FINF; sc.e = 0;
-        } else {
-            Shell c;
-            c.dmin = (float)pc->dmin; c.dmax = (float)pc->dmax; c.nstep = pc->nstep; c.ezero = 0;
-            const int s0 = pc->step0;
-            for (int k = 0; k < c.nstep; k++) c.ezero |= (G(S.se)[s0 + k] == 0 ? 1u : 0u) << k;
-            sc = screen_shell(c, [&](int k) { return (float)G(S.sd)[s0 + k]; }, true, rr, b, v2);
-        }
+    const bool con = cb & SDMD_CONSTRAINT_CONNECT;
+    Shell c;
+    const float *rad;
+    if (con) {
+        const int q = (cb >> 2) - 1;
+        o.slot = q;
+        if (q < 0) { o.flag = true; return; }             // not staged: FP64 decides
+        c.dmin = wm.con_dmin[q]; c.dmax = wm.con_dmax[q]; c.nstep = wm.con_nstep[q]; c.ezero = wm.con_ez[q];
+        rad = wm.con_rad[q];
     } else {
         const ScrPair sp = T.pr[A.type * NT + tj];
-        const int ri = sp.rp;
-        o.rp = ri;
-        if (ri < 0) {
-            sc.flag = true; sc.t = FINF; sc.e = 0;
-        } else {
-            Shell c;
-            c.dmin = sp.dmin; c.dmax = sp.dmax; c.nstep = sp.nstep; c.ezero = sp.ezero;
-            const float *rad = T.rad + sp.off;
-            sc = screen_shell(c, [&](int k) { return rad[k]; }, false, rr, b, v2);
-        }
+        o.rp = sp.rp;
+        if (sp.rp < 0 || sp.off == 0xffff) { o.flag = true; return; }
+        c.dmin = sp.dmin; c.dmax = sp.dmax; c.nstep = sp.nstep; c.ezero = sp.ezero;
+        rad = T.rad + sp.off;
     }
-    o.t = sc.t; o.e = sc.e; o.flag = sc.flag || (rr > calib - cband);
+    const Scr sc = screen_shell(c, [&](int k) { return rad[k]; }, con, rr, b, v2);
+    o.t = sc.t; o.e = sc.e; o.ks = sc.ks; o.flag = sc.flag || (rr > rsafe);
 }
 
-// FQ: candidates per lane held in registers (64*FQ per wave in one pass)
+// One screened candidate in FP64 (TimePrediction.c:79-179) in the shell the
+// screen found: no radius lies inside the screen's band around the pair's
+// distance, so the FP64 search would end in the same shell, and the shell's
+// limits and energies load together with j's state (one round trip).
+// Returns +inf when it does not reach JobAssign.
+template <class FW>
+__device__ __forceinline__ double coli64_shell(const FSys &F, const ScrTab &T, const FW &wm, const FAtom &A, int id, int ks,
+                                               int slot, double &pot, int &sub, long long &pc, bool &late) {
+    const Sys &S = F.s;
+    const int j = id >> 8;
+    const bool con = slot >= 0;
+    const ScrPair sp = T.pr[A.type * NT + (id & 255)];
+    const int nstep = con ? wm.con_nstep[slot & (FCON - 1)] : (int)sp.nstep, stride = con ? FCONSTEP : PROW;
+    const double *row = con ? F.crow + (size_t)(A.co + slot) * (2 + 2 * FCONSTEP)
+                            : F.prow + (size_t)max((int)sp.rp, 0) * (2 + 2 * PROW);
+    const int kl = max(ks - 1, 0), kh = min(ks, stride - 1);
+    const double dmin = G(row)[0], dmax = G(row)[1];
+    const double dl = G(row)[2 + kl], el = G(row)[2 + stride + kl], dh = G(row)[2 + kh], eh = G(row)[2 + stride + kh];
+    pc = G(S.evc)[j];
+    Kin k;
+    kin_local(F, A, j, k, &late);
+    const double lo = ks > 0 ? dl : dmin, lopot = ks > 0 ? el : 0;
+    double hi, hipot;
+    int cs;
+    if (ks < nstep) { hi = dh; hipot = -1 * eh; cs = ks == 0 ? 0 : -1; }
+    else if (dmax > 0) { hi = dmax; hipot = 0; cs = (nstep == 0 && k.b < 0) ? 0 : 1; }
+    else { hi = INFINIT; hipot = INFINIT; cs = 1; }
+    pot = 0;
+    sub = SDMD_INVALID_INTER;
+    if (!con && lopot == 0 && hipot == 0) return __builtin_inf();
+    int s;
+    double d2;
+    if (k.b < 0 && calc_disc(k, lo) > 0) {
+        s = -1; d2 = lo; pot = lopot;
+        sub = (cs == 0) ? SDMD_CORECOLLI : SDMD_TBDCAPTR;
+    } else {
+        s = 1; d2 = hi; pot = hipot;
+        if (con) sub = (cs == 1) ? SDMD_WELLBOUNC : SDMD_TBDESCAP;
+        else if (cs == 1) return __builtin_inf();
+        else sub = SDMD_TBDESCAP;
+    }
+    const double t = calc_time(k, s, d2);
+    return (t > 0) ? t : __builtin_inf();
+}
 
-// screened CollisionTime: FP32 screen of the neighbourhood, FP64 re-solve of
-// the marked candidates and of those whose interval reaches the smallest
-// upper bound; the FP64 minimum (first in scan order on ties) competes with
-// the running best under JobAssign's strict '<'
+// FQ: candidates per lane whose records are loaded together
+
+// Screened CollisionTime: the candidates inside the scan radius are listed
+// in LDS (a quarter of the neighbourhood), screened in FP32 one per lane, and
+// the marked ones and those whose interval reaches the smallest upper bound
+// are re-solved in FP64; the FP64 minimum (first in scan order on ties)
+// competes with the running best under JobAssign's strict '<'.
+// A lone wavefront issues one instruction in about five cycles, so what
+// counts is how often the long screen runs: once per 64 listed candidates
+// instead of once per 64 scanned.
 // VAL: validation mode (every live candidate also solved in FP64 and the
 // full scan's winner compared), a separate instantiation so that the
 // screened path carries none of its state
-template <int FQ, bool VAL>
-__device__ __forceinline__ void collision_fast(FSys &F, const ScrTab &T, FWave &wm, const FAtom &A, Best &best, long long &nscreen,
+template <int FQ, bool VAL, class FW>
+__device__ __forceinline__ void collision_fast(FSys &F, const ScrTab &T, FW &wm, const FAtom &A, Best &best, long long &nscreen,
                                long long &nconf, int *err) {
     const Sys &S = F.s;
     unsigned long long pt = S.prof ? wall_clock64() : 0;
     const int lane = threadIdx.x & 63;
-    const int n = wm.coff[27];
+    const int n = uni(wm.coff[27]);
     const double calib64 = (S.cutoffr * SDMD_EXTEND_RATIO) * (S.cutoffr * SDMD_EXTEND_RATIO);
     const float calib = (float)calib64;
-    const float cband = 2e-5f * calib + 1e-5f;
+    const float cband = 2e-5f * calib + 1e-5f, rscan = calib + cband, rsafe = calib - cband;
     const float tA = (float)(A.t - F.Te);
-    const fvec4 s0 = A.s0, s1 = A.s1;
     int my_screen = 0, my_causal = 0, my_conf = 0;
     Best mine;
     mine.t = __builtin_inf(); mine.pot = 0; mine.pc = 0; mine.partner = INVALID; mine.type = SDMD_COLI; mine.sub = 0;
@@ -903,118 +886,118 @@ __device__ __forceinline__ void collision_fast(FSys &F, const ScrTab &T, FWave &
     int fullk = 0x7fffffff;
     float myt32 = FINF;
     // FP64 re-solve of candidate k (and the validation scan)
-    auto confirm = [&](int k, const CandS &o, bool need) {
-        double pot;
+    auto confirm = [&](int k, int id, int bits, int rp, float t32, int ks, int slot, bool flag, bool need) {
+        double pot, t;
         int sub;
-        bool reached, late;
-        const double t = coli64(F, A, o.j, o.bits, o.rp, calib64, pot, sub, reached, late, err);
-        my_causal += late ? 1 : 0;                 // FP64 check of the screen's FP32 time order
+        bool late;
+        long long pc = 0;
         if (need) {
+            if (flag) {
+                bool reached;
+                t = coli64(F, A, id >> 8, bits, rp, calib64, pot, sub, reached, late, err);
+                pc = G(S.evc)[id >> 8];
+            } else {
+                t = coli64_shell(F, T, wm, A, id, ks, slot, pot, sub, pc, late);
+            }
+            my_causal += late ? 1 : 0;             // FP64 check of the screen's FP32 time order
             my_conf++;
-            if (t < mine.t) { mine.t = t; mine.pot = pot; mine.sub = sub; mine.partner = o.j; mink = k; myt32 = o.t; }
+            if (t < mine.t) { mine.t = t; mine.pot = pot; mine.sub = sub; mine.partner = id >> 8; mine.pc = pc; mink = k; myt32 = t32; }
         }
         if constexpr (VAL) {
-            if (t < full.t) { full.t = t; full.pot = pot; full.sub = sub; full.partner = o.j; fullk = k; }
+            bool reached;
+            t = coli64(F, A, id >> 8, bits, rp, calib64, pot, sub, reached, late, err);
+            if (!need) my_causal += late ? 1 : 0;
+            if (t < full.t) { full.t = t; full.pot = pot; full.sub = sub; full.partner = id >> 8; fullk = k; }
         }
     };
-    if (n <= 64 * FQ) {
-        // one pass: all record loads issued together, screens kept in registers
+    // ---- the candidates inside the scan radius, in candidate order
+    int near = 0;
+    for (int base = 0; base < n; base += 64 * FQ) {
         fvec4 r0[FQ], r1[FQ];
         int cq[FQ];
         // every lane loads a record for every slot (slots past the last
         // candidate re-read the last one), so the loads issue together
 #pragma unroll
         for (int q = 0; q < FQ; q++) {
-            const int k = min(lane + 64 * q, n - 1);
+            const int k = min(base + lane + 64 * q, n - 1);
             const int c = cand_cell(wm, k);
             const size_t at = (size_t)wm.cell[c] * F.cap + (k - wm.coff[c]);
             cq[q] = c;
             r0[q] = G(F.rec)[2 * at];
             r1[q] = G(F.rec)[2 * at + 1];
         }
-        if (A.role == 'A' || A.role == 'D' || A.role == 'S') {
-            // a free H-bond atom scans the same neighbourhood for HBTime:
-            // list the candidates inside the scan radius (FP32 with the
-            // screen's band, so the list holds every candidate the FP64
-            // test keeps), in candidate order, for that scan
-            int off = 0;
-#pragma unroll
-            for (int q = 0; q < FQ; q++) {
-                const int k = lane + 64 * q;
-                const int j = __float_as_int(r1[q].w) >> 8;
-                bool nr = false;
-                if (k < n && j >= 1 && j <= S.N && j != A.i) {
-                    const float dtj = tA - r0[q].w;
-                    const fvec4 co = wm.cof[cq[q]];
-                    const float rx = s0.x - (r0[q].x + r1[q].x * dtj) - co.x;
-                    const float ry = s0.y - (r0[q].y + r1[q].y * dtj) - co.y;
-                    const float rz = s0.z - (r0[q].z + r1[q].z * dtj) - co.z;
-                    nr = rx * rx + ry * ry + rz * rz <= calib + cband;
-                }
-                const unsigned long long m = __ballot(nr);
-                const int r = off + __builtin_amdgcn_mbcnt_hi((unsigned int)(m >> 32),
-                                                              __builtin_amdgcn_mbcnt_lo((unsigned int)m, 0));
-                if (nr && r < 128) { wm.hbl_j[r] = j; wm.hbl_k[r] = k; }
-                off += __popcll(m);
-            }
-            if (lane == 0) wm.hbl_n = off <= 128 ? off : -1;
-            __builtin_amdgcn_wave_barrier();
-        }
-        CandS o[FQ];
-        float thi = FINF;
 #pragma unroll
         for (int q = 0; q < FQ; q++) {
-            o[q].live = false; o[q].t = FINF; o[q].flag = false;
-            if (lane + 64 * q < n) {
-                screen_at(F, T, wm, A, cq[q], r0[q], r1[q], s0, s1, tA, calib, cband, o[q], my_causal);
-                my_screen += o[q].live;
-                if (o[q].live && !o[q].flag && o[q].t < FINF) thi = fminf(thi, o[q].t + o[q].e);
+            const int k = base + lane + 64 * q;
+            if (base + 64 * q < n) {                       // uniform
+                const int id = __float_as_int(r1[q].w), j = id >> 8;
+                const Near d = near_at(wm, A, cq[q], r0[q], r1[q], tA);
+                const bool nr = k < n && j >= 1 && j <= S.N && j != A.i && (id & 255) < NT && d.rr <= rscan;
+                const unsigned long long m = __ballot(nr);
+                const int r = near + __builtin_amdgcn_mbcnt_hi((unsigned int)(m >> 32),
+                                                               __builtin_amdgcn_mbcnt_lo((unsigned int)m, 0));
+                if (nr && r < FW::LIST) {
+                    wm.l_rr[r] = d.rr; wm.l_b[r] = d.b; wm.l_v2[r] = d.v2;
+                    wm.l_id[r] = id;
+                    wm.l_k[r] = k | (d.dt < 0.f ? (int)0x80000000 : 0);
+                }
+                near += __popcll(m);
             }
         }
+    }
+    wave_sync();
+    if (near <= FW::LIST) {
+        float thi = FINF;
+        for (int r = lane; r < near; r += 64) {
+            CandS o;
+            screen_near(F, T, wm, A, wm.l_id[r], wm.l_rr[r], wm.l_b[r], wm.l_v2[r], rsafe, o);
+            my_screen += o.live;
+            my_causal += (o.live && wm.l_k[r] < 0) ? 1 : 0;
+            if (o.live && !o.flag && o.t < FINF) thi = fminf(thi, o.t + o.e);
+            wm.l_t[r] = o.live ? o.t : FINF;
+            wm.l_e[r] = (o.live && o.flag) ? -1.f : o.e;
+            wm.l_sh[r] = o.ks | ((o.slot + 1) << 8) | (o.live ? 1 << 16 : 0);
+        }
+        if (lane == 0) wm.hbl_n = near;
         thi = wave_min_f(thi);
         PROF_MARK(S, FPH_SCREEN, pt);
-        // one copy of the FP64 re-solve, looped over the marked slots
-        unsigned needm = 0, valm = 0;
-#pragma unroll
-        for (int q = 0; q < FQ; q++) {
-            const bool need = o[q].live && (o[q].flag || (o[q].t < FINF && o[q].t - o[q].e <= thi));
-            needm |= (need ? 1u : 0u) << q;
-            valm |= ((o[q].live && VAL) ? 1u : 0u) << q;
-        }
-        unsigned todo = needm | valm;
-        while (todo) {
-            const int q = __builtin_ctz(todo);
-            todo &= todo - 1;
-            CandS oq;
-            oq.j = o[0].j; oq.bits = o[0].bits; oq.t = o[0].t; oq.rp = o[0].rp;
-#pragma unroll
-            for (int r = 1; r < FQ; r++)
-                if (q == r) { oq.j = o[r].j; oq.bits = o[r].bits; oq.t = o[r].t; oq.rp = o[r].rp; }
-            confirm(lane + 64 * q, oq, (needm >> q) & 1);
+        for (int r = lane; r < near; r += 64) {
+            const float t = wm.l_t[r], e = wm.l_e[r];
+            const int sh = wm.l_sh[r];
+            const bool flag = e < 0.f, need = flag || (t < FINF && t - e <= thi);
+            if (need || (VAL && (sh >> 16))) {
+                const int id = wm.l_id[r], slot = ((sh >> 8) & 255) - 1;
+                // what the FP64 search of a marked candidate needs
+                const int bits = coli_bits(wm, S, A, id >> 8) & (SDMD_BOND_CONNECT | SDMD_CONSTRAINT_CONNECT);
+                const int rp = (bits & SDMD_CONSTRAINT_CONNECT) ? -1 : T.pr[A.type * NT + (id & 255)].rp;
+                confirm(wm.l_k[r] & 0x7fffffff, id, bits, rp, t, sh & 255, slot, flag, need);
+            }
         }
     } else {
-        // large neighbourhoods: bound first, then re-screen and confirm
+        // more candidates inside the radius than the list holds: bound
+        // first, then re-screen and confirm
         float thi = FINF;
-        for (int k = lane; k < n; k += 64) {
-            const int c = cand_cell(wm, k);
-            const size_t at = (size_t)wm.cell[c] * F.cap + (k - wm.coff[c]);
-            CandS o;
-            const fvec4 q0 = G(F.rec)[2 * at], q1 = G(F.rec)[2 * at + 1];
-            screen_at(F, T, wm, A, c, q0, q1, s0, s1, tA, calib, cband, o, my_causal);
-            my_screen += o.live;
-            if (o.live && !o.flag && o.t < FINF) thi = fminf(thi, o.t + o.e);
-        }
-        thi = wave_min_f(thi);
-        int dummy = 0;
-        for (int k = lane; k < n; k += 64) {
-            const int c = cand_cell(wm, k);
-            const size_t at = (size_t)wm.cell[c] * F.cap + (k - wm.coff[c]);
-            CandS o;
-            const fvec4 q0 = G(F.rec)[2 * at], q1 = G(F.rec)[2 * at + 1];
-            screen_at(F, T, wm, A, c, q0, q1, s0, s1, tA, calib, cband, o, dummy);
-            if (!o.live) continue;
-            const bool need = o.flag || (o.t < FINF && o.t - o.e <= thi);
-            if (need || VAL) confirm(k, o, need);
+        for (int pass = 0; pass < 2; pass++) {
+            for (int k = lane; k < n; k += 64) {
+                const int c = cand_cell(wm, k);
+                const size_t at = (size_t)wm.cell[c] * F.cap + (k - wm.coff[c]);
+                const fvec4 q0 = G(F.rec)[2 * at], q1 = G(F.rec)[2 * at + 1];
+                const int id = __float_as_int(q1.w), j = id >> 8;
+                const Near d = near_at(wm, A, c, q0, q1, tA);
+                if (!(j >= 1 && j <= S.N && j != A.i && (id & 255) < NT && d.rr <= rscan)) continue;
+                CandS o;
+                screen_near(F, T, wm, A, id, d.rr, d.b, d.v2, rsafe, o);
+                if (!o.live) continue;
+                if (pass == 0) {
+                    my_screen++;
+                    my_causal += d.dt < 0.f ? 1 : 0;
+                    if (!o.flag && o.t < FINF) thi = fminf(thi, o.t + o.e);
+                } else {
+                    const bool need = o.flag || (o.t < FINF && o.t - o.e <= thi);
+                    if (need || VAL) confirm(k, id, o.bits, o.rp, o.t, o.ks, o.slot, o.flag, need);
+                }
+            }
+            if (pass == 0) thi = wave_min_f(thi);
         }
     }
     PROF_MARK(S, FPH_CONFIRM, pt);
@@ -1055,37 +1038,10 @@ __device__ __forceinline__ void collision_fast(FSys &F, const ScrTab &T, FWave &
             else if (fw.t < __builtin_inf()) cnt_max(F.max_time_err, fabs(win.t - fw.t) / fw.t);
         }
     }
-    if (win.t < __builtin_inf() && win.partner > 0) {
-        if (win.t > 0 && best.t > win.t) {
-            best.t = win.t; best.pot = win.pot; best.sub = win.sub; best.type = SDMD_COLI;
-            best.partner = win.partner; best.pc = G(S.evc)[win.partner];
-        }
+    if (win.t < __builtin_inf() && win.partner > 0 && win.t > 0 && best.t > win.t) {
+        best.t = win.t; best.pot = win.pot; best.sub = win.sub; best.type = SDMD_COLI;
+        best.partner = win.partner; best.pc = win.pc;
     }
-}
-
-// one BondTime entry (TimePrediction.c:219-293) at local time
-__device__ double bond64(const FSys &F, const FAtom &A, int e, int &sub) {
-    const Sys &S = F.s;
-    const int j = G(S.bond_j)[e];
-    const double lo = G(S.bond_dmin)[e], hi = G(S.bond_dmax)[e];
-    Kin k;
-    kin_local(F, A, j, k);
-    double t;
-    if (k.rr - hi > ZERO && k.b >= 0) {
-        sub = SDMD_WELLBOUNC;
-        t = 1e-16 * A.i * j;
-    } else if (!(k.rr - hi > ZERO) && lo - k.rr > ZERO && k.b < 0) {
-        sub = SDMD_CORECOLLI;
-        t = 1e-16 * A.i * j;
-    } else {
-        int s;
-        double d2;
-        if (k.b < 0 && calc_disc(k, lo) > 0) { s = -1; d2 = lo; sub = SDMD_CORECOLLI; }
-        else { s = 1; d2 = hi; sub = SDMD_WELLBOUNC; }
-        t = calc_time(k, s, d2);
-        if (t < 0) t = INFINIT;
-    }
-    return (t > 0) ? t : __builtin_inf();
 }
 
 // free-atom HBTime candidate (TimePrediction.c:414-478) at local time, in
@@ -1154,8 +1110,8 @@ __device__ double hbfree64(const FSys &F, const FAtom &A, int j, double calib, d
 }
 
 // Predict for atom i at time t (its state is at t); writes the event record
-template <int FQ>
-__device__ __forceinline__ void predict_fast(FSys &F, const ScrTab &T, FWave &wm, int i, double t, WStats &ws, int *err) {
+template <int FQ, class FW>
+__device__ __forceinline__ void predict_fast(FSys &F, const ScrTab &T, FW &wm, int i, double t, WStats &ws, int *err) {
     Sys &S = F.s;
     const int lane = threadIdx.x & 63;
     long long &nscreen = ws.screen, &nconf = ws.conf, &nfp64 = ws.fp64;
@@ -1198,7 +1154,7 @@ __device__ __forceinline__ void predict_fast(FSys &F, const ScrTab &T, FWave &wm
     PROF_MARK(S, FPH_BOND, pt);
     // CollisionTime (screened), against no running best yet
     if (lane == 0) wm.hbl_n = -1;
-    __builtin_amdgcn_wave_barrier();
+    wave_sync();
     Best cw = init;
     cw.t = __builtin_inf();
     if (F.validate) collision_fast<FQ, true>(F, T, wm, A, cw, nscreen, nconf, err);
@@ -1226,16 +1182,19 @@ __device__ __forceinline__ void predict_fast(FSys &F, const ScrTab &T, FWave &wm
     }
     // ThermostatTime, TimePrediction.c:582-595
     if (S.thermostat) {
-        double z = 0;
-        if (lane == 0) z = fast_normal_at(F, i, A.rctr);
-        z = lane_get(z, 0);
-        const double tt = S.thermoF * ((z < 0) ? (-z) : (z));
-        take(best, S, tt, 0, SDMD_INVALID_INTER, SDMD_THER, 0);
+        const unsigned int ctr = uni((int)A.rctr);
+        if (lane == 0) G(F.rctr)[i] = ctr + 1;
+        unsigned int c[4];
+        normal_words(F, uni(i), ctr, c);
+        if (!(S.thermoF * (double)normal_floor(c[0], c[2]) > best.t)) {
+            const double z = normal_of(c[0], c[1], c[2], c[3]);
+            const double tt = S.thermoF * ((z < 0) ? (-z) : (z));
+            take(best, S, tt, 0, SDMD_INVALID_INTER, SDMD_THER, 0);
+        }
     }
     // HBTime head, TimePrediction.c:309-330
     const double calib = (S.cutoffr * SDMD_EXTEND_RATIO) * (S.cutoffr * SDMD_EXTEND_RATIO);
-    const int hbit = G(S.hbitype)[i];
-    __builtin_amdgcn_wave_barrier();
+    const int hbit = A.hbit;
     if (lane == 0) G(S.hbitype)[i] = SDMD_NOEVENT;
     // The bonded H-bond partner's time (lane 32) and HBNeighborTime's pair
     // times over neighborPartner[1..4] (lane q - 1 for slot q) read state
@@ -1307,7 +1266,7 @@ __device__ __forceinline__ void predict_fast(FSys &F, const ScrTab &T, FWave &wm
             // the candidates the screen listed inside the scan radius, in
             // candidate order; otherwise every candidate, filtered below
             for (int r = lane; r < nl; r += 64) {
-                const int j = wm.hbl_j[r], k = wm.hbl_k[r];
+                const int j = wm.l_id[r] >> 8, k = wm.l_k[r] & 0x7fffffff;
                 double pot;
                 bool reached;
                 const double tt = hbfree_all(F, A, j, calib, pot, reached, err);
@@ -1337,19 +1296,19 @@ __device__ __forceinline__ void predict_fast(FSys &F, const ScrTab &T, FWave &wm
                                                          __builtin_amdgcn_mbcnt_lo((unsigned int)m0 & lo, 0));
                 const int r1 = n0 + __builtin_amdgcn_mbcnt_hi((unsigned int)(m1 >> 32) & hi,
                                                               __builtin_amdgcn_mbcnt_lo((unsigned int)m1 & lo, 0));
-                __builtin_amdgcn_wave_barrier();
-                if (ok[0]) { wm.hbl_j[r0] = jj[0]; wm.hbl_k[r0] = base + lane; }
-                if (ok[1]) { wm.hbl_j[r1] = jj[1]; wm.hbl_k[r1] = base + 64 + lane; }
-                __builtin_amdgcn_wave_barrier();
+                wave_sync();
+                if (ok[0]) { wm.l_id[r0] = jj[0] << 8; wm.l_k[r0] = base + lane; }
+                if (ok[1]) { wm.l_id[r1] = jj[1] << 8; wm.l_k[r1] = base + 64 + lane; }
+                wave_sync();
                 for (int r = lane; r < npass; r += 64) {
-                    const int j = wm.hbl_j[r], k = wm.hbl_k[r];
+                    const int j = wm.l_id[r] >> 8, k = wm.l_k[r];
                     double pot;
                     bool reached;
                     const double tt = hbfree64(F, A, j, calib, pot, reached, err);
                     my += reached;
                     if (tt < mine.t) { mine.t = tt; mine.pot = pot; mine.partner = j; mink = k; }
                 }
-                __builtin_amdgcn_wave_barrier();
+                wave_sync();
             }
             nfp64 += wave_sum_i(my);
             double tw = mine.t;
@@ -1594,22 +1553,10 @@ __device__ __forceinline__ int exec_pair(FSys &F, int a, int p, int ty, double t
     return 2;
 }
 
-__device__ __forceinline__ int exec_fast(FSys &F, int a, double t, int *renew, int *err, bool *recs) {
+// every other event (H-bond, thermostat, cell crossing, wall): about 1 % of
+// them, kept out of line so that its registers do not count in the loop
+__device__ __attribute__((noinline)) int exec_general(FSys &F, int a, int partner, double t, int *renew, int *err) {
     Sys &S = F.s;
-    // the record and state of a, loaded together with its partner id
-    const int p = G(S.evp)[a];
-    const int ty0 = G(S.evtype)[a];
-    const long long pca = G(S.evpc)[a];
-    const double pot0 = G(S.evpot)[a];
-    const int sub0 = G(S.evsub)[a];
-    PairAtom a0;
-    pair_load(F, a, a0);
-    const int partner = (p > 0 && p <= S.N) ? p : 0;
-    *recs = false;
-    if (partner && partner != a && (ty0 == SDMD_COLI || ty0 == SDMD_BOND || ty0 == SDMD_HBNE)) {
-        *recs = true;
-        return exec_pair(F, a, partner, ty0, t, a0, pca, pot0, sub0, renew, err);
-    }
     advance(F, a, t);
     renew[0] = a;
     if (partner && G(S.evpc)[a] < G(S.evc)[partner]) {          // HazardCheck, SGThread.c:215-235
@@ -1651,6 +1598,25 @@ __device__ __forceinline__ int exec_fast(FSys &F, int a, double t, int *renew, i
     if (partner) G(S.evc)[partner]++;
     if (partner) { renew[1] = partner; return 2; }
     return 1;
+}
+
+__device__ __forceinline__ int exec_fast(FSys &F, int a, double t, int *renew, int *err, bool *recs) {
+    Sys &S = F.s;
+    // the record and state of a, loaded together with its partner id
+    const int p = G(S.evp)[a];
+    const int ty0 = G(S.evtype)[a];
+    const long long pca = G(S.evpc)[a];
+    const double pot0 = G(S.evpot)[a];
+    const int sub0 = G(S.evsub)[a];
+    PairAtom a0;
+    pair_load(F, a, a0);
+    const int partner = (p > 0 && p <= S.N) ? p : 0;
+    *recs = false;
+    if (partner && partner != a && (ty0 == SDMD_COLI || ty0 == SDMD_BOND || ty0 == SDMD_HBNE)) {
+        *recs = true;
+        return exec_pair(F, a, partner, ty0, t, a0, pca, pot0, sub0, renew, err);
+    }
+    return exec_general(F, a, partner, t, renew, err);
 }
 
 // ---------------------------------------------------------------- tree blocks
@@ -1773,12 +1739,13 @@ __device__ __forceinline__ void job_done(FJobs *J) {
 }
 
 // ---------------------------------------------------------------- shared memory
+template <int W>
 struct FShared {
     long long run_clock_end, run_count_end;   // the launch's bounds (thread 0)
     double b1[FMAXBLK], b2[FMAXBLK], b3[FMAXBLK];
     int ba[FMAXBLK], bb[FMAXBLK];
-    double red_t[FMAXW], red_t1[FMAXW], red_t3[FMAXW];
-    int red_a[FMAXW], red_n[FMAXW];
+    double red_t[W], red_t1[W], red_t3[W];
+    int red_a[W];
     double sel_t[FSEL];
     int sel_a[FSEL], sel_rank[FSEL];  // selected set: atom, number of earlier events in the set
     // per selected event: cells of target and partner (packed x<<20|y<<10|z),
@@ -1797,7 +1764,7 @@ struct FShared {
     double ren_t[2 * FSEL];
     int dirty[4 * FSEL];
     unsigned int dmask[FMAXBLK / 32];   // blocks touched this round (bit per block)
-    FWave w[FMAXW];
+    FWave<flist(W)> w[W];
 };
 
 template <int W>
@@ -1861,7 +1828,7 @@ __global__ __launch_bounds__(256) void k_fast_records(FSys *systems) {
 template <int W>
 __global__ __launch_bounds__(64 * W) void k_fast_predict(FSys *systems) {
     __shared__ FSys Fl;
-    __shared__ FWave w[W];
+    __shared__ FWave<flist(W)> w[W];
     __shared__ ScrTab tab;
     FSys &Fg = systems[blockIdx.x];
     fsys_load<W>(Fl, &Fg);
@@ -1877,7 +1844,7 @@ __global__ __launch_bounds__(64 * W) void k_fast_predict(FSys *systems) {
     __syncthreads();
     WStats &ws = w[wave].st;                // in LDS: no registers held across the loop
     ws.screen = ws.conf = ws.fp64 = ws.cand = 0;
-    __builtin_amdgcn_wave_barrier();
+    wave_sync();
     int err = 0;
     for (int i = 1 + blockIdx.y * W + wave; i <= S.N; i += W * gridDim.y) {
         predict_fast<4>(F, tab, w[wave], i, G(F.t0)[i], ws, &err);
@@ -1967,11 +1934,11 @@ __global__ __launch_bounds__(64 * EWAVES) void k_fast_energy(FSys *systems, doub
 // A helper workgroup: its wavefronts claim the owner's published jobs
 // (re-predictions) until the owner stops, then add their statistics to hp.
 template <int W, int FQ>
-__device__ __forceinline__ void helper_loop(FSys &F, const ScrTab &tab, FShared &sh, FJobs *J, FHelp *hp, int xcc) {
+__device__ __forceinline__ void helper_loop(FSys &F, const ScrTab &tab, FShared<W> &sh, FJobs *J, FHelp *hp, int xcc) {
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     WStats &ws = sh.w[wave].st;             // in LDS: no registers held across the loop
     ws.screen = ws.conf = ws.fp64 = ws.cand = 0;
-    __builtin_amdgcn_wave_barrier();
+    wave_sync();
     for (;;) {
         int q = -1, quit = 0;
         if (lane == 0) {
@@ -2027,7 +1994,7 @@ template <int W, int FQ>
 __global__ __launch_bounds__(64 * W) void k_fast_run(FSys *systems, FJobs *jobs, FHelp *help, int nsys, int H,
                                                      long long npops, long long budget, double t_end) {
     __shared__ FSys Fl;
-    __shared__ FShared sh;
+    __shared__ FShared<W> sh;
     __shared__ ScrTab tab;
     const int sys = (blockIdx.x & 7) + 8 * ((blockIdx.x >> 3) / (H + 1));
     const int role = (blockIdx.x >> 3) % (H + 1);
@@ -2068,7 +2035,7 @@ __global__ __launch_bounds__(64 * W) void k_fast_run(FSys *systems, FJobs *jobs,
     }
     WStats &ws = sh.w[wave].st;             // in LDS: no registers held across the loop
     ws.screen = ws.conf = ws.fp64 = ws.cand = 0;
-    __builtin_amdgcn_wave_barrier();
+    wave_sync();
     const int cap = F.max_batch > 0 ? min(F.max_batch, FSEL) : FSEL;
     unsigned long long pt = S.prof ? wall_clock64() : 0;
     while (true) {
@@ -2464,6 +2431,7 @@ struct sdmd::FastState {
     FSys *host;
     FSys *dev;
     int waves;                 // wavefronts per workgroup (events in flight per round per pass)
+    int tuned;                 // waves is the autotuner's choice
     int depth;                 // candidates per lane staged in registers (FQ)
     int validate;
     hipGraph_t graph;          // captured launch sequence (sdmd_gpu_run_graph)
@@ -2598,15 +2566,45 @@ int sdmd_fast_open(sdmd_gpu_ctx *c, const sdmd_gpu_opts *o) {
             if (rc == SDMD_OK) rc = fdev_alloc(c, &F.crad, cr, (size_t)(nc > 0 ? nc : 1));
             free(hj); free(hl); free(hh); free(cr);
             if (rc) return rc;
+            // FP64 shells at a fixed stride (a constraint of more steps than
+            // a row holds is not staged, and then not read from here)
+            const int CR = 2 + 2 * FCONSTEP, PR = 2 + 2 * PROW;
+            double *rows = (double *)calloc((size_t)(nc > 0 ? nc : 1) * CR, sizeof(double));
+            // the collision table's rows are one copy for systems of equal tables
+            const sdmd_system_desc *d0 = c->desc[0];
+            int top = 0;
+            for (int k = 0; k < NT * NT; k++)
+                top = d->pair[k].step0 + d->pair[k].nstep > top ? d->pair[k].step0 + d->pair[k].nstep : top;
+            const bool shared = s > 0 && top <= d0->nstep_pool && !memcmp(d->pair, d0->pair, sizeof(sdmd_pair) * NT * NT) &&
+                                !memcmp(d->step_d, d0->step_d, sizeof(double) * top) &&
+                                !memcmp(d->step_e, d0->step_e, sizeof(double) * top);
+            double *prows = (double *)calloc(shared ? 1 : (size_t)NT * NT * PR, sizeof(double));
+            if (!rows || !prows) { free(rows); free(prows); return SDMD_ENOMEM; }
+            auto fill = [&](double *r, const sdmd_pair &p, int stride) {
+                r[0] = p.dmin;
+                r[1] = p.dmax;
+                for (int k = 0; k < p.nstep && k < stride; k++) {
+                    r[2 + k] = d->step_d[p.step0 + k];
+                    r[2 + stride + k] = d->step_e[p.step0 + k];
+                }
+            };
+            for (int k = 0; k < nc; k++) fill(rows + (size_t)k * CR, d->con[k], FCONSTEP);
+            for (int k = 0; k < NT * NT && !shared; k++) fill(prows + (size_t)k * PR, d->pair[k], PROW);
+            rc = fdev_alloc(c, &F.crow, rows, (size_t)(nc > 0 ? nc : 1) * CR);
+            if (shared) F.prow = fs->host[0].prow;
+            else if (rc == SDMD_OK) rc = fdev_alloc(c, &F.prow, prows, (size_t)NT * NT * PR);
+            free(rows); free(prows);
+            if (rc) return rc;
         }
         // FP32 screen table: RightPair (ToolFunctions.c:278-292) resolved for
         // every type pair, the pair's limits and its step radii
         ScrTab *tb = (ScrTab *)calloc(1, sizeof(ScrTab));
         if (!tb) return SDMD_ENOMEM;
         auto back = [](int t) { return t == 3 ? 1 : t == 4 ? 2 : t == 27 ? 26 : t; };
-        int pool = 0;
+        int pool = 0, stored = 0, nlist = 0;
+        static thread_local int lists[NT * NT][3];      // first step, steps, place in the pool
         rc = SDMD_OK;
-        // every defined pair's entry, radii in the pool once
+        // every defined pair's entry; equal lists of radii stored once
         ScrPair *ent = (ScrPair *)calloc(NT * NT, sizeof(ScrPair));
         if (!ent) { free(tb); return SDMD_ENOMEM; }
         for (int p = 0; p < NT * NT; p++) {
@@ -2618,14 +2616,24 @@ int sdmd_fast_open(sdmd_gpu_ctx *c, const sdmd_gpu_opts *o) {
             sp.dmin = (float)pp.dmin;
             sp.dmax = (float)pp.dmax;
             sp.nstep = (unsigned short)pp.nstep;
-            sp.off = (unsigned short)pool;
             sp.ezero = 0;
             sp.rp = (short)p;
+            float list[16];
             for (int k = 0; k < pp.nstep; k++) {
-                tb->rad[pool + k] = (float)d->step_d[pp.step0 + k];
+                list[k] = (float)d->step_d[pp.step0 + k];
                 if (d->step_e[pp.step0 + k] == 0) sp.ezero |= (unsigned short)(1u << k);
             }
             pool += pp.nstep;
+            // a list already stored: that of an earlier pair with the same steps
+            int q = 0;
+            while (q < nlist && (lists[q][0] != pp.step0 || lists[q][1] != pp.nstep)) q++;
+            if (q == nlist && stored + pp.nstep <= FRADL) {
+                lists[q][0] = pp.step0; lists[q][1] = pp.nstep; lists[q][2] = stored;
+                memcpy(tb->rad + stored, list, sizeof(float) * pp.nstep);
+                stored += pp.nstep;
+                nlist++;
+            }
+            sp.off = q < nlist ? (unsigned short)lists[q][2] : 0xffff;
         }
         for (int t1 = 0; t1 < NT; t1++)
             for (int t2 = 0; t2 < NT; t2++) {
@@ -2660,10 +2668,7 @@ int sdmd_fast_open(sdmd_gpu_ctx *c, const sdmd_gpu_opts *o) {
             setg(24, Sh.cmap_off, 1, 0, 0); setg(25, Sh.cmap_off, 1, 1, 0);
             setg(26, Sh.bond_off, 1, 0, 0); setg(27, Sh.bond_off, 1, 1, 0);
             setg(28, Sh.con_off, 1, 0, 0); setg(29, Sh.con_off, 1, 1, 0);
-            for (int k = 0; k < SDMD_DYNSLOTS; k++) {
-                setg(32 + k, Sh.dynj, SDMD_DYNSLOTS, k, 0);
-                setg(40 + k, Sh.dynb, SDMD_DYNSLOTS, k, 0);
-            }
+            setg(30, Sh.hbitype, 1, 0, 0);
         }
         if (rc == SDMD_OK) {
             ScrTab *dt = nullptr;
@@ -2702,7 +2707,18 @@ static int fast_sync_from(sdmd_gpu_ctx *c) {
 
 int sdmd_fast_sync(sdmd_gpu_ctx *c) { return fast_sync_from(c); }
 
-#define FDISPATCH(fn, ...) do { switch (fs->waves) { \
+// Wavefronts per workgroup of a launch.  With helper workgroups a round's
+// re-predictions (10 to 40) find more wavefronts than they need, and one
+// wavefront per SIMD, with all registers of the SIMD, is the fastest a
+// prediction gets: us per round with 4 / 8 wavefronts per workgroup 20 / 28
+// (59 atoms), 35 / 40 (64 systems of 1 536), 47 / 52 (26 080).  Without
+// helpers the owner's wavefronts are all there are: 51 / 34 ms for 6 000
+// events of 26 080 atoms.  The autotuner's choice is taken as it is.
+static int run_waves(const FastState *fs) {
+    return (!fs->tuned && fs->helpers > 0 && fs->waves > 4) ? 4 : fs->waves;
+}
+
+#define FDISPATCH(fn, ...) do { switch (run_waves(fs)) { \
     case 4: fn<4>(__VA_ARGS__); break; \
     case 8: fn<8>(__VA_ARGS__); break; \
     case 12: fn<12>(__VA_ARGS__); break; \
@@ -2896,7 +2912,7 @@ int sdmd_fast_run_graph(sdmd_gpu_ctx *c, int launches, double max_ms) {
     FastState *fs = c->fast;
     long long budget;
     if (launches < 1 || budget_ticks(max_ms, &budget)) return SDMD_EINVAL;
-    const int key = ((launches * 16 + fs->helpers) * 64 + fs->waves) * 8 + fs->depth;
+    const int key = ((launches * 16 + fs->helpers) * 64 + run_waves(fs)) * 8 + fs->depth;
     if (!fs->gexec || fs->g_launches != key || fs->g_budget != budget) {
         if (fs->gexec) { HIPV(hipGraphExecDestroy(fs->gexec)); fs->gexec = nullptr; }
         if (fs->graph) { HIPV(hipGraphDestroy(fs->graph)); fs->graph = nullptr; }
@@ -2937,6 +2953,7 @@ int sdmd_fast_autotune(sdmd_gpu_ctx *c, double trial_ms, int32_t *block_out, int
     static const int shapes[][2] = {{4, 4}, {8, 4}, {12, 4}, {16, 4}, {4, 2}, {8, 2}, {12, 2}, {16, 2}};
     double best = -1;
     int bw = fs->waves, bq = fs->depth;
+    fs->tuned = 1;                               // the trials run the shapes as named
     for (const auto &sh : shapes) {
         fs->waves = sh[0];
         fs->depth = sh[1];

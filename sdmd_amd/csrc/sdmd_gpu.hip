@@ -189,37 +189,6 @@ __device__ __forceinline__ int in_nb_list(const Atom &A, int j, int *err) {   //
 }
 
 // ---------------------------------------------------------------- wave helpers
-// LDS written by some lanes of a wave, read next by others of the same wave:
-// the wave's LDS operations run in order, so only the compiler is held
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
-
-// lane of the wave's smallest t, the lowest one on equal t; every t is
-// positive or +inf (no NaN, no -0).  The order of such doubles is that of
-// their bits, so the high words are reduced first (six DPP minima) and the
-// low words only where several lanes share the smallest high word.
-__device__ __forceinline__ unsigned wave_umin(unsigned v) {
-    v = min(v, (unsigned)__builtin_amdgcn_update_dpp(-1, (int)v, 0x111, 0xF, 0xF, false));   // row_shr:1
-    v = min(v, (unsigned)__builtin_amdgcn_update_dpp(-1, (int)v, 0x112, 0xF, 0xF, false));   // row_shr:2
-    v = min(v, (unsigned)__builtin_amdgcn_update_dpp(-1, (int)v, 0x114, 0xF, 0xF, false));   // row_shr:4
-    v = min(v, (unsigned)__builtin_amdgcn_update_dpp(-1, (int)v, 0x118, 0xF, 0xF, false));   // row_shr:8
-    v = min(v, (unsigned)__builtin_amdgcn_update_dpp(-1, (int)v, 0x142, 0xA, 0xF, false));   // row_bcast:15
-    v = min(v, (unsigned)__builtin_amdgcn_update_dpp(-1, (int)v, 0x143, 0xC, 0xF, false));   // row_bcast:31
-    return (unsigned)__builtin_amdgcn_readlane((int)v, 63);
-}
-__device__ __forceinline__ int wave_first_min(double t) {
-    const unsigned long long b = (unsigned long long)__double_as_longlong(t);
-    const unsigned hi = (unsigned)(b >> 32), lo = (unsigned)b;
-    unsigned long long m = __ballot(hi == wave_umin(hi));
-    if (m & (m - 1)) {
-        const unsigned l = ((m >> (threadIdx.x & 63)) & 1) ? lo : 0xffffffffu;
-        m &= __ballot(l == wave_umin(l));
-    }
-    return __ffsll((long long)m) - 1;
-}
-
 // Ordered selection over n entries in program order, run by one full wave.
 // Entry k offers its computed time ct[k] (+inf when it would not reach
 // JobAssign or fails `t > 0`); flagged entries (bit 0) first offer j's
@@ -1585,15 +1554,9 @@ static int upload_system(sdmd_gpu_ctx *c, Sys *S, const sdmd_system_desc *d, con
     UP(node, (const int *)nullptr, 2 * N1);
     UP(leaf, (const int *)nullptr, N1 + 1);
     S->win = (o && o->window > 0) ? o->window : MAXC;
-    if (!o || o->mode == SDMD_MODE_PLAIN) {
-        // the plain engine's derived tables: cell arrays (filled by k_cells),
-        // pops each atom has taken, the constraint entry of each connection
-        // row entry (the first of its partner, as FindPair finds it), the
-        // collision table with RightPair resolved (ToolFunctions.c:278-292)
-        const size_t ncell = (size_t)d->cellnum[0] * d->cellnum[1] * d->cellnum[2];
-        UP(ccnt, (const int *)nullptr, ncell + 1);
-        UP(cmem, (const int *)nullptr, (ncell + 1) * CELL_CAP);
-        UP(lag, (const unsigned char *)nullptr, N1);
+    {
+        // the constraint entry of each connection row entry (the first of
+        // its partner, as FindPair finds it)
         int *cc = (int *)malloc(sizeof(int) * (size_t)(ncm > 0 ? ncm : 1));
         if (!cc) return SDMD_ENOMEM;
         for (int a = 1; a <= N; a++)
@@ -1606,6 +1569,14 @@ static int upload_system(sdmd_gpu_ctx *c, Sys *S, const sdmd_system_desc *d, con
         rc = dev_upload(c, &S->cmap_con, cc, (size_t)ncm);
         free(cc);
         if (rc) return rc;
+    }
+    if (!o || o->mode == SDMD_MODE_PLAIN) {
+        // the plain engine's derived tables: cell arrays (filled by k_cells),
+        // pops each atom has taken, the collision table with RightPair resolved (ToolFunctions.c:278-292)
+        const size_t ncell = (size_t)d->cellnum[0] * d->cellnum[1] * d->cellnum[2];
+        UP(ccnt, (const int *)nullptr, ncell + 1);
+        UP(cmem, (const int *)nullptr, (ncell + 1) * CELL_CAP);
+        UP(lag, (const unsigned char *)nullptr, N1);
         sdmd_pair rp[NT * NT];
         auto back = [](int t) { return t == 3 ? 1 : t == 4 ? 2 : t == 27 ? 26 : t; };
         int pool = 0, most = 0;
