@@ -95,6 +95,8 @@ struct Sys {
     int *ccnt, *cmem, *cmap_con;
     unsigned char *lag;
     sdmd_pair *rpair;
+    double *bulk_t2;            // bulk prediction: see k_bulk_resolve
+    int *bulk_head, *bulk_next, *bulk_flag;
     int ltab, logk;             // step pool entries held in LDS (0: none); pops between sweeps
     const int *gbase[48];       // gather table of a staged atom
     int gstride[48];

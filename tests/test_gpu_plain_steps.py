@@ -66,3 +66,33 @@ def test_single_operations_between_runs(require_gpu, name):
         assert np.array_equal(whole.state(0).arr[f], mixed.state(0).arr[f]), f
     whole.close()
     mixed.close()
+
+
+# helix: H bonds formed (records that depend on H-bond slots); window 5: every
+# atom predicted in windows; 0.9 of the box edge from a wall; an odd and an
+# even number of atoms
+@pytest.mark.parametrize("name,pops,window", [("ala10helix", 0, 0), ("ala10helix", 3000, 0), ("mix4x20", 2000, 0),
+                                              ("cyl8x20", 3001, 0), ("dense30", 500, 0), ("dense30", 500, 100),
+                                              ("ala10cyl", 1000, 5)])
+def test_bulk_prediction_of_evolved_states(require_gpu, name, pops, window):
+    """The bulk prediction of a state reached by a run, atom for atom and
+    the tree, as the oracle predicts it in order."""
+    import oracle_lib
+    from sdmd_amd.engine import GpuEngine, System
+
+    eng = engine(name, pops + 10, 256)
+    eng.run(pops)
+    arr = eng.state(0)
+    eng.close()
+    sysm = System(None, arr)
+    again = GpuEngine([sysm, sysm], window=window, max_pops=10)     # two systems share the launch
+    again.prepare()
+    o = oracle_lib.Oracle(arr)
+    assert o.bulk() == 0
+    ref = o.state()
+    for k in range(2):
+        got = again.state(k)
+        for f in ("ev_partner", "ev_type", "ev_sub", "ev_time", "ev_pot", "ev_pcounter", "nb_partnernum", "hb_itype"):
+            assert np.array_equal(got.arr[f][1:], ref.arr[f][1:]), (k, f)
+        assert again.stats(k)["error"] == 0
+    again.close()
