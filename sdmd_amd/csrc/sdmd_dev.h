@@ -857,6 +857,10 @@ static __global__ __launch_bounds__(64) void k_energy_reduce(const double *part,
 // ---------------------------------------------------------------- host side
 namespace sdmd { struct FastState; }
 
+// a system's arrays that a run changes lie in one device block, so that a
+// download is one copy
+struct sdmd_dyn_block { char *dev; size_t bytes; };
+
 struct sdmd_gpu_ctx {
     int nsys;
     int block;
@@ -869,7 +873,10 @@ struct sdmd_gpu_ctx {
     const sdmd_system_desc **desc;
     void **allocs;
     int nalloc, capalloc;
-    int *dev_renew;
+    struct sdmd_op_status *status;  // pinned host memory: what a single operation reports
+    sdmd_dyn_block *dyn;       // per system: the arrays a run changes, one device block
+    char *hostbuf;             // pinned host copy of one such block (allocated at the first download)
+    size_t hostbuf_bytes;
     double *dev_energy;        // 3 planes of nsys doubles (kinetic, potential, error flag)
     double *epart;             // partial energy sums: 3 doubles per system and workgroup
     int echunks;               // energy workgroups per system
@@ -879,16 +886,25 @@ struct sdmd_gpu_ctx {
 
 static int hip_ok(hipError_t e) { return e == hipSuccess ? SDMD_OK : SDMD_EDEVICE; }
 
+static int dev_keep(sdmd_gpu_ctx *c, void *p) {          // freed when the context closes
+    if (c->nalloc == c->capalloc) {
+        const int cap = c->capalloc ? 2 * c->capalloc : 128;
+        void **a = (void **)realloc(c->allocs, sizeof(void *) * cap);
+        if (!a) { HIPV(hipFree(p)); return SDMD_ENOMEM; }
+        c->allocs = a;
+        c->capalloc = cap;
+    }
+    c->allocs[c->nalloc++] = p;
+    return SDMD_OK;
+}
+
 template <typename T>
 static int dev_upload(sdmd_gpu_ctx *c, T **dst, const T *src, size_t n) {
-    if (c->nalloc == c->capalloc) {
-        c->capalloc = c->capalloc ? 2 * c->capalloc : 128;
-        c->allocs = (void **)realloc(c->allocs, sizeof(void *) * c->capalloc);
-    }
-    size_t bytes = sizeof(T) * (n ? n : 1);
+    const size_t bytes = sizeof(T) * (n ? n : 1);
     void *p = nullptr;
     if (hipMalloc(&p, bytes) != hipSuccess) return SDMD_EDEVICE;
-    c->allocs[c->nalloc++] = p;
+    int rc = dev_keep(c, p);
+    if (rc) return rc;
     if (src && n) {
         if (hipMemcpy(p, src, sizeof(T) * n, hipMemcpyHostToDevice) != hipSuccess) return SDMD_EDEVICE;
     } else if (hipMemset(p, 0, bytes) != hipSuccess) {
@@ -898,9 +914,63 @@ static int dev_upload(sdmd_gpu_ctx *c, T **dst, const T *src, size_t n) {
     return SDMD_OK;
 }
 
+// Many small arrays as one allocation and one copy: arena_add appends an
+// array (zeros where src is null) on a 256-byte boundary and remembers the
+// pointer to set; arena_commit uploads the block and sets the pointers.  A
+// system has about 60 arrays; one hipMalloc and one copy each made opening 64
+// systems of 1 536 atoms take 100 ms.
+struct sdmd_arena {
+    char *data;
+    size_t used, cap;
+    struct { void **dst; size_t at; } fix[96];
+    int nfix, failed;
+    ~sdmd_arena() { free(data); }
+};
+
+static void arena_add_bytes(sdmd_arena *a, void **dst, const void *src, size_t bytes) {
+    const size_t at = (a->used + 255) & ~(size_t)255, end = at + (bytes ? bytes : 1);
+    if (a->failed || a->nfix == (int)(sizeof a->fix / sizeof a->fix[0])) { a->failed = 1; return; }
+    if (end > a->cap) {
+        const size_t cap = end > 2 * a->cap ? end : 2 * a->cap;
+        char *d = (char *)realloc(a->data, cap);
+        if (!d) { a->failed = 1; return; }
+        a->data = d;
+        a->cap = cap;
+    }
+    memset(a->data + a->used, 0, at - a->used);
+    if (src && bytes) memcpy(a->data + at, src, bytes);
+    else memset(a->data + at, 0, end - at);
+    a->used = end;
+    a->fix[a->nfix].dst = dst;
+    a->fix[a->nfix++].at = at;
+}
+template <typename T>
+static void arena_add(sdmd_arena *a, T **dst, const T *src, size_t n) {
+    arena_add_bytes(a, (void **)dst, src, sizeof(T) * n);
+}
+static int arena_commit(sdmd_gpu_ctx *c, sdmd_arena *a) {
+    int rc = a->failed ? SDMD_ENOMEM : SDMD_OK;
+    char *d = nullptr;
+    if (!rc && hipMalloc((void **)&d, a->used ? a->used : 1) != hipSuccess) rc = SDMD_EDEVICE;
+    if (!rc) rc = dev_keep(c, d);
+    if (!rc && a->used && hipMemcpy(d, a->data, a->used, hipMemcpyHostToDevice) != hipSuccess) rc = SDMD_EDEVICE;
+    for (int k = 0; !rc && k < a->nfix; k++) *a->fix[k].dst = d + a->fix[k].at;
+    a->used = 0;
+    a->nfix = a->failed = 0;
+    return rc;
+}
+
+// what a single operation reports to the host (pinned memory, written by the
+// kernel): the system's error word and, for a pop, the event
+struct sdmd_op_status {
+    int error;
+    sdmd_gpu_event ev;
+};
 
 // screened local-time engine (sdmd_fast.hip)
 int sdmd_fast_open(sdmd_gpu_ctx *c, const sdmd_gpu_opts *o);
+int sdmd_dyn_download(sdmd_gpu_ctx *c, int s);
+void sdmd_dyn_scatter(const sdmd_gpu_ctx *c, int s, sdmd_system_desc *d);
 int sdmd_fast_prepare(sdmd_gpu_ctx *c);
 int sdmd_fast_run(sdmd_gpu_ctx *c, long long pops, double max_ms, double t_end);
 int sdmd_fast_download(sdmd_gpu_ctx *c, int s, sdmd_system_desc *out);

@@ -1814,6 +1814,35 @@ __device__ __forceinline__ void tab_load(ScrTab &dst, const void *src) {
 }
 
 #ifndef SDMD_FAST_WAVES
+// cell arrays from the reference's linked lists (list order), every cell
+__global__ __launch_bounds__(256) void k_fast_cells(FSys *systems) {
+    FSys &F = systems[blockIdx.x];
+    const Sys &S = F.s;
+    for (int c = 1 + blockIdx.y * 256 + threadIdx.x; c <= F.ncell; c += 256 * gridDim.y) {
+        int q = 0;
+        for (int a = G(S.celllist)[S.N + c]; a && q < F.cap; a = G(S.celllist)[a], q++) {
+            G(F.cmem)[(size_t)c * F.cap + q] = a;
+            G(F.slot)[a] = q;
+        }
+        G(F.ccnt)[c] = q;
+    }
+}
+
+// linked cell lists from the cell arrays of one system, for a download
+__global__ __launch_bounds__(256) void k_fast_lists(FSys *systems, int sys) {
+    FSys &F = systems[sys];
+    const Sys &S = F.s;
+    for (int c = 1 + blockIdx.x * 256 + threadIdx.x; c <= F.ncell; c += 256 * gridDim.x) {
+        int head = 0;
+        for (int q = G(F.ccnt)[c] - 1; q >= 0; q--) {
+            const int a = G(F.cmem)[(size_t)c * F.cap + q];
+            G(S.celllist)[a] = head;
+            head = a;
+        }
+        G(S.celllist)[S.N + c] = head;
+    }
+}
+
 // mirror records of every atom, before the bulk prediction reads them
 __global__ __launch_bounds__(256) void k_fast_records(FSys *systems) {
     FSys &F = systems[blockIdx.x];
@@ -2474,6 +2503,7 @@ int sdmd_fast_open(sdmd_gpu_ctx *c, const sdmd_gpu_opts *o) {
     fs->host = (FSys *)calloc((size_t)c->nsys, sizeof(FSys));
     if (!fs->host) return SDMD_ENOMEM;
     int rc;
+    sdmd_arena ar = {};
     for (int s = 0; s < c->nsys; s++) {
         const sdmd_system_desc *d = c->desc[s];
         FSys &F = fs->host[s];
@@ -2502,7 +2532,8 @@ int sdmd_fast_open(sdmd_gpu_ctx *c, const sdmd_gpu_opts *o) {
         int fullest = 0;
         for (long cell = 1; cell <= ncell; cell++) {
             int n = 0;
-            for (int a = d->celllist[N + cell]; a && n <= N; a = d->celllist[a]) n++;
+            for (int a = d->celllist[N + cell]; a && n <= N; a = d->celllist[a], n++)
+                if (a < 0 || a > N) return SDMD_EINVAL;
             if (n > N) return SDMD_EINVAL;                 // a cycle in the list
             fullest = n > fullest ? n : fullest;
         }
@@ -2510,34 +2541,23 @@ int sdmd_fast_open(sdmd_gpu_ctx *c, const sdmd_gpu_opts *o) {
         while (cap < 2 * fullest && cap < FCAP_MAX) cap *= 2;
         if (fullest > cap) return SDMD_EUNSUPPORTED;
         F.cap = cap;
-        int *cnt = (int *)calloc((size_t)ncell + 1, sizeof(int));
-        int *mem = (int *)calloc(((size_t)ncell + 1) * cap, sizeof(int));
-        int *slot = (int *)calloc((size_t)N + 1, sizeof(int));
         double *t0 = (double *)malloc(sizeof(double) * ((size_t)N + 1));
-        if (!cnt || !mem || !slot || !t0) { free(cnt); free(mem); free(slot); free(t0); return SDMD_ENOMEM; }
-        rc = SDMD_OK;
-        for (long cell = 1; cell <= ncell && rc == SDMD_OK; cell++) {
-            int guard = 0;
-            for (int a = d->celllist[N + cell]; a; a = d->celllist[a]) {
-                if (++guard > N || cnt[cell] >= cap) { rc = SDMD_EUNSUPPORTED; break; }
-                mem[cell * cap + cnt[cell]] = a;
-                slot[a] = cnt[cell]++;
-            }
-        }
+        if (!t0) return SDMD_ENOMEM;
         for (int a = 0; a <= N; a++) t0[a] = d->currenttime;
-        if (rc == SDMD_OK) rc = fdev_alloc(c, &F.ccnt, cnt, (size_t)ncell + 1);
-        if (rc == SDMD_OK) rc = fdev_alloc(c, &F.cmem, mem, ((size_t)ncell + 1) * cap);
-        if (rc == SDMD_OK) rc = fdev_alloc(c, &F.slot, slot, (size_t)N + 1);
-        if (rc == SDMD_OK) rc = fdev_alloc(c, &F.t0, t0, (size_t)N + 1);
-        free(cnt); free(mem); free(slot); free(t0);
-        if (rc) return rc;
-        if ((rc = fdev_alloc(c, &F.rec, (const fvec4 *)nullptr, ((size_t)ncell + 1) * cap * 2))) return rc;
-        if ((rc = fdev_alloc(c, &F.b1, (const double *)nullptr, (size_t)F.nblk))) return rc;
-        if ((rc = fdev_alloc(c, &F.b2, (const double *)nullptr, (size_t)F.nblk))) return rc;
-        if ((rc = fdev_alloc(c, &F.ba, (const int *)nullptr, (size_t)F.nblk))) return rc;
-        if ((rc = fdev_alloc(c, &F.b3, (const double *)nullptr, (size_t)F.nblk))) return rc;
-        if ((rc = fdev_alloc(c, &F.bb, (const int *)nullptr, (size_t)F.nblk))) return rc;
-        if ((rc = fdev_alloc(c, &F.rctr, (const unsigned int *)nullptr, (size_t)N + 1))) return rc;
+        arena_add(&ar, &F.t0, (const double *)t0, (size_t)N + 1);
+        free(t0);
+        arena_add(&ar, &F.ccnt, (const int *)nullptr, (size_t)ncell + 1);
+        arena_add(&ar, &F.slot, (const int *)nullptr, (size_t)N + 1);
+        if ((rc = fdev_alloc(c, &F.cmem, (const int *)nullptr, ((size_t)ncell + 1) * cap)) ||
+            (rc = fdev_alloc(c, &F.rec, (const fvec4 *)nullptr, ((size_t)ncell + 1) * cap * 2))) {
+                    return rc;
+        }
+        arena_add(&ar, &F.b1, (const double *)nullptr, (size_t)F.nblk);
+        arena_add(&ar, &F.b2, (const double *)nullptr, (size_t)F.nblk);
+        arena_add(&ar, &F.b3, (const double *)nullptr, (size_t)F.nblk);
+        arena_add(&ar, &F.ba, (const int *)nullptr, (size_t)F.nblk);
+        arena_add(&ar, &F.bb, (const int *)nullptr, (size_t)F.nblk);
+        arena_add(&ar, &F.rctr, (const unsigned int *)nullptr, (size_t)N + 1);
         {
             // bond lists at a fixed stride of 16 (BondTime's connect[16]);
             // constraint step radii inline (CONSTRn lists, <= 8 steps staged)
@@ -2560,12 +2580,11 @@ int sdmd_fast_open(sdmd_gpu_ctx *c, const sdmd_gpu_opts *o) {
                     if (d->step_e[pc.step0 + q] == 0) cr[k].ez |= 1u << q;
                 }
             }
-            rc = fdev_alloc(c, &F.bj16, hj, n16);
-            if (rc == SDMD_OK) rc = fdev_alloc(c, &F.blo16, hl, n16);
-            if (rc == SDMD_OK) rc = fdev_alloc(c, &F.bhi16, hh, n16);
-            if (rc == SDMD_OK) rc = fdev_alloc(c, &F.crad, cr, (size_t)(nc > 0 ? nc : 1));
+            arena_add(&ar, &F.bj16, (const int *)hj, n16);
+            arena_add(&ar, &F.blo16, (const double *)hl, n16);
+            arena_add(&ar, &F.bhi16, (const double *)hh, n16);
+            arena_add(&ar, &F.crad, (const ConRad *)cr, (size_t)(nc > 0 ? nc : 1));
             free(hj); free(hl); free(hh); free(cr);
-            if (rc) return rc;
             // FP64 shells at a fixed stride (a constraint of more steps than
             // a row holds is not staged, and then not read from here)
             const int CR = 2 + 2 * FCONSTEP, PR = 2 + 2 * PROW;
@@ -2590,12 +2609,12 @@ int sdmd_fast_open(sdmd_gpu_ctx *c, const sdmd_gpu_opts *o) {
             };
             for (int k = 0; k < nc; k++) fill(rows + (size_t)k * CR, d->con[k], FCONSTEP);
             for (int k = 0; k < NT * NT && !shared; k++) fill(prows + (size_t)k * PR, d->pair[k], PROW);
-            rc = fdev_alloc(c, &F.crow, rows, (size_t)(nc > 0 ? nc : 1) * CR);
+            arena_add(&ar, &F.crow, (const double *)rows, (size_t)(nc > 0 ? nc : 1) * CR);
             if (shared) F.prow = fs->host[0].prow;
-            else if (rc == SDMD_OK) rc = fdev_alloc(c, &F.prow, prows, (size_t)NT * NT * PR);
+            else arena_add(&ar, &F.prow, (const double *)prows, (size_t)NT * NT * PR);
             free(rows); free(prows);
-            if (rc) return rc;
         }
+        if ((rc = arena_commit(c, &ar))) return rc;
         // FP32 screen table: RightPair (ToolFunctions.c:278-292) resolved for
         // every type pair, the pair's limits and its step radii
         ScrTab *tb = (ScrTab *)calloc(1, sizeof(ScrTab));
@@ -2679,6 +2698,8 @@ int sdmd_fast_open(sdmd_gpu_ctx *c, const sdmd_gpu_opts *o) {
         if (rc) return rc;
     }
     if ((rc = fdev_alloc(c, &fs->dev, fs->host, (size_t)c->nsys))) return rc;
+    hipLaunchKernelGGL(k_fast_cells, dim3(c->nsys, 64), dim3(256), 0, c->stream, fs->dev);
+    if (hipGetLastError() != hipSuccess) return SDMD_EDEVICE;
     if ((rc = fdev_alloc(c, &fs->jobs, (const FJobs *)nullptr, (size_t)c->nsys))) return rc;
     if ((rc = fdev_alloc(c, &fs->help, (const FHelp *)nullptr, (size_t)c->nsys))) return rc;
     fs->hhelp = (FHelp *)calloc((size_t)c->nsys, sizeof(FHelp));
@@ -2809,31 +2830,30 @@ int sdmd_fast_download(sdmd_gpu_ctx *c, int s, sdmd_system_desc *out) {
     const FSys &F = fs->host[s];
     const Sys &S = F.s;
     if (S.error) return SDMD_ESTATE;         // e.g. an incomplete drain: not a snapshot at one time
+    // every array is wanted here (the plain engine leaves out missing ones)
+    for (const void *p : {(void *)out->x, (void *)out->y, (void *)out->z, (void *)out->vx, (void *)out->vy, (void *)out->vz,
+                          (void *)out->type, (void *)out->cellx, (void *)out->celly, (void *)out->cellz,
+                          (void *)out->hb_bond, (void *)out->hb_itype, (void *)out->nb_partner,
+                          (void *)out->nb_partnernum, (void *)out->nb_status, (void *)out->dyn_j, (void *)out->dyn_bits,
+                          (void *)out->ev_partner, (void *)out->ev_type, (void *)out->ev_sub, (void *)out->ev_counter,
+                          (void *)out->ev_pcounter, (void *)out->ev_time, (void *)out->ev_pot, (void *)out->celllist})
+        if (!p) return SDMD_EDEVICE;
     const int N = S.N;
     const size_t N1 = (size_t)N + 1;
     double *t0 = (double *)malloc(sizeof(double) * N1);
     double *b1 = (double *)malloc(sizeof(double) * (size_t)F.nblk);
-    int *cnt = (int *)malloc(sizeof(int) * ((size_t)F.ncell + 1));
-    int *mem = (int *)malloc(sizeof(int) * ((size_t)F.ncell + 1) * F.cap);
-    if (!t0 || !b1 || !cnt || !mem) { free(t0); free(b1); free(cnt); free(mem); return SDMD_ENOMEM; }
-    int rc = SDMD_OK;
-#define FDOWN(dst, src, n) if (rc == SDMD_OK && hipMemcpy(dst, src, sizeof(*(dst)) * (n), hipMemcpyDeviceToHost) != hipSuccess) rc = SDMD_EDEVICE
-    FDOWN(t0, F.t0, N1);
-    FDOWN(b1, F.b1, (size_t)F.nblk);
-    FDOWN(cnt, F.ccnt, (size_t)F.ncell + 1);
-    FDOWN(mem, F.cmem, ((size_t)F.ncell + 1) * F.cap);
-    FDOWN(out->x, S.x, N1); FDOWN(out->y, S.y, N1); FDOWN(out->z, S.z, N1);
-    FDOWN(out->vx, S.vx, N1); FDOWN(out->vy, S.vy, N1); FDOWN(out->vz, S.vz, N1);
-    FDOWN(out->type, S.type, N1);
-    FDOWN(out->cellx, S.cx, N1); FDOWN(out->celly, S.cy, N1); FDOWN(out->cellz, S.cz, N1);
-    FDOWN(out->hb_bond, S.hbbond, N1); FDOWN(out->hb_itype, S.hbitype, N1);
-    FDOWN(out->nb_partner, S.nbp, N1 * SDMD_NBSLOTS); FDOWN(out->nb_partnernum, S.nbnum, N1);
-    FDOWN(out->nb_status, S.nbstat, N1);
-    FDOWN(out->dyn_j, S.dynj, N1 * SDMD_DYNSLOTS); FDOWN(out->dyn_bits, S.dynb, N1 * SDMD_DYNSLOTS);
-    FDOWN(out->ev_partner, S.evp, N1); FDOWN(out->ev_type, S.evtype, N1); FDOWN(out->ev_sub, S.evsub, N1);
-    FDOWN((long long *)out->ev_counter, S.evc, N1); FDOWN((long long *)out->ev_pcounter, S.evpc, N1);
-    FDOWN(out->ev_time, S.evt, N1); FDOWN(out->ev_pot, S.evpot, N1);
-#undef FDOWN
+    if (!t0 || !b1) { free(t0); free(b1); return SDMD_ENOMEM; }
+    // the lists from the cell arrays on the device, then every array that a
+    // run changes in one copy
+    const int blocks = (F.ncell + 255) / 256;
+    hipLaunchKernelGGL(k_fast_lists, dim3(blocks < 1024 ? blocks : 1024), dim3(256), 0, c->stream, fs->dev, s);
+    int rc = hip_ok(hipGetLastError());
+    if (rc == SDMD_OK) rc = hip_ok(hipMemcpyAsync(t0, F.t0, sizeof(double) * N1, hipMemcpyDeviceToHost, c->stream));
+    if (rc == SDMD_OK)
+        rc = hip_ok(hipMemcpyAsync(b1, F.b1, sizeof(double) * (size_t)F.nblk, hipMemcpyDeviceToHost, c->stream));
+    if (rc == SDMD_OK) rc = sdmd_dyn_download(c, s);
+    if (rc != SDMD_OK) HIPV(hipStreamSynchronize(c->stream));   // no copy in flight when the buffers go
+    if (rc == SDMD_OK) sdmd_dyn_scatter(c, s, out);
     if (rc == SDMD_OK) {
         double T = INFINIT;
         for (int b = 0; b < F.nblk; b++) if (b1[b] < T) T = b1[b];
@@ -2845,19 +2865,9 @@ int sdmd_fast_download(sdmd_gpu_ctx *c, int s, sdmd_system_desc *out) {
             out->z[a] = out->z[a] + out->vz[a] * dt;
             out->ev_time[a] -= T;
         }
-        // linked cell lists from the cell arrays
-        for (long cell = 1; cell <= F.ncell; cell++) {
-            int head = 0;
-            for (int q = cnt[cell] - 1; q >= 0; q--) {
-                const int a = mem[cell * F.cap + q];
-                out->celllist[a] = head;
-                head = a;
-            }
-            out->celllist[N + cell] = head;
-        }
         out->currenttime = T;
     }
-    free(t0); free(b1); free(cnt); free(mem);
+    free(t0); free(b1);
     return rc;
 }
 

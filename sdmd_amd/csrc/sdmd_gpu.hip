@@ -1009,24 +1009,6 @@ __device__ __forceinline__ void cbt_update(Sys &S, Smem &sm, int n, int a0, int 
     }
 }
 
-// one atom's path (lane 0), for single operations
-__device__ void cbt_update_run(Sys &S, int a) {
-    int father, left, right, old;
-    for (father = G(S.leaf)[a] / 2; father > 0; father /= 2) {
-        if (G(S.node)[father] != a) break;
-        left = G(S.node)[father * 2];
-        right = G(S.node)[father * 2 + 1];
-        G(S.node)[father] = (G(S.evt)[left] < G(S.evt)[right]) ? left : right;
-    }
-    for (; father > 0; father /= 2) {
-        old = G(S.node)[father];
-        left = G(S.node)[father * 2];
-        right = G(S.node)[father * 2 + 1];
-        G(S.node)[father] = (G(S.evt)[left] < G(S.evt)[right]) ? left : right;
-        if (G(S.node)[father] == old) return;
-    }
-}
-
 // CreateCBT (CBT.c:16-30).  Inserting atom a splits leaf a - 1: its atom
 // moves to node 2 (a - 1), a takes node 2 (a - 1) + 1.  So the atom of a
 // leaf depends on the leaf's number alone (the right child 2c + 1 holds c +
@@ -1565,7 +1547,7 @@ __global__ __launch_bounds__(256) void k_cells(const Sys *systems) {
 }
 
 // single operations behind the fine-grained entry points
-enum { OP_PREDICT, OP_CREATE_TREE, OP_UPDATE_TREE, OP_ADVANCE, OP_DO_EVENT, OP_CELL_MOVE };
+enum { OP_PREDICT, OP_CREATE_TREE, OP_UPDATE_TREE, OP_DO_EVENT, OP_CELL_MOVE };
 
 // CalKinetE + CalPotenE (ToolFunctions.c:626-752) of every system at its
 // current time: one wavefront per atom i, one lane per neighbour cell
@@ -1604,8 +1586,11 @@ __global__ __launch_bounds__(64 * EWAVES) void k_energy(Sys *systems, double *pa
     energy_partial(ke, pe, err || S.error, part);
 }
 
+struct Renew { int a[4]; };                // a renew list by value (at most two atoms, zero-terminated)
+
 template <int B>
-__global__ __launch_bounds__(B) void k_op(Sys *systems, int sys, int op, const int *renew, double dt, int a, int b) {
+__global__ __launch_bounds__(B) void k_op(Sys *systems, int sys, int op, Renew renew, int a, int b,
+                                          sdmd_op_status *status) {
     __shared__ Smem sm;
     __shared__ Sys Sl;
     sys_load<B>(Sl, &systems[sys]);
@@ -1615,20 +1600,16 @@ __global__ __launch_bounds__(B) void k_op(Sys *systems, int sys, int op, const i
     __syncthreads();
     if (op == OP_CREATE_TREE) cbt_create<B>(S);
     if (op == OP_PREDICT) {
-        predict_list<B, false>(S, sm, nullptr, renew);
-    } else if (op == OP_ADVANCE) {
-        for (int i = tid + 1; i <= S.N; i += B) {
-            G(S.x)[i] += G(S.vx)[i] * dt;
-            G(S.y)[i] += G(S.vy)[i] * dt;
-            G(S.z)[i] += G(S.vz)[i] * dt;
-            G(S.evt)[i] -= dt;
+        predict_list<B, false>(S, sm, nullptr, renew.a);
+    } else if (op == OP_UPDATE_TREE) {
+        const int n = renew.a[0];
+        if (tid < 64 && n > 0) {
+            const int a0 = renew.a[1], a1 = n > 1 ? renew.a[2] : a0;
+            cbt_update(S, sm, n, a0, G(S.leaf)[a0], G(S.evt)[a0], a1, G(S.leaf)[a1], G(S.evt)[a1]);
         }
-        __syncthreads();
-        if (tid == 0) S.currenttime += dt;
     } else if (tid == 0) {
         int err = 0;
-        if (op == OP_UPDATE_TREE) { for (int k = 1; renew[k]; k++) cbt_update_run(S, renew[k]); }
-        else if (op == OP_DO_EVENT) {
+        if (op == OP_DO_EVENT) {
             // SingleThreadRun, SGThread.c:100-104
             S.frame++;
             do_event(S, sm, a, b, &err);
@@ -1641,8 +1622,43 @@ __global__ __launch_bounds__(B) void k_op(Sys *systems, int sys, int op, const i
     if (tid == 0) {
         S.zpos = sm.zpos;
         if (sm.err) S.error = sm.err;
+        status->error = S.error;
     }
     sys_store<B>(&systems[sys], Sl);
+}
+
+// UpdateData + TimeForward (ToolFunctions.c:23-36) of one system by dt
+__global__ __launch_bounds__(256) void k_advance(Sys *systems, int sys, double dt, sdmd_op_status *status) {
+    Sys &S = systems[sys];
+    for (int i = 1 + blockIdx.x * 256 + threadIdx.x; i <= S.N; i += 256 * gridDim.x) {
+        G(S.x)[i] += G(S.vx)[i] * dt;
+        G(S.y)[i] += G(S.vy)[i] * dt;
+        G(S.z)[i] += G(S.vz)[i] * dt;
+        G(S.evt)[i] -= dt;
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        S.currenttime += dt;
+        status->error = S.error;
+    }
+}
+
+// AssignJob's event and HazardCheck's verdict (SGThread.c:215-259); target 0:
+// the tree holds no event
+__global__ __launch_bounds__(64) void k_pop(const Sys *systems, int sys, sdmd_op_status *status) {
+    const Sys &S = systems[sys];
+    if (threadIdx.x != 0) return;
+    const int root = G(S.node)[1];
+    sdmd_gpu_event ev = {};
+    if (root >= 1 && root <= S.N) {
+        ev.target = root;
+        ev.partner = G(S.evp)[root];
+        ev.type = G(S.evtype)[root];
+        ev.sub = G(S.evsub)[root];
+        ev.time = G(S.evt)[root];
+        ev.potential = G(S.evpot)[root];
+        if (ev.partner > 0 && ev.partner <= S.N) ev.stale = G(S.evpc)[root] < G(S.evc)[ev.partner];
+    }
+    status->ev = ev;
 }
 
 }  // namespace sdmd
@@ -1666,7 +1682,8 @@ static void atom_gather_table(Sys *S) {
     word(S->leaf, 1);
 }
 
-static int upload_system(sdmd_gpu_ctx *c, Sys *S, const sdmd_system_desc *d, const sdmd_gpu_opts *o) {
+static int upload_system(sdmd_gpu_ctx *c, sdmd_arena *ar, int s, const sdmd_system_desc *d, const sdmd_gpu_opts *o) {
+    Sys *S = &c->host_sys[s];
     memset(S, 0, sizeof *S);
     const int N = d->natom;
     const size_t N1 = (size_t)N + 1;
@@ -1699,19 +1716,23 @@ static int upload_system(sdmd_gpu_ctx *c, Sys *S, const sdmd_system_desc *d, con
         for (int k = 0; k < d->con_off[d->natom + 1]; k++) check_list(d->con[k]);
     }
     int rc = 0;
-#define UP(field, src, n) if ((rc = dev_upload(c, &S->field, src, n))) return rc
+#define UP(field, src, n) arena_add(ar, &S->field, src, n)
+#define UPBIG(field, n) if ((rc = dev_upload(c, &S->field, (decltype(+S->field))nullptr, n))) return rc
+    // what a run changes, first and in the order sdmd_dyn_scatter copies it back
     UP(x, d->x, N1); UP(y, d->y, N1); UP(z, d->z, N1);
-    UP(vx, d->vx, N1); UP(vy, d->vy, N1); UP(vz, d->vz, N1); UP(mass, d->mass, N1);
-    UP(type, d->type, N1); UP(aatype, d->aatype, N1); UP(protein, d->protein, N1); UP(aanum, d->aanum, N1);
-    UP(cx, d->cellx, N1); UP(cy, d->celly, N1); UP(cz, d->cellz, N1);
-    UP(role, (const signed char *)d->hb_role, N1);
-    UP(hbnb, d->hb_neighbor, N1); UP(hbbond, d->hb_bond, N1); UP(hbitype, d->hb_itype, N1);
+    UP(vx, d->vx, N1); UP(vy, d->vy, N1); UP(vz, d->vz, N1);
+    UP(type, d->type, N1); UP(cx, d->cellx, N1); UP(cy, d->celly, N1); UP(cz, d->cellz, N1);
+    UP(hbbond, d->hb_bond, N1); UP(hbitype, d->hb_itype, N1);
     UP(nbp, d->nb_partner, N1 * SDMD_NBSLOTS); UP(nbnum, d->nb_partnernum, N1); UP(nbstat, d->nb_status, N1);
     UP(dynj, d->dyn_j, N1 * SDMD_DYNSLOTS); UP(dynb, d->dyn_bits, N1 * SDMD_DYNSLOTS);
     UP(evp, d->ev_partner, N1); UP(evtype, d->ev_type, N1); UP(evsub, d->ev_sub, N1);
     UP(evc, (const long long *)d->ev_counter, N1); UP(evpc, (const long long *)d->ev_pcounter, N1);
     UP(evt, d->ev_time, N1); UP(evpot, d->ev_pot, N1);
     UP(celllist, d->celllist, (size_t)d->ncelllist);
+    c->dyn[s].bytes = ar->used;
+    UP(mass, d->mass, N1); UP(aatype, d->aatype, N1); UP(protein, d->protein, N1); UP(aanum, d->aanum, N1);
+    UP(role, (const signed char *)d->hb_role, N1);
+    UP(hbnb, d->hb_neighbor, N1);
     const int nb = d->bond_off[N + 1], nc = d->con_off[N + 1], ncm = d->cmap_off[N + 1];
     UP(bond_off, d->bond_off, N1 + 1); UP(bond_j, d->bond_j, (size_t)nb);
     UP(bond_dmin, d->bond_dmin, (size_t)nb); UP(bond_dmax, d->bond_dmax, (size_t)nb);
@@ -1736,16 +1757,15 @@ static int upload_system(sdmd_gpu_ctx *c, Sys *S, const sdmd_system_desc *d, con
                 for (int q = d->con_off[a]; q < d->con_off[a + 1]; q++)
                     if (d->con_j[q] == d->cmap_j[k]) { cc[k] = q; break; }
             }
-        rc = dev_upload(c, &S->cmap_con, cc, (size_t)ncm);
+        UP(cmap_con, (const int *)cc, (size_t)ncm);
         free(cc);
-        if (rc) return rc;
     }
     if (!o || o->mode == SDMD_MODE_PLAIN) {
         // the plain engine's derived tables: cell arrays (filled by k_cells),
         // pops each atom has taken, the collision table with RightPair resolved (ToolFunctions.c:278-292)
         const size_t ncell = (size_t)d->cellnum[0] * d->cellnum[1] * d->cellnum[2];
         UP(ccnt, (const int *)nullptr, ncell + 1);
-        UP(cmem, (const int *)nullptr, (ncell + 1) * CELL_CAP);
+        UPBIG(cmem, (ncell + 1) * CELL_CAP);
         UP(lag, (const unsigned char *)nullptr, N1);
         UP(bulk_t2, (const double *)nullptr, N1);
         UP(bulk_head, (const int *)nullptr, N1); UP(bulk_next, (const int *)nullptr, N1);
@@ -1770,11 +1790,10 @@ static int upload_system(sdmd_gpu_ctx *c, Sys *S, const sdmd_system_desc *d, con
         // memory traffic), frequent for small ones (an atom read late takes
         // the steps it lacks one by one, about 20 ns each)
         S->logk = N / 64 < 8 ? 8 : (N / 64 > LOGK ? LOGK : N / 64);
-        atom_gather_table(S);
     }
     if (o && o->trace) {
         S->trace_cap = o->trace_capacity > 0 ? o->trace_capacity : 100000;
-        UP(trace, (const sdmd_gpu_pop_rec *)nullptr, (size_t)S->trace_cap);
+        UPBIG(trace, (size_t)S->trace_cap);
     }
     if (o && (o->profile & 1)) {
         UP(prof, (const unsigned long long *)nullptr, (size_t)PH_NPH);
@@ -1782,10 +1801,51 @@ static int upload_system(sdmd_gpu_ctx *c, Sys *S, const sdmd_system_desc *d, con
     if (o && o->hash_every > 0) {
         S->hash_every = o->hash_every;
         S->hash_cap = (o->trace_capacity > 0 ? o->trace_capacity : 1000000) / o->hash_every + 1;
-        UP(hashes, (const long long *)nullptr, (size_t)S->hash_cap * 2);
+        UPBIG(hashes, (size_t)S->hash_cap * 2);
     }
 #undef UP
+#undef UPBIG
+    if ((rc = arena_commit(c, ar))) return rc;
+    c->dyn[s].dev = (char *)S->x;
+    if (!o || o->mode == SDMD_MODE_PLAIN) atom_gather_table(S);
     return SDMD_OK;
+}
+
+// One system's block of changing arrays into c->hostbuf (on the context's
+// stream, waited for), and from there into the caller's arrays.
+int sdmd_dyn_download(sdmd_gpu_ctx *c, int s) {
+    if (!c->hostbuf) {
+        size_t most = 0;
+        for (int k = 0; k < c->nsys; k++) most = c->dyn[k].bytes > most ? c->dyn[k].bytes : most;
+        if (hipHostMalloc((void **)&c->hostbuf, most, hipHostMallocDefault) != hipSuccess) {
+            c->hostbuf = nullptr;
+            return SDMD_EDEVICE;
+        }
+        c->hostbuf_bytes = most;
+    }
+    int rc = hip_ok(hipMemcpyAsync(c->hostbuf, c->dyn[s].dev, c->dyn[s].bytes, hipMemcpyDeviceToHost, c->stream));
+    return rc ? rc : hip_ok(hipStreamSynchronize(c->stream));
+}
+
+void sdmd_dyn_scatter(const sdmd_gpu_ctx *c, int s, sdmd_system_desc *d) {
+    const Sys &S = c->host_sys[s];
+    const size_t N1 = (size_t)S.N + 1;
+    auto get = [&](void *dst, const void *dev, size_t bytes) {
+        if (dst) memcpy(dst, c->hostbuf + ((const char *)dev - c->dyn[s].dev), bytes);
+    };
+#define DOWN(dst, src, n) get(dst, src, sizeof(*(src)) * (n))
+    DOWN(d->x, S.x, N1); DOWN(d->y, S.y, N1); DOWN(d->z, S.z, N1);
+    DOWN(d->vx, S.vx, N1); DOWN(d->vy, S.vy, N1); DOWN(d->vz, S.vz, N1);
+    DOWN(d->type, S.type, N1);
+    DOWN(d->cellx, S.cx, N1); DOWN(d->celly, S.cy, N1); DOWN(d->cellz, S.cz, N1);
+    DOWN(d->hb_bond, S.hbbond, N1); DOWN(d->hb_itype, S.hbitype, N1);
+    DOWN(d->nb_partner, S.nbp, N1 * SDMD_NBSLOTS); DOWN(d->nb_partnernum, S.nbnum, N1); DOWN(d->nb_status, S.nbstat, N1);
+    DOWN(d->dyn_j, S.dynj, N1 * SDMD_DYNSLOTS); DOWN(d->dyn_bits, S.dynb, N1 * SDMD_DYNSLOTS);
+    DOWN(d->ev_partner, S.evp, N1); DOWN(d->ev_type, S.evtype, N1); DOWN(d->ev_sub, S.evsub, N1);
+    DOWN(d->ev_counter, S.evc, N1); DOWN(d->ev_pcounter, S.evpc, N1);
+    DOWN(d->ev_time, S.evt, N1); DOWN(d->ev_pot, S.evpot, N1);
+    DOWN(d->celllist, S.celllist, (size_t)S.ncelllist);
+#undef DOWN
 }
 
 static int sync_to_device(sdmd_gpu_ctx *c) {
@@ -1834,13 +1894,16 @@ extern "C" int sdmd_gpu_open(const sdmd_system_desc *const *systems, int32_t nsy
     HIPV(hipEventCreate(&c->ev1));
     c->host_sys = (Sys *)calloc((size_t)nsys, sizeof(Sys));
     c->desc = (const sdmd_system_desc **)calloc((size_t)nsys, sizeof(void *));
-    int rc = SDMD_OK;
+    c->dyn = (sdmd_dyn_block *)calloc((size_t)nsys, sizeof(sdmd_dyn_block));
+    int rc = (c->host_sys && c->desc && c->dyn) ? SDMD_OK : SDMD_ENOMEM;
+    if (rc == SDMD_OK)
+        rc = hip_ok(hipHostMalloc((void **)&c->status, sizeof *c->status, hipHostMallocCoherent));
+    sdmd_arena ar = {};
     for (int s = 0; s < nsys && rc == SDMD_OK; s++) {
         c->desc[s] = systems[s];
-        rc = upload_system(c, &c->host_sys[s], systems[s], opts);
+        rc = upload_system(c, &ar, s, systems[s], opts);
     }
     if (rc == SDMD_OK) rc = dev_upload(c, &c->dev_sys, (const Sys *)nullptr, (size_t)nsys);
-    if (rc == SDMD_OK) rc = dev_upload(c, &c->dev_renew, (const int *)nullptr, 8);
     if (rc == SDMD_OK) {
         // energy workgroups per system: about 2048 in all (8 per CU), each
         // with an atom per wavefront at least
@@ -1866,6 +1929,8 @@ extern "C" int sdmd_gpu_close(sdmd_gpu_ctx *c) {
     if (!c) return SDMD_EINVAL;
     if (c->stream) HIPV(hipStreamSynchronize(c->stream));
     for (int k = 0; k < c->nalloc; k++) HIPV(hipFree(c->allocs[k]));
+    if (c->status) HIPV(hipHostFree(c->status));
+    if (c->hostbuf) HIPV(hipHostFree(c->hostbuf));
     free(c->allocs);
     if (c->ev0) HIPV(hipEventDestroy(c->ev0));
     if (c->ev1) HIPV(hipEventDestroy(c->ev1));
@@ -1873,6 +1938,7 @@ extern "C" int sdmd_gpu_close(sdmd_gpu_ctx *c) {
     sdmd_fast_close(c);
     free(c->host_sys);
     free(c->desc);
+    free(c->dyn);
     free(c);
     return SDMD_OK;
 }
@@ -1916,8 +1982,8 @@ static void launch_run(sdmd_gpu_ctx *c, long long n, long long budget, double t_
     hipLaunchKernelGGL((k_run<B>), dim3(c->nsys), dim3(B), 0, c->stream, c->dev_sys, n, budget, t_end, t_out);
 }
 template <int B>
-static void launch_op(sdmd_gpu_ctx *c, int s, int op, double dt, int a, int b) {
-    hipLaunchKernelGGL((k_op<B>), dim3(1), dim3(B), 0, c->stream, c->dev_sys, s, op, c->dev_renew, dt, a, b);
+static void launch_op(sdmd_gpu_ctx *c, int s, int op, Renew renew, int a, int b) {
+    hipLaunchKernelGGL((k_op<B>), dim3(1), dim3(B), 0, c->stream, c->dev_sys, s, op, renew, a, b, c->status);
 }
 
 #define DISPATCH(fn, ...) do { switch (c->block) { \
@@ -1995,66 +2061,65 @@ static int run_bounded(sdmd_gpu_ctx *c, int64_t pops, double max_ms, double t_en
     return check_errors(c);
 }
 
-static int run_op(sdmd_gpu_ctx *c, int s, int op, const int32_t *renew, double dt, int a, int b) {
+// After a single operation: its launch, its end and, from the pinned status
+// word, its error; errors other systems carry from earlier calls are known on
+// the host (every run and prepare copies them back).  One wait per call: the
+// struct copy and second wait of a run cost as much as the operation.
+static int op_result(sdmd_gpu_ctx *c, int s) {
+    if (hipGetLastError() != hipSuccess || hipStreamSynchronize(c->stream) != hipSuccess) return SDMD_EDEVICE;
+    c->host_sys[s].error = c->status->error;
+    for (int k = 0; k < c->nsys; k++)
+        if (c->host_sys[k].error) return SDMD_ESTATE;
+    return SDMD_OK;
+}
+
+static int run_op(sdmd_gpu_ctx *c, int s, int op, const int32_t *renew, int a, int b) {
     if (!c || s < 0 || s >= c->nsys) return SDMD_EINVAL;
     if (c->mode != SDMD_MODE_PLAIN) return SDMD_EUNSUPPORTED;
+    Renew list = {};
     if (renew) {
-        int n = renew[0];
+        const int n = renew[0];
         if (n < 0 || n > 2) return SDMD_EINVAL;
-        int buf[8] = {0};
-        for (int k = 0; k <= n; k++) buf[k] = renew[k];
+        for (int k = 0; k <= n; k++) list.a[k] = renew[k];
         for (int k = 1; k <= n; k++)
-            if (buf[k] < 1 || buf[k] > c->host_sys[s].N) return SDMD_EINVAL;
-        if (hipMemcpyAsync(c->dev_renew, buf, sizeof buf, hipMemcpyHostToDevice, c->stream) != hipSuccess) return SDMD_EDEVICE;
+            if (list.a[k] < 1 || list.a[k] > c->host_sys[s].N) return SDMD_EINVAL;
     }
-    DISPATCH(launch_op, c, s, op, dt, a, b);
-    if (hipGetLastError() != hipSuccess) return SDMD_EDEVICE;
-    if (hipStreamSynchronize(c->stream) != hipSuccess) return SDMD_EDEVICE;
-    return check_errors(c);
+    DISPATCH(launch_op, c, s, op, list, a, b);
+    return op_result(c, s);
 }
 
 extern "C" int sdmd_gpu_predict(sdmd_gpu_ctx *c, int32_t s, const int32_t *renew) {
     if (!renew) return SDMD_EINVAL;
-    return run_op(c, s, OP_PREDICT, renew, 0, 0, 0);
+    return run_op(c, s, OP_PREDICT, renew, 0, 0);
 }
-extern "C" int sdmd_gpu_create_tree(sdmd_gpu_ctx *c, int32_t s) { return run_op(c, s, OP_CREATE_TREE, nullptr, 0, 0, 0); }
+extern "C" int sdmd_gpu_create_tree(sdmd_gpu_ctx *c, int32_t s) { return run_op(c, s, OP_CREATE_TREE, nullptr, 0, 0); }
 extern "C" int sdmd_gpu_update_tree(sdmd_gpu_ctx *c, int32_t s, const int32_t *renew) {
     if (!renew) return SDMD_EINVAL;
-    return run_op(c, s, OP_UPDATE_TREE, renew, 0, 0, 0);
+    return run_op(c, s, OP_UPDATE_TREE, renew, 0, 0);
 }
-extern "C" int sdmd_gpu_advance(sdmd_gpu_ctx *c, int32_t s, double dt) { return run_op(c, s, OP_ADVANCE, nullptr, dt, 0, 0); }
+extern "C" int sdmd_gpu_advance(sdmd_gpu_ctx *c, int32_t s, double dt) {
+    if (!c || s < 0 || s >= c->nsys) return SDMD_EINVAL;
+    if (c->mode != SDMD_MODE_PLAIN) return SDMD_EUNSUPPORTED;
+    const int blocks = (c->host_sys[s].N + 255) / 256;
+    hipLaunchKernelGGL(k_advance, dim3(blocks < 1024 ? blocks : 1024), dim3(256), 0, c->stream, c->dev_sys, s, dt, c->status);
+    return op_result(c, s);
+}
 extern "C" int sdmd_gpu_do_event(sdmd_gpu_ctx *c, int32_t s, int32_t t, int32_t p) {
     if (!c || s < 0 || s >= c->nsys || t < 1 || t > c->host_sys[s].N || p < 0 || p > c->host_sys[s].N) return SDMD_EINVAL;
-    return run_op(c, s, OP_DO_EVENT, nullptr, 0, t, p);
+    return run_op(c, s, OP_DO_EVENT, nullptr, t, p);
 }
 extern "C" int sdmd_gpu_cell_move(sdmd_gpu_ctx *c, int32_t s, int32_t a) {
     if (!c || s < 0 || s >= c->nsys || a < 1 || a > c->host_sys[s].N) return SDMD_EINVAL;
-    return run_op(c, s, OP_CELL_MOVE, nullptr, 0, a, 0);
+    return run_op(c, s, OP_CELL_MOVE, nullptr, a, 0);
 }
 
 extern "C" int sdmd_gpu_pop(sdmd_gpu_ctx *c, int32_t s, sdmd_gpu_event *out) {
     if (!c || s < 0 || s >= c->nsys || !out) return SDMD_EINVAL;
     if (c->mode != SDMD_MODE_PLAIN) return SDMD_EUNSUPPORTED;
-    const Sys &S = c->host_sys[s];
-    int root = 0;
-    if (hipMemcpy(&root, S.node + 1, sizeof(int), hipMemcpyDeviceToHost) != hipSuccess) return SDMD_EDEVICE;
-    if (root < 1 || root > S.N) return SDMD_ESTATE;
-    out->target = root;
-    if (hipMemcpy(&out->partner, S.evp + root, sizeof(int), hipMemcpyDeviceToHost) != hipSuccess ||
-        hipMemcpy(&out->type, S.evtype + root, sizeof(int), hipMemcpyDeviceToHost) != hipSuccess ||
-        hipMemcpy(&out->sub, S.evsub + root, sizeof(int), hipMemcpyDeviceToHost) != hipSuccess ||
-        hipMemcpy(&out->time, S.evt + root, sizeof(double), hipMemcpyDeviceToHost) != hipSuccess ||
-        hipMemcpy(&out->potential, S.evpot + root, sizeof(double), hipMemcpyDeviceToHost) != hipSuccess)
-        return SDMD_EDEVICE;
-    out->stale = 0;
-    out->pad = 0;
-    if (out->partner > 0) {   // HazardCheck, SGThread.c:224-227
-        long long pc = 0, cnt = 0;
-        if (hipMemcpy(&pc, S.evpc + root, sizeof pc, hipMemcpyDeviceToHost) != hipSuccess ||
-            hipMemcpy(&cnt, S.evc + out->partner, sizeof cnt, hipMemcpyDeviceToHost) != hipSuccess)
-            return SDMD_EDEVICE;
-        out->stale = pc < cnt;
-    }
+    hipLaunchKernelGGL(k_pop, dim3(1), dim3(64), 0, c->stream, c->dev_sys, s, c->status);
+    if (hipGetLastError() != hipSuccess || hipStreamSynchronize(c->stream) != hipSuccess) return SDMD_EDEVICE;
+    if (c->status->ev.target == 0) return SDMD_ESTATE;
+    *out = c->status->ev;
     return SDMD_OK;
 }
 
@@ -2068,20 +2133,8 @@ extern "C" int sdmd_gpu_download(sdmd_gpu_ctx *c, int32_t s, sdmd_system_desc *d
     if (rc) return rc;
     const Sys &S = c->host_sys[s];
     if (d->natom != S.N) return SDMD_EINVAL;
-    const size_t N1 = (size_t)S.N + 1;
-#define DOWN(dst, src, n) if (dst && hipMemcpy(dst, src, sizeof(*(dst)) * (n), hipMemcpyDeviceToHost) != hipSuccess) return SDMD_EDEVICE
-    DOWN(d->x, S.x, N1); DOWN(d->y, S.y, N1); DOWN(d->z, S.z, N1);
-    DOWN(d->vx, S.vx, N1); DOWN(d->vy, S.vy, N1); DOWN(d->vz, S.vz, N1);
-    DOWN(d->type, S.type, N1);
-    DOWN(d->cellx, S.cx, N1); DOWN(d->celly, S.cy, N1); DOWN(d->cellz, S.cz, N1);
-    DOWN(d->hb_bond, S.hbbond, N1); DOWN(d->hb_itype, S.hbitype, N1);
-    DOWN(d->nb_partner, S.nbp, N1 * SDMD_NBSLOTS); DOWN(d->nb_partnernum, S.nbnum, N1); DOWN(d->nb_status, S.nbstat, N1);
-    DOWN(d->dyn_j, S.dynj, N1 * SDMD_DYNSLOTS); DOWN(d->dyn_bits, S.dynb, N1 * SDMD_DYNSLOTS);
-    DOWN(d->ev_partner, S.evp, N1); DOWN(d->ev_type, S.evtype, N1); DOWN(d->ev_sub, S.evsub, N1);
-    DOWN((long long *)d->ev_counter, S.evc, N1); DOWN((long long *)d->ev_pcounter, S.evpc, N1);
-    DOWN(d->ev_time, S.evt, N1); DOWN(d->ev_pot, S.evpot, N1);
-    DOWN(d->celllist, S.celllist, (size_t)S.ncelllist);
-#undef DOWN
+    if ((rc = sdmd_dyn_download(c, s))) return rc;
+    sdmd_dyn_scatter(c, s, d);
     d->currenttime = S.currenttime;
     return SDMD_OK;
 }
