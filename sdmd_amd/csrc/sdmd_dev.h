@@ -37,8 +37,21 @@ enum { ERR_NONE = 0, ERR_TABLE = 1, ERR_HBMODEL = 2, ERR_SUBTYPE = 3, ERR_PHI_NA
 // (not flat) loads and stores, which do not serialise against LDS traffic.
 template <class T>
 using gptr_t = __attribute__((address_space(1))) T *;
+// An int index becomes a 32-bit unsigned byte offset, which the load takes
+// beside a base in scalar registers (every array indexed by an int is below
+// 4 GiB; longer ones are indexed by 64-bit integers).
 template <class T>
-__device__ __forceinline__ gptr_t<T> G(T *p) { return (gptr_t<T>)p; }
+struct GP {
+    gptr_t<T> p;
+    __device__ __forceinline__ __attribute__((address_space(1))) T &operator[](int j) const {
+        return *(gptr_t<T>)((gptr_t<char>)p + (unsigned)j * (unsigned)sizeof(T));
+    }
+    __device__ __forceinline__ gptr_t<T> operator->() const { return p; }
+    __device__ __forceinline__ __attribute__((address_space(1))) T &operator[](size_t j) const { return p[j]; }
+    __device__ __forceinline__ __attribute__((address_space(1))) T &operator[](long long j) const { return p[j]; }
+};
+template <class T>
+__device__ __forceinline__ GP<T> G(T *p) { return {(gptr_t<T>)p}; }
 
 static __constant__ int c_OX[27] = {0, 1, 0, 0, 0, 1, 1, 1, -1, 0, 0, 0, -1, -1, -1, 0, 0, 1, -1, 1, -1, -1, -1, 1, 1, 1, -1};
 static __constant__ int c_OY[27] = {0, 0, 1, 0, 1, 0, 1, 1, 0, -1, 0, -1, 0, -1, -1, -1, 1, 0, 0, -1, 1, -1, 1, -1, 1, -1, 1};
@@ -123,7 +136,8 @@ static __device__ __forceinline__ int type_change(int t, int direct) {   // Atom
     return t;
 }
 
-static __device__ const sdmd_pair *right_pair(const Sys &S, int t1, int t2) {   // RightPair, ToolFunctions.c:278-292
+template <class SYS>
+static __device__ const sdmd_pair *right_pair(SYS &S, int t1, int t2) {   // RightPair, ToolFunctions.c:278-292
     const sdmd_pair *p = &S.pair[t1 * NT + t2];
     if (p->dmin > 0) return p;
     int a = type_change(t1, 0), b = type_change(t2, 0);
@@ -136,7 +150,8 @@ static __device__ const sdmd_pair *right_pair(const Sys &S, int t1, int t2) {   
     return nullptr;
 }
 
-static __device__ int hb_model(const Sys &S, int a1, int a2, int *err) {   // HBModel, Models.c:212-290
+template <class SYS>
+static __device__ int hb_model(SYS &S, int a1, int a2, int *err) {   // HBModel, Models.c:212-290
     if (G(S.role)[a1] == 'A' || G(S.role)[a1] == 'S') { int t = a1; a1 = a2; a2 = t; }
     int o1 = type_change(G(S.type)[a1], 0), o2 = type_change(G(S.type)[a2], 0);
     if (o1 == 2 && o2 == 26) return 1;
@@ -166,7 +181,8 @@ static __device__ int hb_model(const Sys &S, int a1, int a2, int *err) {   // HB
     return 0;
 }
 
-static __device__ double hb_barrier(const Sys &S, int a1, int a2) {   // HBBarrier, Events.c:1097-1119
+template <class SYS>
+static __device__ double hb_barrier(SYS &S, int a1, int a2) {   // HBBarrier, Events.c:1097-1119
     if (G(S.role)[a1] == 'A' || G(S.role)[a1] == 'S') { int t = a1; a1 = a2; a2 = t; }
     int o1 = type_change(G(S.type)[a1], 0), o2 = type_change(G(S.type)[a2], 0);
     if (o1 == 2 && o2 == 26) return S.hbpot[1];
@@ -178,10 +194,12 @@ static __device__ double hb_barrier(const Sys &S, int a1, int a2) {   // HBBarri
 struct FP { double lo, hi, lopot, hipot, acc; };
 
 // FindPair, ToolFunctions.c:39-224, on the flattened tables
-static __device__ __forceinline__ int shell_lookup(const Sys &S, const sdmd_pair *c, int kind, double direction,
+template <class SYS>
+static __device__ __forceinline__ int shell_lookup(SYS &S, const sdmd_pair *c, int kind, double direction,
                                                    double d2, FP &f, int a1, int a2, int *err);
 
-static __device__ int find_pair(const Sys &S, int a1, int a2, int kind, double direction, double d2, FP &f,
+template <class SYS>
+static __device__ int find_pair(SYS &S, int a1, int a2, int kind, double direction, double d2, FP &f,
                          int hbpartner, int typechange, int *err) {
     const sdmd_pair *c = nullptr;
     if (kind == K_COLLISION) {
@@ -204,7 +222,8 @@ static __device__ int find_pair(const Sys &S, int a1, int a2, int kind, double d
 }
 
 // the shell search of FindPair (ToolFunctions.c:104-224) on a resolved pair
-static __device__ __forceinline__ int shell_lookup(const Sys &S, const sdmd_pair *c, int kind, double direction,
+template <class SYS>
+static __device__ __forceinline__ int shell_lookup(SYS &S, const sdmd_pair *c, int kind, double direction,
                                                    double d2, FP &f, int a1, int a2, int *err) {
     int cs = -1;
     direction = (direction < 0) ? 1 : -1;
@@ -293,7 +312,8 @@ struct Kin { double r1, r2, r3, b, v2, rr; };
 
 // PBCShift (ToolFunctions.c:801-817) + CalculateParameters (TimePrediction.c:1081-1090)
 // with atom j's position and velocity given
-static __device__ __forceinline__ void calc_params_at(const Sys &S, double xi, double yi, double zi, double vxi,
+template <class SYS>
+static __device__ __forceinline__ void calc_params_at(SYS &S, double xi, double yi, double zi, double vxi,
                                                       double vyi, double vzi, int cxi, int cyi, int czi, int j,
                                                       double xj, double yj, double zj, double vxj, double vyj,
                                                       double vzj, Kin &k) {
@@ -322,7 +342,8 @@ static __device__ __forceinline__ void calc_params_at(const Sys &S, double xi, d
 }
 
 // the same with j's stored position and velocity
-static __device__ __forceinline__ void calc_params(const Sys &S, double xi, double yi, double zi, double vxi,
+template <class SYS>
+static __device__ __forceinline__ void calc_params(SYS &S, double xi, double yi, double zi, double vxi,
                                                    double vyi, double vzi, int cxi, int cyi, int czi, int j,
                                                    Kin &k) {
     calc_params_at(S, xi, yi, zi, vxi, vyi, vzi, cxi, cyi, czi, j, G(S.x)[j], G(S.y)[j], G(S.z)[j], G(S.vx)[j], G(S.vy)[j],
@@ -348,7 +369,8 @@ static __device__ __forceinline__ double calc_time(const Kin &k, int s, double d
 // shell, TBDEscap elsewhere).  Returns 0 when no wall event is offered.
 struct WallEv { double t, pot; int sub; };
 
-static __device__ __forceinline__ int wall_time(const Sys &S, double y, double z, double vy, double vz, int type,
+template <class SYS>
+static __device__ __forceinline__ int wall_time(SYS &S, double y, double z, double vy, double vz, int type,
                                                 WallEv &w, int *err) {
     Kin k;
     k.r1 = 0.0 - S.wallpos[1];
@@ -389,7 +411,8 @@ static __device__ __forceinline__ int wall_time(const Sys &S, double y, double z
 // immovable wall, phi = (-b + s*sqrt(b^2 - 2 d^2 U / m)) / d^2 with d^2 the
 // squared radius; WellBounc reflects, TBDCaptr / TBDEscap cross or bounce by
 // the energy test.  (y, z) is the atom's position at the event.
-static __device__ __forceinline__ void wall_event(const Sys &S, double y, double z, double &vx, double &vy,
+template <class SYS>
+static __device__ __forceinline__ void wall_event(SYS &S, double y, double z, double &vx, double &vy,
                                                   double &vz, double m, double U, int sub, int *err) {
     const double r1 = 0.0 - S.wallpos[1], r2 = y - S.wallpos[2], r3 = z - S.wallpos[3];
     const double v1 = 0.0 - 0.0, v2 = vy - 0.0, v3 = vz - 0.0;
@@ -415,7 +438,8 @@ static __device__ __forceinline__ void wall_event(const Sys &S, double y, double
     vz = vz + phi * r3;
 }
 
-static __device__ __forceinline__ int cell_index(const Sys &S, int cx, int cy, int cz, int c) {
+template <class SYS>
+static __device__ __forceinline__ int cell_index(SYS &S, int cx, int cy, int cz, int c) {
     int n1 = cx + c_OX[c], n2 = cy + c_OY[c], n3 = cz + c_OZ[c];
     if (n1 < 0) n1 = S.cellnum[1] - 1; else if (n1 >= S.cellnum[1]) n1 = 0;
     if (n2 < 0) n2 = S.cellnum[2] - 1; else if (n2 >= S.cellnum[2]) n2 = 0;
@@ -424,7 +448,8 @@ static __device__ __forceinline__ int cell_index(const Sys &S, int cx, int cy, i
 }
 
 // static + dynamic connection-map bits of row i (binary search + slots)
-static __device__ int cmap_get(const Sys &S, int i, int j) {
+template <class SYS>
+static __device__ int cmap_get(SYS &S, int i, int j) {
     int lo = G(S.cmap_off)[i], hi = G(S.cmap_off)[i + 1] - 1, bits = 0;
     while (lo <= hi) {
         int m = (lo + hi) >> 1;
@@ -446,7 +471,8 @@ static __device__ int cmap_get(const Sys &S, int i, int j) {
 // the collision table.  The shell is looked up with the direction taken from
 // the (possibly swapped) pair's velocities against the unswapped r, and the
 // accumulated energy of that shell is added.
-static __device__ double pair_energy(const Sys &S, int i, int j, double r1, double r2, double r3, double rr,
+template <class SYS>
+static __device__ double pair_energy(SYS &S, int i, int j, double r1, double r2, double r3, double rr,
                                      const double *vi, const double *vj, int *err) {
     const int bits = cmap_get(S, i, j);
     if (bits & SDMD_BOND_CONNECT) return 0;
@@ -602,7 +628,8 @@ static __device__ __forceinline__ int scan32_incl(int x) {
     return x;
 }
 
-static __device__ int check_pair_match(const Sys &S, int i, int j, int *err) {   // CheckPairMatch 1119-1138
+template <class SYS>
+static __device__ int check_pair_match(SYS &S, int i, int j, int *err) {   // CheckPairMatch 1119-1138
     int t = hb_model(S, i, j, err);
     if (t < 0) return -1;
     int ti = G(S.type)[i], tj = G(S.type)[j];

@@ -71,6 +71,9 @@ enum { FERR_SELECT = 20, FERR_SLOT = 21, FERR_ROW = 22, FERR_CAND = 23, FERR_NBL
 enum { FPH_SELECT, FPH_EXEC, FPH_STAGE, FPH_SCREEN, FPH_CONFIRM, FPH_OTHER, FPH_TREE, FPH_EVENT, FPH_BOND,
        FPH_SCAN, FPH_COLLECT };
 
+#define FPROF(prof, ph, t) do { if ((prof) && threadIdx.x == 0) { unsigned long long _n = wall_clock64(); \
+    (prof)[ph] += _n - (t); (t) = _n; } } while (0)
+
 // step radii (squared, FP32) of one constraint entry and bit k set when
 // step k carries no energy
 constexpr int PROW = 16;          // steps per collision pair at most
@@ -112,6 +115,24 @@ struct FSys {
     double max_screen_err, max_time_err, tlast;
 };
 
+// ---------------------------------------------------------------- fixed view
+// A system's struct as constant memory: what a launch does not change
+// (pointers, sizes, tables) is read through this view into scalar registers,
+// where the copy in LDS costs a wait per use.  Counters, epoch and clock are
+// read and written in the LDS copy only.
+typedef const __attribute__((address_space(4))) FSys FV;
+typedef const __attribute__((address_space(4))) Sys SV;
+__device__ __forceinline__ FV &fixed_view(const FSys *p) { return *(FV *)p; }
+// the same view, read anew: the compiler keeps nothing it read before across
+// this point (a hundred values held over the whole event loop would be moved
+// through vector registers, two instructions per use; a scalar load fetches
+// sixteen words with one)
+__device__ __forceinline__ FV &view_anew(FV &F) {
+    FV *p = &F;
+    asm volatile("" : "+s"(p));
+    return *p;
+}
+
 // ---------------------------------------------------------------- RNG
 // Philox4x32-10 (Salmon, Moraes, Dror, Shaw, SC'11), Box-Muller normal.
 __device__ __forceinline__ void philox10(unsigned int c[4], unsigned int k0, unsigned int k1) {
@@ -127,7 +148,8 @@ __device__ __forceinline__ void philox10(unsigned int c[4], unsigned int k0, uns
 }
 
 // the four words of draw number `ctr` of atom a
-__device__ __forceinline__ void normal_words(const FSys &F, int a, unsigned int ctr, unsigned int c[4]) {
+template <class FS>
+__device__ __forceinline__ void normal_words(FS &F, int a, unsigned int ctr, unsigned int c[4]) {
     c[0] = (unsigned int)a; c[1] = ctr; c[2] = 0x5344u; c[3] = 0x4d44u;
     philox10(c, F.key0, F.key1);
 }
@@ -189,7 +211,8 @@ __device__ __forceinline__ double uni(double v) { return __longlong_as_double(un
 __device__ __forceinline__ float uni(float v) { return __int_as_float(uni(__float_as_int(v))); }
 
 // ---------------------------------------------------------------- state access
-__device__ __forceinline__ int cell_id(const Sys &S, int cx, int cy, int cz) {
+template <class SYS>
+__device__ __forceinline__ int cell_id(SYS &S, int cx, int cy, int cz) {
     return cz * S.cellnum[1] * S.cellnum[2] + cy * S.cellnum[1] + cx + 1;
 }
 
@@ -220,15 +243,15 @@ __device__ __forceinline__ void advance(FSys &F, int a, double t) {
 }
 
 // mirror record of atom a (position at t0, expressed at epoch Te)
-__device__ void put_record(FSys &F, int a) {
-    const Sys &S = F.s;
+__device__ __forceinline__ void put_record(FV &F, double Te, int a) {
+    SV &S = F.s;
     const int cx = G(S.cx)[a], cy = G(S.cy)[a], cz = G(S.cz)[a];
     const size_t at = (size_t)cell_id(S, cx, cy, cz) * F.cap + G(F.slot)[a];
     fvec4 r0, r1;
     r0.x = (float)(G(S.x)[a] - cx * S.cellsize[1]);
     r0.y = (float)(G(S.y)[a] - cy * S.cellsize[2]);
     r0.z = (float)(G(S.z)[a] - cz * S.cellsize[3]);
-    r0.w = (float)(G(F.t0)[a] - F.Te);
+    r0.w = (float)(G(F.t0)[a] - Te);
     r1.x = (float)G(S.vx)[a];
     r1.y = (float)G(S.vy)[a];
     r1.z = (float)G(S.vz)[a];
@@ -238,21 +261,20 @@ __device__ void put_record(FSys &F, int a) {
 }
 
 // ---------------------------------------------------------------- predicted atom
-// The first members are loaded by one wavefront, one per lane: lanes 0..6
-// eight bytes each, lanes 7..31 four (ScrTab's gather map).
+// Its fields are loaded by one wavefront, one per lane (ScrTab's gather map:
+// lanes 0..6 eight bytes each, lanes 7..31 four), and kept in scalar
+// registers: every lane uses them, and an LDS read costs a lone wavefront
+// more than a hundred cycles each time it is waited for.
 struct FAtom {
-    double x, y, z, vx, vy, vz;
-    long long counter;
+    double x, y, z, vx, vy, vz, t;
+    int i, role, cx, cy, cz, type, hbbond, hbnb, protein, aanum, nbstat, nbnum, nb1, hbit;
+    int co;                      // con_off at i
     unsigned int rctr;           // its thermostat draw counter
-    int cx, cy, cz, type, hbbond, hbnb, protein, aanum, nbstat, nbnum;
-    int nbp[SDMD_NBSLOTS];
-    int pad23, ro, ro1, bo, bo1, co, co1, hbit, pad31;   // cmap_off, bond_off, con_off at i and i + 1
-    double t;
-    int i, role, rowlo, ncon;
-    int spanok;                  // the static row spans < 128 atom ids: byte lookup
-    float s0[3], s1[3];          // the atom's own mirror record (position at t, velocity)
+    int rowlo, spanok;           // static row: first column; its span is < 128 atom ids (byte lookup)
+    bool hbscan;                 // a free H-bond atom: its neighbourhood is scanned for partners
+    float tfloor;                // lower bound of the next thermostat draw's |normal|
+    double pcc;                  // lane 0..2: cell-crossing time along that axis (or infinite)
 };
-static_assert(offsetof(FAtom, rctr) == 56 && offsetof(FAtom, pad31) == 56 + 4 * 24, "lane map of the gather");
 
 // statistics accumulated per wave, added to the system at the end
 struct WStats { long long screen, conf, fp64, cand; };
@@ -263,7 +285,8 @@ struct Best {
     int partner, type, sub;
 };
 
-__device__ __forceinline__ void take(Best &B, const Sys &S, double t, double pot, int sub, int type, int j) {
+template <class SYS>
+__device__ __forceinline__ void take(Best &B, SYS &S, double t, double pot, int sub, int type, int j) {
     // JobAssign, TimePrediction.c:1140-1158: strictly earlier and positive
     if (t > 0 && B.t > t) {
         B.t = t; B.pot = pot; B.sub = sub; B.type = type;
@@ -274,13 +297,14 @@ __device__ __forceinline__ void take(Best &B, const Sys &S, double t, double pot
 
 constexpr int FCON = 16;          // constraint partners staged per predicted atom
 constexpr int FCONSTEP = 8;       // steps per staged constraint
+constexpr int FMARK = 32;         // words of first-candidate marks
 
 // Per-wavefront LDS.  NL: candidates inside the scan radius listed for the
 // screen (25 to 60 at most sizes; a longer list takes the unlisted path).
 template <int NL>
 struct FWave {
     static constexpr int LIST = NL;
-    FAtom a;                     // the atom being predicted (uniform across the wave)
+    int nbp[SDMD_NBSLOTS];       // the predicted atom's neighborPartner
     union {
         // its bonded partners' states (lanes 32..47 stage bond q = lane - 32)
         struct {
@@ -300,9 +324,15 @@ struct FWave {
     int l_k[NL];                 // candidate index; bit 31: its local time is later than the reader's
     long long bcj[16];
     int bjj[16];
+    // the neighbour cells that hold candidates, in scan order: candidate k of
+    // cell c has its record at slot cbase[c] + k; coff[c] is the cell's first
+    // candidate (the number of candidates past the last cell)
     int coff[28];
-    int cell[27];
-    fvec4 cof[27];               // neighbour cell c's offset times the cell size (x, y, z)
+    long long cbase[27];
+    fvec4 cof[27];               // cell c's offset times the cell size (x, y, z)
+    // bit p: candidate p + 1 is the first of its cell (a window of 64 * FMARK
+    // candidates), so that a lane counts bits instead of searching coff
+    unsigned long long mark[FMARK];
     // the predicted atom's constraint shells (FP32), CONSTRn lists
     int con_nstep[FCON];
     unsigned int con_ez[FCON];
@@ -321,7 +351,7 @@ constexpr int flist(int W) { return W <= 8 ? 256 : 128; }
 // tests (TimePrediction.c:96-118), with the staged constraint's slot; the
 // dynamic slots carry H-bond bits only
 template <class FW>
-__device__ __forceinline__ int coli_bits(const FW &wm, const Sys &S, const FAtom &A, int j) {
+__device__ __forceinline__ int coli_bits(const FW &wm, SV &S, const FAtom &A, int j) {
     if (A.spanok) {
         const unsigned off = (unsigned)(j - A.rowlo);
         return off < 128u ? wm.conn[off] : 0;
@@ -329,10 +359,11 @@ __device__ __forceinline__ int coli_bits(const FW &wm, const Sys &S, const FAtom
     return cmap_get(S, A.i, j) & (SDMD_BOND_CONNECT | SDMD_CONSTRAINT_CONNECT);
 }
 
-__device__ __forceinline__ int fin_nb_list(const FAtom &A, int j) {
+template <class FW>
+__device__ __forceinline__ int fin_nb_list(const FW &wm, const FAtom &A, int j) {
     for (int k = 1; k < SDMD_NBSLOTS; k++) {
-        if (A.nbp[k] == 0) return 0;
-        if (A.nbp[k] == j) return k;
+        if (wm.nbp[k] == 0) return 0;
+        if (wm.nbp[k] == j) return k;
     }
     if (A.nbnum == 0) return 0;
     if (A.nbnum == j) return 5;
@@ -342,8 +373,8 @@ __device__ __forceinline__ int fin_nb_list(const FAtom &A, int j) {
 }
 
 // pair kinematics for atom A (at its time) and j (local state advanced to A.t)
-__device__ __forceinline__ void kin_local(const FSys &F, const FAtom &A, int j, Kin &k, bool *late = nullptr) {
-    const Sys &S = F.s;
+__device__ __forceinline__ void kin_local(FV &F, const FAtom &A, int j, Kin &k, bool *late = nullptr) {
+    SV &S = F.s;
     const double dt = A.t - G(F.t0)[j];
     if (late) *late = dt < 0;                  // j's state is later than A's time
     const double vxj = G(S.vx)[j], vyj = G(S.vy)[j], vzj = G(S.vz)[j];
@@ -356,9 +387,9 @@ __device__ __forceinline__ void kin_local(const FSys &F, const FAtom &A, int j, 
 // rp: the resolved collision pair of (A.type, type of j) (RightPair,
 // ToolFunctions.c:278-292), known from the screen, so the table entry loads
 // with j's state instead of after it
-__device__ double coli64(const FSys &F, const FAtom &A, int j, int bits, int rp, double calib, double &pot, int &sub,
+__device__ __forceinline__ double coli64(FV &F, const FAtom &A, int j, int bits, int rp, double calib, double &pot, int &sub,
                          bool &reached, bool &late, int *err) {
-    const Sys &S = F.s;
+    SV &S = F.s;
     reached = false;
     pot = 0;
     sub = SDMD_INVALID_INTER;
@@ -562,6 +593,9 @@ __device__ __forceinline__ void wave_best(Best &mine, int k, const Best &running
 // the bond entry of this lane (lanes < bond count).  No memory fence: the
 // LDS data is shared within the wave only, whose LDS operations execute in
 // order, so independent global loads stay in flight across the stages.
+// the predicted atom's mirror record (position, velocity, time since the epoch)
+struct Own { float x, y, z, vx, vy, vz, t; };
+
 struct BondPre {
     int j, sub;
     double lo, hi, xj, yj, zj, vxj, vyj, vzj, t0j;
@@ -583,8 +617,8 @@ __device__ __forceinline__ int rl32(int v, int L) { return __builtin_amdgcn_read
 // all lanes (indices clamped into range, results masked afterwards), so a
 // level costs one memory latency.
 template <class FW>
-__device__ __forceinline__ void fstage(FSys &F, const ScrTab &T, FW &wm, FAtom &A, int i, double t, int &nb) {
-    const Sys &S = F.s;
+__device__ __forceinline__ void fstage(FV &F, const ScrTab &T, FW &wm, FAtom &A, int i, double t, int &nb, Own &own) {
+    SV &S = F.s;
     const int lane = threadIdx.x & 63;
     i = uni(i);
     t = uni(t);
@@ -600,16 +634,22 @@ __device__ __forceinline__ void fstage(FSys &F, const ScrTab &T, FW &wm, FAtom &
     const int o = rl32(lo, 24), nrow = rl32(lo, 25) - o;
     nb = rl32(lo, 27) - rl32(lo, 26);
     const int co = rl32(lo, 28), ncon = rl32(lo, 29) - co;
-    if (lane < 7) ((long long *)&A)[lane] = w;
-    else if (lane < 32) ((int *)&A.rctr)[lane - 7] = lo;
-    if (lane < 3) {
+    if (lane >= 18 && lane < 18 + SDMD_NBSLOTS) wm.nbp[lane - 18] = lo;
+    const double p = __longlong_as_double(w);
+    A.x = lane_get(p, 0); A.y = lane_get(p, 1); A.z = lane_get(p, 2);
+    A.vx = lane_get(p, 3); A.vy = lane_get(p, 4); A.vz = lane_get(p, 5);
+    A.t = t; A.i = i; A.role = uni(role); A.cx = cx; A.cy = cy; A.cz = cz; A.co = co;
+    A.rctr = (unsigned)rl32(lo, 7);
+    A.type = rl32(lo, 11); A.hbbond = rl32(lo, 12); A.hbnb = rl32(lo, 13); A.protein = rl32(lo, 14);
+    A.aanum = rl32(lo, 15); A.nbstat = rl32(lo, 16); A.nbnum = rl32(lo, 17); A.nb1 = rl32(lo, 19);
+    A.hbit = rl32(lo, 30);
+    A.hbscan = A.hbit != SDMD_HBSKIP && A.hbbond <= 0 && (A.role == 'A' || A.role == 'D' || A.role == 'S');
+    {
         // own mirror record, as put_record writes it for a state at time t
-        const int c = lane == 0 ? cx : lane == 1 ? cy : cz;
-        A.s0[lane] = (float)(__longlong_as_double(w) - c * S.cellsize[lane + 1]);
-    } else if (lane < 6) {
-        A.s1[lane - 3] = (float)__longlong_as_double(w);
-    } else if (lane == 6) {
-        A.i = i; A.t = t; A.role = role; A.ncon = ncon;
+        const int ax = min(lane, 2), c = ax == 0 ? cx : ax == 1 ? cy : cz;
+        const float f = (float)(lane < 3 ? p - c * S.cellsize[ax + 1] : p);
+        own.x = lane_get(f, 0); own.y = lane_get(f, 1); own.z = lane_get(f, 2);
+        own.vx = lane_get(f, 3); own.vy = lane_get(f, 4); own.vz = lane_get(f, 5);
     }
     // ---- level 2
     int rj = 0, rb = 0, rc = 0;
@@ -658,6 +698,38 @@ __device__ __forceinline__ void fstage(FSys &F, const ScrTab &T, FW &wm, FAtom &
     }
     int cnt = G(F.ccnt)[cell];
     if (lane >= 27) cnt = 0;
+    if (lane < FMARK) wm.mark[lane] = 0;
+    // a cell farther from the atom than the scan radius holds no candidate:
+    // an atom lies inside its cell until its cell-crossing event (FP32
+    // rounding and the crossing's 1e-8 A are far below the margin).  The scan
+    // radius is 0.9 cells or less, which leaves 17 cells of 27.
+    bool reach;
+    {
+        const float lx = own.x, ly = own.y, lz = own.z;
+        const int cl = lane < 27 ? lane : 0, ox = c_OX[cl], oy = c_OY[cl], oz = c_OZ[cl];
+        const float m = 0.02f;
+        const float dx = ox == 0 ? 0.f : fmaxf((ox < 0 ? lx : F.L32[0] - lx) - m, 0.f);
+        const float dy = oy == 0 ? 0.f : fmaxf((oy < 0 ? ly : F.L32[1] - ly) - m, 0.f);
+        const float dz = oz == 0 ? 0.f : fmaxf((oz < 0 ? lz : F.L32[2] - lz) - m, 0.f);
+        const float c2 = (float)((S.cutoffr * SDMD_EXTEND_RATIO) * (S.cutoffr * SDMD_EXTEND_RATIO));
+        reach = dx * dx + dy * dy + dz * dz <= c2 + (2e-5f * c2 + 1e-5f);
+    }
+    // PBCandCrossCellTime, TimePrediction.c:598-632, one axis per lane
+    {
+        const int ax = min(lane, 2);
+        const double v = ax == 0 ? A.vx : ax == 1 ? A.vy : A.vz;
+        const int ci = ax == 0 ? cx : ax == 1 ? cy : cz;
+        const double cs = S.cellsize[ax + 1];
+        const double tt = (v > 0 ? (ci + 1) * cs - p + ZERO : ci * cs - p - ZERO) / v;
+        A.pcc = (v != 0 && tt > 0) ? tt : __builtin_inf();
+    }
+    // the thermostat draw's lower bound (while the loads above are in flight)
+    A.tfloor = 0.f;
+    if (S.thermostat) {
+        unsigned int c[4];
+        normal_words(F, i, A.rctr, c);
+        A.tfloor = normal_floor(c[0], c[2]);
+    }
     // bonded partners' states (any valid atom on other lanes)
     {
         const int j = bj;
@@ -688,7 +760,8 @@ __device__ __forceinline__ void fstage(FSys &F, const ScrTab &T, FW &wm, FAtom &
             wm.conn[rj - rowlo] = (unsigned char)((rb & (SDMD_BOND_CONNECT | SDMD_CONSTRAINT_CONNECT)) |
                                                   (staged ? (slot + 1) << 2 : 0));
         }
-        if (lane == 0) { A.rowlo = rowlo; A.spanok = spanok; }
+        A.rowlo = rowlo;
+        A.spanok = spanok;
         if (own_con) {
             wm.con_dmin[lane] = (float)cdmin;
             wm.con_dmax[lane] = (float)cdmax;
@@ -698,24 +771,37 @@ __device__ __forceinline__ void fstage(FSys &F, const ScrTab &T, FW &wm, FAtom &
             for (int k = 0; k < FCONSTEP; k++) wm.con_rad[lane][k] = rad[k];
         }
     }
-    if (lane < 27) {
-        wm.cell[lane] = cell;
-        fvec4 co4;
-        co4.x = c_OX[lane] * F.L32[0];
-        co4.y = c_OY[lane] * F.L32[1];
-        co4.z = c_OZ[lane] * F.L32[2];
-        co4.w = 0.f;
-        wm.cof[lane] = co4;
+    // the cells in reach that hold atoms, packed in scan order, and the marks
+    // of their first candidates; one prefix sum for the candidates in reach
+    // (high half) and for those of all 27 cells (low half)
+    {
+        const bool keep = reach && cnt > 0;
+        const int incl = scan32_incl(cnt | (keep ? cnt << 16 : 0));
+        const int tot = lane_get(incl, 26), n = tot >> 16;
+        const int start = (incl >> 16) - cnt;
+        const unsigned km = (unsigned)(__ballot(keep) & 0x7ffffffu), below = (1u << (lane & 31)) - 1;
+        const int nc = __popc(km), at = __popc(km & below);
+        if (lane < 27 && keep) {
+            fvec4 co4;
+            co4.x = c_OX[lane] * F.L32[0];
+            co4.y = c_OY[lane] * F.L32[1];
+            co4.z = c_OZ[lane] * F.L32[2];
+            co4.w = 0.f;
+            wm.cof[at] = co4;
+            wm.cbase[at] = (long long)cell * F.cap - start;
+            wm.coff[at] = start;
+            if (start > 0 && start <= 64 * FMARK) atomicOr(&wm.mark[(start - 1) >> 6], 1ull << ((start - 1) & 63));
+        } else if (lane < 28) {
+            wm.coff[nc + __popc(~km & below)] = n;
+        }
+        if (lane == 0) wm.st.cand += (tot & 0xffff) - 1;
     }
-    const int incl = scan32_incl(cnt);
-    if (lane < 27) wm.coff[lane + 1] = incl;
-    if (lane == 0) wm.coff[0] = 0;
     wave_sync();
 }
 
 // BondTime entry (TimePrediction.c:219-293) from the staged partner state
-__device__ __forceinline__ double bond64_pre(const FSys &F, const FAtom &A, const BondPre &bp, int &sub) {
-    const Sys &S = F.s;
+__device__ __forceinline__ double bond64_pre(FV &F, const FAtom &A, const BondPre &bp, int &sub) {
+    SV &S = F.s;
     const int j = bp.j;
     const double dt = A.t - bp.t0j;
     Kin k;
@@ -740,6 +826,7 @@ __device__ __forceinline__ double bond64_pre(const FSys &F, const FAtom &A, cons
     return (t > 0) ? t : __builtin_inf();
 }
 
+// cell of candidate k by search (the scans that do not go in order)
 template <class FW>
 __device__ __forceinline__ int cand_cell(const FW &wm, int k) {
     int lo = 0, hi = 26;                 // largest c with coff[c] <= k
@@ -750,19 +837,57 @@ __device__ __forceinline__ int cand_cell(const FW &wm, int k) {
     return lo;
 }
 
+// the marks of the window of candidates that begins at `base`
+template <class FW>
+__device__ __forceinline__ void mark_window(FW &wm, int base, int n) {
+    const int lane = threadIdx.x & 63;
+    if (lane < FMARK) wm.mark[lane] = 0;
+    wave_sync();
+    if (lane < 27) {
+        const int s = wm.coff[lane], p = s - 1 - base;
+        if (s < n && p >= 0 && p < 64 * FMARK) atomicOr(&wm.mark[p >> 6], 1ull << (p & 63));
+    }
+    wave_sync();
+}
+
+// the mirror records of candidates base .. base + 64 * FQ - 1, whose loads
+// issue together; `first`: cells that begin at or before candidate `base`,
+// less one.  Lanes past the last candidate re-read it.
+template <int FQ>
+struct Group {
+    fvec4 r0[FQ], r1[FQ];
+    int cq[FQ];
+};
+template <int FQ, class FW>
+__device__ __forceinline__ void load_group(FV &F, const FW &wm, int base, int n, int &first, Group<FQ> &g) {
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int q = 0; q < FQ; q++) {
+        if (base + 64 * q < n) {                           // uniform
+            const unsigned long long m = (unsigned long long)uni((long long)wm.mark[((base >> 6) + q) & (FMARK - 1)]);
+            const int c = first + __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0));
+            first += __popcll(m);
+            const size_t at = (size_t)(wm.cbase[c] + min(base + lane + 64 * q, n - 1));
+            g.cq[q] = c;
+            g.r0[q] = G(F.rec)[2 * at];
+            g.r1[q] = G(F.rec)[2 * at + 1];
+        }
+    }
+}
+
 // kinematics of a candidate from its mirror record (r0, r1) in neighbour
-// cell c, in FP32
+// cell c, in FP32, against the atom's own record
 struct Near { float rr, b, v2, dt; };
 template <class FW>
-__device__ __forceinline__ Near near_at(const FW &wm, const FAtom &A, int c, const fvec4 &r0, const fvec4 &r1, float tA) {
+__device__ __forceinline__ Near near_at(const FW &wm, const Own &A, int c, const fvec4 &r0, const fvec4 &r1) {
     Near o;
-    o.dt = tA - r0.w;
+    o.dt = A.t - r0.w;
     const fvec4 co = wm.cof[c];
-    const float rx = A.s0[0] - (r0.x + r1.x * o.dt) - co.x;
-    const float ry = A.s0[1] - (r0.y + r1.y * o.dt) - co.y;
-    const float rz = A.s0[2] - (r0.z + r1.z * o.dt) - co.z;
+    const float rx = A.x - (r0.x + r1.x * o.dt) - co.x;
+    const float ry = A.y - (r0.y + r1.y * o.dt) - co.y;
+    const float rz = A.z - (r0.z + r1.z * o.dt) - co.z;
     o.rr = rx * rx + ry * ry + rz * rz;
-    const float vx = A.s1[0] - r1.x, vy = A.s1[1] - r1.y, vz = A.s1[2] - r1.z;
+    const float vx = A.vx - r1.x, vy = A.vy - r1.y, vz = A.vz - r1.z;
     o.b = rx * vx + ry * vy + rz * vz;
     o.v2 = vx * vx + vy * vy + vz * vz;
     return o;
@@ -779,15 +904,15 @@ struct CandS {
 };
 
 template <class FW>
-__device__ __forceinline__ void screen_near(const FSys &F, const ScrTab &T, const FW &wm, const FAtom &A, int id, float rr,
-                                            float b, float v2, float rsafe, CandS &o) {
-    const Sys &S = F.s;
+__device__ __forceinline__ void screen_near(FV &F, const ScrTab &T, const FW &wm, const FAtom &A, int id,
+                                            float rr, float b, float v2, float rsafe, CandS &o) {
+    SV &S = F.s;
     o.t = FINF; o.e = 0; o.flag = false; o.live = false; o.rp = -1; o.ks = 0; o.slot = -1;
     const int j = id >> 8, tj = id & 255;
     o.j = j;
     const int cb = coli_bits(wm, S, A, j);
     o.bits = cb & (SDMD_BOND_CONNECT | SDMD_CONSTRAINT_CONNECT);
-    if ((cb & SDMD_BOND_CONNECT) || A.hbbond == j || fin_nb_list(A, j)) return;
+    if ((cb & SDMD_BOND_CONNECT) || A.hbbond == j || (A.nb1 && fin_nb_list(wm, A, j))) return;
     o.live = true;
     const bool con = cb & SDMD_CONSTRAINT_CONNECT;
     Shell c;
@@ -815,9 +940,9 @@ __device__ __forceinline__ void screen_near(const FSys &F, const ScrTab &T, cons
 // limits and energies load together with j's state (one round trip).
 // Returns +inf when it does not reach JobAssign.
 template <class FW>
-__device__ __forceinline__ double coli64_shell(const FSys &F, const ScrTab &T, const FW &wm, const FAtom &A, int id, int ks,
+__device__ __forceinline__ double coli64_shell(FV &F, const ScrTab &T, const FW &wm, const FAtom &A, int id, int ks,
                                                int slot, double &pot, int &sub, long long &pc, bool &late) {
-    const Sys &S = F.s;
+    SV &S = F.s;
     const int j = id >> 8;
     const bool con = slot >= 0;
     const ScrPair sp = T.pr[A.type * NT + (id & 255)];
@@ -856,6 +981,9 @@ __device__ __forceinline__ double coli64_shell(const FSys &F, const ScrTab &T, c
 
 // FQ: candidates per lane whose records are loaded together
 
+// HBTime's bookkeeping of listed candidate `lane`
+struct HBPre { int role, aanum, protein, hbbond; };
+
 // Screened CollisionTime: the candidates inside the scan radius are listed
 // in LDS (a quarter of the neighbourhood), screened in FP32 one per lane, and
 // the marked ones and those whose interval reaches the smallest upper bound
@@ -868,17 +996,18 @@ __device__ __forceinline__ double coli64_shell(const FSys &F, const ScrTab &T, c
 // full scan's winner compared), a separate instantiation so that the
 // screened path carries none of its state
 template <int FQ, bool VAL, class FW>
-__device__ __forceinline__ void collision_fast(FSys &F, const ScrTab &T, FW &wm, const FAtom &A, Best &best, long long &nscreen,
-                               long long &nconf, int *err) {
-    const Sys &S = F.s;
-    unsigned long long pt = S.prof ? wall_clock64() : 0;
+__device__ __forceinline__ void collision_fast(FSys &M, FV &F, unsigned long long *prof, const ScrTab &T, FW &wm, const FAtom &A, const Own &own,
+                                               Group<FQ> &g, int first, HBPre &hp, Best &best, long long &nscreen,
+                                               long long &nconf, int *err) {
+    SV &S = F.s;
+    unsigned long long pt = prof ? wall_clock64() : 0;
     const int lane = threadIdx.x & 63;
     const int n = uni(wm.coff[27]);
     const double calib64 = (S.cutoffr * SDMD_EXTEND_RATIO) * (S.cutoffr * SDMD_EXTEND_RATIO);
     const float calib = (float)calib64;
     const float cband = 2e-5f * calib + 1e-5f, rscan = calib + cband, rsafe = calib - cband;
-    const float tA = (float)(A.t - F.Te);
-    int my_screen = 0, my_causal = 0, my_conf = 0;
+    int screened = 0, confirmed = 0;                       // wave-uniform
+    int my_causal = 0;
     Best mine;
     mine.t = __builtin_inf(); mine.pot = 0; mine.pc = 0; mine.partner = INVALID; mine.type = SDMD_COLI; mine.sub = 0;
     int mink = 0x7fffffff;
@@ -900,7 +1029,6 @@ __device__ __forceinline__ void collision_fast(FSys &F, const ScrTab &T, FW &wm,
                 t = coli64_shell(F, T, wm, A, id, ks, slot, pot, sub, pc, late);
             }
             my_causal += late ? 1 : 0;             // FP64 check of the screen's FP32 time order
-            my_conf++;
             if (t < mine.t) { mine.t = t; mine.pot = pot; mine.sub = sub; mine.partner = id >> 8; mine.pc = pc; mink = k; myt32 = t32; }
         }
         if constexpr (VAL) {
@@ -912,26 +1040,13 @@ __device__ __forceinline__ void collision_fast(FSys &F, const ScrTab &T, FW &wm,
     };
     // ---- the candidates inside the scan radius, in candidate order
     int near = 0;
-    for (int base = 0; base < n; base += 64 * FQ) {
-        fvec4 r0[FQ], r1[FQ];
-        int cq[FQ];
-        // every lane loads a record for every slot (slots past the last
-        // candidate re-read the last one), so the loads issue together
-#pragma unroll
-        for (int q = 0; q < FQ; q++) {
-            const int k = min(base + lane + 64 * q, n - 1);
-            const int c = cand_cell(wm, k);
-            const size_t at = (size_t)wm.cell[c] * F.cap + (k - wm.coff[c]);
-            cq[q] = c;
-            r0[q] = G(F.rec)[2 * at];
-            r1[q] = G(F.rec)[2 * at + 1];
-        }
+    for (int base = 0; base < n;) {
 #pragma unroll
         for (int q = 0; q < FQ; q++) {
             const int k = base + lane + 64 * q;
             if (base + 64 * q < n) {                       // uniform
-                const int id = __float_as_int(r1[q].w), j = id >> 8;
-                const Near d = near_at(wm, A, cq[q], r0[q], r1[q], tA);
+                const int id = __float_as_int(g.r1[q].w), j = id >> 8;
+                const Near d = near_at(wm, own, g.cq[q], g.r0[q], g.r1[q]);
                 const bool nr = k < n && j >= 1 && j <= S.N && j != A.i && (id & 255) < NT && d.rr <= rscan;
                 const unsigned long long m = __ballot(nr);
                 const int r = near + __builtin_amdgcn_mbcnt_hi((unsigned int)(m >> 32),
@@ -944,28 +1059,45 @@ __device__ __forceinline__ void collision_fast(FSys &F, const ScrTab &T, FW &wm,
                 near += __popcll(m);
             }
         }
+        base += 64 * FQ;
+        if (base >= n) break;
+        if ((base & (64 * FMARK - 1)) == 0) mark_window(wm, base, n);
+        load_group<FQ>(F, wm, base, n, first, g);
     }
     wave_sync();
     if (near <= FW::LIST) {
+        // HBTime's bookkeeping of the first 64 listed candidates, in flight
+        // during the screen
+        hp.role = 0;
+        if (A.hbscan && lane < near) {
+            const int j = wm.l_id[lane] >> 8;
+            hp.role = G(S.role)[j]; hp.aanum = G(S.aanum)[j]; hp.protein = G(S.protein)[j]; hp.hbbond = G(S.hbbond)[j];
+        }
         float thi = FINF;
-        for (int r = lane; r < near; r += 64) {
+        for (int r0 = 0; r0 < near; r0 += 64) {
+            const int r = r0 + lane;
             CandS o;
+            o.live = false;
+            if (r < near) {
             screen_near(F, T, wm, A, wm.l_id[r], wm.l_rr[r], wm.l_b[r], wm.l_v2[r], rsafe, o);
-            my_screen += o.live;
             my_causal += (o.live && wm.l_k[r] < 0) ? 1 : 0;
             if (o.live && !o.flag && o.t < FINF) thi = fminf(thi, o.t + o.e);
             wm.l_t[r] = o.live ? o.t : FINF;
             wm.l_e[r] = (o.live && o.flag) ? -1.f : o.e;
             wm.l_sh[r] = o.ks | ((o.slot + 1) << 8) | (o.live ? 1 << 16 : 0);
+            }
+            screened += __popcll(__ballot(o.live));
         }
         if (lane == 0) wm.hbl_n = near;
         thi = wave_min_f(thi);
-        PROF_MARK(S, FPH_SCREEN, pt);
-        for (int r = lane; r < near; r += 64) {
-            const float t = wm.l_t[r], e = wm.l_e[r];
-            const int sh = wm.l_sh[r];
-            const bool flag = e < 0.f, need = flag || (t < FINF && t - e <= thi);
-            if (need || (VAL && (sh >> 16))) {
+        FPROF(prof, FPH_SCREEN, pt);
+        for (int r0 = 0; r0 < near; r0 += 64) {
+            const int r = r0 + lane, rl = min(r, near - 1);
+            const float t = wm.l_t[rl], e = wm.l_e[rl];
+            const int sh = wm.l_sh[rl];
+            const bool flag = e < 0.f, need = r < near && (flag || (t < FINF && t - e <= thi));
+            confirmed += __popcll(__ballot(need));
+            if (need || (VAL && r < near && (sh >> 16))) {
                 const int id = wm.l_id[r], slot = ((sh >> 8) & 255) - 1;
                 // what the FP64 search of a marked candidate needs
                 const int bits = coli_bits(wm, S, A, id >> 8) & (SDMD_BOND_CONNECT | SDMD_CONSTRAINT_CONNECT);
@@ -978,35 +1110,41 @@ __device__ __forceinline__ void collision_fast(FSys &F, const ScrTab &T, FW &wm,
         // first, then re-screen and confirm
         float thi = FINF;
         for (int pass = 0; pass < 2; pass++) {
-            for (int k = lane; k < n; k += 64) {
-                const int c = cand_cell(wm, k);
-                const size_t at = (size_t)wm.cell[c] * F.cap + (k - wm.coff[c]);
+            for (int k0 = 0; k0 < n; k0 += 64) {
+                const int k = k0 + lane, kl = min(k, n - 1);
+                const int c = cand_cell(wm, kl);
+                const size_t at = (size_t)(wm.cbase[c] + kl);
                 const fvec4 q0 = G(F.rec)[2 * at], q1 = G(F.rec)[2 * at + 1];
                 const int id = __float_as_int(q1.w), j = id >> 8;
-                const Near d = near_at(wm, A, c, q0, q1, tA);
-                if (!(j >= 1 && j <= S.N && j != A.i && (id & 255) < NT && d.rr <= rscan)) continue;
+                const Near d = near_at(wm, own, c, q0, q1);
                 CandS o;
-                screen_near(F, T, wm, A, id, d.rr, d.b, d.v2, rsafe, o);
-                if (!o.live) continue;
+                o.live = false;
+                if (k < n && j >= 1 && j <= S.N && j != A.i && (id & 255) < NT && d.rr <= rscan)
+                    screen_near(F, T, wm, A, id, d.rr, d.b, d.v2, rsafe, o);
                 if (pass == 0) {
-                    my_screen++;
-                    my_causal += d.dt < 0.f ? 1 : 0;
-                    if (!o.flag && o.t < FINF) thi = fminf(thi, o.t + o.e);
+                    screened += __popcll(__ballot(o.live));
+                    if (o.live) {
+                        my_causal += d.dt < 0.f ? 1 : 0;
+                        if (!o.flag && o.t < FINF) thi = fminf(thi, o.t + o.e);
+                    }
                 } else {
-                    const bool need = o.flag || (o.t < FINF && o.t - o.e <= thi);
-                    if (need || VAL) confirm(k, id, o.bits, o.rp, o.t, o.ks, o.slot, o.flag, need);
+                    const bool need = o.live && (o.flag || (o.t < FINF && o.t - o.e <= thi));
+                    confirmed += __popcll(__ballot(need));
+                    if (need || (VAL && o.live)) confirm(k, id, o.bits, o.rp, o.t, o.ks, o.slot, o.flag, need);
                 }
             }
             if (pass == 0) thi = wave_min_f(thi);
         }
     }
-    PROF_MARK(S, FPH_CONFIRM, pt);
-    nscreen += wave_sum_i(my_screen);
-    nconf += wave_sum_i(my_conf);
-    my_causal = wave_sum_i(my_causal);
-    if (my_causal && lane == 0) {
-        cnt_add(F.causal, my_causal);
-        *err = FERR_CAUSAL;
+    FPROF(prof, FPH_CONFIRM, pt);
+    nscreen += screened;
+    nconf += confirmed;
+    if (__ballot(my_causal != 0)) {
+        my_causal = wave_sum_i(my_causal);
+        if (lane == 0) {
+            cnt_add(M.causal, my_causal);
+            *err = FERR_CAUSAL;
+        }
     }
     // wave argmin (first minimal candidate)
     double tw = mine.t;
@@ -1018,7 +1156,7 @@ __device__ __forceinline__ void collision_fast(FSys &F, const ScrTab &T, FW &wm,
         const int src = m ? __ffsll((long long)m) - 1 : 0;
         bcast(win, src);
         const float w32 = lane_get(myt32, src);
-        if (m && lane == 0 && win.t > 0 && w32 < FINF) cnt_max(F.max_screen_err, fabs((double)w32 - win.t) / win.t);
+        if (m && lane == 0 && win.t > 0 && w32 < FINF) cnt_max(M.max_screen_err, fabs((double)w32 - win.t) / win.t);
         if (!m) win.t = __builtin_inf();
     }
     if constexpr (VAL) {
@@ -1031,11 +1169,11 @@ __device__ __forceinline__ void collision_fast(FSys &F, const ScrTab &T, FW &wm,
         bcast(fw, src);
         if (!m) fw.t = __builtin_inf();
         if (lane == 0) {
-            cnt_add(F.validated, 1);
+            cnt_add(M.validated, 1);
             const bool same = (!m && win.t == __builtin_inf()) ||
                               (fw.partner == win.partner && fw.t == win.t && fw.sub == win.sub);
-            if (same) cnt_add(F.agree, 1);
-            else if (fw.t < __builtin_inf()) cnt_max(F.max_time_err, fabs(win.t - fw.t) / fw.t);
+            if (same) cnt_add(M.agree, 1);
+            else if (fw.t < __builtin_inf()) cnt_max(M.max_time_err, fabs(win.t - fw.t) / fw.t);
         }
     }
     if (win.t < __builtin_inf() && win.partner > 0 && win.t > 0 && best.t > win.t) {
@@ -1048,50 +1186,24 @@ __device__ __forceinline__ void collision_fast(FSys &F, const ScrTab &T, FW &wm,
 // two parts: the conditions on j's bookkeeping alone (role pairing, j not
 // H-bonded, sequence separation within a chain: TimePrediction.c:420-430),
 // then distance, CheckPairMatch, FindPair and the contact time
-__device__ __forceinline__ bool hbfree_pass(const FSys &F, const FAtom &A, int j) {
-    const Sys &S = F.s;
-    if (j < 1 || j > S.N || j == A.i) return false;
-    const signed char ri = A.role, rj = G(S.role)[j];
-    const bool pairok = (ri == 'A' && rj == 'D') || (ri == 'D' && rj == 'A') ||
-                        (ri == 'S' && G(S.type)[j] == 2) || (rj == 'S' && A.type == 2) || (ri == 'S' && rj == 'S');
-    int sep = A.aanum - G(S.aanum)[j];
-    if (sep < 0) sep = -sep;
-    const int pj = G(S.protein)[j];
-    return pairok && G(S.hbbond)[j] == 0 && ((A.protein == pj && sep >= 4) || A.protein != pj);
-}
-
-// the whole candidate with j's bookkeeping and state loaded together (for
-// candidates already known to lie near A)
-__device__ __forceinline__ double hbfree_all(const FSys &F, const FAtom &A, int j, double calib, double &pot, bool &reached,
-                                             int *err) {
-    const Sys &S = F.s;
-    reached = false;
-    pot = 0;
-    const signed char rj = G(S.role)[j];
-    const int tj = G(S.type)[j], aj = G(S.aanum)[j], pj = G(S.protein)[j], hj = G(S.hbbond)[j];
-    Kin k;
-    kin_local(F, A, j, k);
-    const signed char ri = A.role;
+__device__ __forceinline__ bool hbfree_pre(const FAtom &A, const HBPre &h, int tj) {
+    const int ri = A.role, rj = h.role;
     const bool pairok = (ri == 'A' && rj == 'D') || (ri == 'D' && rj == 'A') || (ri == 'S' && tj == 2) ||
                         (rj == 'S' && A.type == 2) || (ri == 'S' && rj == 'S');
-    int sep = A.aanum - aj;
+    int sep = A.aanum - h.aanum;
     if (sep < 0) sep = -sep;
-    if (!(pairok && hj == 0 && ((A.protein == pj && sep >= 4) || A.protein != pj))) return __builtin_inf();
-    if (!(k.rr <= calib) || check_pair_match(S, A.i, j, err) < 0) return __builtin_inf();
-    FP f;
-    const int cs = find_pair(S, A.i, j, K_HB, k.b, k.rr, f, 0, 0, err);
-    reached = true;
-    if (k.b < 0 && cs == 1 && calc_disc(k, f.lo) > 0) {
-        pot = f.lopot;
-        double t = calc_time(k, -1, f.lo);
-        if (t < 0) t = INFINIT;
-        return (t > 0) ? t : __builtin_inf();
-    }
-    return __builtin_inf();
+    return pairok && h.hbbond == 0 && ((A.protein == h.protein && sep >= 4) || A.protein != h.protein);
 }
 
-__device__ double hbfree64(const FSys &F, const FAtom &A, int j, double calib, double &pot, bool &reached, int *err) {
-    const Sys &S = F.s;
+__device__ __forceinline__ bool hbfree_pass(FV &F, const FAtom &A, int j) {
+    SV &S = F.s;
+    if (j < 1 || j > S.N || j == A.i) return false;
+    const HBPre h = {G(S.role)[j], G(S.aanum)[j], G(S.protein)[j], G(S.hbbond)[j]};
+    return hbfree_pre(A, h, G(S.type)[j]);
+}
+
+__device__ __forceinline__ double hbfree64(FV &F, const FAtom &A, int j, double calib, double &pot, bool &reached, int *err) {
+    SV &S = F.s;
     reached = false;
     pot = 0;
     Kin k;
@@ -1111,16 +1223,24 @@ __device__ double hbfree64(const FSys &F, const FAtom &A, int j, double calib, d
 
 // Predict for atom i at time t (its state is at t); writes the event record
 template <int FQ, class FW>
-__device__ __forceinline__ void predict_fast(FSys &F, const ScrTab &T, FW &wm, int i, double t, WStats &ws, int *err) {
-    Sys &S = F.s;
+__device__ __forceinline__ void predict_fast(FSys &M, FV &F0, unsigned long long *prof, const ScrTab &T, FW &wm, int i,
+                                             double t, WStats &ws, int *err) {
     const int lane = threadIdx.x & 63;
     long long &nscreen = ws.screen, &nconf = ws.conf, &nfp64 = ws.fp64;
-    unsigned long long pt = S.prof ? wall_clock64() : 0;
-    FAtom &A = wm.a;
+    unsigned long long pt = prof ? wall_clock64() : 0;
+    FAtom A;
+    Own own;
     int nb = 0;
-    fstage(F, T, wm, A, i, t, nb);
-    ws.cand += wm.coff[27] - 1;
-    PROF_MARK(S, FPH_STAGE, pt);
+    fstage(view_anew(F0), T, wm, A, i, t, nb, own);
+    FV &F = view_anew(F0);
+    SV &S = F.s;
+    // the first candidates' records load during the bond times
+    const int n = uni(wm.coff[27]);
+    int first = 0;
+    Group<FQ> g;
+    load_group<FQ>(F, wm, 0, n, first, g);
+    own.t = (float)(A.t - M.Te);
+    FPROF(prof, FPH_STAGE, pt);
     if (nb > 16 && lane == 0) *err = ERR_CELLCAP;      // BondTime's connect[16], TimePrediction.c:188
     Best init;
     init.t = INFINIT; init.pot = 0; init.pc = 0; init.partner = INVALID; init.type = SDMD_INVD; init.sub = 0;
@@ -1151,42 +1271,30 @@ __device__ __forceinline__ void predict_fast(FSys &F, const ScrTab &T, FW &wm, i
         best = out;
         nfp64 += nb;
     }
-    PROF_MARK(S, FPH_BOND, pt);
+    FPROF(prof, FPH_BOND, pt);
     // CollisionTime (screened), against no running best yet
     if (lane == 0) wm.hbl_n = -1;
     wave_sync();
     Best cw = init;
     cw.t = __builtin_inf();
-    if (F.validate) collision_fast<FQ, true>(F, T, wm, A, cw, nscreen, nconf, err);
-    else collision_fast<FQ, false>(F, T, wm, A, cw, nscreen, nconf, err);
-    if (S.prof) pt = wall_clock64();
+    HBPre hp;
+    if (F.validate) collision_fast<FQ, true>(M, F, prof, T, wm, A, own, g, first, hp, cw, nscreen, nconf, err);
+    else collision_fast<FQ, false>(M, F, prof, T, wm, A, own, g, first, hp, cw, nscreen, nconf, err);
+    if (prof) pt = wall_clock64();
     // JobAssign order: bonds first, then the collision winner if strictly earlier
     if (cw.partner > 0 && cw.t > 0 && best.t > cw.t) best = cw;
-    // PBCandCrossCellTime, TimePrediction.c:598-632
+    // PBCandCrossCellTime (each axis's time from the staging)
     {
-        double t_ev = INFINIT;
-        const double pos[3] = {A.x, A.y, A.z}, v[3] = {A.vx, A.vy, A.vz};
-        const int ci[3] = {A.cx, A.cy, A.cz};
-        for (int n = 0; n < 3; n++) {
-            const double lo = ci[n] * S.cellsize[n + 1], hi = (ci[n] + 1) * S.cellsize[n + 1];
-            double tt;
-            if (v[n] > 0) {
-                tt = (hi - pos[n] + ZERO) / v[n];
-                if (t_ev > tt && tt > 0) t_ev = tt;
-            } else if (v[n] < 0) {
-                tt = (lo - pos[n] - ZERO) / v[n];
-                if (t_ev > tt && tt > 0) t_ev = tt;
-            }
-        }
+        const double t_ev = fmin(fmin(lane_get(A.pcc, 0), lane_get(A.pcc, 1)), fmin(lane_get(A.pcc, 2), INFINIT));
         take(best, S, t_ev, 0, SDMD_INVALID_INTER, SDMD_PCC, 0);
     }
     // ThermostatTime, TimePrediction.c:582-595
     if (S.thermostat) {
-        const unsigned int ctr = uni((int)A.rctr);
+        const unsigned int ctr = A.rctr;
         if (lane == 0) G(F.rctr)[i] = ctr + 1;
-        unsigned int c[4];
-        normal_words(F, uni(i), ctr, c);
-        if (!(S.thermoF * (double)normal_floor(c[0], c[2]) > best.t)) {
+        if (!(S.thermoF * (double)A.tfloor > best.t)) {
+            unsigned int c[4];
+            normal_words(F, A.i, ctr, c);
             const double z = normal_of(c[0], c[1], c[2], c[3]);
             const double tt = S.thermoF * ((z < 0) ? (-z) : (z));
             take(best, S, tt, 0, SDMD_INVALID_INTER, SDMD_THER, 0);
@@ -1206,7 +1314,7 @@ __device__ __forceinline__ void predict_fast(FSys &F, const ScrTab &T, FW &wm, i
     int pt_sub = 0;
     if (lane < nq) {
         // HBNeighborTime slot q, TimePrediction.c:486-579
-        const int j = A.nbp[lane + 1];
+        const int j = wm.nbp[lane + 1];
         Kin k;
         kin_local(F, A, j, k);
         int host, nb, partner;
@@ -1257,7 +1365,6 @@ __device__ __forceinline__ void predict_fast(FSys &F, const ScrTab &T, FW &wm, i
             // per lane (their loads issued together), then the FP64 part for
             // the candidates that pass, packed onto the wave's lanes in
             // candidate order (most candidates fail the role pairing)
-            const int n = wm.coff[27];
             Best mine = best;
             mine.t = __builtin_inf();
             int mink = 0x7fffffff;
@@ -1266,10 +1373,11 @@ __device__ __forceinline__ void predict_fast(FSys &F, const ScrTab &T, FW &wm, i
             // the candidates the screen listed inside the scan radius, in
             // candidate order; otherwise every candidate, filtered below
             for (int r = lane; r < nl; r += 64) {
-                const int j = wm.l_id[r] >> 8, k = wm.l_k[r] & 0x7fffffff;
+                const int id = wm.l_id[r], j = id >> 8, k = wm.l_k[r] & 0x7fffffff;
+                if (!(r == lane ? hbfree_pre(A, hp, id & 255) : hbfree_pass(F, A, j))) continue;
                 double pot;
                 bool reached;
-                const double tt = hbfree_all(F, A, j, calib, pot, reached, err);
+                const double tt = hbfree64(F, A, j, calib, pot, reached, err);
                 my += reached;
                 if (tt < mine.t) { mine.t = tt; mine.pot = pot; mine.partner = j; mink = k; }
             }
@@ -1282,7 +1390,7 @@ __device__ __forceinline__ void predict_fast(FSys &F, const ScrTab &T, FW &wm, i
                     jj[u] = 0;
                     if (k < n) {
                         const int c = cand_cell(wm, k);
-                        const size_t at = (size_t)wm.cell[c] * F.cap + (k - wm.coff[c]);
+                        const size_t at = (size_t)(wm.cbase[c] + k);
                         jj[u] = __float_as_int(G(F.rec)[2 * at + 1].w) >> 8;
                     }
                 }
@@ -1334,7 +1442,7 @@ __device__ __forceinline__ void predict_fast(FSys &F, const ScrTab &T, FW &wm, i
             if (flag == 0) A.nbnum = q;
             nfp64 += 1;
             if (tt > 0 && best.t > tt) {
-                take(best, S, tt, pot, sub, SDMD_HBNE, A.nbp[q]);
+                take(best, S, tt, pot, sub, SDMD_HBNE, wm.nbp[q]);
                 A.nbnum = q;
                 flag = 1;
             }
@@ -1345,7 +1453,7 @@ __device__ __forceinline__ void predict_fast(FSys &F, const ScrTab &T, FW &wm, i
         WallEv w;
         if (wall_time(S, A.y, A.z, A.vy, A.vz, A.type, w, err)) take(best, S, w.t, w.pot, w.sub, SDMD_WALL, 0);
     }
-    PROF_MARK(S, FPH_OTHER, pt);
+    FPROF(prof, FPH_OTHER, pt);
     if (lane == 0) {
         G(S.evt)[i] = t + best.t;
         G(S.evpot)[i] = best.pot;
@@ -1429,15 +1537,15 @@ __device__ void thermostat_fast(FSys &F, int i) {
 // execute one popped event on lane 0 (DoEvent, Events.c:25-114, with the
 // counter increments of SGThread.c:100-104); returns the renew count
 // mirror record of atom a from values the caller holds (as put_record)
-__device__ __forceinline__ void put_record_v(FSys &F, int a, int cx, int cy, int cz, int slot, int type, double x,
+__device__ __forceinline__ void put_record_v(FV &F, double Te, int a, int cx, int cy, int cz, int slot, int type, double x,
                                              double y, double z, double vx, double vy, double vz, double t0) {
-    const Sys &S = F.s;
+    SV &S = F.s;
     const size_t at = (size_t)cell_id(S, cx, cy, cz) * F.cap + slot;
     fvec4 r0, r1;
     r0.x = (float)(x - cx * S.cellsize[1]);
     r0.y = (float)(y - cy * S.cellsize[2]);
     r0.z = (float)(z - cz * S.cellsize[3]);
-    r0.w = (float)(t0 - F.Te);
+    r0.w = (float)(t0 - Te);
     r1.x = (float)vx;
     r1.y = (float)vy;
     r1.z = (float)vz;
@@ -1453,8 +1561,8 @@ struct PairAtom {
     int cx, cy, cz, slot, type;
 };
 
-__device__ __forceinline__ void pair_load(const FSys &F, int j, PairAtom &q) {
-    const Sys &S = F.s;
+__device__ __forceinline__ void pair_load(FV &F, int j, PairAtom &q) {
+    SV &S = F.s;
     q.x = G(S.x)[j]; q.y = G(S.y)[j]; q.z = G(S.z)[j];
     q.vx = G(S.vx)[j]; q.vy = G(S.vy)[j]; q.vz = G(S.vz)[j];
     q.t0 = G(F.t0)[j]; q.m = G(S.mass)[j]; q.c = G(S.evc)[j];
@@ -1463,8 +1571,8 @@ __device__ __forceinline__ void pair_load(const FSys &F, int j, PairAtom &q) {
 }
 
 // advance to t (as advance()) in registers, stored
-__device__ __forceinline__ void pair_advance(FSys &F, int j, PairAtom &q, double t) {
-    Sys &S = F.s;
+__device__ __forceinline__ void pair_advance(FV &F, int j, PairAtom &q, double t) {
+    SV &S = F.s;
     const double dt = t - q.t0;
     q.x = q.x + q.vx * dt;
     q.y = q.y + q.vy * dt;
@@ -1480,20 +1588,21 @@ __device__ __forceinline__ void pair_advance(FSys &F, int j, PairAtom &q, double
 // arithmetic as exec_fast's general path (advance, PosLocal, image_near,
 // interaction_event): both mirror records are written here.  Returns the
 // renewed atoms (1 when the event is stale).
-__device__ __forceinline__ int exec_pair(FSys &F, int a, int p, int ty, double t, const PairAtom &a0, long long pca,
+__device__ __forceinline__ int exec_pair(FSys &M, FV &F, int a, int p, int ty, double t, const PairAtom &a0, long long pca,
                                          double pot0, int sub0, int *renew, int *err) {
-    Sys &S = F.s;
+    SV &S = F.s;
+    const double Te = M.Te;
     PairAtom A = a0, P;
     pair_load(F, p, P);
     pair_advance(F, a, A, t);
     renew[0] = a;
     if (pca < P.c) {                                           // HazardCheck, SGThread.c:215-235
-        cnt_add(S.recal, 1);
-        put_record_v(F, a, A.cx, A.cy, A.cz, A.slot, A.type, A.x, A.y, A.z, A.vx, A.vy, A.vz, A.t0);
+        cnt_add(M.s.recal, 1);
+        put_record_v(F, Te, a, A.cx, A.cy, A.cz, A.slot, A.type, A.x, A.y, A.z, A.vx, A.vy, A.vz, A.t0);
         return 1;
     }
     if (P.t0 > t) {
-        cnt_add(F.causal, 1);
+        cnt_add(M.causal, 1);
         *err = FERR_CAUSAL;
     }
     pair_advance(F, p, P, t);
@@ -1543,12 +1652,12 @@ __device__ __forceinline__ int exec_pair(FSys &F, int a, int p, int ty, double t
             G(S.vx)[p] = P.vx; G(S.vy)[p] = P.vy; G(S.vz)[p] = P.vz;
         }
     }
-    cnt_add(S.per_type[ty], 1);
-    cnt_add(S.frame, 1);
+    cnt_add(M.s.per_type[ty], 1);
+    cnt_add(M.s.frame, 1);
     G(S.evc)[a] = A.c + 1;
     G(S.evc)[p] = P.c + 1;
-    put_record_v(F, a, A.cx, A.cy, A.cz, A.slot, A.type, A.x, A.y, A.z, A.vx, A.vy, A.vz, A.t0);
-    put_record_v(F, p, P.cx, P.cy, P.cz, P.slot, P.type, P.x, P.y, P.z, P.vx, P.vy, P.vz, P.t0);
+    put_record_v(F, Te, a, A.cx, A.cy, A.cz, A.slot, A.type, A.x, A.y, A.z, A.vx, A.vy, A.vz, A.t0);
+    put_record_v(F, Te, p, P.cx, P.cy, P.cz, P.slot, P.type, P.x, P.y, P.z, P.vx, P.vy, P.vz, P.t0);
     renew[1] = p;
     return 2;
 }
@@ -1600,8 +1709,8 @@ __device__ __attribute__((noinline)) int exec_general(FSys &F, int a, int partne
     return 1;
 }
 
-__device__ __forceinline__ int exec_fast(FSys &F, int a, double t, int *renew, int *err, bool *recs) {
-    Sys &S = F.s;
+__device__ __forceinline__ int exec_fast(FSys &M, FV &F, int a, double t, int *renew, int *err, bool *recs) {
+    SV &S = F.s;
     // the record and state of a, loaded together with its partner id
     const int p = G(S.evp)[a];
     const int ty0 = G(S.evtype)[a];
@@ -1614,9 +1723,9 @@ __device__ __forceinline__ int exec_fast(FSys &F, int a, double t, int *renew, i
     *recs = false;
     if (partner && partner != a && (ty0 == SDMD_COLI || ty0 == SDMD_BOND || ty0 == SDMD_HBNE)) {
         *recs = true;
-        return exec_pair(F, a, partner, ty0, t, a0, pca, pot0, sub0, renew, err);
+        return exec_pair(M, F, a, partner, ty0, t, a0, pca, pot0, sub0, renew, err);
     }
-    return exec_general(F, a, partner, t, renew, err);
+    return exec_general(M, a, partner, t, renew, err);
 }
 
 // ---------------------------------------------------------------- tree blocks
@@ -1647,7 +1756,7 @@ __device__ __forceinline__ void block_min3(int b, bool in, double t, int p, doub
     t1 = m; a1 = km; t2 = u; a2 = ku; t3 = w;
 }
 
-__device__ void block_scan(const FSys &F, int b, double &t1, int &a1, double &t2, int &a2, double &t3) {
+__device__ void block_scan(FV &F, int b, double &t1, int &a1, double &t2, int &a2, double &t3) {
     const int lane = threadIdx.x & 63;
     const int a = b * 64 + lane + 1;
     const bool in = a <= F.s.N;
@@ -1657,7 +1766,7 @@ __device__ void block_scan(const FSys &F, int b, double &t1, int &a1, double &t2
 }
 
 // block_scan of two blocks with their loads issued together (b1 < 0: none)
-__device__ __forceinline__ void block_scan2(const FSys &F, int b0, int b1, double &t1, int &a1, double &t2, int &a2,
+__device__ __forceinline__ void block_scan2(FV &F, int b0, int b1, double &t1, int &a1, double &t2, int &a2,
                                             double &t3, double &u1, int &c1, double &u2, int &c2, double &u3) {
     const int lane = threadIdx.x & 63;
     const int N = F.s.N;
@@ -1784,11 +1893,11 @@ __device__ __forceinline__ void fsys_store(FSys *dst, const FSys &src) {
 // FP32 mirror re-expressed at a new epoch (positions at Te, time offsets 0);
 // the FP64 state is not touched
 template <int W>
-__device__ void rebase(FSys &F, double Te) {
+__device__ void rebase(FSys &M, FV &F, double Te) {
     __syncthreads();
-    if (threadIdx.x == 0) { F.Te = Te; F.rebases++; }   // single writer between barriers
+    if (threadIdx.x == 0) { M.Te = Te; M.rebases++; }   // single writer between barriers
     __syncthreads();
-    const Sys &S = F.s;
+    SV &S = F.s;
     for (int a = threadIdx.x + 1; a <= S.N; a += 64 * W) {
         const int cx = G(S.cx)[a], cy = G(S.cy)[a], cz = G(S.cz)[a];
         const size_t at = (size_t)cell_id(S, cx, cy, cz) * F.cap + G(F.slot)[a];
@@ -1845,8 +1954,8 @@ __global__ __launch_bounds__(256) void k_fast_lists(FSys *systems, int sys) {
 
 // mirror records of every atom, before the bulk prediction reads them
 __global__ __launch_bounds__(256) void k_fast_records(FSys *systems) {
-    FSys &F = systems[blockIdx.x];
-    for (int a = 1 + blockIdx.y * 256 + threadIdx.x; a <= F.s.N; a += 256 * gridDim.y) put_record(F, a);
+    FV &F = fixed_view(systems + blockIdx.x);
+    for (int a = 1 + blockIdx.y * 256 + threadIdx.x; a <= F.s.N; a += 256 * gridDim.y) put_record(F, F.Te, a);
 }
 
 // Bulk Predict(1..N): a prediction reads positions, velocities and counters
@@ -1860,6 +1969,7 @@ __global__ __launch_bounds__(64 * W) void k_fast_predict(FSys *systems) {
     __shared__ FWave<flist(W)> w[W];
     __shared__ ScrTab tab;
     FSys &Fg = systems[blockIdx.x];
+    FV &C = fixed_view(systems + blockIdx.x);
     fsys_load<W>(Fl, &Fg);
     tab_load<W>(tab, Fl.scrtab);
     FSys &F = Fl;
@@ -1868,7 +1978,6 @@ __global__ __launch_bounds__(64 * W) void k_fast_predict(FSys *systems) {
     if (tid == 0) {                         // statistics of this workgroup only
         F.validated = F.agree = F.causal = 0;
         F.max_screen_err = F.max_time_err = 0;
-        S.prof = nullptr;
     }
     __syncthreads();
     WStats &ws = w[wave].st;                // in LDS: no registers held across the loop
@@ -1876,7 +1985,7 @@ __global__ __launch_bounds__(64 * W) void k_fast_predict(FSys *systems) {
     wave_sync();
     int err = 0;
     for (int i = 1 + blockIdx.y * W + wave; i <= S.N; i += W * gridDim.y) {
-        predict_fast<4>(F, tab, w[wave], i, G(F.t0)[i], ws, &err);
+        predict_fast<4>(F, C, nullptr, tab, w[wave], i, G(F.t0)[i], ws, &err);
         if (__ballot(err != 0)) break;              // uniform across the wave
     }
     if (err) atomicCAS(&Fg.s.error, 0, err);
@@ -1898,7 +2007,7 @@ __global__ __launch_bounds__(64 * W) void k_fast_predict(FSys *systems) {
 
 // the block minima of every system, one wavefront per 64-atom block
 __global__ __launch_bounds__(256) void k_fast_blocks(FSys *systems) {
-    FSys &F = systems[blockIdx.x];
+    FV &F = fixed_view(systems + blockIdx.x);
     for (int b = blockIdx.y * 4 + (threadIdx.x >> 6); b < F.nblk; b += 4 * gridDim.y) {
         double t1, t2, t3;
         int a1, a2;
@@ -1963,7 +2072,7 @@ __global__ __launch_bounds__(64 * EWAVES) void k_fast_energy(FSys *systems, doub
 // A helper workgroup: its wavefronts claim the owner's published jobs
 // (re-predictions) until the owner stops, then add their statistics to hp.
 template <int W, int FQ>
-__device__ __forceinline__ void helper_loop(FSys &F, const ScrTab &tab, FShared<W> &sh, FJobs *J, FHelp *hp, int xcc) {
+__device__ __forceinline__ void helper_loop(FSys &F, FV &C, const ScrTab &tab, FShared<W> &sh, FJobs *J, FHelp *hp, int xcc) {
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     WStats &ws = sh.w[wave].st;             // in LDS: no registers held across the loop
     ws.screen = ws.conf = ws.fp64 = ws.cand = 0;
@@ -1993,7 +2102,7 @@ __device__ __forceinline__ void helper_loop(FSys &F, const ScrTab &tab, FShared<
         const double t = J->t[q];
         if (lane == 0) F.Te = J->Te;             // every wave of the round writes the same epoch
         int err = 0;
-        predict_fast<FQ>(F, tab, sh.w[wave], a, t, ws, &err);
+        predict_fast<FQ>(F, C, nullptr, tab, sh.w[wave], a, t, ws, &err);
         if (lane == 0 && err) atomicCAS(&J->err, 0, err);
         wait_stores();                           // the event record is in the L2 before the count
         if (lane == 0) job_done(J);
@@ -2033,40 +2142,42 @@ __global__ __launch_bounds__(64 * W) void k_fast_run(FSys *systems, FJobs *jobs,
     if (threadIdx.x == 0) Fl.t_stop = t_end;
     tab_load<W>(tab, Fl.scrtab);
     FSys &F = Fl;
-    Sys &S = F.s;
+    FV &C = fixed_view(systems + sys);
+    Sys &M = F.s;                              // counters
+    SV &S = C.s;
+    unsigned long long *const prof = S.prof;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int xcc = xcc_id();
     if (role > 0) {
         if (tid == 0) {                          // statistics of this helper only; no phase clocks
-            S.prof = nullptr;
             F.validated = F.agree = F.causal = 0;
             F.max_screen_err = F.max_time_err = 0;
         }
         __syncthreads();
-        helper_loop<W, FQ>(F, tab, sh, J, help + sys, xcc);
+        helper_loop<W, FQ>(F, C, tab, sh, J, help + sys, xcc);
         return;
     }
     if (H > 0 && tid == 0) {                     // helpers on this XCD may join
         __hip_atomic_store(&J->xcc, xcc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         wait_stores();
     }
-    const int nblk = F.nblk;
+    const int nblk = C.nblk;
     for (int b = tid; b < nblk; b += 64 * W) {
-        sh.b1[b] = G(F.b1)[b]; sh.b2[b] = G(F.b2)[b]; sh.b3[b] = G(F.b3)[b];
-        sh.ba[b] = G(F.ba)[b]; sh.bb[b] = G(F.bb)[b];
+        sh.b1[b] = G(C.b1)[b]; sh.b2[b] = G(C.b2)[b]; sh.b3[b] = G(C.b3)[b];
+        sh.ba[b] = G(C.ba)[b]; sh.bb[b] = G(C.bb)[b];
     }
-    if (tid == 0) { sh.err = S.error; sh.stop = 0; sh.drain = 0; }
+    if (tid == 0) { sh.err = M.error; sh.stop = 0; sh.drain = 0; }
     if (tid < FMAXBLK / 32) sh.dmask[tid] = 0;
     __syncthreads();
     if (tid == 0) {                       // npops < 0: -npops executed events
         sh.run_clock_end = (long long)wall_clock64() + budget;
-        sh.run_count_end = npops < 0 ? S.frame - npops : S.pops + npops;
+        sh.run_count_end = npops < 0 ? M.frame - npops : M.pops + npops;
     }
     WStats &ws = sh.w[wave].st;             // in LDS: no registers held across the loop
     ws.screen = ws.conf = ws.fp64 = ws.cand = 0;
     wave_sync();
-    const int cap = F.max_batch > 0 ? min(F.max_batch, FSEL) : FSEL;
-    unsigned long long pt = S.prof ? wall_clock64() : 0;
+    const int cap = C.max_batch > 0 ? min(C.max_batch, FSEL) : FSEL;
+    unsigned long long pt = prof ? wall_clock64() : 0;
     while (true) {
         // ---- selection: every event earlier than the smallest third time of
         // any block (each block's two earliest), or, when that set is too
@@ -2092,27 +2203,27 @@ __global__ __launch_bounds__(64 * W) void k_fast_run(FSys *systems, FJobs *jobs,
             theta3 = fmin(theta3, sh.red_t3[w]);
             if (sh.red_t1[w] < tmin || (sh.red_t1[w] == tmin && sh.red_a[w] < amin)) { tmin = sh.red_t1[w]; amin = sh.red_a[w]; }
         }
-        PROF_MARK(S, FPH_SCAN, pt);
+        FPROF(prof, FPH_SCAN, pt);
         if (tid == 0) {
             // Once the pop or time budget is spent, drain: execute what is
             // still pending up to the latest executed time, so that every
             // atom's local time is at most that time and every pending event
             // is later -- the state is then a snapshot at one time.
-            const bool spent = (npops < 0 ? S.frame : S.pops) >= sh.run_count_end;
+            const bool spent = (npops < 0 ? M.frame : M.pops) >= sh.run_count_end;
             if (!sh.drain && (spent || (long long)wall_clock64() > sh.run_clock_end)) {
                 sh.drain = 1;
                 if (F.tlast < F.t_stop) F.t_stop = F.tlast;
-                sh.drain_end = S.pops + FDRAIN;
+                sh.drain_end = M.pops + FDRAIN;
             }
             const bool pending = tmin < INFINIT && tmin <= F.t_stop;
-            if (sh.drain && S.pops >= sh.drain_end && pending && !sh.err) sh.err = FERR_DRAIN;
-            if (sh.err || !pending || amin < 1 || amin > S.N || (sh.drain && S.pops >= sh.drain_end))
+            if (sh.drain && M.pops >= sh.drain_end && pending && !sh.err) sh.err = FERR_DRAIN;
+            if (sh.err || !pending || amin < 1 || amin > S.N || (sh.drain && M.pops >= sh.drain_end))
                 sh.stop = 1;
             sh.nsel = 0;
         }
         __syncthreads();
         if (sh.stop) break;
-        if (tmin - F.Te > F.rebase_dt) rebase<W>(F, tmin);
+        if (tmin - F.Te > C.rebase_dt) rebase<W>(F, C, tmin);
         // collect the prefix set
         for (int b = tid; b < nblk; b += 64 * W) {
             if (sh.b1[b] < theta3) {
@@ -2137,7 +2248,7 @@ __global__ __launch_bounds__(64 * W) void k_fast_run(FSys *systems, FJobs *jobs,
             }
             __syncthreads();
         }
-        PROF_MARK(S, FPH_COLLECT, pt);
+        FPROF(prof, FPH_COLLECT, pt);
         if (wave == 0) {
             int nsel = sh.nsel;
             bool single = (nsel == 0 || nsel > FSEL);
@@ -2159,7 +2270,7 @@ __global__ __launch_bounds__(64 * W) void k_fast_run(FSys *systems, FJobs *jobs,
                 sh.pre_ca[lane] = (G(S.cx)[a] << 20) | (G(S.cy)[a] << 10) | G(S.cz)[a];
                 sh.pre_cp[lane] = (G(S.cx)[p] << 20) | (G(S.cy)[p] << 10) | G(S.cz)[p];
                 sh.pre_fl[lane] = (ty == SDMD_PCC || ty == SDMD_HB) ? 1 : 0;
-                const double da = t - G(F.t0)[a], dp = t - G(F.t0)[p];
+                const double da = t - G(C.t0)[a], dp = t - G(C.t0)[p];
                 sh.pre_pa[lane][0] = (float)(G(S.x)[a] + G(S.vx)[a] * da);
                 sh.pre_pa[lane][1] = (float)(G(S.y)[a] + G(S.vy)[a] * da);
                 sh.pre_pa[lane][2] = (float)(G(S.z)[a] + G(S.vz)[a] * da);
@@ -2246,7 +2357,7 @@ __global__ __launch_bounds__(64 * W) void k_fast_run(FSys *systems, FJobs *jobs,
             }
         }
         __syncthreads();
-        PROF_MARK(S, FPH_SELECT, pt);
+        FPROF(prof, FPH_SELECT, pt);
         // ---- execution: one lane per event
         const int nex = sh.nex;
         if (nex < 1) {                                     // no selectable event: stop with an error
@@ -2267,10 +2378,10 @@ __global__ __launch_bounds__(64 * W) void k_fast_run(FSys *systems, FJobs *jobs,
                 const signed char ra = G(S.role)[a], rb = G(S.role)[min(max(p, 0), S.N)];
                 int renew[2] = {0, 0};
                 bool recs;
-                const int nr = exec_fast(F, a, t, renew, &err, &recs);
+                const int nr = exec_fast(F, C, a, t, renew, &err, &recs);
                 if (!recs) {                               // the pair path writes its own records
-                    put_record(F, renew[0]);
-                    if (nr > 1) put_record(F, renew[1]);
+                    put_record(C, F.Te, renew[0]);
+                    if (nr > 1) put_record(C, F.Te, renew[1]);
                 }
                 cnt_max(F.tlast, t);
                 for (int r = 0; r < nr; r++) {
@@ -2284,7 +2395,7 @@ __global__ __launch_bounds__(64 * W) void k_fast_run(FSys *systems, FJobs *jobs,
         }
         if (err) atomicCAS(&sh.err, 0, err);
         __syncthreads();
-        PROF_MARK(S, FPH_EVENT, pt);
+        FPROF(prof, FPH_EVENT, pt);
         // re-prediction of every renewed atom, one wave per atom; a wave takes
         // the next atom when it finishes one (prediction times vary)
         const int nheavy = sh.nren, nlight = sh.nlight;
@@ -2327,7 +2438,7 @@ __global__ __launch_bounds__(64 * W) void k_fast_run(FSys *systems, FJobs *jobs,
             r = lane_get(r, 0);
             if (r < 0) break;
             const int q = ren_at(r);
-            predict_fast<FQ>(F, tab, sh.w[wave], sh.ren_a[q], sh.ren_t[q], ws, &err);
+            predict_fast<FQ>(F, C, prof, tab, sh.w[wave], sh.ren_a[q], sh.ren_t[q], ws, &err);
             if (H > 0 && lane == 0) job_done(J);
             if (__ballot(err != 0)) break;          // uniform across the wave
         }
@@ -2352,7 +2463,7 @@ __global__ __launch_bounds__(64 * W) void k_fast_run(FSys *systems, FJobs *jobs,
         }
         if (err) atomicCAS(&sh.err, 0, err);
         __syncthreads();
-        if (tid == 0) S.pops += nex;
+        if (tid == 0) M.pops += nex;
         // the touched blocks, each once, in ascending order (mask cleared for
         // the next round)
         if (wave == 0) {
@@ -2366,7 +2477,7 @@ __global__ __launch_bounds__(64 * W) void k_fast_run(FSys *systems, FJobs *jobs,
             if (lane == 31) sh.ndirty = incl;
         }
         __syncthreads();
-        PROF_MARK(S, FPH_EXEC, pt);
+        FPROF(prof, FPH_EXEC, pt);
         // ---- tree: rescan the touched blocks, two per wavefront at a time
         // so their loads overlap
         const int nd = min(sh.ndirty, 4 * FSEL);
@@ -2376,31 +2487,31 @@ __global__ __launch_bounds__(64 * W) void k_fast_run(FSys *systems, FJobs *jobs,
             const int b1 = d1 < nd ? sh.dirty[d1] : -1;
             double t1, t2, t3, u1, u2, u3;
             int a1b, a2b, c1b, c2b;
-            block_scan2(F, b0, b1, t1, a1b, t2, a2b, t3, u1, c1b, u2, c2b, u3);
+            block_scan2(C, b0, b1, t1, a1b, t2, a2b, t3, u1, c1b, u2, c2b, u3);
             if (lane == 0) {
                 sh.b1[b0] = t1; sh.ba[b0] = a1b; sh.b2[b0] = t2; sh.bb[b0] = a2b; sh.b3[b0] = t3;
                 if (b1 >= 0) { sh.b1[b1] = u1; sh.ba[b1] = c1b; sh.b2[b1] = u2; sh.bb[b1] = c2b; sh.b3[b1] = u3; }
             }
         }
         __syncthreads();
-        PROF_MARK(S, FPH_TREE, pt);
+        FPROF(prof, FPH_TREE, pt);
     }
     if (H > 0 && tid == 0)                        // helpers leave once their current job is done
         __hip_atomic_store(&J->stop, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     for (int b = tid; b < nblk; b += 64 * W) {
-        G(F.b1)[b] = sh.b1[b]; G(F.b2)[b] = sh.b2[b]; G(F.b3)[b] = sh.b3[b];
-        G(F.ba)[b] = sh.ba[b]; G(F.bb)[b] = sh.bb[b];
+        G(C.b1)[b] = sh.b1[b]; G(C.b2)[b] = sh.b2[b]; G(C.b3)[b] = sh.b3[b];
+        G(C.ba)[b] = sh.ba[b]; G(C.bb)[b] = sh.bb[b];
     }
     if (lane == 0) {
         atomicAdd((unsigned long long *)&F.screens, (unsigned long long)ws.screen);
         atomicAdd((unsigned long long *)&F.confirms, (unsigned long long)ws.conf);
-        atomicAdd((unsigned long long *)&S.pair_evals, (unsigned long long)(ws.fp64 + ws.conf));
-        atomicAdd((unsigned long long *)&S.candidates, (unsigned long long)ws.cand);
+        atomicAdd((unsigned long long *)&M.pair_evals, (unsigned long long)(ws.fp64 + ws.conf));
+        atomicAdd((unsigned long long *)&M.candidates, (unsigned long long)ws.cand);
     }
     __syncthreads();
     if (tid == 0) {
-        if (sh.err) S.error = sh.err;
-        S.currenttime = F.tlast;
+        if (sh.err) M.error = sh.err;
+        M.currenttime = F.tlast;
     }
     fsys_store<W>(&systems[sys], Fl);
 }
