@@ -1799,17 +1799,26 @@ __device__ __forceinline__ void block_scan2(FV &F, int b0, int b1, double &t1, i
 constexpr long long FHELP_IDLE = 1000000000LL;   // ticks (10 s at 100 MHz): a helper with no owner activity leaves
 constexpr long long FJOB_WAIT = 200000000LL;     // ticks (2 s): the owner's bound on one round's predictions
 
+// What helpers poll, what they count and what they read lie in cache lines of
+// their own: with the done count beside the polled word a round of 64 systems
+// of 1 536 atoms spent 2.7 us before a helper's prediction began and 3.5 us
+// after the last one ended.
+struct FJob {                   // one re-prediction: its time, the FP32 mirror's epoch, the atom
+    double t, Te;
+    int a, pad[3];
+};
 struct __attribute__((aligned(256))) FJobs {
-    unsigned long long word;    // jobs of the round << 32 | next job index
-    int done;                   // jobs of the round completed
-    int stop;                   // the owner has left its loop
+    unsigned long long word;    // jobs of the round << 32 | next job index; JOB_STOP in the index: the owner has left
+    unsigned long long pad0[31];
+    int done;                   // helper jobs of the round completed, + JOB_FAILED for a failed one
+    int pad1[63];
     int err;                    // first error of a helper's prediction
     int xcc;                    // the owner's XCD (-1: helpers stay out)
-    double Te;                  // FP32-mirror epoch of the round
-    unsigned long long pad[28];
-    int a[2 * FSEL];            // job q: atom and time
-    double t[2 * FSEL];
+    int pad2[62];
+    FJob job[2 * FSEL];
 };
+constexpr unsigned JOB_STOP = 0x80000000u;   // (a late claim's increments do not reach it)
+constexpr int JOB_FAILED = 0x10000;
 
 // helpers' statistics (the owner's live in FSys), summed by the host
 struct FHelp {
@@ -1837,14 +1846,14 @@ __device__ __forceinline__ void acquire_agent() { __builtin_amdgcn_fence(__ATOMI
 // the XCD this wavefront runs on (hwreg XCC_ID, bits 3:0)
 __device__ __forceinline__ int xcc_id() { return __builtin_amdgcn_s_getreg((3 << 11) | (0 << 6) | 20) & 15; }
 
-// claim the next job of the published round (-1: none left)
+// claim the next unassigned job of the published round (-1: none left)
 __device__ __forceinline__ int job_claim(FJobs *J) {
     const unsigned long long old = __hip_atomic_fetch_add(&J->word, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     return (unsigned)old < (unsigned)(old >> 32) ? (int)(unsigned)old : -1;
 }
 
-__device__ __forceinline__ void job_done(FJobs *J) {
-    __hip_atomic_fetch_add(&J->done, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+__device__ __forceinline__ void job_done(FJobs *J, bool failed) {
+    __hip_atomic_fetch_add(&J->done, failed ? 1 + JOB_FAILED : 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // ---------------------------------------------------------------- shared memory
@@ -2077,6 +2086,7 @@ __device__ __forceinline__ void helper_loop(FSys &F, FV &C, const ScrTab &tab, F
     WStats &ws = sh.w[wave].st;             // in LDS: no registers held across the loop
     ws.screen = ws.conf = ws.fp64 = ws.cand = 0;
     wave_sync();
+    int near = -1;                               // 1: on the owner's XCD (fixed for the launch, set before any job)
     for (;;) {
         int q = -1, quit = 0;
         if (lane == 0) {
@@ -2084,12 +2094,13 @@ __device__ __forceinline__ void helper_loop(FSys &F, FV &C, const ScrTab &tab, F
             for (;;) {
                 const unsigned long long w = job_load(&J->word);
                 if ((unsigned)w < (unsigned)(w >> 32)) {
-                    if (int_load(&J->xcc) != xcc) { quit = 1; break; }   // not the owner's XCD
+                    if (near < 0) near = int_load(&J->xcc) == xcc;
+                    if (!near) { quit = 1; break; }
                     q = job_claim(J);
                     if (q >= 0) break;
                     continue;
                 }
-                if (int_load(&J->stop)) { quit = 1; break; }
+                if ((unsigned)w & JOB_STOP) { quit = 1; break; }
                 if ((long long)wall_clock64() - idle0 > FHELP_IDLE) { quit = 1; break; }
                 __builtin_amdgcn_s_sleep(2);
             }
@@ -2098,14 +2109,15 @@ __device__ __forceinline__ void helper_loop(FSys &F, FV &C, const ScrTab &tab, F
         quit = lane_get(quit, 0);
         if (quit) break;
         acquire_agent();                         // drop stale L1 lines: the owner's writes, from the L2
-        const int a = J->a[q];
-        const double t = J->t[q];
-        if (lane == 0) F.Te = J->Te;             // every wave of the round writes the same epoch
+        const int a = J->job[q].a;
+        const double t = J->job[q].t, Te = J->job[q].Te;
+        if (lane == 0) F.Te = Te;                // every wave of the round writes the same epoch
         int err = 0;
         predict_fast<FQ>(F, C, nullptr, tab, sh.w[wave], a, t, ws, &err);
-        if (lane == 0 && err) atomicCAS(&J->err, 0, err);
+        const bool failed = __ballot(err != 0) != 0;
+        if (err) atomicCAS(&J->err, 0, err);
         wait_stores();                           // the event record is in the L2 before the count
-        if (lane == 0) job_done(J);
+        if (lane == 0) job_done(J, failed);
     }
     if (lane == 0) {
         atomicAdd((unsigned long long *)&hp->screens, (unsigned long long)ws.screen);
@@ -2402,59 +2414,62 @@ __global__ __launch_bounds__(64 * W) void k_fast_run(FSys *systems, FJobs *jobs,
         const int nren = nheavy + nlight;             // <= 2 * nex <= 2 * FSEL: the two ends do not meet
         auto ren_at = [&](int r) { return r < nheavy ? r : 2 * FSEL - nlight + (r - nheavy); };
         err = 0;
-        if (H > 0) {
-            // publish the round's jobs, then claim them alongside the helpers
+        // Jobs 0 .. W - 1 are the owner's wavefronts' own; the others are
+        // published for the helpers and for owner wavefronts that finish
+        // early.  A round with no more jobs than wavefronts stays on this CU:
+        // nothing is published or waited for (59 atoms: 14.2 -> 11.2 us per
+        // round's predictions).
+        const bool shared = H > 0 && nren > W;
+        if (shared) {
             for (int r = tid; r < nren; r += 64 * W) {
                 const int q = ren_at(r);
-                J->a[r] = sh.ren_a[q];
-                J->t[r] = sh.ren_t[q];
+                J->job[r].a = sh.ren_a[q];
+                J->job[r].t = sh.ren_t[q];
+                J->job[r].Te = F.Te;
             }
-            if (tid == 0) {
-                J->Te = F.Te;
-                J->done = 0;
-            }
+            if (tid == 0) J->done = 0;
             // the barrier does not wait for other wavefronts' stores: each
             // wave waits for its own (event execution, job list) to complete
             // in the L2 before the word announces the round
             wait_stores();
             __syncthreads();
             if (tid == 0)
-                __hip_atomic_store(&J->word, (unsigned long long)nren << 32, __ATOMIC_RELAXED,
+                __hip_atomic_store(&J->word, (unsigned long long)nren << 32 | W, __ATOMIC_RELAXED,
                                    __HIP_MEMORY_SCOPE_AGENT);
-            __syncthreads();
         }
-        // one prediction call site for both forms: a wave takes the next job
-        // from the LDS counter (no helpers) or from the system's job word
-        for (;;) {
-            int r = -1;
-            if (lane == 0 && sh.err == 0) {
-                if (H == 0) {
-                    r = atomicAdd(&sh.next_ren, 1);
-                    if (r >= nren) r = -1;
-                } else {
+        // one prediction call site for all forms: after its own job a wave
+        // takes the next one from the LDS counter or from the job word
+        for (int r = wave < nren ? wave : -1; r >= 0;) {
+            const int q = ren_at(r);
+            predict_fast<FQ>(F, C, prof, tab, sh.w[wave], sh.ren_a[q], sh.ren_t[q], ws, &err);
+            if (shared && r >= W && lane == 0) job_done(J, false);
+            if (__ballot(err != 0)) break;          // uniform across the wave
+            r = -1;
+            if (lane == 0 && sh.err == 0 && nren > W) {
+                if (shared) {
                     r = job_claim(J);
+                } else {
+                    r = W + atomicAdd(&sh.next_ren, 1);
+                    if (r >= nren) r = -1;
                 }
             }
             r = lane_get(r, 0);
-            if (r < 0) break;
-            const int q = ren_at(r);
-            predict_fast<FQ>(F, C, prof, tab, sh.w[wave], sh.ren_a[q], sh.ren_t[q], ws, &err);
-            if (H > 0 && lane == 0) job_done(J);
-            if (__ballot(err != 0)) break;          // uniform across the wave
         }
-        if (H > 0) {
+        if (shared) {
             if (err) atomicCAS(&sh.err, 0, err);
             if (tid == 0) {
                 // every claimed job completes (its wavefront is running); an
                 // error ends the wait, and the loop with it
                 const long long w0 = (long long)wall_clock64();
-                while (int_load(&J->done) < nren && *(volatile int *)&sh.err == 0 && int_load(&J->err) == 0) {
+                int done;
+                while ((done = int_load(&J->done)) < nren - W && *(volatile int *)&sh.err == 0) {
                     if ((long long)wall_clock64() - w0 > FJOB_WAIT) { atomicCAS(&sh.err, 0, FERR_JOBS); break; }
-                    __builtin_amdgcn_s_sleep(1);
                 }
                 acquire_agent();                        // the helpers' event records, from the L2
-                const int he = int_load(&J->err);
-                if (he) atomicCAS(&sh.err, 0, he);
+                if (done >= JOB_FAILED) {
+                    const int he = int_load(&J->err);
+                    atomicCAS(&sh.err, 0, he ? he : (int)FERR_JOBS);
+                }
             }
         }
         for (int r = tid; r < nren; r += 64 * W) {
@@ -2497,7 +2512,7 @@ __global__ __launch_bounds__(64 * W) void k_fast_run(FSys *systems, FJobs *jobs,
         FPROF(prof, FPH_TREE, pt);
     }
     if (H > 0 && tid == 0)                        // helpers leave once their current job is done
-        __hip_atomic_store(&J->stop, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(&J->word, (unsigned long long)JOB_STOP, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     for (int b = tid; b < nblk; b += 64 * W) {
         G(C.b1)[b] = sh.b1[b]; G(C.b2)[b] = sh.b2[b]; G(C.b3)[b] = sh.b3[b];
         G(C.ba)[b] = sh.ba[b]; G(C.bb)[b] = sh.bb[b];
@@ -2558,7 +2573,6 @@ __global__ void k_fast_jobs_reset(FJobs *jobs, int nsys) {
     if (s < nsys) {
         jobs[s].word = 0;
         jobs[s].done = 0;
-        jobs[s].stop = 0;
         jobs[s].err = 0;
         jobs[s].xcc = -1;
     }
