@@ -54,6 +54,7 @@ constexpr int FCAP_MIN = 64;      // slots per cell at least (a system's capacit
 constexpr int FCAP_MAX = 1024;    // ... at most
 constexpr int FMAXBLK = 1024;     // 64-atom blocks per system (N <= 65535)
 constexpr int FSEL = 64;          // events considered per round
+constexpr int FSMALL = 32;        // 64-atom blocks up to which one wavefront selects and executes a round
 constexpr int FMAXW = 16;         // wavefronts per workgroup at most
 constexpr long long FDRAIN = 1 << 20;   // bound on the pops of a closing drain
 constexpr float FINF = 3.0e38f;
@@ -1584,16 +1585,14 @@ __device__ __forceinline__ void pair_advance(FV &F, int j, PairAtom &q, double t
 
 // A collision, bond or H-bond-neighbour event of atoms a and p (DoEvent ->
 // InteractionEvent without its H-bond branch, Events.c:770-1025), with
-// both atoms' state loaded in two round trips (a's, then p's) and the same
+// both atoms' state given (loaded with the selection) and the same
 // arithmetic as exec_fast's general path (advance, PosLocal, image_near,
 // interaction_event): both mirror records are written here.  Returns the
 // renewed atoms (1 when the event is stale).
-__device__ __forceinline__ int exec_pair(FSys &M, FV &F, int a, int p, int ty, double t, const PairAtom &a0, long long pca,
-                                         double pot0, int sub0, int *renew, int *err) {
+__device__ __forceinline__ int exec_pair(FSys &M, FV &F, int a, int p, int ty, double t, PairAtom &A, PairAtom &P,
+                                         long long pca, double pot0, int sub0, int *renew, int *err) {
     SV &S = F.s;
     const double Te = M.Te;
-    PairAtom A = a0, P;
-    pair_load(F, p, P);
     pair_advance(F, a, A, t);
     renew[0] = a;
     if (pca < P.c) {                                           // HazardCheck, SGThread.c:215-235
@@ -1709,23 +1708,35 @@ __device__ __attribute__((noinline)) int exec_general(FSys &F, int a, int partne
     return 1;
 }
 
-__device__ __forceinline__ int exec_fast(FSys &M, FV &F, int a, double t, int *renew, int *err, bool *recs) {
+// a selected event's record and the state of its atoms (P of the partner, or
+// of the atom itself)
+struct Pending {
+    int a, p, ty, sub;           // p: partner, 0 = none
+    double t, pot;
+    long long pca;
+    signed char ra, rp;          // roles
+    PairAtom A, P;
+};
+__device__ __forceinline__ void pending_load(FV &F, int a, double t, Pending &e) {
     SV &S = F.s;
-    // the record and state of a, loaded together with its partner id
-    const int p = G(S.evp)[a];
-    const int ty0 = G(S.evtype)[a];
-    const long long pca = G(S.evpc)[a];
-    const double pot0 = G(S.evpot)[a];
-    const int sub0 = G(S.evsub)[a];
-    PairAtom a0;
-    pair_load(F, a, a0);
-    const int partner = (p > 0 && p <= S.N) ? p : 0;
-    *recs = false;
-    if (partner && partner != a && (ty0 == SDMD_COLI || ty0 == SDMD_BOND || ty0 == SDMD_HBNE)) {
-        *recs = true;
-        return exec_pair(M, F, a, partner, ty0, t, a0, pca, pot0, sub0, renew, err);
-    }
-    return exec_general(M, a, partner, t, renew, err);
+    const int p0 = G(S.evp)[a];
+    e.a = a; e.t = t;
+    e.ty = G(S.evtype)[a]; e.sub = G(S.evsub)[a]; e.pot = G(S.evpot)[a]; e.pca = G(S.evpc)[a];
+    e.ra = G(S.role)[a];
+    pair_load(F, a, e.A);
+    e.p = (p0 > 0 && p0 <= S.N) ? p0 : 0;
+    const int q = e.p ? e.p : a;
+    e.rp = G(S.role)[q];
+    pair_load(F, q, e.P);
+}
+
+__device__ __forceinline__ int exec_fast(FSys &M, FV &F, Pending &e, int *renew, int *err) {
+    if (e.p && e.p != e.a && (e.ty == SDMD_COLI || e.ty == SDMD_BOND || e.ty == SDMD_HBNE))
+        return exec_pair(M, F, e.a, e.p, e.ty, e.t, e.A, e.P, e.pca, e.pot, e.sub, renew, err);
+    const int nr = exec_general(M, e.a, e.p, e.t, renew, err);
+    put_record(F, M.Te, renew[0]);                     // the pair path writes its own records
+    if (nr > 1) put_record(F, M.Te, renew[1]);
+    return nr;
 }
 
 // ---------------------------------------------------------------- tree blocks
@@ -1735,48 +1746,62 @@ __device__ __forceinline__ int exec_fast(FSys &M, FV &F, int a, double t, int *r
 // pair event seen from the other side: the earlier one's execution
 // re-predicts it, and the earlier one's independence test covers its atoms,
 // so it is skipped when ranking.
-// the block's earliest (t1, a1) and second (t2, a2) events that are not the
-// mirror of an earlier one, and its third time t3, from each lane's atom
-// b*64 + lane + 1 (event time t, partner p; `in` false past the last atom)
-__device__ __forceinline__ void block_min3(int b, bool in, double t, int p, double &t1, int &a1, double &t2, int &a2,
-                                           double &t3) {
-    const int k = in ? b * 64 + (threadIdx.x & 63) + 1 : 0x7fffffff;
-    if (!in) p = 0;
-    double m = t;
-    int km = k;
-    wave_argmin(m, km);
-    const int pm = lane_get(p, (km - 1 - b * 64) & 63);
-    const bool out1 = (k == km) || (k == pm && p == km);
-    double u = out1 ? __builtin_inf() : t;
-    int ku = out1 ? 0x7fffffff : k;
-    wave_argmin(u, ku);
-    const int pu = lane_get(p, (ku - 1 - b * 64) & 63);
-    const bool out2 = out1 || (k == ku) || (k == pu && p == ku);
-    const double w = wave_min_d(out2 ? __builtin_inf() : t);
-    t1 = m; a1 = km; t2 = u; a2 = ku; t3 = w;
+//
+// A wavefront scans four blocks at once, one per row of 16 lanes with four
+// atoms per lane: the reductions stay inside rows (DPP moves only) and serve
+// four blocks with the instructions that one block takes.
+struct RowMin { double t; int k, p; };       // time, atom, the atom's partner
+__device__ __forceinline__ bool earlier(double t, int k, double u, int l) { return t < u || (t == u && k < l); }
+template <int S>
+__device__ __forceinline__ void row_min_step(RowMin &m) {
+    unsigned own, tl, th, k, p;
+    const unsigned long long w = (unsigned long long)__double_as_longlong(m.t);
+    xpair<S>((unsigned)w, own, tl);
+    xpair<S>((unsigned)(w >> 32), own, th);
+    xpair<S>((unsigned)m.k, own, k);
+    xpair<S>((unsigned)m.p, own, p);
+    const double t = __longlong_as_double((long long)(((unsigned long long)th << 32) | tl));
+    if (earlier(t, (int)k, m.t, m.k)) { m.t = t; m.k = (int)k; m.p = (int)p; }
+}
+// smallest (t, k) of the row from each lane's four
+__device__ __forceinline__ RowMin row_min(const double (&t)[4], const int (&k)[4], const int (&p)[4]) {
+    RowMin m = {t[0], k[0], p[0]};
+#pragma unroll
+    for (int u = 1; u < 4; u++)
+        if (earlier(t[u], k[u], m.t, m.k)) { m.t = t[u]; m.k = k[u]; m.p = p[u]; }
+    row_min_step<0>(m); row_min_step<1>(m); row_min_step<2>(m); row_min_step<3>(m);
+    return m;
 }
 
-__device__ void block_scan(FV &F, int b, double &t1, int &a1, double &t2, int &a2, double &t3) {
-    const int lane = threadIdx.x & 63;
-    const int a = b * 64 + lane + 1;
-    const bool in = a <= F.s.N;
-    const double t = in ? G(F.s.evt)[a] : __builtin_inf();
-    const int p = in ? G(F.s.evp)[a] : 0;
-    block_min3(b, in, t, p, t1, a1, t2, a2, t3);
-}
-
-// block_scan of two blocks with their loads issued together (b1 < 0: none)
-__device__ __forceinline__ void block_scan2(FV &F, int b0, int b1, double &t1, int &a1, double &t2, int &a2,
-                                            double &t3, double &u1, int &c1, double &u2, int &c2, double &u3) {
-    const int lane = threadIdx.x & 63;
-    const int N = F.s.N;
-    const int x0 = b0 * 64 + lane + 1, x1 = b1 * 64 + lane + 1;
-    const bool in0 = x0 <= N, in1 = b1 >= 0 && x1 <= N;
-    const int r0 = in0 ? x0 : 1, r1 = in1 ? x1 : 1;
-    const double e0 = G(F.s.evt)[r0], e1 = G(F.s.evt)[r1];
-    const int p0 = G(F.s.evp)[r0], p1 = G(F.s.evp)[r1];
-    block_min3(b0, in0, in0 ? e0 : __builtin_inf(), in0 ? p0 : 0, t1, a1, t2, a2, t3);
-    if (b1 >= 0) block_min3(b1, in1, in1 ? e1 : __builtin_inf(), in1 ? p1 : 0, u1, c1, u2, c2, u3);
+// the earliest (t1, a1) and second (t2, a2) events of this row's block b that
+// are not the mirror of an earlier one, and its third time t3 (b < 0: none)
+__device__ __forceinline__ void block_scan4(FV &F, int b, double &t1, int &a1, double &t2, int &a2, double &t3) {
+    const int l = threadIdx.x & 15, N = F.s.N;
+    const double inf = __builtin_inf();
+    double t[4];
+    int k[4], p[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+        const int a = b * 64 + 16 * u + l + 1;
+        const bool in = b >= 0 && a <= N;
+        const int r = in ? a : 1;
+        t[u] = G(F.s.evt)[r];
+        p[u] = G(F.s.evp)[r];
+        k[u] = in ? a : 0x7fffffff;
+    }
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+        if (k[u] == 0x7fffffff) { t[u] = inf; p[u] = 0; }
+    const RowMin m = row_min(t, k, p);
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+        if (k[u] == m.k || (k[u] == m.p && p[u] == m.k)) { t[u] = inf; k[u] = 0x7fffffff; p[u] = 0; }
+    const RowMin n = row_min(t, k, p);
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+        if (k[u] == n.k || (k[u] == n.p && p[u] == n.k)) { t[u] = inf; k[u] = 0x7fffffff; p[u] = 0; }
+    const RowMin o = row_min(t, k, p);
+    t1 = m.t; a1 = m.k; t2 = n.t; a2 = n.k; t3 = o.t;
 }
 
 // ---------------------------------------------------------------- helper workgroups
@@ -1873,14 +1898,12 @@ struct FShared {
     float pre_pa[FSEL][3], pre_pp[FSEL][3];
     unsigned long long conflict;
     int nset;                          // events in the selected set
-    int nsel, nex, ndirty, nren, nlight, next_ren, err, stop, drain;
+    int nsel, nex, nren, nlight, next_ren, err, stop, drain;
     long long drain_end;
-    int ex_a[FSEL];
     // renewed atoms: H-bond-capable ones from the front (nren), the others
     // from the back (nlight)
     int ren_a[2 * FSEL];
     double ren_t[2 * FSEL];
-    int dirty[4 * FSEL];
     unsigned int dmask[FMAXBLK / 32];   // blocks touched this round (bit per block)
     FWave<flist(W)> w[W];
 };
@@ -2014,14 +2037,15 @@ __global__ __launch_bounds__(64 * W) void k_fast_predict(FSys *systems) {
     }
 }
 
-// the block minima of every system, one wavefront per 64-atom block
+// the block minima of every system, four 64-atom blocks per wavefront
 __global__ __launch_bounds__(256) void k_fast_blocks(FSys *systems) {
     FV &F = fixed_view(systems + blockIdx.x);
-    for (int b = blockIdx.y * 4 + (threadIdx.x >> 6); b < F.nblk; b += 4 * gridDim.y) {
+    for (int b0 = 4 * (blockIdx.y * 4 + (threadIdx.x >> 6)); b0 < F.nblk; b0 += 16 * gridDim.y) {
+        const int b = b0 + ((threadIdx.x & 63) >> 4);
         double t1, t2, t3;
         int a1, a2;
-        block_scan(F, b, t1, a1, t2, a2, t3);
-        if ((threadIdx.x & 63) == 0) {
+        block_scan4(F, b < F.nblk ? b : -1, t1, a1, t2, a2, t3);
+        if ((threadIdx.x & 15) == 0 && b < F.nblk) {
             G(F.b1)[b] = t1; G(F.ba)[b] = a1; G(F.b2)[b] = t2; G(F.bb)[b] = a2; G(F.b3)[b] = t3;
         }
     }
@@ -2189,14 +2213,22 @@ __global__ __launch_bounds__(64 * W) void k_fast_run(FSys *systems, FJobs *jobs,
     ws.screen = ws.conf = ws.fp64 = ws.cand = 0;
     wave_sync();
     const int cap = C.max_batch > 0 ? min(C.max_batch, FSEL) : FSEL;
+    const bool small = nblk <= FSMALL;
     unsigned long long pt = prof ? wall_clock64() : 0;
     while (true) {
         // ---- selection: every event earlier than the smallest third time of
         // any block (each block's two earliest), or, when that set is too
         // large, earlier than the smallest second time (each block's earliest)
+        //
+        // Wavefront 0 collects the set, loads the events' atoms, tests their
+        // independence and executes them, one event per lane, with the loaded
+        // state in registers: a barrier or a hand-over through LDS costs as
+        // much as 50 instructions.  Up to FSMALL blocks (few events) no other
+        // wavefront takes part before the re-predictions; of more blocks the
+        // scans and the pair tests are spread over the workgroup.
         double m3 = __builtin_inf(), m2 = __builtin_inf(), m1 = __builtin_inf();
         int a1 = 0x7fffffff;
-        for (int b = tid; b < nblk; b += 64 * W) {
+        for (int b = small ? lane : tid; b < nblk; b += small ? 64 : 64 * W) {
             m3 = fmin(m3, sh.b3[b]);
             m2 = fmin(m2, sh.b2[b]);
             const double t = sh.b1[b];
@@ -2205,17 +2237,20 @@ __global__ __launch_bounds__(64 * W) void k_fast_run(FSys *systems, FJobs *jobs,
         m3 = wave_min_d(m3);
         m2 = wave_min_d(m2);
         wave_argmin(m1, a1);
-        if (lane == 0) { sh.red_t[wave] = m2; sh.red_t3[wave] = m3; sh.red_t1[wave] = m1; sh.red_a[wave] = a1; }
-        __syncthreads();
         const double tcap = nextafter(F.t_stop, __builtin_inf());
-        double theta = fmin(sh.red_t[0], tcap), theta3 = fmin(sh.red_t3[0], tcap), tmin = sh.red_t1[0];
-        int amin = sh.red_a[0];
-        for (int w = 1; w < W; w++) {
-            theta = fmin(theta, sh.red_t[w]);
-            theta3 = fmin(theta3, sh.red_t3[w]);
-            if (sh.red_t1[w] < tmin || (sh.red_t1[w] == tmin && sh.red_a[w] < amin)) { tmin = sh.red_t1[w]; amin = sh.red_a[w]; }
+        double theta = fmin(m2, tcap), theta3 = fmin(m3, tcap), tmin = m1;
+        int amin = a1;
+        if (!small) {
+            if (lane == 0) { sh.red_t[wave] = m2; sh.red_t3[wave] = m3; sh.red_t1[wave] = m1; sh.red_a[wave] = a1; }
+            __syncthreads();
+            for (int w = 0; w < W; w++) {
+                theta = fmin(theta, sh.red_t[w]);
+                theta3 = fmin(theta3, sh.red_t3[w]);
+                if (sh.red_t1[w] < tmin || (sh.red_t1[w] == tmin && sh.red_a[w] < amin)) { tmin = sh.red_t1[w]; amin = sh.red_a[w]; }
+            }
         }
         FPROF(prof, FPH_SCAN, pt);
+        const bool old_epoch = tmin - F.Te > C.rebase_dt;     // uniform
         if (tid == 0) {
             // Once the pop or time budget is spent, drain: execute what is
             // still pending up to the latest executed time, so that every
@@ -2232,78 +2267,84 @@ __global__ __launch_bounds__(64 * W) void k_fast_run(FSys *systems, FJobs *jobs,
             if (sh.err || !pending || amin < 1 || amin > S.N || (sh.drain && M.pops >= sh.drain_end))
                 sh.stop = 1;
             sh.nsel = 0;
+            sh.nren = 0;
+            sh.nlight = 0;
+            sh.next_ren = 0;
+            sh.conflict = 0;
         }
-        __syncthreads();
-        if (sh.stop) break;
-        if (tmin - F.Te > C.rebase_dt) rebase<W>(F, C, tmin);
+        if (!small || old_epoch) {
+            __syncthreads();
+            if (sh.stop) break;
+            if (old_epoch) rebase<W>(F, C, tmin);
+        }
         // collect the prefix set
-        for (int b = tid; b < nblk; b += 64 * W) {
-            if (sh.b1[b] < theta3) {
-                const int slotk = atomicAdd(&sh.nsel, 1);
-                if (slotk < FSEL) { sh.sel_t[slotk] = sh.b1[b]; sh.sel_a[slotk] = sh.ba[b]; }
-            }
-            if (sh.b2[b] < theta3) {
-                const int slotk = atomicAdd(&sh.nsel, 1);
-                if (slotk < FSEL) { sh.sel_t[slotk] = sh.b2[b]; sh.sel_a[slotk] = sh.bb[b]; }
-            }
-        }
-        __syncthreads();
-        if (sh.nsel > FSEL) {
-            __syncthreads();
-            if (tid == 0) sh.nsel = 0;
-            __syncthreads();
-            for (int b = tid; b < nblk; b += 64 * W) {
-                if (sh.b1[b] < theta) {
+        auto collect = [&](double before, bool second) {
+            for (int b = small ? lane : tid; b < nblk; b += small ? 64 : 64 * W) {
+                if (sh.b1[b] < before) {
                     const int slotk = atomicAdd(&sh.nsel, 1);
                     if (slotk < FSEL) { sh.sel_t[slotk] = sh.b1[b]; sh.sel_a[slotk] = sh.ba[b]; }
                 }
+                if (second && sh.b2[b] < before) {
+                    const int slotk = atomicAdd(&sh.nsel, 1);
+                    if (slotk < FSEL) { sh.sel_t[slotk] = sh.b2[b]; sh.sel_a[slotk] = sh.bb[b]; }
+                }
             }
+        };
+        if (small) {
+            wave_sync();                                      // at most 2 * FSMALL events: no overflow
+            if (wave == 0 && !sh.stop) collect(theta3, true);
+            wave_sync();
+        } else {
+            collect(theta3, true);
             __syncthreads();
+            if (sh.nsel > FSEL) {
+                __syncthreads();
+                if (tid == 0) sh.nsel = 0;
+                __syncthreads();
+                collect(theta, false);
+                __syncthreads();
+            }
         }
         FPROF(prof, FPH_COLLECT, pt);
-        if (wave == 0) {
-            int nsel = sh.nsel;
-            bool single = (nsel == 0 || nsel > FSEL);
-            double t = __builtin_inf();
-            int a = 0x7fffffff;
+        int ns = 0;
+        Pending ev;
+        ev.a = 0x7fffffff;
+        ev.t = __builtin_inf();
+        if (wave == 0 && !sh.stop) {
+            ns = sh.nsel;
+            const bool single = (ns == 0 || ns > FSEL);
             if (single) {
-                if (lane == 0) { t = tmin; a = amin; }
-                nsel = 1;
-            } else if (lane < nsel) {
-                t = sh.sel_t[lane]; a = sh.sel_a[lane];
+                if (lane == 0) { ev.t = tmin; ev.a = amin; }
+                ns = 1;
+            } else if (lane < ns) {
+                ev.t = sh.sel_t[lane]; ev.a = sh.sel_a[lane];
             }
             // cells, kind and positions (at the event time) of each event's
             // target and partner, for the independence test
-            const bool valid = lane < nsel && a >= 1 && a <= S.N;
-            if (valid) {
-                const int p0 = G(S.evp)[a];
-                const int p = (p0 > 0 && p0 <= S.N) ? p0 : a;
-                const int ty = G(S.evtype)[a];
-                sh.pre_ca[lane] = (G(S.cx)[a] << 20) | (G(S.cy)[a] << 10) | G(S.cz)[a];
-                sh.pre_cp[lane] = (G(S.cx)[p] << 20) | (G(S.cy)[p] << 10) | G(S.cz)[p];
-                sh.pre_fl[lane] = (ty == SDMD_PCC || ty == SDMD_HB) ? 1 : 0;
-                const double da = t - G(C.t0)[a], dp = t - G(C.t0)[p];
-                sh.pre_pa[lane][0] = (float)(G(S.x)[a] + G(S.vx)[a] * da);
-                sh.pre_pa[lane][1] = (float)(G(S.y)[a] + G(S.vy)[a] * da);
-                sh.pre_pa[lane][2] = (float)(G(S.z)[a] + G(S.vz)[a] * da);
-                sh.pre_pp[lane][0] = (float)(G(S.x)[p] + G(S.vx)[p] * dp);
-                sh.pre_pp[lane][1] = (float)(G(S.y)[p] + G(S.vy)[p] * dp);
-                sh.pre_pp[lane][2] = (float)(G(S.z)[p] + G(S.vz)[p] * dp);
+            if (lane < ns && ev.a >= 1 && ev.a <= S.N) {
+                pending_load(C, ev.a, ev.t, ev);
+                sh.pre_ca[lane] = (ev.A.cx << 20) | (ev.A.cy << 10) | ev.A.cz;
+                sh.pre_cp[lane] = (ev.P.cx << 20) | (ev.P.cy << 10) | ev.P.cz;
+                sh.pre_fl[lane] = (ev.ty == SDMD_PCC || ev.ty == SDMD_HB) ? 1 : 0;
+                const double da = ev.t - ev.A.t0, dp = ev.t - ev.P.t0;
+                sh.pre_pa[lane][0] = (float)(ev.A.x + ev.A.vx * da);
+                sh.pre_pa[lane][1] = (float)(ev.A.y + ev.A.vy * da);
+                sh.pre_pa[lane][2] = (float)(ev.A.z + ev.A.vz * da);
+                sh.pre_pp[lane][0] = (float)(ev.P.x + ev.P.vx * dp);
+                sh.pre_pp[lane][1] = (float)(ev.P.y + ev.P.vy * dp);
+                sh.pre_pp[lane][2] = (float)(ev.P.z + ev.P.vz * dp);
             }
-            sh.sel_a[lane] = a;
-            sh.sel_t[lane] = t;
+            sh.sel_a[lane] = ev.a;
+            sh.sel_t[lane] = ev.t;
             sh.sel_rank[lane] = 0;
-            if (lane == 0) { sh.nset = nsel; sh.conflict = 0; }
             if (lane == 0) {
+                sh.nset = ns;
                 F.batches++;
                 if (single) F.single++;
-                sh.ndirty = 0;
-                sh.nren = 0;
-                sh.nlight = 0;
-                sh.next_ren = 0;
             }
         }
-        __syncthreads();
+        if (small) wave_sync();
+        else __syncthreads();
         // independence: every pair of the set, spread over the workgroup (no
         // sorting: the pair's time order is compared directly); the later
         // event k of a pair conflicts with the earlier one l when an atom of
@@ -2314,22 +2355,22 @@ __global__ __launch_bounds__(64 * W) void k_fast_run(FSys *systems, FJobs *jobs,
         // its neighbours' bookkeeping) -- or when the two atoms are closer
         // than two cell widths (>= twice the cut-off, so an event created by
         // one cannot reach the other's atoms through a single partner)
-        {
-            const int ns = sh.nset;
-            const int npair = ns * (ns - 1) / 2;
+        if (!small || wave == 0) {
+            const int nset = small ? ns : sh.nset;
+            const int npair = nset * (nset - 1) / 2;
             const int n1 = S.cellnum[1], n2 = S.cellnum[2], n3 = S.cellnum[3];
             const float bx = (float)S.box[1], by = (float)S.box[2], bz = (float)S.box[3];
             const float cmin = (float)fmin(S.cellsize[1], fmin(S.cellsize[2], S.cellsize[3]));
             const float R2 = 4.f * cmin * cmin;
             unsigned long long mine = 0;
-            for (int q = tid; q < npair; q += 64 * W) {
+            for (int q = small ? lane : tid; q < npair; q += small ? 64 : 64 * W) {
                 int i = (int)((1.f + sqrtf(1.f + 8.f * (float)q)) * 0.5f);
                 while (i * (i - 1) / 2 > q) i--;
                 while ((i + 1) * i / 2 <= q) i++;
                 const int j = q - i * (i - 1) / 2;
                 const bool jfirst = sh.sel_t[j] < sh.sel_t[i] || (sh.sel_t[j] == sh.sel_t[i] && sh.sel_a[j] < sh.sel_a[i]);
                 const int k = jfirst ? i : j, l = jfirst ? j : i;      // l is the earlier event
-                atomicAdd(&sh.sel_rank[k], 1);
+                if (nset > cap) atomicAdd(&sh.sel_rank[k], 1);
                 const int D = 2 + ((sh.pre_fl[k] | sh.pre_fl[l]) ? 1 : 0);
                 auto far = [&](int u, int v) {
                     int dx = abs((u >> 20) - (v >> 20)), dy = abs(((u >> 10) & 1023) - ((v >> 10) & 1023)),
@@ -2353,60 +2394,44 @@ __global__ __launch_bounds__(64 * W) void k_fast_run(FSys *systems, FJobs *jobs,
             mine = wave_or64(mine);
             if (lane == 0 && mine) atomicOr(&sh.conflict, mine);
         }
-        __syncthreads();
-        if (wave == 0) {
-            const int ns = sh.nset;
-            const int a = sh.sel_a[lane];
-            // the independent events among the `cap` earliest of the set
-            const bool ok = lane < ns && a >= 1 && a <= S.N && !((sh.conflict >> lane) & 1) && sh.sel_rank[lane] < cap;
-            const unsigned long long okm = __ballot(ok);
-            const int rank = __popcll(okm & ((1ULL << lane) - 1));
-            if (ok && rank < cap) sh.ex_a[rank] = a;
-            if (lane == 0) {
-                const int nok = __popcll(okm);
-                sh.nex = min(nok, cap);
-                F.deferred += ns - sh.nex;
-            }
-        }
-        __syncthreads();
+        if (small) wave_sync();
+        else __syncthreads();
         FPROF(prof, FPH_SELECT, pt);
-        // ---- execution: one lane per event
+        // ---- execution: the independent events among the `cap` earliest of
+        // the set, one lane per event
+        int err = 0;
+        if (wave == 0) {
+            const bool ok = lane < ns && ev.a >= 1 && ev.a <= S.N && !((sh.conflict >> lane) & 1) && sh.sel_rank[lane] < cap;
+            const int nex = __popcll(__ballot(ok));
+            if (lane == 0) {
+                sh.nex = nex;
+                F.deferred += ns - nex;
+            }
+            if (ok) {
+                // H-bond-capable atoms (acceptor, donor, sulfur) scan their
+                // neighbourhood for H-bond partners: the longest predictions
+                // of a round, queued first so the waves finish together
+                int renew[2] = {0, 0};
+                const int nr = exec_fast(F, C, ev, renew, &err);
+                for (int r = 0; r < nr; r++) {
+                    const signed char ro = r ? ev.rp : ev.ra;    // renew[1] is the partner
+                    const bool heavy = ro == 'A' || ro == 'D' || ro == 'S';
+                    const int slot = heavy ? atomicAdd(&sh.nren, 1) : 2 * FSEL - 1 - atomicAdd(&sh.nlight, 1);
+                    sh.ren_a[slot] = renew[r];
+                    sh.ren_t[slot] = ev.t;
+                }
+            }
+            const double last = -wave_min_d(ok ? -ev.t : __builtin_inf());
+            if (lane == 0 && nex > 0 && F.tlast < last) F.tlast = last;
+        }
+        if (err) atomicCAS(&sh.err, 0, err);
+        __syncthreads();
+        if (sh.stop) break;
         const int nex = sh.nex;
         if (nex < 1) {                                     // no selectable event: stop with an error
             if (tid == 0) sh.err = FERR_SELECT;
             break;
         }
-        // events spread over the waves' lanes (event e on wave e % W, lane e / W)
-        int err = 0;
-        {
-            const int e = lane * W + wave;
-            if (e < nex) {
-                const int a = sh.ex_a[e];
-                const double t = G(S.evt)[a];
-                // H-bond-capable atoms (acceptor, donor, sulfur) scan their
-                // neighbourhood for H-bond partners: the longest predictions
-                // of a round, queued first so the waves finish together
-                const int p = G(S.evp)[a];
-                const signed char ra = G(S.role)[a], rb = G(S.role)[min(max(p, 0), S.N)];
-                int renew[2] = {0, 0};
-                bool recs;
-                const int nr = exec_fast(F, C, a, t, renew, &err, &recs);
-                if (!recs) {                               // the pair path writes its own records
-                    put_record(C, F.Te, renew[0]);
-                    if (nr > 1) put_record(C, F.Te, renew[1]);
-                }
-                cnt_max(F.tlast, t);
-                for (int r = 0; r < nr; r++) {
-                    const signed char ro = r ? rb : ra;          // renew[1] is the partner p
-                    const bool heavy = ro == 'A' || ro == 'D' || ro == 'S';
-                    const int slot = heavy ? atomicAdd(&sh.nren, 1) : 2 * FSEL - 1 - atomicAdd(&sh.nlight, 1);
-                    sh.ren_a[slot] = renew[r];
-                    sh.ren_t[slot] = t;
-                }
-            }
-        }
-        if (err) atomicCAS(&sh.err, 0, err);
-        __syncthreads();
         FPROF(prof, FPH_EVENT, pt);
         // re-prediction of every renewed atom, one wave per atom; a wave takes
         // the next atom when it finishes one (prediction times vary)
@@ -2479,36 +2504,34 @@ __global__ __launch_bounds__(64 * W) void k_fast_run(FSys *systems, FJobs *jobs,
         if (err) atomicCAS(&sh.err, 0, err);
         __syncthreads();
         if (tid == 0) M.pops += nex;
-        // the touched blocks, each once, in ascending order (mask cleared for
-        // the next round)
-        if (wave == 0) {
-            const unsigned int m = (lane < FMAXBLK / 32) ? sh.dmask[lane] : 0u;
+        // the touched blocks, each once, in ascending order (every wavefront
+        // makes its own list from the mask)
+        int *dirty = sh.w[wave].l_id;
+        int nd;
+        {
             static_assert(FMAXBLK / 32 <= 32, "the touched-block mask fits lanes 0..31");
+            static_assert(FWave<flist(W)>::LIST >= 2 * FSEL, "a round touches at most 2 * FSEL blocks");
+            const unsigned int m = (lane < FMAXBLK / 32) ? sh.dmask[lane] : 0u;
             const int c = __popc(m);
             const int incl = scan32_incl(c);
             int o = incl - c;
-            for (unsigned int mm = m; mm; mm &= mm - 1) sh.dirty[o++] = lane * 32 + __builtin_ctz(mm);
-            if (lane < FMAXBLK / 32) sh.dmask[lane] = 0u;
-            if (lane == 31) sh.ndirty = incl;
+            for (unsigned int mm = m; mm; mm &= mm - 1) dirty[o++] = lane * 32 + __builtin_ctz(mm);
+            nd = lane_get(incl, 31);
+            wave_sync();
         }
-        __syncthreads();
         FPROF(prof, FPH_EXEC, pt);
-        // ---- tree: rescan the touched blocks, two per wavefront at a time
-        // so their loads overlap
-        const int nd = min(sh.ndirty, 4 * FSEL);
-        for (int d = wave; d < nd; d += 2 * W) {
-            const int b0 = sh.dirty[d];
-            const int d1 = d + W;
-            const int b1 = d1 < nd ? sh.dirty[d1] : -1;
-            double t1, t2, t3, u1, u2, u3;
-            int a1b, a2b, c1b, c2b;
-            block_scan2(C, b0, b1, t1, a1b, t2, a2b, t3, u1, c1b, u2, c2b, u3);
-            if (lane == 0) {
-                sh.b1[b0] = t1; sh.ba[b0] = a1b; sh.b2[b0] = t2; sh.bb[b0] = a2b; sh.b3[b0] = t3;
-                if (b1 >= 0) { sh.b1[b1] = u1; sh.ba[b1] = c1b; sh.b2[b1] = u2; sh.bb[b1] = c2b; sh.b3[b1] = u3; }
+        // ---- tree: rescan the touched blocks, four per wavefront at a time
+        for (int d0 = 4 * wave; d0 < nd; d0 += 4 * W) {
+            const int d = d0 + (lane >> 4), b = d < nd ? dirty[d] : -1;
+            double t1, t2, t3;
+            int a1b, a2b;
+            block_scan4(C, b, t1, a1b, t2, a2b, t3);
+            if ((lane & 15) == 0 && b >= 0) {
+                sh.b1[b] = t1; sh.ba[b] = a1b; sh.b2[b] = t2; sh.bb[b] = a2b; sh.b3[b] = t3;
             }
         }
         __syncthreads();
+        if (tid < FMAXBLK / 32) sh.dmask[tid] = 0u;       // next set after the coming barriers
         FPROF(prof, FPH_TREE, pt);
     }
     if (H > 0 && tid == 0)                        // helpers leave once their current job is done
