@@ -825,57 +825,75 @@ static __device__ void hb_event(Sys &S, int i, int j, int nbi, int nbj, int *err
 
 // Energy sums: workgroup (x, y) of EWAVES wavefronts leaves the sums of its
 // threads' a and b and the OR of their error flags for system x in
-// part[3 * (x * gridDim.y + y) ..]; k_energy_reduce adds a system's
-// workgroups.  Both run in a fixed order (butterfly within a wavefront, then
-// by index), so the energies of a state are the same on every call.
+// part[ENERGY_PART * (x * gridDim.y + y) ..]; k_energy_reduce adds a system's
+// workgroups.  Every addition keeps its rounding error (Knuth's TwoSum), so
+// the result is the exact sum of the terms rounded once whatever the split,
+// and the energies of a state are the same on every call.
 constexpr int EWAVES = 4;
+constexpr int ENERGY_PART = 5;            // two sums with their errors, the flag
+struct Sum2 {
+    double s, c;
+    __device__ __forceinline__ void add(double x) {
+        const double t = s + x, z = t - s;
+        c += (s - (t - z)) + (x - z);
+        s = t;
+    }
+    __device__ __forceinline__ void add(const Sum2 &o) { add(o.s); c += o.c; }
+    __device__ __forceinline__ double value() const { return __builtin_isfinite(s) ? s + c : s; }
+};
 template <int S>
-static __device__ __forceinline__ void dsum_step(double &v) {
-    unsigned long long a, b;
-    xpair64<S>((unsigned long long)__double_as_longlong(v), a, b);
-    v = __longlong_as_double((long long)a) + __longlong_as_double((long long)b);
+static __device__ __forceinline__ void sum2_step(Sum2 &v) {
+    unsigned long long sa, sb, ca, cb;
+    xpair64<S>((unsigned long long)__double_as_longlong(v.s), sa, sb);
+    xpair64<S>((unsigned long long)__double_as_longlong(v.c), ca, cb);
+    Sum2 o = {__longlong_as_double((long long)sa), __longlong_as_double((long long)ca)};
+    o.add(Sum2{__longlong_as_double((long long)sb), __longlong_as_double((long long)cb)});
+    v = o;
 }
-static __device__ __forceinline__ double wave_sum_d(double v) {
-    dsum_step<0>(v); dsum_step<1>(v); dsum_step<2>(v); dsum_step<3>(v); dsum_step<4>(v); dsum_step<5>(v);
-    return lane_get(v, 0);
+static __device__ __forceinline__ Sum2 wave_sum2(Sum2 v) {
+    sum2_step<0>(v); sum2_step<1>(v); sum2_step<2>(v); sum2_step<3>(v); sum2_step<4>(v); sum2_step<5>(v);
+    return Sum2{lane_get(v.s, 0), lane_get(v.c, 0)};
 }
-static __device__ __forceinline__ void energy_partial(double a, double b, int err, double *part) {
-    __shared__ double red[2 * EWAVES];
+static __device__ __forceinline__ void energy_partial(Sum2 a, Sum2 b, int err, double *part) {
+    __shared__ Sum2 red[2 * EWAVES];
     __shared__ int any_err[EWAVES];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    a = wave_sum_d(a);
-    b = wave_sum_d(b);
+    a = wave_sum2(a);
+    b = wave_sum2(b);
     const bool bad = __ballot(err != 0) != 0;
     if (lane == 0) { red[2 * wave] = a; red[2 * wave + 1] = b; any_err[wave] = bad; }
     __syncthreads();
     if (threadIdx.x == 0) {
-        double sa = 0, sb = 0;
+        Sum2 sa = {0, 0}, sb = {0, 0};
         int se = 0;
-        for (int w = 0; w < EWAVES; w++) { sa += red[2 * w]; sb += red[2 * w + 1]; se |= any_err[w]; }
-        double *p = part + 3 * ((size_t)blockIdx.x * gridDim.y + blockIdx.y);
-        G(p)[0] = sa;
-        G(p)[1] = sb;
-        G(p)[2] = se ? 1.0 : 0.0;
+        for (int w = 0; w < EWAVES; w++) { sa.add(red[2 * w]); sb.add(red[2 * w + 1]); se |= any_err[w]; }
+        double *p = part + ENERGY_PART * ((size_t)blockIdx.x * gridDim.y + blockIdx.y);
+        G(p)[0] = sa.s;
+        G(p)[1] = sa.c;
+        G(p)[2] = sb.s;
+        G(p)[3] = sb.c;
+        G(p)[4] = se ? 1.0 : 0.0;
     }
 }
 
 // one wavefront per system: out's three planes (kinetic, potential, error)
 static __global__ __launch_bounds__(64) void k_energy_reduce(const double *part, int chunks, double *out) {
     const int s = blockIdx.x, n = gridDim.x, lane = threadIdx.x;
-    double a = 0, b = 0, e = 0;
+    Sum2 a = {0, 0}, b = {0, 0};
+    bool e = false;
     for (int k = lane; k < chunks; k += 64) {
-        const double *p = part + 3 * ((size_t)s * chunks + k);
-        a += G(p)[0];
-        b += G(p)[1];
-        e += G(p)[2];
+        const double *p = part + ENERGY_PART * ((size_t)s * chunks + k);
+        a.add(Sum2{G(p)[0], G(p)[1]});
+        b.add(Sum2{G(p)[2], G(p)[3]});
+        e |= G(p)[4] != 0;
     }
-    a = wave_sum_d(a);
-    b = wave_sum_d(b);
-    e = wave_sum_d(e);
+    a = wave_sum2(a);
+    b = wave_sum2(b);
+    const bool bad = __ballot(e) != 0;
     if (lane == 0) {
-        G(out)[s] = a;
-        G(out)[n + s] = b;
-        G(out)[2 * n + s] = e != 0 ? 1.0 : 0.0;
+        G(out)[s] = a.value();
+        G(out)[n + s] = b.value();
+        G(out)[2 * n + s] = bad ? 1.0 : 0.0;
     }
 }
 
@@ -905,7 +923,7 @@ struct sdmd_gpu_ctx {
     char *hostbuf;             // pinned host copy of one such block (allocated at the first download)
     size_t hostbuf_bytes;
     double *dev_energy;        // 3 planes of nsys doubles (kinetic, potential, error flag)
-    double *epart;             // partial energy sums: 3 doubles per system and workgroup
+    double *epart;             // partial energy sums: ENERGY_PART doubles per system and workgroup
     int echunks;               // energy workgroups per system
     double *scratch;           // device address of the allocation-free energy planes on this GPU
     double last_ms;

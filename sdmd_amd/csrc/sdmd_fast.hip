@@ -1969,6 +1969,41 @@ __global__ __launch_bounds__(256) void k_fast_cells(FSys *systems) {
     }
 }
 
+// bond lists at a fixed stride of 16 (BondTime's connect[16]) and the
+// constraints' tables: FP32 radii and energy bits inline (up to 8 steps are
+// staged) and FP64 shells at a fixed stride (a constraint of more steps than
+// a row holds is not staged, and then not read from here).  Derived on the
+// device: 17 MB for 26 080 atoms, which took longer to write on the host and
+// to copy than all the rest of opening a system.
+__global__ __launch_bounds__(256) void k_fast_derive(FSys *systems) {
+    FV &F = fixed_view(systems + blockIdx.x);
+    SV &S = F.s;
+    const int tid = blockIdx.y * 256 + threadIdx.x, all = 256 * gridDim.y, N = S.N;
+    for (int k = tid; k < (N + 1) * 16; k += all) {
+        const int a = k >> 4, e = a > 0 ? G(S.bond_off)[a] + (k & 15) : 0;
+        const bool in = a > 0 && e < G(S.bond_off)[a + 1];
+        G(F.bj16)[k] = in ? G(S.bond_j)[e] : 0;
+        G(F.blo16)[k] = in ? G(S.bond_dmin)[e] : 0.0;
+        G(F.bhi16)[k] = in ? G(S.bond_dmax)[e] : 0.0;
+    }
+    const int nc = G(S.con_off)[N + 1];
+    for (int k = tid; k < nc; k += all) {
+        const int step0 = G(S.con)[k].step0, nstep = min((int)G(S.con)[k].nstep, FCONSTEP);
+        double *row = F.crow + (size_t)k * (2 + 2 * FCONSTEP);
+        G(row)[0] = G(S.con)[k].dmin;
+        G(row)[1] = G(S.con)[k].dmax;
+        unsigned ez = 0;
+        for (int q = 0; q < FCONSTEP; q++) {
+            const double dq = q < nstep ? G(S.sd)[step0 + q] : 0.0, eq = q < nstep ? G(S.se)[step0 + q] : 0.0;
+            G(row)[2 + q] = dq;
+            G(row)[2 + FCONSTEP + q] = eq;
+            G(F.crad)[k].rad[q] = (float)dq;
+            if (q < nstep && eq == 0) ez |= 1u << q;
+        }
+        G(F.crad)[k].ez = ez;
+    }
+}
+
 // linked cell lists from the cell arrays of one system, for a download
 __global__ __launch_bounds__(256) void k_fast_lists(FSys *systems, int sys) {
     FSys &F = systems[sys];
@@ -2056,8 +2091,7 @@ __global__ __launch_bounds__(256) void k_fast_blocks(FSys *systems) {
 // positions are x + v (T - t0); one wavefront per atom i, two lanes per
 // neighbour cell, for partners j > i.  A chain of dependent loads per pair
 // bounds it, so the atoms are spread over the GPU: gridDim.y workgroups per
-// system, each leaving its sums in `part` (energy_reduce adds them in a fixed
-// order).  One workgroup per system with one thread per atom took 4.0 ms for
+// system, each leaving its sums in `part` (k_energy_reduce adds them).  One workgroup per system with one thread per atom took 4.0 ms for
 // 64 systems of 1 536 atoms.
 __global__ __launch_bounds__(64 * EWAVES) void k_fast_energy(FSys *systems, double *part) {
     const FSys &F = systems[blockIdx.x];
@@ -2070,13 +2104,13 @@ __global__ __launch_bounds__(64 * EWAVES) void k_fast_energy(FSys *systems, doub
     const int N = S.N;
     const double cut2 = S.cutoffr * S.cutoffr;
     const int c = min(lane >> 1, 26);
-    double ke = 0, pe = 0;
+    Sum2 ke = {0, 0}, pe = {0, 0};
     int err = 0;
     for (int i = 1 + blockIdx.y * EWAVES + (tid >> 6); i <= N; i += EWAVES * gridDim.y) {
         const double dti = T - G(F.t0)[i];
         const double vi[3] = {G(S.vx)[i], G(S.vy)[i], G(S.vz)[i]};
         const double xi = G(S.x)[i] + vi[0] * dti, yi = G(S.y)[i] + vi[1] * dti, zi = G(S.z)[i] + vi[2] * dti;
-        if (lane == 0) ke += 0.5 * G(S.mass)[i] * (vi[0] * vi[0] + vi[1] * vi[1] + vi[2] * vi[2]);
+        if (lane == 0) ke.add(0.5 * G(S.mass)[i] * (vi[0] * vi[0] + vi[1] * vi[1] + vi[2] * vi[2]));
         int cc[3] = {G(S.cx)[i] + c_OX[c], G(S.cy)[i] + c_OY[c], G(S.cz)[i] + c_OZ[c]};
         double sh[3] = {0, 0, 0};
         for (int k = 0; k < 3; k++) {
@@ -2094,7 +2128,7 @@ __global__ __launch_bounds__(64 * EWAVES) void k_fast_energy(FSys *systems, doub
             const double r1 = xi - (xj + sh[0]), r2 = yi - (yj + sh[1]), r3 = zi - (zj + sh[2]);
             const double rr = r1 * r1 + r2 * r2 + r3 * r3;
             if (rr > cut2) continue;
-            pe += pair_energy(S, i, j, r1, r2, r3, rr, vi, vj, &err);
+            pe.add(pair_energy(S, i, j, r1, r2, r3, rr, vi, vj, &err));
         }
     }
     energy_partial(ke, pe, err || S.error, part);
@@ -2707,36 +2741,19 @@ int sdmd_fast_open(sdmd_gpu_ctx *c, const sdmd_gpu_opts *o) {
         arena_add(&ar, &F.bb, (const int *)nullptr, (size_t)F.nblk);
         arena_add(&ar, &F.rctr, (const unsigned int *)nullptr, (size_t)N + 1);
         {
-            // bond lists at a fixed stride of 16 (BondTime's connect[16]);
-            // constraint step radii inline (CONSTRn lists, <= 8 steps staged)
-            const size_t n16 = ((size_t)N + 1) * 16;
-            int *hj = (int *)calloc(n16, sizeof(int));
-            double *hl = (double *)calloc(n16, sizeof(double)), *hh = (double *)calloc(n16, sizeof(double));
-            const int nc = d->con_off[N + 1];
-            ConRad *cr = (ConRad *)calloc(nc > 0 ? nc : 1, sizeof(ConRad));
-            if (!hj || !hl || !hh || !cr) { free(hj); free(hl); free(hh); free(cr); return SDMD_ENOMEM; }
-            for (int a = 1; a <= N; a++)
-                for (int k = d->bond_off[a], q = 0; k < d->bond_off[a + 1] && q < 16; k++, q++) {
-                    hj[(size_t)a * 16 + q] = d->bond_j[k];
-                    hl[(size_t)a * 16 + q] = d->bond_dmin[k];
-                    hh[(size_t)a * 16 + q] = d->bond_dmax[k];
-                }
-            for (int k = 0; k < nc; k++) {
-                const sdmd_pair &pc = d->con[k];
-                for (int q = 0; q < pc.nstep && q < 8; q++) {
-                    cr[k].rad[q] = (float)d->step_d[pc.step0 + q];
-                    if (d->step_e[pc.step0 + q] == 0) cr[k].ez |= 1u << q;
-                }
-            }
-            arena_add(&ar, &F.bj16, (const int *)hj, n16);
-            arena_add(&ar, &F.blo16, (const double *)hl, n16);
-            arena_add(&ar, &F.bhi16, (const double *)hh, n16);
-            arena_add(&ar, &F.crad, (const ConRad *)cr, (size_t)(nc > 0 ? nc : 1));
-            free(hj); free(hl); free(hh); free(cr);
-            // FP64 shells at a fixed stride (a constraint of more steps than
-            // a row holds is not staged, and then not read from here)
-            const int CR = 2 + 2 * FCONSTEP, PR = 2 + 2 * PROW;
-            double *rows = (double *)calloc((size_t)(nc > 0 ? nc : 1) * CR, sizeof(double));
+            // bond lists and constraint tables at fixed strides, written by
+            // k_fast_derive from the lists already on the device
+            const size_t nc = (size_t)(d->con_off[N + 1] > 0 ? d->con_off[N + 1] : 1), n16 = ((size_t)N + 1) * 16;
+            const size_t bytes[5] = {n16 * sizeof(int), n16 * sizeof(double), n16 * sizeof(double), nc * sizeof(ConRad),
+                                     nc * (2 + 2 * FCONSTEP) * sizeof(double)};
+            void **dst[5] = {(void **)&F.bj16, (void **)&F.blo16, (void **)&F.bhi16, (void **)&F.crad, (void **)&F.crow};
+            size_t at[5], all = 0;
+            for (int k = 0; k < 5; k++) { at[k] = all; all += (bytes[k] + 255) & ~(size_t)255; }
+            char *block = nullptr;
+            if (hipMalloc((void **)&block, all) != hipSuccess) return SDMD_EDEVICE;
+            if ((rc = dev_keep(c, block))) return rc;
+            for (int k = 0; k < 5; k++) *dst[k] = block + at[k];
+            const int PR = 2 + 2 * PROW;
             // the collision table's rows are one copy for systems of equal tables
             const sdmd_system_desc *d0 = c->desc[0];
             int top = 0;
@@ -2746,7 +2763,7 @@ int sdmd_fast_open(sdmd_gpu_ctx *c, const sdmd_gpu_opts *o) {
                                 !memcmp(d->step_d, d0->step_d, sizeof(double) * top) &&
                                 !memcmp(d->step_e, d0->step_e, sizeof(double) * top);
             double *prows = (double *)calloc(shared ? 1 : (size_t)NT * NT * PR, sizeof(double));
-            if (!rows || !prows) { free(rows); free(prows); return SDMD_ENOMEM; }
+            if (!prows) return SDMD_ENOMEM;
             auto fill = [&](double *r, const sdmd_pair &p, int stride) {
                 r[0] = p.dmin;
                 r[1] = p.dmax;
@@ -2755,12 +2772,10 @@ int sdmd_fast_open(sdmd_gpu_ctx *c, const sdmd_gpu_opts *o) {
                     r[2 + stride + k] = d->step_e[p.step0 + k];
                 }
             };
-            for (int k = 0; k < nc; k++) fill(rows + (size_t)k * CR, d->con[k], FCONSTEP);
             for (int k = 0; k < NT * NT && !shared; k++) fill(prows + (size_t)k * PR, d->pair[k], PROW);
-            arena_add(&ar, &F.crow, (const double *)rows, (size_t)(nc > 0 ? nc : 1) * CR);
             if (shared) F.prow = fs->host[0].prow;
             else arena_add(&ar, &F.prow, (const double *)prows, (size_t)NT * NT * PR);
-            free(rows); free(prows);
+            free(prows);
         }
         if ((rc = arena_commit(c, &ar))) return rc;
         // FP32 screen table: RightPair (ToolFunctions.c:278-292) resolved for
@@ -2847,6 +2862,7 @@ int sdmd_fast_open(sdmd_gpu_ctx *c, const sdmd_gpu_opts *o) {
     }
     if ((rc = fdev_alloc(c, &fs->dev, fs->host, (size_t)c->nsys))) return rc;
     hipLaunchKernelGGL(k_fast_cells, dim3(c->nsys, 64), dim3(256), 0, c->stream, fs->dev);
+    hipLaunchKernelGGL(k_fast_derive, dim3(c->nsys, 64), dim3(256), 0, c->stream, fs->dev);
     if (hipGetLastError() != hipSuccess) return SDMD_EDEVICE;
     if ((rc = fdev_alloc(c, &fs->jobs, (const FJobs *)nullptr, (size_t)c->nsys))) return rc;
     if ((rc = fdev_alloc(c, &fs->help, (const FHelp *)nullptr, (size_t)c->nsys))) return rc;

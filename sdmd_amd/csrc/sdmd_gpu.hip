@@ -1560,12 +1560,12 @@ __global__ __launch_bounds__(64 * EWAVES) void k_energy(Sys *systems, double *pa
     const int N = S.N, tid = threadIdx.x, lane = tid & 63;
     const double cut2 = S.cutoffr * S.cutoffr;
     const int c = min(lane, 26);
-    double ke = 0, pe = 0;
+    Sum2 ke = {0, 0}, pe = {0, 0};
     int err = 0;
     for (int i = 1 + blockIdx.y * EWAVES + (tid >> 6); i <= N; i += EWAVES * gridDim.y) {
         const double xi = G(S.x)[i], yi = G(S.y)[i], zi = G(S.z)[i];
         const double vi[3] = {G(S.vx)[i], G(S.vy)[i], G(S.vz)[i]};
-        if (lane == 0) ke += 0.5 * G(S.mass)[i] * (vi[0] * vi[0] + vi[1] * vi[1] + vi[2] * vi[2]);
+        if (lane == 0) ke.add(0.5 * G(S.mass)[i] * (vi[0] * vi[0] + vi[1] * vi[1] + vi[2] * vi[2]));
         int cc[3] = {G(S.cx)[i] + c_OX[c], G(S.cy)[i] + c_OY[c], G(S.cz)[i] + c_OZ[c]};
         double sh[3] = {0, 0, 0};
         for (int k = 0; k < 3; k++) {
@@ -1580,7 +1580,7 @@ __global__ __launch_bounds__(64 * EWAVES) void k_energy(Sys *systems, double *pa
             const double rr = r1 * r1 + r2 * r2 + r3 * r3;
             if (rr > cut2) continue;
             const double vj[3] = {G(S.vx)[j], G(S.vy)[j], G(S.vz)[j]};
-            pe += pair_energy(S, i, j, r1, r2, r3, rr, vi, vj, &err);
+            pe.add(pair_energy(S, i, j, r1, r2, r3, rr, vi, vj, &err));
         }
     }
     energy_partial(ke, pe, err || S.error, part);
@@ -1911,7 +1911,7 @@ extern "C" int sdmd_gpu_open(const sdmd_system_desc *const *systems, int32_t nsy
         for (int s = 0; s < nsys; s++) maxn = systems[s]->natom > maxn ? systems[s]->natom : maxn;
         const int want = (maxn + EWAVES - 1) / EWAVES, fit = (2048 + nsys - 1) / nsys;
         c->echunks = want < fit ? want : fit;
-        rc = dev_upload(c, &c->epart, (const double *)nullptr, (size_t)3 * nsys * c->echunks);
+        rc = dev_upload(c, &c->epart, (const double *)nullptr, (size_t)ENERGY_PART * nsys * c->echunks);
     }
     if (rc == SDMD_OK) rc = sync_to_device(c);
     if (rc == SDMD_OK && mode == SDMD_MODE_PLAIN) {
