@@ -1750,58 +1750,75 @@ __device__ __forceinline__ int exec_fast(FSys &M, FV &F, Pending &e, int *renew,
 // A wavefront scans four blocks at once, one per row of 16 lanes with four
 // atoms per lane: the reductions stay inside rows (DPP moves only) and serve
 // four blocks with the instructions that one block takes.
-struct RowMin { double t; int k, p; };       // time, atom, the atom's partner
-__device__ __forceinline__ bool earlier(double t, int k, double u, int l) { return t < u || (t == u && k < l); }
-template <int S>
-__device__ __forceinline__ void row_min_step(RowMin &m) {
-    unsigned own, tl, th, k, p;
-    const unsigned long long w = (unsigned long long)__double_as_longlong(m.t);
-    xpair<S>((unsigned)w, own, tl);
-    xpair<S>((unsigned)(w >> 32), own, th);
-    xpair<S>((unsigned)m.k, own, k);
-    xpair<S>((unsigned)m.p, own, p);
-    const double t = __longlong_as_double((long long)(((unsigned long long)th << 32) | tl));
-    if (earlier(t, (int)k, m.t, m.k)) { m.t = t; m.k = (int)k; m.p = (int)p; }
+// Times are compared as two ordered unsigned words, high words first.
+template <int CTRL>
+__device__ __forceinline__ unsigned row_umin_step(unsigned v) {
+    return min(v, (unsigned)__builtin_amdgcn_update_dpp(-1, (int)v, CTRL, 0xF, 0xF, false));
 }
-// smallest (t, k) of the row from each lane's four
-__device__ __forceinline__ RowMin row_min(const double (&t)[4], const int (&k)[4], const int (&p)[4]) {
-    RowMin m = {t[0], k[0], p[0]};
+// the row's smallest word, in all its lanes (quad permutations, half-row and
+// row mirrors)
+__device__ __forceinline__ unsigned row_umin(unsigned v) {
+    return row_umin_step<0x140>(row_umin_step<0x141>(row_umin_step<0x4E>(row_umin_step<0xB1>(v))));
+}
+struct RowScan {
+    unsigned hi[4], lo[4];       // times of this lane's atoms as ordered words
+    int k[4], p[4];              // atoms (0x7fffffff: none) and their partners
+};
+// the row's smallest time; with TAKE also its atom (the lowest on equal
+// times), which leaves the scan with its mirror
+template <bool TAKE>
+__device__ __forceinline__ double row_first(RowScan &r, int &atom) {
+    const unsigned H = row_umin(min(min(r.hi[0], r.hi[1]), min(r.hi[2], r.hi[3])));
+    unsigned l = 0xffffffffu;
 #pragma unroll
-    for (int u = 1; u < 4; u++)
-        if (earlier(t[u], k[u], m.t, m.k)) { m.t = t[u]; m.k = k[u]; m.p = p[u]; }
-    row_min_step<0>(m); row_min_step<1>(m); row_min_step<2>(m); row_min_step<3>(m);
-    return m;
+    for (int u = 0; u < 4; u++) l = min(l, r.hi[u] == H ? r.lo[u] : 0xffffffffu);
+    const unsigned L = row_umin(l);
+    if (TAKE) {
+        unsigned a = 0x7fffffffu;
+#pragma unroll
+        for (int u = 0; u < 4; u++) a = min(a, (r.hi[u] == H && r.lo[u] == L) ? (unsigned)r.k[u] : 0x7fffffffu);
+        const int K = (int)row_umin(a);
+        unsigned q = 0xffffffffu;                // the atom's partner (one lane holds it)
+#pragma unroll
+        for (int u = 0; u < 4; u++) q = min(q, r.k[u] == K ? (unsigned)r.p[u] : 0xffffffffu);
+        const int P = (int)row_umin(q);
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+            if (r.k[u] == K || (r.k[u] == P && r.p[u] == K)) {
+                order_words(__builtin_inf(), r.hi[u], r.lo[u]);
+                r.k[u] = 0x7fffffff;
+                r.p[u] = 0;
+            }
+        atom = K;
+    }
+    const unsigned s = (H >> 31) ? 0u : 0xffffffffu;             // order_words undone
+    return __longlong_as_double((long long)(((unsigned long long)(H ^ (s | 0x80000000u)) << 32) | (L ^ s)));
 }
 
 // the earliest (t1, a1) and second (t2, a2) events of this row's block b that
 // are not the mirror of an earlier one, and its third time t3 (b < 0: none)
 __device__ __forceinline__ void block_scan4(FV &F, int b, double &t1, int &a1, double &t2, int &a2, double &t3) {
     const int l = threadIdx.x & 15, N = F.s.N;
-    const double inf = __builtin_inf();
+    RowScan r;
     double t[4];
-    int k[4], p[4];
 #pragma unroll
     for (int u = 0; u < 4; u++) {
         const int a = b * 64 + 16 * u + l + 1;
         const bool in = b >= 0 && a <= N;
-        const int r = in ? a : 1;
-        t[u] = G(F.s.evt)[r];
-        p[u] = G(F.s.evp)[r];
-        k[u] = in ? a : 0x7fffffff;
+        const int q = in ? a : 1;
+        t[u] = G(F.s.evt)[q];
+        r.p[u] = G(F.s.evp)[q];
+        r.k[u] = in ? a : 0x7fffffff;
     }
 #pragma unroll
-    for (int u = 0; u < 4; u++)
-        if (k[u] == 0x7fffffff) { t[u] = inf; p[u] = 0; }
-    const RowMin m = row_min(t, k, p);
-#pragma unroll
-    for (int u = 0; u < 4; u++)
-        if (k[u] == m.k || (k[u] == m.p && p[u] == m.k)) { t[u] = inf; k[u] = 0x7fffffff; p[u] = 0; }
-    const RowMin n = row_min(t, k, p);
-#pragma unroll
-    for (int u = 0; u < 4; u++)
-        if (k[u] == n.k || (k[u] == n.p && p[u] == n.k)) { t[u] = inf; k[u] = 0x7fffffff; p[u] = 0; }
-    const RowMin o = row_min(t, k, p);
-    t1 = m.t; a1 = m.k; t2 = n.t; a2 = n.k; t3 = o.t;
+    for (int u = 0; u < 4; u++) {
+        if (r.k[u] == 0x7fffffff) { t[u] = __builtin_inf(); r.p[u] = 0; }
+        order_words(t[u], r.hi[u], r.lo[u]);
+    }
+    int none;
+    t1 = row_first<true>(r, a1);
+    t2 = row_first<true>(r, a2);
+    t3 = row_first<false>(r, none);
 }
 
 // ---------------------------------------------------------------- helper workgroups
@@ -2269,7 +2286,7 @@ __global__ __launch_bounds__(64 * W) void k_fast_run(FSys *systems, FJobs *jobs,
             if (t < m1 || (t == m1 && sh.ba[b] < a1)) { m1 = t; a1 = sh.ba[b]; }
         }
         m3 = wave_min_d(m3);
-        m2 = wave_min_d(m2);
+        if (!small) m2 = wave_min_d(m2);                      // only needed where a set can be too large
         wave_argmin(m1, a1);
         const double tcap = nextafter(F.t_stop, __builtin_inf());
         double theta = fmin(m2, tcap), theta3 = fmin(m3, tcap), tmin = m1;
@@ -2301,8 +2318,6 @@ __global__ __launch_bounds__(64 * W) void k_fast_run(FSys *systems, FJobs *jobs,
             if (sh.err || !pending || amin < 1 || amin > S.N || (sh.drain && M.pops >= sh.drain_end))
                 sh.stop = 1;
             sh.nsel = 0;
-            sh.nren = 0;
-            sh.nlight = 0;
             sh.next_ren = 0;
             sh.conflict = 0;
         }
@@ -2312,23 +2327,32 @@ __global__ __launch_bounds__(64 * W) void k_fast_run(FSys *systems, FJobs *jobs,
             if (old_epoch) rebase<W>(F, C, tmin);
         }
         // collect the prefix set
-        auto collect = [&](double before, bool second) {
-            for (int b = small ? lane : tid; b < nblk; b += small ? 64 : 64 * W) {
-                if (sh.b1[b] < before) {
-                    const int slotk = atomicAdd(&sh.nsel, 1);
-                    if (slotk < FSEL) { sh.sel_t[slotk] = sh.b1[b]; sh.sel_a[slotk] = sh.ba[b]; }
-                }
-                if (second && sh.b2[b] < before) {
-                    const int slotk = atomicAdd(&sh.nsel, 1);
-                    if (slotk < FSEL) { sh.sel_t[slotk] = sh.b2[b]; sh.sel_a[slotk] = sh.bb[b]; }
-                }
+        if (small) {                                          // at most 2 * FSMALL events: no overflow
+            wave_sync();
+            if (wave == 0 && !sh.stop) {
+                const int b = min(lane, nblk - 1);
+                const double u1 = sh.b1[b], u2 = sh.b2[b];
+                const bool in1 = lane < nblk && u1 < theta3, in2 = lane < nblk && u2 < theta3;
+                const unsigned long long k1 = __ballot(in1), k2 = __ballot(in2), below = (1ull << lane) - 1;
+                const int n1 = __popcll(k1), s1 = __popcll(k1 & below), s2 = n1 + __popcll(k2 & below);
+                if (in1) { sh.sel_t[s1] = u1; sh.sel_a[s1] = sh.ba[b]; }
+                if (in2) { sh.sel_t[s2] = u2; sh.sel_a[s2] = sh.bb[b]; }
+                if (lane == 0) sh.nsel = n1 + __popcll(k2);
             }
-        };
-        if (small) {
-            wave_sync();                                      // at most 2 * FSMALL events: no overflow
-            if (wave == 0 && !sh.stop) collect(theta3, true);
             wave_sync();
         } else {
+            auto collect = [&](double before, bool second) {
+                for (int b = tid; b < nblk; b += 64 * W) {
+                    if (sh.b1[b] < before) {
+                        const int slotk = atomicAdd(&sh.nsel, 1);
+                        if (slotk < FSEL) { sh.sel_t[slotk] = sh.b1[b]; sh.sel_a[slotk] = sh.ba[b]; }
+                    }
+                    if (second && sh.b2[b] < before) {
+                        const int slotk = atomicAdd(&sh.nsel, 1);
+                        if (slotk < FSEL) { sh.sel_t[slotk] = sh.b2[b]; sh.sel_a[slotk] = sh.bb[b]; }
+                    }
+                }
+            };
             collect(theta3, true);
             __syncthreads();
             if (sh.nsel > FSEL) {
@@ -2343,6 +2367,7 @@ __global__ __launch_bounds__(64 * W) void k_fast_run(FSys *systems, FJobs *jobs,
         int ns = 0;
         Pending ev;
         ev.a = 0x7fffffff;
+        ev.ra = ev.rp = 0;
         ev.t = __builtin_inf();
         if (wave == 0 && !sh.stop) {
             ns = sh.nsel;
@@ -2441,20 +2466,27 @@ __global__ __launch_bounds__(64 * W) void k_fast_run(FSys *systems, FJobs *jobs,
                 sh.nex = nex;
                 F.deferred += ns - nex;
             }
-            if (ok) {
-                // H-bond-capable atoms (acceptor, donor, sulfur) scan their
-                // neighbourhood for H-bond partners: the longest predictions
-                // of a round, queued first so the waves finish together
-                int renew[2] = {0, 0};
-                const int nr = exec_fast(F, C, ev, renew, &err);
-                for (int r = 0; r < nr; r++) {
-                    const signed char ro = r ? ev.rp : ev.ra;    // renew[1] is the partner
-                    const bool heavy = ro == 'A' || ro == 'D' || ro == 'S';
-                    const int slot = heavy ? atomicAdd(&sh.nren, 1) : 2 * FSEL - 1 - atomicAdd(&sh.nlight, 1);
+            int renew[2] = {0, 0}, nr = 0;
+            if (ok) nr = exec_fast(F, C, ev, renew, &err);
+            // H-bond-capable atoms (acceptor, donor, sulfur) scan their
+            // neighbourhood for H-bond partners: the longest predictions of a
+            // round, queued first so the waves finish together
+            const unsigned long long below = (1ull << lane) - 1;
+            int nh = 0, nl = 0;
+#pragma unroll
+            for (int r = 0; r < 2; r++) {
+                const signed char ro = r ? ev.rp : ev.ra;        // renew[1] is the partner
+                const bool heavy = ro == 'A' || ro == 'D' || ro == 'S';
+                const unsigned long long mh = __ballot(r < nr && heavy), ml = __ballot(r < nr && !heavy);
+                if (r < nr) {
+                    const int slot = heavy ? nh + __popcll(mh & below) : 2 * FSEL - 1 - (nl + __popcll(ml & below));
                     sh.ren_a[slot] = renew[r];
                     sh.ren_t[slot] = ev.t;
                 }
+                nh += __popcll(mh);
+                nl += __popcll(ml);
             }
+            if (lane == 0) { sh.nren = nh; sh.nlight = nl; }
             const double last = -wave_min_d(ok ? -ev.t : __builtin_inf());
             if (lane == 0 && nex > 0 && F.tlast < last) F.tlast = last;
         }
