@@ -54,6 +54,7 @@ constexpr int FCAP_MIN = 64;      // slots per cell at least (a system's capacit
 constexpr int FCAP_MAX = 1024;    // ... at most
 constexpr int FMAXBLK = 1024;     // 64-atom blocks per system (N <= 65535)
 constexpr int FSEL = 64;          // events considered per round
+constexpr int FSEL_AIM = 54;      // ... aimed at where a window of time bounds the set
 constexpr int FSMALL = 32;        // 64-atom blocks up to which one wavefront selects and executes a round
 constexpr int FMAXW = 16;         // wavefronts per workgroup at most
 constexpr long long FDRAIN = 1 << 20;   // bound on the pops of a closing drain
@@ -1902,6 +1903,7 @@ __device__ __forceinline__ void job_done(FJobs *J, bool failed) {
 template <int W>
 struct FShared {
     long long run_clock_end, run_count_end;   // the launch's bounds (thread 0)
+    double window;                            // span of event times collected per round
     double b1[FMAXBLK], b2[FMAXBLK], b3[FMAXBLK];
     int ba[FMAXBLK], bb[FMAXBLK];
     double red_t[W], red_t1[W], red_t3[W];
@@ -2257,6 +2259,7 @@ __global__ __launch_bounds__(64 * W) void k_fast_run(FSys *systems, FJobs *jobs,
     if (tid < FMAXBLK / 32) sh.dmask[tid] = 0;
     __syncthreads();
     if (tid == 0) {                       // npops < 0: -npops executed events
+        sh.window = __builtin_inf();
         sh.run_clock_end = (long long)wall_clock64() + budget;
         sh.run_count_end = npops < 0 ? M.frame - npops : M.pops + npops;
     }
@@ -2265,6 +2268,10 @@ __global__ __launch_bounds__(64 * W) void k_fast_run(FSys *systems, FJobs *jobs,
     wave_sync();
     const int cap = C.max_batch > 0 ? min(C.max_batch, FSEL) : FSEL;
     const bool small = nblk <= FSMALL;
+    // A run of a number of pops or events ends with the round that reaches
+    // it, so its rounds keep their sets; a run up to a time has the same
+    // result whatever they are.
+    const bool wide = !small && llabs(npops) >= (1LL << 32);
     unsigned long long pt = prof ? wall_clock64() : 0;
     while (true) {
         // ---- selection: every event earlier than the smallest third time of
@@ -2353,9 +2360,32 @@ __global__ __launch_bounds__(64 * W) void k_fast_run(FSys *systems, FJobs *jobs,
                     }
                 }
             };
-            collect(theta3, true);
+            // Any time up to theta3 bounds a prefix of the event order.  Where
+            // that of theta3 is too large (more than about 200 blocks), the
+            // events of a window of time are taken that holds about FSEL_AIM
+            // of them, the window following the counts seen: a round costs
+            // 20 us beside its predictions, and the blocks' second times,
+            // the other bound at hand, leave only 27 events of 408 blocks.
+            const double reach = wide ? fmin(theta3, tmin + sh.window) : theta3;
+            collect(reach, true);
             __syncthreads();
-            if (sh.nsel > FSEL) {
+            int found = sh.nsel;
+            if (wide) {
+                double w = sh.window;
+                if (found > FSEL) {
+                    __syncthreads();
+                    w = (reach - tmin) * ((double)FSEL_AIM / found);
+                    if (tid == 0) sh.nsel = 0;
+                    __syncthreads();
+                    collect(fmax(theta, tmin + w), true);
+                    __syncthreads();
+                    found = sh.nsel;
+                } else if (reach < theta3) {                  // the window was the bound
+                    w *= fmin(fmax((double)FSEL_AIM / max(found, 1), 0.8), 1.25);
+                }
+                if (tid == 0) sh.window = w;                  // read next after the coming barriers
+            }
+            if (found > FSEL) {
                 __syncthreads();
                 if (tid == 0) sh.nsel = 0;
                 __syncthreads();
