@@ -957,6 +957,25 @@ __device__ void predict_list(Sys &S, Smem &sm, const PairTab *T, const int *rene
 }
 
 // ---------------------------------------------------------------- CBT, CBT.c
+// the winner of a stretch of a path: its time, atom << 1 | (its level's
+// sibling is to the right of all below)
+struct PathMin {
+    double t;
+    int v;
+    // this stretch above another one
+    __device__ __forceinline__ void after(const PathMin &o) {
+        if (!(t < o.t || (t == o.t && (v & 1)))) { t = o.t; v = o.v; }
+    }
+    // that of the lane a DPP move reads from (none: one that never wins)
+    template <int CTRL, int ROWS>
+    __device__ __forceinline__ PathMin from() const {
+        const unsigned long long w = (unsigned long long)__double_as_longlong(t);
+        const unsigned lo = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)w, CTRL, ROWS, 0xF, false);
+        const unsigned hi = (unsigned)__builtin_amdgcn_update_dpp(0x7ff00000, (int)(unsigned)(w >> 32), CTRL, ROWS, 0xF, false);
+        return {__longlong_as_double((long long)(((unsigned long long)hi << 32) | lo)),
+                __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xF, false)};
+    }
+};
 // UpdateCBT (CBT.c:33-39, 56-83) for one or two renewed atoms, by one wave.
 // A path's nodes follow from the leaf's index alone, so each lane holds one
 // level (lanes 0..31 the first atom's path, 32..63 the second's): the path's
@@ -987,23 +1006,30 @@ __device__ __forceinline__ void cbt_update(Sys &S, Smem &sm, int n, int a0, int 
             if (qs >= 0 && ds) { sv = sn; st = tn; }
             if (qf >= 0 && df) { of = fn; nv = fn; }
         }
-        const int a = h ? a1 : a0, Lh = h ? l1 : l0, d = 31 - __clz(Lh);
-        int cur = a;
-        double tc = h ? t1 : t0;
-        bool own = true;       // still on nodes that held the atom itself
-        for (int q = 0; q < d; q++) {
-            const int src = 32 * h + q;
-            const int o = lane_get(of, src), s = lane_get(sv, src);
-            const double ts = lane_get(st, src);
-            const bool left = !((Lh >> q) & 1);
-            own = own && o == a;
-            // node = (evt[left] < evt[right]) ? left : right
-            const bool keep = left ? tc < ts : !(ts < tc);
-            if (!keep) { cur = s; tc = ts; }
-            if (lane == src) { nv = cur; nt = tc; done = true; }
-            if (!own && cur == o) break;
+        const int a = h ? a1 : a0, d = 31 - __clz(h ? l1 : l0);
+        const bool here = half == h && on;
+        // node = (evt[left] < evt[right]) ? left : right: on equal times the
+        // one to the right, so a level's winner is the smallest (time, place)
+        // of the atom and the siblings up to there, and the sibling is to the
+        // right where the path is the left child
+        PathMin e = {here ? st : __builtin_inf(), here ? (sv << 1) | (int)!((L >> k) & 1) : 0};
+        if (here && k == 0) e.after({h ? t1 : t0, a << 1});
+        e.after(e.from<0x111, 0xF>());                 // row_shr:1, 2, 4, 8
+        e.after(e.from<0x112, 0xF>());
+        e.after(e.from<0x114, 0xF>());
+        e.after(e.from<0x118, 0xF>());
+        e.after(e.from<0x142, 0xA>());                 // row_bcast:15
+        const int cur = e.v >> 1;
+        // the walk ends where a node keeps its value, except on nodes that
+        // held the atom itself from the leaf on
+        const unsigned changed = (unsigned)(__ballot(here && of != a) >> (32 * h));
+        const int first = changed ? __builtin_ctz(changed) : 32;
+        const unsigned kept = (unsigned)(__ballot(here && k >= first && cur == of) >> (32 * h));
+        const int last = kept ? __builtin_ctz(kept) : d - 1;
+        if (here && k <= last) {
+            nv = cur; nt = e.t; done = true;
+            if (nv != of) G(S.node)[f] = nv;
         }
-        if (half == h && on && done && nv != of) G(S.node)[f] = nv;
         if (lane == 32 * h + d - 1) sm.root = nv;      // the top level: node 1
         wave_sync();
     }
