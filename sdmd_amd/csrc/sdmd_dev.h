@@ -115,12 +115,19 @@ struct Sys {
     int gstride[48];
 };
 
+// A system's struct as constant memory: what a launch does not change
+// (pointers, sizes, tables) is read through this view into scalar registers,
+// where a copy in LDS costs a wait per use.  Counters and clocks are read and
+// written in the LDS copy only.
+typedef const __attribute__((address_space(4))) Sys SV;
+__device__ __forceinline__ SV &fixed_view(const Sys *p) { return *(SV *)p; }
+
 // phases timed when a context is opened with profiling on
 enum { PH_POP, PH_SWEEP, PH_EVENT, PH_STAGE, PH_GATHER, PH_BONDSEL, PH_EVAL, PH_SELECT, PH_HB, PH_TAIL,
        PH_TREE, PH_NPH };
 
-#define PROF_MARK(S, ph, t) do { if ((S).prof && threadIdx.x == 0) { unsigned long long _n = wall_clock64(); \
-    (S).prof[ph] += _n - (t); (t) = _n; } } while (0)
+#define FPROF(prof, ph, t) do { if ((prof) && threadIdx.x == 0) { unsigned long long _n = wall_clock64(); \
+    (prof)[ph] += _n - (t); (t) = _n; } } while (0)
 
 // ---------------------------------------------------------------- models
 static __device__ __forceinline__ int type_change(int t, int direct) {   // AtomTypeChange, ToolFunctions.c:233-270

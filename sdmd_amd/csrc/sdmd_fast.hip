@@ -73,9 +73,6 @@ enum { FERR_SELECT = 20, FERR_SLOT = 21, FERR_ROW = 22, FERR_CAND = 23, FERR_NBL
 enum { FPH_SELECT, FPH_EXEC, FPH_STAGE, FPH_SCREEN, FPH_CONFIRM, FPH_OTHER, FPH_TREE, FPH_EVENT, FPH_BOND,
        FPH_SCAN, FPH_COLLECT };
 
-#define FPROF(prof, ph, t) do { if ((prof) && threadIdx.x == 0) { unsigned long long _n = wall_clock64(); \
-    (prof)[ph] += _n - (t); (t) = _n; } } while (0)
-
 // step radii (squared, FP32) of one constraint entry and bit k set when
 // step k carries no energy
 constexpr int PROW = 16;          // steps per collision pair at most
@@ -118,12 +115,8 @@ struct FSys {
 };
 
 // ---------------------------------------------------------------- fixed view
-// A system's struct as constant memory: what a launch does not change
-// (pointers, sizes, tables) is read through this view into scalar registers,
-// where the copy in LDS costs a wait per use.  Counters, epoch and clock are
-// read and written in the LDS copy only.
+// (see fixed_view of Sys)
 typedef const __attribute__((address_space(4))) FSys FV;
-typedef const __attribute__((address_space(4))) Sys SV;
 __device__ __forceinline__ FV &fixed_view(const FSys *p) { return *(FV *)p; }
 // the same view, read anew: the compiler keeps nothing it read before across
 // this point (a hundred values held over the whole event loop would be moved

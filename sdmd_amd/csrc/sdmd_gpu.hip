@@ -114,7 +114,8 @@ struct PairTab {
 // The same operations in the same order give the same bits; the sweep's
 // memory traffic is paid once per LOGK pops (a sweep per pop cost 33 us of a
 // 73 us pop at 26 080 atoms).
-__device__ __forceinline__ int lag_of(const Sys &S, int n, int j) { return n ? (int)G(S.lag)[j] : 0; }
+template <class SYS>
+__device__ __forceinline__ int lag_of(SYS &S, int n, int j) { return n ? (int)G(S.lag)[j] : 0; }
 
 __device__ __forceinline__ void steps_pos(const double *log, int l, int n, double &x, double &y, double &z, double vx,
                                           double vy, double vz) {
@@ -125,13 +126,15 @@ __device__ __forceinline__ void steps_pos(const double *log, int l, int n, doubl
         z = z + vz * dt;
     }
 }
-__device__ __forceinline__ double evt_now(const Sys &S, const Smem &sm, int j) {
+template <class SYS>
+__device__ __forceinline__ double evt_now(SYS &S, const Smem &sm, int j) {
     double t = G(S.evt)[j];
     const int n = sm.nlog;
     for (int l = lag_of(S, n, j); l < n; l++) t = t - sm.log[l];
     return t;
 }
-__device__ __forceinline__ void pos_now(const Sys &S, const Smem &sm, int j, double *p) {
+template <class SYS>
+__device__ __forceinline__ void pos_now(SYS &S, const Smem &sm, int j, double *p) {
     const int n = sm.nlog, l = lag_of(S, n, j);
     double x = G(S.x)[j], y = G(S.y)[j], z = G(S.z)[j];
     if (l < n) steps_pos(sm.log, l, n, x, y, z, G(S.vx)[j], G(S.vy)[j], G(S.vz)[j]);
@@ -147,7 +150,7 @@ struct PosLazy {      // PosStored with the steps an atom has not taken yet
 };
 
 // pair kinematics of the staged atom and j's current state
-__device__ __forceinline__ void calc_params_now(const Sys &S, const Smem &sm, const Atom &A, int j, Kin &k) {
+__device__ __forceinline__ void calc_params_now(SV &S, const Smem &sm, const Atom &A, int j, Kin &k) {
     double p[3];
     pos_now(S, sm, j, p);
     calc_params_at(S, A.x, A.y, A.z, A.vx, A.vy, A.vz, A.cx, A.cy, A.cz, j, p[0], p[1], p[2], G(S.vx)[j], G(S.vy)[j],
@@ -156,7 +159,7 @@ __device__ __forceinline__ void calc_params_now(const Sys &S, const Smem &sm, co
 
 // UpdateData + TimeForward over all atoms: each takes the steps it still lacks
 template <int B>
-__device__ __forceinline__ void sweep(const Sys &S, Smem &sm) {
+__device__ __forceinline__ void sweep(SV &S, Smem &sm) {
     const int n = sm.nlog, N = S.N;
     for (int i = threadIdx.x + 1; i <= N; i += B) {
         int l = G(S.lag)[i];
@@ -225,13 +228,13 @@ __device__ __forceinline__ void wave_select(int n, const double *ct, const unsig
 }
 
 // JobAssign / CheckDuplication result applied to the staged record (lane 0)
-__device__ __forceinline__ void take_computed(Atom &A, const Sys &S, double t, double pot, int sub, int type, int j) {
+__device__ __forceinline__ void take_computed(Atom &A, SV &S, double t, double pot, int sub, int type, int j) {
     A.pot = pot; A.sub = sub; A.t = t; A.evtype = type;
     if (j) { A.partner = j; A.pc = G(S.evc)[j]; }
     else A.partner = INVALID;
 }
 
-__device__ __forceinline__ void take_inherited(Atom &A, const Sys &S, const Smem &sm, int j, int type) {
+__device__ __forceinline__ void take_inherited(Atom &A, SV &S, const Smem &sm, int j, int type) {
     A.partner = j; A.pot = G(S.evpot)[j]; A.sub = G(S.evsub)[j]; A.t = evt_now(S, sm, j); A.evtype = type;
     A.pc = G(S.evc)[j];
 }
@@ -239,13 +242,13 @@ __device__ __forceinline__ void take_inherited(Atom &A, const Sys &S, const Smem
 // CheckDuplication's condition; A.exclude is an atom whose record is being
 // written by another wavefront (it held none when A's prediction began)
 __device__ __forceinline__ bool dup_open(const Atom &A, int j) { return A.exclude >= 0 && j != A.exclude && j < A.below; }
-__device__ __forceinline__ bool dupable(const Sys &S, const Atom &A, int j, int type) {
+__device__ __forceinline__ bool dupable(SV &S, const Atom &A, int j, int type) {
     return dup_open(A, j) && G(S.evp)[j] == A.i && G(S.evtype)[j] == type && G(S.evpc)[j] == A.counter;
 }
 
 // ---------------------------------------------------------------- candidate evaluation
 // one BondTime entry, TimePrediction.c:219-293
-__device__ __forceinline__ void eval_bond(const Sys &S, const Smem &sm, const Atom &A, Cand &C, int q) {
+__device__ __forceinline__ void eval_bond(SV &S, const Smem &sm, const Atom &A, Cand &C, int q) {
     const int e = A.bo + q;
     const int j = G(S.bond_j)[e];
     const double lo = G(S.bond_dmin)[e], hi = G(S.bond_dmax)[e];
@@ -325,7 +328,7 @@ __device__ __forceinline__ int shell_fast(double dmin, double dmax, int nstep, c
 // Every field of j that either may need is loaded at once (one round trip);
 // shells come from LDS.
 template <bool TAB>
-__device__ __forceinline__ void eval_candidate(const Sys &S, const Smem &sm, const PairTab *T, const Atom &A, Cand &C,
+__device__ __forceinline__ void eval_candidate(SV &S, const Smem &sm, const PairTab *T, const Atom &A, Cand &C,
                                                int kidx, double calib, int *err) {
     const int j = C.j[kidx], i = A.i;
     double tout = __builtin_inf(), pot = 0, ht = __builtin_inf(), hpot = 0;
@@ -434,7 +437,7 @@ __device__ __forceinline__ void eval_candidate(const Sys &S, const Smem &sm, con
 }
 
 // ---------------------------------------------------------------- lane-0 pieces
-__device__ void job_assign_atom(Atom &A, const Sys &S, double t, double pot, int sub, int type, int j) {
+__device__ void job_assign_atom(Atom &A, SV &S, double t, double pot, int sub, int type, int j) {
     if (t > 0 && A.t > t) take_computed(A, S, t, pot, sub, type, j);
 }
 
@@ -444,7 +447,7 @@ __device__ double next_normal(Sys &S, Smem &sm) {
 }
 
 // PBCandCrossCellTime along axis n, TimePrediction.c:598-632 (INFINIT: none)
-__device__ __forceinline__ double pcc_axis(const Sys &S, double pos, double v, int ci, int n) {
+__device__ __forceinline__ double pcc_axis(SV &S, double pos, double v, int ci, int n) {
     double t = -1;
     const double lo = ci * S.cellsize[n + 1], hi = (ci + 1) * S.cellsize[n + 1];
     if (v > 0) t = (hi - pos + ZERO) / v;
@@ -453,7 +456,7 @@ __device__ __forceinline__ double pcc_axis(const Sys &S, double pos, double v, i
 }
 
 // HBTime for a bonded HB atom, TimePrediction.c:330-383
-__device__ void hb_time_bonded(const Sys &S, const Smem &sm, Atom &A, int *err) {
+__device__ void hb_time_bonded(SV &S, const Smem &sm, Atom &A, int *err) {
     const int j = A.hbbond;
     if (dupable(S, A, j, SDMD_HB) && A.t > evt_now(S, sm, j)) { take_inherited(A, S, sm, j, SDMD_HB); return; }
     Kin k;
@@ -475,7 +478,7 @@ __device__ void hb_time_bonded(const Sys &S, const Smem &sm, Atom &A, int *err) 
 }
 
 // HBNeighborTime, TimePrediction.c:486-579
-__device__ void hb_neighbor_time(const Sys &S, const Smem &sm, Atom &A, int *err) {
+__device__ void hb_neighbor_time(SV &S, const Smem &sm, Atom &A, int *err) {
     int flag = 0;
     for (int n = 1; n <= A.nbstat; n++) {
         const int j = A.nbp[n];
@@ -534,7 +537,7 @@ __device__ __forceinline__ void stage_atom(const Sys &S, Atom &A, int i, int exc
 // has several, and the candidates of the 27 cells (DMD.c:117-121 order, each
 // in list order: the cell arrays hold a list back to front) on all of them.
 template <bool CELLS>
-__device__ __forceinline__ void stage_neighbours(const Sys &S, const Smem &sm, Atom &A, Cand &C, int r, int nw, int *err) {
+__device__ __forceinline__ void stage_neighbours(SV &S, const Smem &sm, Atom &A, Cand &C, int r, int nw, int *err) {
     const int lane = threadIdx.x & 63;
     // occupancy of the 27 cells, by every wave for itself
     const int cl = min(lane, 26);
@@ -638,7 +641,7 @@ __device__ __forceinline__ void stage_neighbours(const Sys &S, const Smem &sm, A
 
 // The predicted atom's record from the evaluated entries, in the reference's
 // order (one wave): bonds and collisions ...
-__device__ __forceinline__ void select_bonds(const Sys &S, const Smem &sm, Atom &A, Cand &C) {
+__device__ __forceinline__ void select_bonds(SV &S, const Smem &sm, Atom &A, Cand &C) {
     double m = A.t;
     int win = -1, inh = 0;
     wave_select(min(A.nb, MAXBOND), C.bt, C.bfl, [&](int d) { return C.bjt[d]; }, m, win, inh);
@@ -647,7 +650,7 @@ __device__ __forceinline__ void select_bonds(const Sys &S, const Smem &sm, Atom 
         else take_computed(A, S, C.bt[win], 0, C.bsub[win], SDMD_BOND, C.bj[win]);
     }
 }
-__device__ __forceinline__ void select_collisions(const Sys &S, const Smem &sm, Atom &A, Cand &C, int n) {
+__device__ __forceinline__ void select_collisions(SV &S, const Smem &sm, Atom &A, Cand &C, int n) {
     double m = A.t;
     int win = -1, inh = 0;
     wave_select(n, C.t, C.fl, [&](int d) { return evt_now(S, sm, C.j[d]); }, m, win, inh);
@@ -657,7 +660,7 @@ __device__ __forceinline__ void select_collisions(const Sys &S, const Smem &sm, 
     }
 }
 // ... cell crossing, thermostat, the bonded H-bond partner (lane 0) ...
-__device__ __forceinline__ void assign_onebody(const Sys &S, const Smem &sm, Atom &A, const Cand &C, int *err) {
+__device__ __forceinline__ void assign_onebody(SV &S, const Smem &sm, Atom &A, const Cand &C, int *err) {
     double t_ev = INFINIT;
     for (int n = 0; n < 3; n++)
         if (t_ev > C.pcc[n]) t_ev = C.pcc[n];
@@ -670,7 +673,7 @@ __device__ __forceinline__ void assign_onebody(const Sys &S, const Smem &sm, Ato
     if (A.hbitype != SDMD_HBSKIP && A.hbbond > 0) hb_time_bonded(S, sm, A, err);
 }
 // ... the free H-bond scan ...
-__device__ __forceinline__ void select_hbonds(const Sys &S, const Smem &sm, Atom &A, Cand &C, int n) {
+__device__ __forceinline__ void select_hbonds(SV &S, const Smem &sm, Atom &A, Cand &C, int n) {
     double m = A.t;
     int win = -1, inh = 0;
     wave_select(n, C.ht, C.hfl, [&](int d) { return evt_now(S, sm, C.j[d]); }, m, win, inh);
@@ -680,7 +683,7 @@ __device__ __forceinline__ void select_hbonds(const Sys &S, const Smem &sm, Atom
     }
 }
 // ... H-bond neighbours and the wall, and the record stored (lane 0)
-__device__ __forceinline__ void assign_tail(Sys &S, const Smem &sm, Atom &A, int *err) {
+__device__ __forceinline__ void assign_tail(SV &S, const Smem &sm, Atom &A, int *err) {
     hb_neighbor_time(S, sm, A, err);
     if (S.wall) {
         WallEv w;
@@ -696,7 +699,7 @@ __device__ __forceinline__ void assign_tail(Sys &S, const Smem &sm, Atom &A, int
     G(S.hbitype)[i] = SDMD_NOEVENT;
 }
 
-__device__ __forceinline__ void finish_atom(Sys &S, const Smem &sm, Atom &A, Cand &C, int *err) {
+__device__ __forceinline__ void finish_atom(SV &S, const Smem &sm, Atom &A, Cand &C, int *err) {
     const int lane = threadIdx.x & 63, n = A.ncand;
     select_bonds(S, sm, A, C);
     wave_sync();
@@ -717,7 +720,7 @@ __device__ __forceinline__ int wants_hbscan(const Atom &A) {
 
 // candidates [w0, w0 + n) of the staged atom's ordered list (all threads)
 template <int B>
-__device__ __forceinline__ void gather_window(const Sys &S, const Atom &A, Cand &C, int w0, int n) {
+__device__ __forceinline__ void gather_window(SV &S, const Atom &A, Cand &C, int w0, int n) {
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     if (!A.over) {
         for (int c = wave; c < 27; c += B / 64) {
@@ -744,7 +747,7 @@ __device__ __forceinline__ void gather_window(const Sys &S, const Atom &A, Cand 
 // minimum (and CheckDuplication against it) carries over, so the result is
 // that of one sequential pass.  All threads.
 template <int B, bool TAB>
-__device__ __forceinline__ void predict_windows(Sys &S, Smem &sm, const PairTab *T, Atom &A, Cand &C, double calib, int *err) {
+__device__ __forceinline__ void predict_windows(SV &S, Smem &sm, const PairTab *T, Atom &A, Cand &C, double calib, int *err) {
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int ntot = A.ncand;
     const int wsz = min(S.win, PWIN);
@@ -781,7 +784,7 @@ __device__ __forceinline__ void predict_windows(Sys &S, Smem &sm, const PairTab 
 // What a bulk prediction's resolution needs to know of an atom besides its
 // record: the earliest time any other entry offered (one wave).  -1 where the
 // record also depends on H-bond slots.
-__device__ __forceinline__ double other_offers(const Sys &S, const Atom &A, const Cand &C) {
+__device__ __forceinline__ double other_offers(SV &S, const Atom &A, const Cand &C) {
     const int lane = threadIdx.x & 63;
     double m = __builtin_inf();
     if (lane < min(A.nb, MAXBOND) && !(A.evtype == SDMD_BOND && C.bj[lane] == A.partner)) m = C.bt[lane];
@@ -815,12 +818,12 @@ enum { M_LOOP, M_BULK, M_AGAIN };
 // candidate's evaluation, not by throughput: 205 candidates occupy four
 // wavefronts.
 template <int B, bool TAB, int MODE = M_LOOP>
-__device__ __forceinline__ void predict_atoms(Sys &S, Smem &sm, const PairTab *T, int n, int i0, int i1) {
+__device__ __forceinline__ void predict_atoms(Sys &M, SV &S, unsigned long long *prof, Smem &sm, const PairTab *T, int n, int i0, int i1) {
     constexpr int W = B / 64;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int nw = (W > 1 && n == 2) ? W / 2 : W;      // waves per team
     const int team = wave / nw, r = wave % nw;
-    unsigned long long pt = S.prof ? wall_clock64() : 0;
+    unsigned long long pt = prof ? wall_clock64() : 0;
     double calib = S.cutoffr * SDMD_EXTEND_RATIO;
     calib *= calib;
     int err = 0;
@@ -828,12 +831,12 @@ __device__ __forceinline__ void predict_atoms(Sys &S, Smem &sm, const PairTab *T
         if ((s == team || (nw == W && team == 0)) && r == 0) {
             Atom &A = sm.A[s];
             const int i = s ? i1 : i0;
-            stage_atom(S, A, i, MODE == M_BULK ? -1 : n == 2 ? (s ? i0 : i1) : 0, MODE == M_AGAIN ? i : INT_MAX);
+            stage_atom(M, A, i, MODE == M_BULK ? -1 : n == 2 ? (s ? i0 : i1) : 0, MODE == M_AGAIN ? i : INT_MAX);
             const long long zp = sm.zpos + (MODE == M_LOOP ? s : i - 1);
             if (lane == 0 && S.thermostat) A.zn = zp < S.nz ? G(S.zn)[zp] : 1.0;
         }
     __syncthreads();
-    PROF_MARK(S, PH_STAGE, pt);
+    FPROF(prof, PH_STAGE, pt);
     for (int s = 0; s < n; s++)
         if (s == team || (nw == W && team == 0)) {
             Atom &A = sm.A[s];
@@ -845,7 +848,7 @@ __device__ __forceinline__ void predict_atoms(Sys &S, Smem &sm, const PairTab *T
         }
     if (err) atomicCAS(&sm.err, 0, err);
     __syncthreads();
-    PROF_MARK(S, PH_GATHER, pt);
+    FPROF(prof, PH_GATHER, pt);
     const int wsz = min(S.win, PWIN);
     bool whole = true;
     for (int s = 0; s < n; s++) whole = whole && !sm.A[s].over && sm.A[s].ncand <= wsz;
@@ -864,7 +867,7 @@ __device__ __forceinline__ void predict_atoms(Sys &S, Smem &sm, const PairTab *T
             }
         if (err) atomicCAS(&sm.err, 0, err);
         __syncthreads();
-        PROF_MARK(S, PH_EVAL, pt);
+        FPROF(prof, PH_EVAL, pt);
         err = 0;
         for (int s = 0; s < n; s++)
             if ((s == team || (nw == W && team == 0)) && r == 0) {
@@ -876,7 +879,7 @@ __device__ __forceinline__ void predict_atoms(Sys &S, Smem &sm, const PairTab *T
                 }
             }
         __syncthreads();
-        PROF_MARK(S, PH_SELECT, pt);
+        FPROF(prof, PH_SELECT, pt);
         if (MODE == M_LOOP && n == 2) {
             const Atom &P = sm.A[0];
             Atom &A = sm.A[1];
@@ -932,16 +935,16 @@ __device__ __forceinline__ void predict_atoms(Sys &S, Smem &sm, const PairTab *T
         // statistics: candidates scanned, quadratic evaluations
         for (int s = 0; s < n; s++) {
             const Atom &A = sm.A[s];
-            S.candidates += A.ncand > 0 ? A.ncand - 1 : 0;
-            S.pair_evals += A.cnt_eval + min(A.nb, MAXBOND) + A.nbstat + (A.hbbond > 0 ? 1 : 0);
+            M.candidates += A.ncand > 0 ? A.ncand - 1 : 0;
+            M.pair_evals += A.cnt_eval + min(A.nb, MAXBOND) + A.nbstat + (A.hbbond > 0 ? 1 : 0);
         }
     __syncthreads();
-    PROF_MARK(S, PH_TAIL, pt);
+    FPROF(prof, PH_TAIL, pt);
 }
 
 // Predict(renewList) with ResetTarget, SGThread.c:158-211
 template <int B, bool TAB>
-__device__ void predict_list(Sys &S, Smem &sm, const PairTab *T, const int *renew) {
+__device__ void predict_list(Sys &M, SV &S, unsigned long long *prof, Smem &sm, const PairTab *T, const int *renew) {
     if (threadIdx.x == 0) {
         for (int n = 1; renew[n]; n++) {
             const int i = renew[n];
@@ -953,7 +956,7 @@ __device__ void predict_list(Sys &S, Smem &sm, const PairTab *T, const int *rene
     __syncthreads();
     const bool two = renew[1] && renew[2] && renew[1] != renew[2];
     for (int n = 1; renew[n]; n += two ? 2 : 1)
-        predict_atoms<B, TAB>(S, sm, T, two ? 2 : 1, renew[n], two ? renew[2] : 0);
+        predict_atoms<B, TAB>(M, S, prof, sm, T, two ? 2 : 1, renew[n], two ? renew[2] : 0);
 }
 
 // ---------------------------------------------------------------- CBT, CBT.c
@@ -983,7 +986,7 @@ struct PathMin {
 // instead of level by level; the walk itself runs on registers.  Where the
 // second path meets nodes the first has just written, it takes their new
 // values.
-__device__ __forceinline__ void cbt_update(Sys &S, Smem &sm, int n, int a0, int l0, double t0, int a1, int l1, double t1) {
+__device__ __forceinline__ void cbt_update(SV &S, Smem &sm, int n, int a0, int l0, double t0, int a1, int l1, double t1) {
     const int lane = threadIdx.x & 63, half = lane >> 5, k = lane & 31;
     const int L = half ? l1 : l0;
     const bool on = half < n && k < 31 - __clz(L);
@@ -1162,7 +1165,7 @@ __device__ void do_event(Sys &S, Smem &sm, int t, int p, int *err) {   // DoEven
 // is loaded side by side, and a collision, bond or H-bond-neighbour event
 // (InteractionEvent without its H-bond branch, Events.c:770-1025) runs on
 // registers.
-__device__ __forceinline__ void pop_event(Sys &S, Smem &sm) {
+__device__ __forceinline__ void pop_event(Sys &M, SV &S, Smem &sm) {
     const int lane = threadIdx.x & 63;
     const int target = sm.root, n0 = sm.nlog;
     const int p0 = G(S.evp)[target], ty = G(S.evtype)[target], sub = G(S.evsub)[target];
@@ -1181,9 +1184,9 @@ __device__ __forceinline__ void pop_event(Sys &S, Smem &sm) {
     }
     const double dt = lane_get(t, 0);
     if (S.trace) {
-        if (S.trace_n < S.trace_cap) {
+        if (M.trace_n < S.trace_cap) {
             if (lane == 0) {
-                sdmd_gpu_pop_rec &r = S.trace[S.trace_n];
+                sdmd_gpu_pop_rec &r = S.trace[M.trace_n];
                 r.target = target; r.partner = p0; r.type = ty; r.sub = sub; r.dt = dt; r.pot = pot0;
             }
         } else {
@@ -1207,14 +1210,14 @@ __device__ __forceinline__ void pop_event(Sys &S, Smem &sm) {
         sm.target = target;
         sm.partner = partner;
         sm.stale = stale;
-        S.currenttime += dt;
+        M.currenttime += dt;
         sm.renew[0] = (partner && !stale) ? 2 : 1;
         sm.renew[1] = target;
         sm.renew[2] = (partner && !stale) ? partner : 0;
         sm.renew[3] = 0;
-        if (stale) S.recal++;
-        else S.frame++;
-        sm.flush = n0 + 1 >= S.logk || (S.hash_every > 0 && (S.pops + 1) % S.hash_every == 0);
+        if (stale) M.recal++;
+        else M.frame++;
+        sm.flush = n0 + 1 >= S.logk || (S.hash_every > 0 && (M.pops + 1) % S.hash_every == 0);
     }
     if (!stale && pair) {
         // InteractionEvent, Events.c:798-1024, from the two lanes' state
@@ -1264,9 +1267,9 @@ __device__ __forceinline__ void pop_event(Sys &S, Smem &sm) {
                 if (mine) { G(S.vx)[a] = vx; G(S.vy)[a] = vy; G(S.vz)[a] = vz; }
             }
         }
-        if (lane == 0) S.per_type[ty]++;
+        if (lane == 0) M.per_type[ty]++;
     } else if (!stale && lane == 0) {
-        do_event(S, sm, target, partner, &err);
+        do_event(M, sm, target, partner, &err);
     }
     if (err && lane == 0) sm.err = err;
     // SGThread.c:100-104, then ResetTarget of the renewed atoms
@@ -1366,18 +1369,18 @@ __global__ __launch_bounds__(B) void k_bulk_predict(Sys *systems, int per) {
     __shared__ Sys Sl;
     __shared__ PairTab tab;
     Sys &Sg = systems[blockIdx.x];
+    SV &V = fixed_view(systems + blockIdx.x);
     sys_load<B>(Sl, &Sg);
     Sys &S = Sl;
     tab_load<B>(tab, S);
     if (threadIdx.x == 0) {
         sm.err = 0; sm.zpos = S.zpos; sm.nlog = 0;
         S.candidates = S.pair_evals = 0;               // this workgroup's counts
-        S.prof = nullptr;
     }
     __syncthreads();
     const int last = min(first + per - 1, S.N);
     for (int i = first; i <= last; i += 2)
-        predict_atoms<B, true, M_BULK>(S, sm, &tab, i < last ? 2 : 1, i, i + 1);
+        predict_atoms<B, true, M_BULK>(S, V, nullptr, sm, &tab, i < last ? 2 : 1, i, i + 1);
     if (threadIdx.x == 0) {
         atomicAdd((unsigned long long *)&Sg.candidates, (unsigned long long)S.candidates);
         atomicAdd((unsigned long long *)&Sg.pair_evals, (unsigned long long)S.pair_evals);
@@ -1433,6 +1436,7 @@ __global__ __launch_bounds__(B) void k_bulk_finish(Sys *systems) {
     __shared__ int next;
     sys_load<B>(Sl, &systems[blockIdx.x]);
     Sys &S = Sl;
+    SV &V = fixed_view(systems + blockIdx.x);
     const int tid = threadIdx.x, N = S.N;
     if (tid == 0) { sm.err = S.error; sm.zpos = S.zpos; sm.nlog = 0; next = INT_MAX; }
     __syncthreads();
@@ -1456,7 +1460,7 @@ __global__ __launch_bounds__(B) void k_bulk_finish(Sys *systems) {
             G(S.evp)[i] = INVALID;
         }
         __syncthreads();
-        predict_atoms<B, true, M_AGAIN>(S, sm, &tab, 1, i, 0);
+        predict_atoms<B, true, M_AGAIN>(S, V, nullptr, sm, &tab, 1, i, 0);
         if (tid == 0) {
             const int p1 = G(S.evp)[i];
             if (p1 != p0 || G(S.evtype)[i] != ty0 || G(S.evt)[i] != t0) {
@@ -1490,7 +1494,9 @@ __global__ __launch_bounds__(B) void k_run(Sys *systems, long long npops, long l
     __shared__ PairTab tab;
     __shared__ int stop;
     sys_load<B>(Sl, &systems[blockIdx.x]);
-    Sys &S = Sl;
+    Sys &S = Sl;                           // counters and clock
+    SV &V = fixed_view(systems + blockIdx.x);
+    unsigned long long *const prof = V.prof;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const unsigned long long t_start = wall_clock64();
     // npops < 0 asks for -npops executed events instead of pops
@@ -1500,7 +1506,7 @@ __global__ __launch_bounds__(B) void k_run(Sys *systems, long long npops, long l
     tab_load<B>(tab, S);
     if (tid == 0) { sm.err = 0; sm.zpos = S.zpos; stop = 0; sm.nlog = 0; sm.root = G(S.node)[1]; }
     __syncthreads();
-    unsigned long long pt = S.prof ? wall_clock64() : 0;
+    unsigned long long pt = prof ? wall_clock64() : 0;
     for (long long pop = 0;; pop++) {
         if (wave == 0) {
             // device-time budget of a bounded run
@@ -1508,25 +1514,25 @@ __global__ __launch_bounds__(B) void k_run(Sys *systems, long long npops, long l
                 S.frame - frame0 >= evgoal || stop) {
                 if (lane == 0) stop = 1;
             } else {
-                pop_event(S, sm);
+                pop_event(S, V, sm);
             }
         }
         __syncthreads();
         if (sm.err || stop) break;
         const int flush = sm.flush;        // wave 0 runs ahead into the next pop's event
-        PROF_MARK(S, PH_EVENT, pt);
-        predict_atoms<B, true>(S, sm, &tab, sm.renew[0], sm.renew[1], sm.renew[2]);
-        if (S.prof) pt = wall_clock64();
-        if (flush) sweep<B>(S, sm);
-        PROF_MARK(S, PH_SWEEP, pt);
+        FPROF(prof, PH_EVENT, pt);
+        predict_atoms<B, true>(S, V, prof, sm, &tab, sm.renew[0], sm.renew[1], sm.renew[2]);
+        if (prof) pt = wall_clock64();
+        if (flush) sweep<B>(V, sm);
+        FPROF(prof, PH_SWEEP, pt);
         if (wave == 0) {
-            cbt_update(S, sm, sm.renew[0], sm.renew[1], sm.A[0].leaf, sm.A[0].t, sm.renew[2], sm.A[1].leaf, sm.A[1].t);
-            PROF_MARK(S, PH_TREE, pt);
+            cbt_update(V, sm, sm.renew[0], sm.renew[1], sm.A[0].leaf, sm.A[0].t, sm.renew[2], sm.A[1].leaf, sm.A[1].t);
+            FPROF(prof, PH_TREE, pt);
             if (lane == 0) {
                 S.pops++;
                 S.last_exec = !sm.stale;
                 if (!sm.stale && S.currenttime >= t_out) stop = 1;
-                if (S.trace && S.trace_n < S.trace_cap) {
+                if (V.trace && S.trace_n < V.trace_cap) {
                     sdmd_gpu_pop_rec &r = S.trace[S.trace_n];
                     r.exec = !sm.stale;
                     r.rand_calls = sm.zpos;
@@ -1540,7 +1546,7 @@ __global__ __launch_bounds__(B) void k_run(Sys *systems, long long npops, long l
                     r.nrenew = n;
                     S.trace_n++;
                 }
-                if (S.hash_every > 0 && S.pops % S.hash_every == 0 && S.hash_n < S.hash_cap) {
+                if (V.hash_every > 0 && S.pops % V.hash_every == 0 && S.hash_n < S.hash_cap) {
                     G(S.hashes)[2 * S.hash_n] = S.pops;
                     G(S.hashes)[2 * S.hash_n + 1] = (long long)state_hash(S);
                     S.hash_n++;
@@ -1550,7 +1556,7 @@ __global__ __launch_bounds__(B) void k_run(Sys *systems, long long npops, long l
         }
     }
     __syncthreads();
-    if (sm.nlog) sweep<B>(S, sm);
+    if (sm.nlog) sweep<B>(V, sm);
     if (tid == 0) {
         S.zpos = sm.zpos;
         if (sm.err) S.error = sm.err;
@@ -1621,17 +1627,18 @@ __global__ __launch_bounds__(B) void k_op(Sys *systems, int sys, int op, Renew r
     __shared__ Sys Sl;
     sys_load<B>(Sl, &systems[sys]);
     Sys &S = Sl;
+    SV &V = fixed_view(systems + sys);
     const int tid = threadIdx.x;
     if (tid == 0) { sm.err = 0; sm.zpos = S.zpos; sm.nlog = 0; }
     __syncthreads();
     if (op == OP_CREATE_TREE) cbt_create<B>(S);
     if (op == OP_PREDICT) {
-        predict_list<B, false>(S, sm, nullptr, renew.a);
+        predict_list<B, false>(S, V, V.prof, sm, nullptr, renew.a);
     } else if (op == OP_UPDATE_TREE) {
         const int n = renew.a[0];
         if (tid < 64 && n > 0) {
             const int a0 = renew.a[1], a1 = n > 1 ? renew.a[2] : a0;
-            cbt_update(S, sm, n, a0, G(S.leaf)[a0], G(S.evt)[a0], a1, G(S.leaf)[a1], G(S.evt)[a1]);
+            cbt_update(V, sm, n, a0, G(S.leaf)[a0], G(S.evt)[a0], a1, G(S.leaf)[a1], G(S.evt)[a1]);
         }
     } else if (tid == 0) {
         int err = 0;
