@@ -2367,10 +2367,12 @@ __global__ __launch_bounds__(64 * W) void k_fast_run(FSys *systems, FJobs *jobs,
                 double w = sh.window;
                 if (found > FSEL) {
                     __syncthreads();
-                    w = (reach - tmin) * ((double)FSEL_AIM / found);
+                    const double fit = (double)FSEL_AIM / found, span = reach - tmin;
+                    // the counts scatter: the window shrinks no faster than it grows
+                    w = w < 1e300 ? span * fmax(fit, 0.8) : span * fit;
                     if (tid == 0) sh.nsel = 0;
                     __syncthreads();
-                    collect(fmax(theta, tmin + w), true);
+                    collect(fmax(theta, tmin + span * fit), true);
                     __syncthreads();
                     found = sh.nsel;
                 } else if (reach < theta3) {                  // the window was the bound
@@ -2444,6 +2446,7 @@ __global__ __launch_bounds__(64 * W) void k_fast_run(FSys *systems, FJobs *jobs,
             const float bx = (float)S.box[1], by = (float)S.box[2], bz = (float)S.box[3];
             const float cmin = (float)fmin(S.cellsize[1], fmin(S.cellsize[2], S.cellsize[3]));
             const float R2 = 4.f * cmin * cmin;
+            const float ix = 1.f / bx, iy = 1.f / by, iz = 1.f / bz;
             unsigned long long mine = 0;
             for (int q = small ? lane : tid; q < npair; q += small ? 64 : 64 * W) {
                 int i = (int)((1.f + sqrtf(1.f + 8.f * (float)q)) * 0.5f);
@@ -2462,9 +2465,9 @@ __global__ __launch_bounds__(64 * W) void k_fast_run(FSys *systems, FJobs *jobs,
                 };
                 auto apart = [&](const float *u, const float *v) {      // minimum image
                     float dx = u[0] - v[0], dy = u[1] - v[1], dz = u[2] - v[2];
-                    dx -= bx * rintf(dx / bx);
-                    dy -= by * rintf(dy / by);
-                    dz -= bz * rintf(dz / bz);
+                    dx -= bx * rintf(dx * ix);
+                    dy -= by * rintf(dy * iy);
+                    dz -= bz * rintf(dz * iz);
                     return dx * dx + dy * dy + dz * dz >= R2;
                 };
                 const int ka = sh.pre_ca[k], kp = sh.pre_cp[k], la = sh.pre_ca[l], lp = sh.pre_cp[l];

@@ -1,6 +1,9 @@
 """The fast engine's list of candidates inside the scan radius: shorter than
 a wavefront, several wavefronts long, and longer than the list holds (the
 unlisted path), on every workgroup shape that has its own list length."""
+import copy
+
+import numpy as np
 import pytest
 
 pytestmark = pytest.mark.gpu
@@ -40,3 +43,21 @@ def test_screens_agree_with_fp64(require_gpu, dense, cutoff, block, helpers):
     assert st["error"] == 0 and fs["causal"] == 0
     assert fs["validated"] > 1500 and fs["agree"] == fs["validated"], fs
     eng.close()
+
+
+# one cut-off wider than 2 048 candidates (two windows of first-candidate
+# marks) in cells of up to a few hundred atoms: 5 014 atoms in 27 cells
+def test_many_candidates_match_oracle(require_gpu, tmp_path):
+    from conftest import fast_bulk_vs_oracle
+    from sdmd_amd import builder
+    from sdmd_amd.engine import System
+
+    chains = builder.build_chains(builder.random_sequences(2, 30, 4), 4, workers=1)
+    unit = [copy.deepcopy(chains[k % 2]) for k in range(16)]
+    edge = 165.0
+    placed = builder.place_chains(unit, (edge,) * 3, np.random.default_rng([4, 0]))
+    d = tmp_path / "wide"
+    builder.write_input_dir(builder.System(placed, (edge,) * 3, "peptides"), str(d), cutoff=54.0, thermostat="no")
+    s = System.load(str(d))
+    assert s.natom > 4000 and min(s.arrays.scalars["cellnum"][:]) == 3
+    fast_bulk_vs_oracle(s)
