@@ -301,11 +301,7 @@ struct FWave {
     static constexpr int LIST = NL;
     int nbp[SDMD_NBSLOTS];       // the predicted atom's neighborPartner
     union {
-        // its bonded partners' states (lanes 32..47 stage bond q = lane - 32)
-        struct {
-            double bxj[16], byj[16], bzj[16], bvx[16], bvy[16], bvz[16], bt0[16], blo[16], bhi[16];
-        };
-        // after the bond phase: the candidates inside the scan radius, in
+        // the candidates inside the scan radius, in
         // candidate order; first their kinematics, then the screen's result
         struct {
             float l_rr[NL], l_b[NL], l_v2[NL];
@@ -317,8 +313,6 @@ struct FWave {
     };
     int l_id[NL];                // atom id << 8 | type, as in the mirror record
     int l_k[NL];                 // candidate index; bit 31: its local time is later than the reader's
-    long long bcj[16];
-    int bjj[16];
     // the neighbour cells that hold candidates, in scan order: candidate k of
     // cell c has its record at slot cbase[c] + k; coff[c] is the cell's first
     // candidate (the number of candidates past the last cell)
@@ -605,6 +599,18 @@ __device__ __forceinline__ long long rl64(long long v, int L) {
 }
 __device__ __forceinline__ int rl32(int v, int L) { return __builtin_amdgcn_readlane(v, L); }
 
+// c_OX, c_OY, c_OZ with two bits per cell (offset + 1)
+constexpr int OFFSETS[3][27] = {
+    {0, 1, 0, 0, 0, 1, 1, 1, -1, 0, 0, 0, -1, -1, -1, 0, 0, 1, -1, 1, -1, -1, -1, 1, 1, 1, -1},
+    {0, 0, 1, 0, 1, 0, 1, 1, 0, -1, 0, -1, 0, -1, -1, -1, 1, 0, 0, -1, 1, -1, 1, -1, 1, -1, 1},
+    {0, 0, 0, 1, 1, 1, 0, 1, 0, 0, -1, -1, -1, 0, -1, 1, -1, -1, 1, 0, 0, 1, -1, -1, -1, 1, 1}};
+constexpr unsigned long long pack_offsets(int axis) {
+    unsigned long long w = 0;
+    for (int c = 0; c < 27; c++) w |= (unsigned long long)(OFFSETS[axis][c] + 1) << (2 * c);
+    return w;
+}
+constexpr unsigned long long OFF_X = pack_offsets(0), OFF_Y = pack_offsets(1), OFF_Z = pack_offsets(2);
+
 // Two memory round trips: (1) every field of atom i, one per lane, through
 // the gather map, with its bonded partners' ids; (2) its connection row,
 // bond limits and partners' states, constraint entries with their FP32 step
@@ -612,7 +618,7 @@ __device__ __forceinline__ int rl32(int v, int L) { return __builtin_amdgcn_read
 // all lanes (indices clamped into range, results masked afterwards), so a
 // level costs one memory latency.
 template <class FW>
-__device__ __forceinline__ void fstage(FV &F, const ScrTab &T, FW &wm, FAtom &A, int i, double t, int &nb, Own &own) {
+__device__ __forceinline__ void fstage(FV &F, const ScrTab &T, FW &wm, FAtom &A, int i, double t, int &nb, Own &own, BondPre &bp) {
     SV &S = F.s;
     const int lane = threadIdx.x & 63;
     i = uni(i);
@@ -683,9 +689,11 @@ __device__ __forceinline__ void fstage(FV &F, const ScrTab &T, FW &wm, FAtom &A,
     }
     const bool own_con = lane < ncon && lane < FCON;
     int cell;
+    int ox, oy, oz;                                        // this lane's neighbour cell (lanes 27.. repeat cell 0)
     {
-        const int cl = lane < 27 ? lane : 0;
-        int n1 = cx + c_OX[cl], n2 = cy + c_OY[cl], n3 = cz + c_OZ[cl];
+        const int sh2 = lane < 27 ? 2 * lane : 0;
+        ox = (int)((OFF_X >> sh2) & 3) - 1; oy = (int)((OFF_Y >> sh2) & 3) - 1; oz = (int)((OFF_Z >> sh2) & 3) - 1;
+        int n1 = cx + ox, n2 = cy + oy, n3 = cz + oz;
         if (n1 < 0) n1 = S.cellnum[1] - 1; else if (n1 >= S.cellnum[1]) n1 = 0;
         if (n2 < 0) n2 = S.cellnum[2] - 1; else if (n2 >= S.cellnum[2]) n2 = 0;
         if (n3 < 0) n3 = S.cellnum[3] - 1; else if (n3 >= S.cellnum[3]) n3 = 0;
@@ -701,7 +709,6 @@ __device__ __forceinline__ void fstage(FV &F, const ScrTab &T, FW &wm, FAtom &A,
     bool reach;
     {
         const float lx = own.x, ly = own.y, lz = own.z;
-        const int cl = lane < 27 ? lane : 0, ox = c_OX[cl], oy = c_OY[cl], oz = c_OZ[cl];
         const float m = 0.02f;
         const float dx = ox == 0 ? 0.f : fmaxf((ox < 0 ? lx : F.L32[0] - lx) - m, 0.f);
         const float dy = oy == 0 ? 0.f : fmaxf((oy < 0 ? ly : F.L32[1] - ly) - m, 0.f);
@@ -732,13 +739,9 @@ __device__ __forceinline__ void fstage(FV &F, const ScrTab &T, FW &wm, FAtom &A,
         const double vxj = G(S.vx)[j], vyj = G(S.vy)[j], vzj = G(S.vz)[j];
         const double t0j = G(F.t0)[j];
         const long long cjj = G(S.evc)[j];
-        if (q >= 0 && q < 16) {            // into the wave's LDS slot: short register lifetimes
-            wm.bxj[q] = xj; wm.byj[q] = yj; wm.bzj[q] = zj;
-            wm.bvx[q] = vxj; wm.bvy[q] = vyj; wm.bvz[q] = vzj;
-            wm.bt0[q] = t0j; wm.bcj[q] = cjj;
-            wm.bjj[q] = bq ? j : 0;
-            wm.blo[q] = blo; wm.bhi[q] = bhi;
-        }
+        bp.j = bq ? j : 0;
+        bp.xj = xj; bp.yj = yj; bp.zj = zj; bp.vxj = vxj; bp.vyj = vyj; bp.vzj = vzj;
+        bp.t0j = t0j; bp.cj = cjj; bp.lo = blo; bp.hi = bhi;
     }
     // ---- connection row as bytes over its span (row and span small enough;
     // otherwise it is searched in memory), with the slots of the staged
@@ -778,9 +781,9 @@ __device__ __forceinline__ void fstage(FV &F, const ScrTab &T, FW &wm, FAtom &A,
         const int nc = __popc(km), at = __popc(km & below);
         if (lane < 27 && keep) {
             fvec4 co4;
-            co4.x = c_OX[lane] * F.L32[0];
-            co4.y = c_OY[lane] * F.L32[1];
-            co4.z = c_OZ[lane] * F.L32[2];
+            co4.x = ox * F.L32[0];
+            co4.y = oy * F.L32[1];
+            co4.z = oz * F.L32[2];
             co4.w = 0.f;
             wm.cof[at] = co4;
             wm.cbase[at] = (long long)cell * F.cap - start;
@@ -1226,7 +1229,8 @@ __device__ __forceinline__ void predict_fast(FSys &M, FV &F0, unsigned long long
     FAtom A;
     Own own;
     int nb = 0;
-    fstage(view_anew(F0), T, wm, A, i, t, nb, own);
+    BondPre bp;                                            // lanes 32 .. 47: one bonded partner each
+    fstage(view_anew(F0), T, wm, A, i, t, nb, own, bp);
     FV &F = view_anew(F0);
     SV &S = F.s;
     // the first candidates' records load during the bond times
@@ -1246,15 +1250,6 @@ __device__ __forceinline__ void predict_fast(FSys &M, FV &F0, unsigned long long
         Best mine = init;
         mine.t = __builtin_inf();
         const int q = lane - 32;
-        BondPre bp;
-        bp.j = 0;
-        if (q >= 0 && q < 16) {
-            bp.j = wm.bjj[q];
-            bp.xj = wm.bxj[q]; bp.yj = wm.byj[q]; bp.zj = wm.bzj[q];
-            bp.vxj = wm.bvx[q]; bp.vyj = wm.bvy[q]; bp.vzj = wm.bvz[q];
-            bp.t0j = wm.bt0[q]; bp.cj = wm.bcj[q];
-            bp.lo = wm.blo[q]; bp.hi = wm.bhi[q];
-        }
         if (bp.j > 0) {
             int sub;
             mine.t = bond64_pre(F, A, bp, sub);
