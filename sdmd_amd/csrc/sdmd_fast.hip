@@ -80,7 +80,8 @@ constexpr int PROW = 16;          // steps per collision pair at most
 struct __attribute__((aligned(16))) ConRad {
     float rad[8];
     unsigned int ez;
-    int pad[3];
+    float dmin, dmax;
+    int nstep;
 };
 
 struct FSys {
@@ -98,6 +99,8 @@ struct FSys {
     int *bj16;
     double *blo16, *bhi16;
     struct ConRad *crad;
+    int *conn;                  // per atom FCONN bytes: its connection row (see FWave)
+    int *rowlo;                 // the row's first column (-1: it does not fit its bytes)
     // FP64 shells at a fixed stride, read at a known shell without a
     // dependent load: dmin, dmax, the radii, the energies
     double *prow;               // [NT*NT][2 + 2 * PROW] by resolved collision pair
@@ -293,6 +296,7 @@ __device__ __forceinline__ void take(Best &B, SYS &S, double t, double pot, int 
 constexpr int FCON = 16;          // constraint partners staged per predicted atom
 constexpr int FCONSTEP = 8;       // steps per staged constraint
 constexpr int FMARK = 32;         // words of first-candidate marks
+constexpr int FCONN = 128;        // atom ids a row's bytes span
 
 // Per-wavefront LDS.  NL: candidates inside the scan radius listed for the
 // screen (25 to 60 at most sizes; a longer list takes the unlisted path).
@@ -323,14 +327,11 @@ struct FWave {
     // candidates), so that a lane counts bits instead of searching coff
     unsigned long long mark[FMARK];
     // the predicted atom's constraint shells (FP32), CONSTRn lists
-    int con_nstep[FCON];
-    unsigned int con_ez[FCON];
-    float con_dmin[FCON], con_dmax[FCON];
-    float con_rad[FCON][FCONSTEP];
+    ConRad con[FCON];
     int hbl_n;                   // entries of l_id / l_k left by the screen, -1: none listed
     // connection row by offset from its first column: bits 0-1 BOND and
     // CONSTRAINT, bits 2-6 the constraint's slot + 1 (0: not staged)
-    unsigned char conn[128];
+    unsigned char conn[FCONN];
     WStats st;                   // the wavefront's statistics (wave-uniform updates)
 };
 // the list's length by workgroup size (the LDS of a CU holds it all)
@@ -582,6 +583,8 @@ __device__ __forceinline__ void wave_best(Best &mine, int k, const Best &running
 // the bond entry of this lane (lanes < bond count).  No memory fence: the
 // LDS data is shared within the wave only, whose LDS operations execute in
 // order, so independent global loads stay in flight across the stages.
+__device__ __forceinline__ fvec4 cv_load(const fvec4 *p) { return *(gptr_t<const fvec4>)p; }
+
 // the predicted atom's mirror record (position, velocity, time since the epoch)
 struct Own { float x, y, z, vx, vy, vz, t; };
 
@@ -632,7 +635,6 @@ __device__ __forceinline__ void fstage(FV &F, const ScrTab &T, FW &wm, FAtom &A,
     const int role = G(S.role)[i];
     const long long w = (long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo);
     const int cx = rl32(lo, 8), cy = rl32(lo, 9), cz = rl32(lo, 10);
-    const int o = rl32(lo, 24), nrow = rl32(lo, 25) - o;
     nb = rl32(lo, 27) - rl32(lo, 26);
     const int co = rl32(lo, 28), ncon = rl32(lo, 29) - co;
     if (lane >= 18 && lane < 18 + SDMD_NBSLOTS) wm.nbp[lane - 18] = lo;
@@ -653,11 +655,7 @@ __device__ __forceinline__ void fstage(FV &F, const ScrTab &T, FW &wm, FAtom &A,
         own.vx = lane_get(f, 3); own.vy = lane_get(f, 4); own.vz = lane_get(f, 5);
     }
     // ---- level 2
-    int rj = 0, rb = 0, rc = 0;
-    if (nrow > 0) {
-        const int k0 = o + min(lane, nrow - 1);
-        rj = G(S.cmap_j)[k0]; rb = G(S.cmap_bits)[k0]; rc = G(S.cmap_con)[k0];
-    }
+    const int row = G(F.conn)[i * (FCONN / 4) + (lane & (FCONN / 4 - 1))];
     // bond q on lane 32 + q: its partner id came with level 1 (lane 48 + q)
     const int q = lane - 32;
     const bool bq = q >= 0 && q < nb && q < 16;
@@ -670,22 +668,10 @@ __device__ __forceinline__ void fstage(FV &F, const ScrTab &T, FW &wm, FAtom &A,
         blo = G(F.blo16)[qq];
         bhi = G(F.bhi16)[qq];
     }
-    double cdmin = 0, cdmax = 0;
-    int cnstep = 0;
-    float rad[FCONSTEP];
-    unsigned int ez = 0;
-#pragma unroll
-    for (int k = 0; k < FCONSTEP; k++) rad[k] = 0.f;
+    fvec4 c0 = {0, 0, 0, 0}, c1 = c0, c2 = c0;
     if (ncon > 0) {
-        const int cc = co + min(lane, ncon - 1);
-        cdmin = G(S.con)[cc].dmin;
-        cdmax = G(S.con)[cc].dmax;
-        cnstep = G(S.con)[cc].nstep;
-        const fvec4 *cv = (const fvec4 *)(F.crad + cc);
-        const fvec4 r03 = G(cv)[0], r47 = G(cv)[1];
-        rad[0] = r03.x; rad[1] = r03.y; rad[2] = r03.z; rad[3] = r03.w;
-        rad[4] = r47.x; rad[5] = r47.y; rad[6] = r47.z; rad[7] = r47.w;
-        ez = G((const unsigned int *)(F.crad + cc))[8];
+        const fvec4 *cv = (const fvec4 *)(F.crad + (co + min(lane, ncon - 1)));
+        c0 = cv_load(cv); c1 = cv_load(cv + 1); c2 = cv_load(cv + 2);
     }
     const bool own_con = lane < ncon && lane < FCON;
     int cell;
@@ -743,32 +729,14 @@ __device__ __forceinline__ void fstage(FV &F, const ScrTab &T, FW &wm, FAtom &A,
         bp.xj = xj; bp.yj = yj; bp.zj = zj; bp.vxj = vxj; bp.vyj = vyj; bp.vzj = vzj;
         bp.t0j = t0j; bp.cj = cjj; bp.lo = blo; bp.hi = bhi;
     }
-    // ---- connection row as bytes over its span (row and span small enough;
-    // otherwise it is searched in memory), with the slots of the staged
-    // constraint shells (one lane each)
-    {
-        if (lane < 32) ((int *)wm.conn)[lane] = 0;
-        const int rowlo = nrow > 0 ? rl32(rj, 0) : 0, rowhi = nrow > 0 ? rl32(rj, min(nrow, 64) - 1) : 0;
-        const bool spanok = nrow <= 64 && rowhi - rowlo < 128;
-        const unsigned long long fits = __ballot(own_con && cnstep <= FCONSTEP);
-        wave_sync();
-        if (lane < nrow && spanok) {
-            const int slot = rc - co;                       // rc < 0: no constraint
-            const bool staged = rc >= 0 && slot >= 0 && slot < FCON && ((fits >> slot) & 1);
-            wm.conn[rj - rowlo] = (unsigned char)((rb & (SDMD_BOND_CONNECT | SDMD_CONSTRAINT_CONNECT)) |
-                                                  (staged ? (slot + 1) << 2 : 0));
-        }
-        A.rowlo = rowlo;
-        A.spanok = spanok;
-        if (own_con) {
-            wm.con_dmin[lane] = (float)cdmin;
-            wm.con_dmax[lane] = (float)cdmax;
-            wm.con_nstep[lane] = cnstep;
-            wm.con_ez[lane] = ez;
-#pragma unroll
-            for (int k = 0; k < FCONSTEP; k++) wm.con_rad[lane][k] = rad[k];
-        }
+    // ---- connection row and constraint shells (one lane each)
+    if (lane < FCONN / 4) ((int *)wm.conn)[lane] = row;
+    if (own_con) {
+        fvec4 *cl = (fvec4 *)&wm.con[lane];
+        cl[0] = c0; cl[1] = c1; cl[2] = c2;
     }
+    A.rowlo = rl32(lo, 31);
+    A.spanok = A.rowlo >= 0;
     // the cells in reach that hold atoms, packed in scan order, and the marks
     // of their first candidates; one prefix sum for the candidates in reach
     // (high half) and for those of all 27 cells (low half)
@@ -919,8 +887,9 @@ __device__ __forceinline__ void screen_near(FV &F, const ScrTab &T, const FW &wm
         const int q = (cb >> 2) - 1;
         o.slot = q;
         if (q < 0) { o.flag = true; return; }             // not staged: FP64 decides
-        c.dmin = wm.con_dmin[q]; c.dmax = wm.con_dmax[q]; c.nstep = wm.con_nstep[q]; c.ezero = wm.con_ez[q];
-        rad = wm.con_rad[q];
+        const ConRad &cr = wm.con[q];
+        c.dmin = cr.dmin; c.dmax = cr.dmax; c.nstep = cr.nstep; c.ezero = cr.ez;
+        rad = cr.rad;
     } else {
         const ScrPair sp = T.pr[A.type * NT + tj];
         o.rp = sp.rp;
@@ -944,7 +913,7 @@ __device__ __forceinline__ double coli64_shell(FV &F, const ScrTab &T, const FW 
     const int j = id >> 8;
     const bool con = slot >= 0;
     const ScrPair sp = T.pr[A.type * NT + (id & 255)];
-    const int nstep = con ? wm.con_nstep[slot & (FCON - 1)] : (int)sp.nstep, stride = con ? FCONSTEP : PROW;
+    const int nstep = con ? wm.con[slot & (FCON - 1)].nstep : (int)sp.nstep, stride = con ? FCONSTEP : PROW;
     const double *row = con ? F.crow + (size_t)(A.co + slot) * (2 + 2 * FCONSTEP)
                             : F.prow + (size_t)max((int)sp.rp, 0) * (2 + 2 * PROW);
     const int kl = max(ks - 1, 0), kh = min(ks, stride - 1);
@@ -1976,11 +1945,11 @@ __global__ __launch_bounds__(256) void k_fast_cells(FSys *systems) {
     }
 }
 
-// bond lists at a fixed stride of 16 (BondTime's connect[16]) and the
-// constraints' tables: FP32 radii and energy bits inline (up to 8 steps are
+// bond lists at a fixed stride of 16 (BondTime's connect[16]), connection
+// rows as bytes and the constraints' tables: FP32 radii and energy bits inline (up to 8 steps are
 // staged) and FP64 shells at a fixed stride (a constraint of more steps than
 // a row holds is not staged, and then not read from here).  Derived on the
-// device: 17 MB for 26 080 atoms, which took longer to write on the host and
+// device: 20 MB for 26 080 atoms, which took longer to write on the host and
 // to copy than all the rest of opening a system.
 __global__ __launch_bounds__(256) void k_fast_derive(FSys *systems) {
     FV &F = fixed_view(systems + blockIdx.x);
@@ -1992,6 +1961,24 @@ __global__ __launch_bounds__(256) void k_fast_derive(FSys *systems) {
         G(F.bj16)[k] = in ? G(S.bond_j)[e] : 0;
         G(F.blo16)[k] = in ? G(S.bond_dmin)[e] : 0.0;
         G(F.bhi16)[k] = in ? G(S.bond_dmax)[e] : 0.0;
+    }
+    // an atom's connection row as bytes over its span (row and span small
+    // enough; otherwise it is searched in memory): bits 0-1 BOND and
+    // CONSTRAINT, bits 2-6 the slot + 1 of a constraint that is staged
+    for (int a = tid; a <= N; a += all) {
+        const int o = a > 0 ? G(S.cmap_off)[a] : 0, n = a > 0 ? G(S.cmap_off)[a + 1] - o : 0;
+        const int lo = n > 0 ? G(S.cmap_j)[o] : 0, hi = n > 0 ? G(S.cmap_j)[o + min(n, 64) - 1] : 0;
+        const bool fits = n <= 64 && hi - lo < FCONN;
+        for (int k = 0; k < FCONN / 4; k++) G(F.conn)[a * (FCONN / 4) + k] = 0;
+        G(F.rowlo)[a] = fits ? lo : -1;
+        unsigned char *bytes = (unsigned char *)(F.conn + a * (FCONN / 4));
+        const int co = a > 0 ? G(S.con_off)[a] : 0;
+        for (int k = o; fits && k < o + n; k++) {
+            const int rc = G(S.cmap_con)[k], slot = rc - co;              // rc < 0: no constraint
+            const bool staged = rc >= 0 && slot >= 0 && slot < FCON && G(S.con)[max(rc, 0)].nstep <= FCONSTEP;
+            G(bytes)[G(S.cmap_j)[k] - lo] = (unsigned char)((G(S.cmap_bits)[k] & (SDMD_BOND_CONNECT | SDMD_CONSTRAINT_CONNECT)) |
+                                                            (staged ? (slot + 1) << 2 : 0));
+        }
     }
     const int nc = G(S.con_off)[N + 1];
     for (int k = tid; k < nc; k += all) {
@@ -2008,6 +1995,9 @@ __global__ __launch_bounds__(256) void k_fast_derive(FSys *systems) {
             if (q < nstep && eq == 0) ez |= 1u << q;
         }
         G(F.crad)[k].ez = ez;
+        G(F.crad)[k].dmin = (float)G(S.con)[k].dmin;
+        G(F.crad)[k].dmax = (float)G(S.con)[k].dmax;
+        G(F.crad)[k].nstep = G(S.con)[k].nstep;
     }
 }
 
@@ -2797,15 +2787,17 @@ int sdmd_fast_open(sdmd_gpu_ctx *c, const sdmd_gpu_opts *o) {
             // bond lists and constraint tables at fixed strides, written by
             // k_fast_derive from the lists already on the device
             const size_t nc = (size_t)(d->con_off[N + 1] > 0 ? d->con_off[N + 1] : 1), n16 = ((size_t)N + 1) * 16;
-            const size_t bytes[5] = {n16 * sizeof(int), n16 * sizeof(double), n16 * sizeof(double), nc * sizeof(ConRad),
-                                     nc * (2 + 2 * FCONSTEP) * sizeof(double)};
-            void **dst[5] = {(void **)&F.bj16, (void **)&F.blo16, (void **)&F.bhi16, (void **)&F.crad, (void **)&F.crow};
-            size_t at[5], all = 0;
-            for (int k = 0; k < 5; k++) { at[k] = all; all += (bytes[k] + 255) & ~(size_t)255; }
+            const size_t bytes[7] = {n16 * sizeof(int), n16 * sizeof(double), n16 * sizeof(double), nc * sizeof(ConRad),
+                                     nc * (2 + 2 * FCONSTEP) * sizeof(double), ((size_t)N + 1) * FCONN,
+                                     ((size_t)N + 1) * sizeof(int)};
+            void **dst[7] = {(void **)&F.bj16, (void **)&F.blo16, (void **)&F.bhi16, (void **)&F.crad,
+                             (void **)&F.crow, (void **)&F.conn, (void **)&F.rowlo};
+            size_t at[7], all = 0;
+            for (int k = 0; k < 7; k++) { at[k] = all; all += (bytes[k] + 255) & ~(size_t)255; }
             char *block = nullptr;
             if (hipMalloc((void **)&block, all) != hipSuccess) return SDMD_EDEVICE;
             if ((rc = dev_keep(c, block))) return rc;
-            for (int k = 0; k < 5; k++) *dst[k] = block + at[k];
+            for (int k = 0; k < 7; k++) *dst[k] = block + at[k];
             const int PR = 2 + 2 * PROW;
             // the collision table's rows are one copy for systems of equal tables
             const sdmd_system_desc *d0 = c->desc[0];
@@ -2903,7 +2895,7 @@ int sdmd_fast_open(sdmd_gpu_ctx *c, const sdmd_gpu_opts *o) {
             setg(24, Sh.cmap_off, 1, 0, 0); setg(25, Sh.cmap_off, 1, 1, 0);
             setg(26, Sh.bond_off, 1, 0, 0); setg(27, Sh.bond_off, 1, 1, 0);
             setg(28, Sh.con_off, 1, 0, 0); setg(29, Sh.con_off, 1, 1, 0);
-            setg(30, Sh.hbitype, 1, 0, 0);
+            setg(30, Sh.hbitype, 1, 0, 0); setg(31, F.rowlo, 1, 0, 0);
         }
         if (rc == SDMD_OK) {
             ScrTab *dt = nullptr;
