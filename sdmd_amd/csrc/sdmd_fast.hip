@@ -956,9 +956,9 @@ struct HBPre { int role, aanum, protein, hbbond; };
 // the marked ones and those whose interval reaches the smallest upper bound
 // are re-solved in FP64; the FP64 minimum (first in scan order on ties)
 // competes with the running best under JobAssign's strict '<'.
-// A lone wavefront issues one instruction in about five cycles, so what
-// counts is how often the long screen runs: once per 64 listed candidates
-// instead of once per 64 scanned.
+// A lone wavefront issues a dependent instruction every 8 cycles and an
+// independent one every 5 (measured), so what counts is how often the long
+// screen runs: once per 64 listed candidates instead of once per 64 scanned.
 // VAL: validation mode (every live candidate also solved in FP64 and the
 // full scan's winner compared), a separate instantiation so that the
 // screened path carries none of its state
@@ -2025,7 +2025,7 @@ __global__ __launch_bounds__(256) void k_fast_records(FSys *systems) {
 // Bulk Predict(1..N): a prediction reads positions, velocities and counters
 // but no other atom's event record, so the atoms are spread over gridDim.y
 // workgroups per system (one wavefront per atom at a time).  Bound by the
-// instruction latency of a prediction (about 16 us on one wavefront); with
+// instruction count of a prediction (about 9 us on one wavefront); with
 // one workgroup per system a 26 080-atom system took 58 ms on one CU.
 template <int W>
 __global__ __launch_bounds__(64 * W) void k_fast_predict(FSys *systems) {
@@ -2088,8 +2088,9 @@ __global__ __launch_bounds__(256) void k_fast_blocks(FSys *systems) {
 // positions are x + v (T - t0); one wavefront per atom i, two lanes per
 // neighbour cell, for partners j > i.  A chain of dependent loads per pair
 // bounds it, so the atoms are spread over the GPU: gridDim.y workgroups per
-// system, each leaving its sums in `part` (k_energy_reduce adds them).  One workgroup per system with one thread per atom took 4.0 ms for
-// 64 systems of 1 536 atoms.
+// system, each leaving its sums in `part` (k_energy_reduce adds them).  One
+// workgroup per system with one thread per atom took 4.0 ms for 64 systems of
+// 1 536 atoms.
 __global__ __launch_bounds__(64 * EWAVES) void k_fast_energy(FSys *systems, double *part) {
     const FSys &F = systems[blockIdx.x];
     const Sys &S = F.s;
