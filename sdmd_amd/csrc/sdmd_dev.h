@@ -110,6 +110,9 @@ struct Sys {
     sdmd_pair *rpair;
     double *bulk_t2;            // bulk prediction: see k_bulk_resolve
     int *bulk_head, *bulk_next, *bulk_flag;
+    double *bulk_pot;           // what a bulk prediction of the atom began with and overwrites
+    long long *bulk_pc;
+    int *bulk_sub, *bulk_nbnum, *bulk_hbit;
     int ltab, logk;             // step pool entries held in LDS (0: none); pops between sweeps
     const int *gbase[48];       // gather table of a staged atom
     int gstride[48];

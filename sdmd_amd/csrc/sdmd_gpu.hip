@@ -806,7 +806,9 @@ __device__ __forceinline__ double other_offers(SV &S, const Atom &A, const Cand 
 // MODE of a prediction: one of the event loop or a single call; the first
 // pass of a bulk prediction (no CheckDuplication, the draw by atom number,
 // other_offers left in S.bulk_t2); a repeated one of a bulk prediction
-// (CheckDuplication against the atoms before it, the same draw, no counting)
+// (CheckDuplication against the atoms before it, the same draw, no counting),
+// which begins with what the first pass began with: the skipped H-bond event's
+// flag above all, which a prediction takes back
 enum { M_LOOP, M_BULK, M_AGAIN };
 
 // Predict of up to two atoms whose records were already reset (ResetTarget),
@@ -841,6 +843,14 @@ __device__ __forceinline__ void predict_atoms(Sys &M, SV &S, unsigned long long 
         if (s == team || (nw == W && team == 0)) {
             Atom &A = sm.A[s];
             if (r == 0 && lane == 0) {
+                if (MODE == M_BULK) {
+                    G(S.bulk_pot)[A.i] = A.pot; G(S.bulk_pc)[A.i] = A.pc; G(S.bulk_sub)[A.i] = A.sub;
+                    G(S.bulk_nbnum)[A.i] = A.nbnum; G(S.bulk_hbit)[A.i] = A.hbitype;
+                }
+                if (MODE == M_AGAIN) {
+                    A.pot = G(S.bulk_pot)[A.i]; A.pc = G(S.bulk_pc)[A.i]; A.sub = G(S.bulk_sub)[A.i];
+                    A.nbnum = G(S.bulk_nbnum)[A.i]; A.hbitype = G(S.bulk_hbit)[A.i];
+                }
                 A.hbscan = wants_hbscan(A);
                 A.pot0 = A.pot; A.pc0 = A.pc; A.sub0 = A.sub; A.nbnum0 = A.nbnum;
             }
@@ -1803,6 +1813,9 @@ static int upload_system(sdmd_gpu_ctx *c, sdmd_arena *ar, int s, const sdmd_syst
         UP(bulk_t2, (const double *)nullptr, N1);
         UP(bulk_head, (const int *)nullptr, N1); UP(bulk_next, (const int *)nullptr, N1);
         UP(bulk_flag, (const int *)nullptr, N1);
+        UP(bulk_pot, (const double *)nullptr, N1); UP(bulk_pc, (const long long *)nullptr, N1);
+        UP(bulk_sub, (const int *)nullptr, N1); UP(bulk_nbnum, (const int *)nullptr, N1);
+        UP(bulk_hbit, (const int *)nullptr, N1);
         sdmd_pair rp[NT * NT];
         auto back = [](int t) { return t == 3 ? 1 : t == 4 ? 2 : t == 27 ? 26 : t; };
         int pool = 0, most = 0;
