@@ -1281,10 +1281,12 @@ __device__ __forceinline__ void pop_event(Sys &M, SV &S, Smem &sm) {
     } else if (!stale && lane == 0) {
         do_event(M, sm, target, partner, &err);
     }
-    if (err && lane == 0) sm.err = err;
-    // SGThread.c:100-104, then ResetTarget of the renewed atoms
+    if (err && lane == 0 && !sm.err) sm.err = err;
+    // SGThread.c:100-104, then ResetTarget of the renewed atoms; a failed
+    // event is the last of the run and leaves the records as they are
     if (mine && !stale) G(S.evc)[a] = counter + 1;
-    if (lane == 0 || (lane == 1 && partner && !stale)) {
+    wave_sync();
+    if (sm.err == 0 && (lane == 0 || (lane == 1 && partner && !stale))) {
         G(S.evtype)[a] = SDMD_INVD;
         G(S.evt)[a] = INFINIT;
         G(S.evp)[a] = INVALID;
@@ -1519,8 +1521,8 @@ __global__ __launch_bounds__(B) void k_run(Sys *systems, long long npops, long l
     unsigned long long pt = prof ? wall_clock64() : 0;
     for (long long pop = 0;; pop++) {
         if (wave == 0) {
-            // device-time budget of a bounded run
-            if (pop >= maxpops || (long long)(wall_clock64() - t_start) > budget || S.currenttime > t_end ||
+            // an error of the last pop, the device-time budget of a bounded run
+            if (sm.err || pop >= maxpops || (long long)(wall_clock64() - t_start) > budget || S.currenttime > t_end ||
                 S.frame - frame0 >= evgoal || stop) {
                 if (lane == 0) stop = 1;
             } else {
