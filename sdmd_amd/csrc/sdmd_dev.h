@@ -113,6 +113,7 @@ struct Sys {
     double *bulk_pot;           // what a bulk prediction of the atom began with and overwrites
     long long *bulk_pc;
     int *bulk_sub, *bulk_nbnum, *bulk_hbit;
+    int bulk_err;               // first error of a bulk prediction
     int ltab, logk;             // step pool entries held in LDS (0: none); pops between sweeps
     const int *gbase[48];       // gather table of a staged atom
     int gstride[48];

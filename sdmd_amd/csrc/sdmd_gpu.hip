@@ -1364,6 +1364,7 @@ __device__ __forceinline__ void tab_load(PairTab &T, const Sys &S) {
 // atoms (9 us each).
 __global__ __launch_bounds__(256) void k_bulk_reset(Sys *systems) {
     const Sys &S = systems[blockIdx.x];
+    if (blockIdx.y == 0 && threadIdx.x == 0) systems[blockIdx.x].bulk_err = 0;
     for (int i = 1 + blockIdx.y * 256 + threadIdx.x; i <= S.N; i += 256 * gridDim.y) {   // ResetTarget for 1..N
         G(S.evtype)[i] = SDMD_INVD;
         G(S.evt)[i] = INFINIT;
@@ -1396,7 +1397,7 @@ __global__ __launch_bounds__(B) void k_bulk_predict(Sys *systems, int per) {
     if (threadIdx.x == 0) {
         atomicAdd((unsigned long long *)&Sg.candidates, (unsigned long long)S.candidates);
         atomicAdd((unsigned long long *)&Sg.pair_evals, (unsigned long long)S.pair_evals);
-        if (sm.err) atomicCAS(&Sg.error, 0, sm.err);
+        if (sm.err) atomicCAS(&Sg.bulk_err, 0, sm.err);
     }
 }
 
@@ -1450,7 +1451,7 @@ __global__ __launch_bounds__(B) void k_bulk_finish(Sys *systems) {
     Sys &S = Sl;
     SV &V = fixed_view(systems + blockIdx.x);
     const int tid = threadIdx.x, N = S.N;
-    if (tid == 0) { sm.err = S.error; sm.zpos = S.zpos; sm.nlog = 0; next = INT_MAX; }
+    if (tid == 0) { sm.err = S.bulk_err; sm.zpos = S.zpos; sm.nlog = 0; next = INT_MAX; }
     __syncthreads();
     bool loaded = false;
     int from = 1;

@@ -80,6 +80,27 @@ def test_normals_used_up_in_an_event(require_gpu, have):
     assert np.array_equal(got["ev_time"][1:], ref["ev_time"][1:] - tr["dt"][pop])
 
 
+# a context in error still predicts: the records and the tree of its state,
+# while the call reports the error
+def test_prepare_of_a_context_in_error(require_gpu):
+    import oracle_lib
+
+    eng = run(59 + 300, 0)
+    o = oracle_lib.Oracle(eng.state(0))
+    assert o.bulk() == 0
+    ref = o.state().arr
+    eng.feed_normals(1000)
+    with pytest.raises(SdmdError):
+        eng.prepare()
+    got = eng.state(0).arr
+    for f in RECORD:
+        assert np.array_equal(got[f][1:], ref[f][1:]), f
+    node, leaf = eng.tree(0)
+    eng.close()
+    want, wleaf = o.tree()
+    assert np.array_equal(node[1:], want[1:]) and np.array_equal(leaf[1:], wleaf[1:])
+
+
 # a record that no event can be made of: the clock moves on, the records stay
 @pytest.mark.parametrize("ty", [0, 1])
 def test_bad_record(require_gpu, ty):
