@@ -718,9 +718,22 @@ __device__ __forceinline__ int wants_hbscan(const Atom &A) {
     return A.hbitype != SDMD_HBSKIP && A.hbbond <= 0 && (A.role == 'A' || A.role == 'D' || A.role == 'S');
 }
 
+// The lists of cells that hold more atoms than their arrays, walked side by
+// side, one lane per cell (the reference's, Events.c:158-200), into `ids`:
+// atom | neighbour cell << 27.  Once per prediction: a walk is a chain of
+// dependent loads (30 us for a cell of 185 atoms), and a window holds the
+// lists of a few cells only.
+__device__ __forceinline__ void walk_lists(SV &S, const Atom &A, const Cand &C, unsigned *ids) {
+    if (threadIdx.x < 27) {
+        const int c = threadIdx.x, end = C.celloff[c + 1];
+        int j = G(S.celllist)[S.N + cell_index(S, A.cx, A.cy, A.cz, c)];
+        for (int g = C.celloff[c]; j && g < end; g++, j = G(S.celllist)[j]) ids[g] = (unsigned)j | (unsigned)c << 27;
+    }
+}
+
 // candidates [w0, w0 + n) of the staged atom's ordered list (all threads)
 template <int B>
-__device__ __forceinline__ void gather_window(SV &S, const Atom &A, Cand &C, int w0, int n) {
+__device__ __forceinline__ void gather_window(SV &S, const Atom &A, Cand &C, const unsigned *ids, int w0, int n) {
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     if (!A.over) {
         for (int c = wave; c < 27; c += B / 64) {
@@ -730,9 +743,14 @@ __device__ __forceinline__ void gather_window(SV &S, const Atom &A, Cand &C, int
                 C.cell[g] = (unsigned char)c;
             }
         }
+    } else if (ids) {
+        for (int k = threadIdx.x; k < n; k += B) {
+            const unsigned v = ids[w0 + k];
+            C.j[k] = (int)(v & 0x7ffffffu);
+            C.cell[k] = (unsigned char)(v >> 27);
+        }
     } else if (wave == 0 && lane < 27) {
-        // a cell holds more atoms than its array: walk the lists (the
-        // reference's, Events.c:158-200)
+        // more candidates than the other atom's arrays hold: the lists again
         int g = C.celloff[lane] - w0;
         if (g < n && C.celloff[lane + 1] > w0) {
             int j = G(S.celllist)[S.N + cell_index(S, A.cx, A.cy, A.cz, lane)];
@@ -748,9 +766,18 @@ __device__ __forceinline__ void gather_window(SV &S, const Atom &A, Cand &C, int
 // that of one sequential pass.  All threads.
 template <int B, bool TAB>
 __device__ __forceinline__ void predict_windows(SV &S, Smem &sm, const PairTab *T, Atom &A, Cand &C, double calib, int *err) {
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int tid = threadIdx.x, wave = tid >> 6;
     const int ntot = A.ncand;
     const int wsz = min(S.win, PWIN);
+    // the other atom's candidate arrays hold nothing while windows are used
+    Cand &other = &C == &sm.c[0] ? sm.c[1] : sm.c[0];
+    static_assert(offsetof(Cand, hpot) == offsetof(Cand, t) + 3 * sizeof(double) * PWIN, "one block of times and energies");
+    constexpr int IDS = 4 * PWIN * (int)(sizeof(double) / sizeof(unsigned));
+    unsigned *ids = (A.over && ntot <= IDS && S.N < (1 << 27)) ? (unsigned *)other.t : nullptr;
+    if (ids) {
+        walk_lists(S, A, C, ids);
+        __syncthreads();
+    }
     if (wave == 0) select_bonds(S, sm, A, C);
     for (int pass = 0; pass < 2; pass++) {
         if (pass == 1) {
@@ -760,7 +787,7 @@ __device__ __forceinline__ void predict_windows(SV &S, Smem &sm, const PairTab *
         }
         for (int w0 = 0; w0 < ntot; w0 += wsz) {
             const int n = min(ntot - w0, wsz);
-            gather_window<B>(S, A, C, w0, n);
+            gather_window<B>(S, A, C, ids, w0, n);
             int ev = 0;
             for (int k = tid; k < n; k += B) {
                 eval_candidate<TAB>(S, sm, T, A, C, k, calib, err);
@@ -777,7 +804,6 @@ __device__ __forceinline__ void predict_windows(SV &S, Smem &sm, const PairTab *
     }
     __syncthreads();
     if (tid == 0) assign_tail(S, sm, A, err);
-    (void)lane;
     __syncthreads();
 }
 
