@@ -1548,8 +1548,8 @@ __global__ __launch_bounds__(B) void k_run(Sys *systems, long long npops, long l
     unsigned long long pt = prof ? wall_clock64() : 0;
     for (long long pop = 0;; pop++) {
         if (wave == 0) {
-            // an error of the last pop, the device-time budget of a bounded run
-            if (sm.err || pop >= maxpops || (long long)(wall_clock64() - t_start) > budget || S.currenttime > t_end ||
+            // device-time budget of a bounded run
+            if (pop >= maxpops || (long long)(wall_clock64() - t_start) > budget || S.currenttime > t_end ||
                 S.frame - frame0 >= evgoal || stop) {
                 if (lane == 0) stop = 1;
             } else {
@@ -1570,7 +1570,8 @@ __global__ __launch_bounds__(B) void k_run(Sys *systems, long long npops, long l
             if (lane == 0) {
                 S.pops++;
                 S.last_exec = !sm.stale;
-                if (!sm.stale && S.currenttime >= t_out) stop = 1;
+                // an error of a prediction ends the run here, before the next pop
+                if (sm.err || (!sm.stale && S.currenttime >= t_out)) stop = 1;
                 if (V.trace && S.trace_n < V.trace_cap) {
                     sdmd_gpu_pop_rec &r = S.trace[S.trace_n];
                     r.exec = !sm.stale;
