@@ -699,16 +699,20 @@ __device__ __forceinline__ void assign_tail(SV &S, const Smem &sm, Atom &A, int 
     G(S.hbitype)[i] = SDMD_NOEVENT;
 }
 
-__device__ __forceinline__ void finish_atom(SV &S, const Smem &sm, Atom &A, Cand &C, int *err) {
+__device__ __forceinline__ void finish_atom(SV &S, unsigned long long *prof, unsigned long long &pt, const Smem &sm, Atom &A,
+                                            Cand &C, int *err) {
     const int lane = threadIdx.x & 63, n = A.ncand;
     select_bonds(S, sm, A, C);
     wave_sync();
+    FPROF(prof, PH_BONDSEL, pt);
     select_collisions(S, sm, A, C, n);
     wave_sync();
     if (lane == 0) assign_onebody(S, sm, A, C, err);
     wave_sync();
+    FPROF(prof, PH_SELECT, pt);
     if (A.hbscan) select_hbonds(S, sm, A, C, n);
     wave_sync();
+    FPROF(prof, PH_HB, pt);
     if (lane == 0) assign_tail(S, sm, A, err);
 }
 
@@ -765,7 +769,8 @@ __device__ __forceinline__ void gather_window(SV &S, const Atom &A, Cand &C, con
 // minimum (and CheckDuplication against it) carries over, so the result is
 // that of one sequential pass.  All threads.
 template <int B, bool TAB>
-__device__ __forceinline__ void predict_windows(SV &S, Smem &sm, const PairTab *T, Atom &A, Cand &C, double calib, int *err) {
+__device__ __forceinline__ void predict_windows(SV &S, unsigned long long *prof, unsigned long long &pt, Smem &sm,
+                                                const PairTab *T, Atom &A, Cand &C, double calib, int *err) {
     const int tid = threadIdx.x, wave = tid >> 6;
     const int ntot = A.ncand;
     const int wsz = min(S.win, PWIN);
@@ -778,11 +783,15 @@ __device__ __forceinline__ void predict_windows(SV &S, Smem &sm, const PairTab *
         walk_lists(S, A, C, ids);
         __syncthreads();
     }
+    FPROF(prof, PH_GATHER, pt);
     if (wave == 0) select_bonds(S, sm, A, C);
+    FPROF(prof, PH_BONDSEL, pt);
     for (int pass = 0; pass < 2; pass++) {
         if (pass == 1) {
+            FPROF(prof, PH_EVAL, pt);
             if (tid == 0) assign_onebody(S, sm, A, C, err);
             __syncthreads();
+            FPROF(prof, PH_SELECT, pt);
             if (!A.hbscan) break;
         }
         for (int w0 = 0; w0 < ntot; w0 += wsz) {
@@ -803,6 +812,7 @@ __device__ __forceinline__ void predict_windows(SV &S, Smem &sm, const PairTab *
         }
     }
     __syncthreads();
+    FPROF(prof, PH_HB, pt);
     if (tid == 0) assign_tail(S, sm, A, err);
     __syncthreads();
 }
@@ -907,7 +917,7 @@ __device__ __forceinline__ void predict_atoms(Sys &M, SV &S, unsigned long long 
         err = 0;
         for (int s = 0; s < n; s++)
             if ((s == team || (nw == W && team == 0)) && r == 0) {
-                finish_atom(S, sm, sm.A[s], sm.c[s], &err);
+                finish_atom(S, prof, pt, sm, sm.A[s], sm.c[s], &err);
                 if (MODE == M_BULK) {
                     wave_sync();
                     const double t2 = other_offers(S, sm.A[s], sm.c[s]);
@@ -915,7 +925,6 @@ __device__ __forceinline__ void predict_atoms(Sys &M, SV &S, unsigned long long 
                 }
             }
         __syncthreads();
-        FPROF(prof, PH_SELECT, pt);
         if (MODE == M_LOOP && n == 2) {
             const Atom &P = sm.A[0];
             Atom &A = sm.A[1];
@@ -940,7 +949,7 @@ __device__ __forceinline__ void predict_atoms(Sys &M, SV &S, unsigned long long 
                         A.exclude = 0;
                     }
                     wave_sync();
-                    finish_atom(S, sm, A, C, &err);
+                    finish_atom(S, prof, pt, sm, A, C, &err);
                 }
                 __syncthreads();
             }
@@ -957,7 +966,7 @@ __device__ __forceinline__ void predict_atoms(Sys &M, SV &S, unsigned long long 
                 if (threadIdx.x < min(A.nb, MAXBOND)) eval_bond(S, sm, A, C, threadIdx.x);
                 __syncthreads();
             }
-            predict_windows<B, TAB>(S, sm, T, A, C, calib, &err);
+            predict_windows<B, TAB>(S, prof, pt, sm, T, A, C, calib, &err);
             if (MODE == M_BULK && threadIdx.x == 0) G(S.bulk_t2)[A.i] = -1;
         }
     }
@@ -1201,7 +1210,7 @@ __device__ void do_event(Sys &S, Smem &sm, int t, int p, int *err) {   // DoEven
 // is loaded side by side, and a collision, bond or H-bond-neighbour event
 // (InteractionEvent without its H-bond branch, Events.c:770-1025) runs on
 // registers.
-__device__ __forceinline__ void pop_event(Sys &M, SV &S, Smem &sm) {
+__device__ __forceinline__ void pop_event(Sys &M, SV &S, unsigned long long *prof, unsigned long long &pt, Smem &sm) {
     const int lane = threadIdx.x & 63;
     const int target = sm.root, n0 = sm.nlog;
     const int p0 = G(S.evp)[target], ty = G(S.evtype)[target], sub = G(S.evsub)[target];
@@ -1230,6 +1239,7 @@ __device__ __forceinline__ void pop_event(Sys &M, SV &S, Smem &sm) {
             return;
         }
     }
+    FPROF(prof, PH_POP, pt);
     x = x + vx * dt; y = y + vy * dt; z = z + vz * dt; t = t - dt;
     const bool mine = lane == 0 || (lane == 1 && partner);
     if (mine) {
@@ -1306,13 +1316,14 @@ __device__ __forceinline__ void pop_event(Sys &M, SV &S, Smem &sm) {
         if (lane == 0) M.per_type[ty]++;
     } else if (!stale && lane == 0) {
         do_event(M, sm, target, partner, &err);
+        if (!err) err = sm.err;                    // a thermostat event's draws used up
     }
-    if (err && lane == 0 && !sm.err) sm.err = err;
+    const bool failed = __ballot(err != 0) != 0;
+    if (failed && lane == 0 && !sm.err) sm.err = err;
     // SGThread.c:100-104, then ResetTarget of the renewed atoms; a failed
     // event is the last of the run and leaves the records as they are
     if (mine && !stale) G(S.evc)[a] = counter + 1;
-    wave_sync();
-    if (sm.err == 0 && (lane == 0 || (lane == 1 && partner && !stale))) {
+    if (!failed && (lane == 0 || (lane == 1 && partner && !stale))) {
         G(S.evtype)[a] = SDMD_INVD;
         G(S.evt)[a] = INFINIT;
         G(S.evp)[a] = INVALID;
@@ -1553,7 +1564,7 @@ __global__ __launch_bounds__(B) void k_run(Sys *systems, long long npops, long l
                 S.frame - frame0 >= evgoal || stop) {
                 if (lane == 0) stop = 1;
             } else {
-                pop_event(S, V, sm);
+                pop_event(S, V, prof, pt, sm);
             }
         }
         __syncthreads();
