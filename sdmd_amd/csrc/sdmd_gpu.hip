@@ -2057,6 +2057,7 @@ static void launch_prepare(sdmd_gpu_ctx *c) {
     }
     int per = 2;
     while (per < 32 && atoms > 256LL * per) per += 2;
+    while ((maxn + per - 1) / per > 65535) per *= 2;   // a grid's y dimension ends at 65 536 (2.1 million atoms)
     const dim3 gp(c->nsys, (maxn + per - 1) / per), ga(c->nsys, maxn < 64 * 256 ? (maxn + 255) / 256 : 64);
     hipLaunchKernelGGL(k_bulk_reset, ga, dim3(256), 0, c->stream, c->dev_sys);
     hipLaunchKernelGGL((k_bulk_predict<256>), gp, dim3(256), 0, c->stream, c->dev_sys, per);
