@@ -66,9 +66,9 @@ typedef struct {
     int32_t block;         /* threads per system workgroup: plain 64..1024 (power of two),
                               fast 64, 256, 512 or 1024 (one re-prediction per wavefront
                               at a time; the autotuner may also pick 768); 0 = 256.  Fast: 512
-                              and more run as 256 where helper workgroups share the
-                              predictions (the faster shape; same results), unless the
-                              autotuner measured otherwise */
+                              and more run as 256 where the number of helpers is left to the
+                              engine too and helpers share the predictions (the faster shape;
+                              same results), unless the autotuner measured otherwise */
     int32_t trace;         /* plain: record every pop (parity checks) */
     int32_t profile;       /* plain, bit 0: accumulate per-phase device time */
     int64_t trace_capacity;
@@ -78,7 +78,8 @@ typedef struct {
     int32_t max_batch;     /* fast: at most this many events per round (0 = 64) */
     uint64_t seed;         /* fast: thermostat stream key (0 = the system's seed) */
     int32_t helpers;       /* fast: helper workgroups per system that take re-predictions on other
-                              CUs (0 = as many as the GPU holds beside the owners, -1 = none) */
+                              CUs (0 = as many as the GPU holds beside the owners, -1 = none;
+                              with a number, `block` is taken as it is) */
     int32_t window;        /* plain: neighbour candidates scanned per pass of a prediction (0 = 1728,
                               the staging area; 1..1728: more passes, the same result) */
 } sdmd_gpu_opts;

@@ -2687,6 +2687,7 @@ struct sdmd::FastState {
     FSys *dev;
     int waves;                 // wavefronts per workgroup (events in flight per round per pass)
     int tuned;                 // waves is the autotuner's choice
+    int autoshape;             // the number of helpers was left to the engine, and the shape with it
     int depth;                 // candidates per lane staged in registers (FQ)
     int validate;
     hipGraph_t graph;          // captured launch sequence (sdmd_gpu_run_graph)
@@ -2918,6 +2919,7 @@ int sdmd_fast_open(sdmd_gpu_ctx *c, const sdmd_gpu_opts *o) {
     const int want = o ? o->helpers : 0;
     if (want < -1) return SDMD_EINVAL;
     fs->helpers = want < 0 ? 0 : (want == 0 ? fs->hmax : (want < fs->hmax ? want : fs->hmax));
+    fs->autoshape = want == 0;
     return SDMD_OK;
 }
 
@@ -2942,11 +2944,14 @@ int sdmd_fast_sync(sdmd_gpu_ctx *c) { return fast_sync_from(c); }
 // re-predictions (10 to 40) find more wavefronts than they need, and one
 // wavefront per SIMD, with all registers of the SIMD, is the fastest a
 // prediction gets: us per round with 4 / 8 wavefronts per workgroup 20 / 28
-// (59 atoms), 35 / 40 (64 systems of 1 536), 47 / 52 (26 080).  Without
-// helpers the owner's wavefronts are all there are: 51 / 34 ms for 6 000
-// events of 26 080 atoms.  The autotuner's choice is taken as it is.
+// (59 atoms), 35 / 40 (64 systems of 1 536), 47 / 52 (26 080); ms for 2 000
+// events of each of 32, 64, 96 and 128 systems of 1 536 atoms (7, 3, 1 and 1
+// helpers) 10.4 / 14.8, 11.2 / 15.0, 14.3 / 16.2 and 14.4 / 16.4.  Without
+// helpers the owner's wavefronts are all there are: 45 / 35 ms for 6 000
+// events of 26 080 atoms.  A caller that asks for a number of helpers gets the
+// workgroups asked for with it; the autotuner's choice is taken as it is.
 static int run_waves(const FastState *fs) {
-    return (!fs->tuned && fs->helpers > 0 && fs->waves > 4) ? 4 : fs->waves;
+    return (!fs->tuned && fs->autoshape && fs->helpers > 0 && fs->waves > 4) ? 4 : fs->waves;
 }
 
 #define FDISPATCH(fn, ...) do { switch (run_waves(fs)) { \

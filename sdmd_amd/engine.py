@@ -111,7 +111,8 @@ class GpuEngine:
                   independent events (one per wavefront); `validate` re-solves
                   every collision candidate in FP64 and counts agreement;
                   `helpers` workgroups per system take re-predictions on
-                  other CUs (0: as many as fit, -1: none).
+                  other CUs (0: as many as fit, in workgroups of at most 256
+                  threads; -1: none; a number: that many, of `block` threads).
     `window` (plain): neighbour candidates per pass of a prediction's
     windowed scan (0: 1728); a smaller window takes more passes and gives
     the same result."""
