@@ -959,9 +959,8 @@ struct HBPre { int role, aanum, protein, hbbond; };
 // A lone wavefront issues a dependent instruction every 8 cycles and an
 // independent one every 5 (measured), so what counts is how often the long
 // screen runs: once per 64 listed candidates instead of once per 64 scanned.
-// VAL: validation mode (every live candidate also solved in FP64 and the
-// full scan's winner compared), a separate instantiation so that the
-// screened path carries none of its state
+// VAL: validation mode (the winner of a full FP64 scan compared), a separate
+// instantiation so that the screened path carries none of its state
 template <int FQ, bool VAL, class FW>
 __device__ __forceinline__ void collision_fast(FSys &M, FV &F, unsigned long long *prof, const ScrTab &T, FW &wm, const FAtom &A, const Own &own,
                                                Group<FQ> &g, int first, HBPre &hp, Best &best, long long &nscreen,
@@ -981,29 +980,21 @@ __device__ __forceinline__ void collision_fast(FSys &M, FV &F, unsigned long lon
     Best full = mine;
     int fullk = 0x7fffffff;
     float myt32 = FINF;
-    // FP64 re-solve of candidate k (and the validation scan)
-    auto confirm = [&](int k, int id, int bits, int rp, float t32, int ks, int slot, bool flag, bool need) {
+    // FP64 re-solve of candidate k
+    auto confirm = [&](int k, int id, int bits, int rp, float t32, int ks, int slot, bool flag) {
         double pot, t;
         int sub;
         bool late;
         long long pc = 0;
-        if (need) {
-            if (flag) {
-                bool reached;
-                t = coli64(F, A, id >> 8, bits, rp, calib64, pot, sub, reached, late, err);
-                pc = G(S.evc)[id >> 8];
-            } else {
-                t = coli64_shell(F, T, wm, A, id, ks, slot, pot, sub, pc, late);
-            }
-            my_causal += late ? 1 : 0;             // FP64 check of the screen's FP32 time order
-            if (t < mine.t) { mine.t = t; mine.pot = pot; mine.sub = sub; mine.partner = id >> 8; mine.pc = pc; mink = k; myt32 = t32; }
-        }
-        if constexpr (VAL) {
+        if (flag) {
             bool reached;
             t = coli64(F, A, id >> 8, bits, rp, calib64, pot, sub, reached, late, err);
-            if (!need) my_causal += late ? 1 : 0;
-            if (t < full.t) { full.t = t; full.pot = pot; full.sub = sub; full.partner = id >> 8; fullk = k; }
+            pc = G(S.evc)[id >> 8];
+        } else {
+            t = coli64_shell(F, T, wm, A, id, ks, slot, pot, sub, pc, late);
         }
+        my_causal += late ? 1 : 0;             // FP64 check of the screen's FP32 time order
+        if (t < mine.t) { mine.t = t; mine.pot = pot; mine.sub = sub; mine.partner = id >> 8; mine.pc = pc; mink = k; myt32 = t32; }
     };
     // ---- the candidates inside the scan radius, in candidate order
     int near = 0;
@@ -1051,7 +1042,7 @@ __device__ __forceinline__ void collision_fast(FSys &M, FV &F, unsigned long lon
             if (o.live && !o.flag && o.t < FINF) thi = fminf(thi, o.t + o.e);
             wm.l_t[r] = o.live ? o.t : FINF;
             wm.l_e[r] = (o.live && o.flag) ? -1.f : o.e;
-            wm.l_sh[r] = o.ks | ((o.slot + 1) << 8) | (o.live ? 1 << 16 : 0);
+            wm.l_sh[r] = o.ks | ((o.slot + 1) << 8);
             }
             screened += __popcll(__ballot(o.live));
         }
@@ -1064,12 +1055,12 @@ __device__ __forceinline__ void collision_fast(FSys &M, FV &F, unsigned long lon
             const int sh = wm.l_sh[rl];
             const bool flag = e < 0.f, need = r < near && (flag || (t < FINF && t - e <= thi));
             confirmed += __popcll(__ballot(need));
-            if (need || (VAL && r < near && (sh >> 16))) {
+            if (need) {
                 const int id = wm.l_id[r], slot = ((sh >> 8) & 255) - 1;
                 // what the FP64 search of a marked candidate needs
                 const int bits = coli_bits(wm, S, A, id >> 8) & (SDMD_BOND_CONNECT | SDMD_CONSTRAINT_CONNECT);
                 const int rp = (bits & SDMD_CONSTRAINT_CONNECT) ? -1 : T.pr[A.type * NT + (id & 255)].rp;
-                confirm(wm.l_k[r] & 0x7fffffff, id, bits, rp, t, sh & 255, slot, flag, need);
+                confirm(wm.l_k[r] & 0x7fffffff, id, bits, rp, t, sh & 255, slot, flag);
             }
         }
     } else {
@@ -1097,10 +1088,46 @@ __device__ __forceinline__ void collision_fast(FSys &M, FV &F, unsigned long lon
                 } else {
                     const bool need = o.live && (o.flag || (o.t < FINF && o.t - o.e <= thi));
                     confirmed += __popcll(__ballot(need));
-                    if (need || (VAL && o.live)) confirm(k, id, o.bits, o.rp, o.t, o.ks, o.slot, o.flag, need);
+                    if (need) confirm(k, id, o.bits, o.rp, o.t, o.ks, o.slot, o.flag);
                 }
             }
             if (pass == 0) thi = wave_min_f(thi);
+        }
+    }
+    if constexpr (VAL) {
+        // every atom of the 27 cells in scan order, from the cell arrays and
+        // the FP64 state alone: what the staging drops (a cell taken to be out
+        // of reach, a record found under another cell) shows as a disagreement
+        const int cl = min(lane, 26);
+        int n1 = A.cx + c_OX[cl], n2 = A.cy + c_OY[cl], n3 = A.cz + c_OZ[cl];
+        if (n1 < 0) n1 = S.cellnum[1] - 1; else if (n1 >= S.cellnum[1]) n1 = 0;
+        if (n2 < 0) n2 = S.cellnum[2] - 1; else if (n2 >= S.cellnum[2]) n2 = 0;
+        if (n3 < 0) n3 = S.cellnum[3] - 1; else if (n3 >= S.cellnum[3]) n3 = 0;
+        const int cell = cell_id(S, n1, n2, n3);
+        const int cnt = lane < 27 ? min(G(F.ccnt)[cell], F.cap) : 0, incl = scan32_incl(cnt);
+        const int all = lane_get(incl, 26);
+        for (int k0 = 0; k0 < all; k0 += 64) {
+            const int k = min(k0 + lane, all - 1);
+            int c = 0;                                     // cells that end at or before candidate k
+#pragma unroll
+            for (int step = 16; step > 0; step >>= 1)
+                if (__shfl(incl, c + step - 1, 64) <= k) c += step;
+            const int before = __shfl(incl - cnt, c, 64), id = __shfl(cell, c, 64);
+            const int j = G(F.cmem)[(size_t)id * F.cap + (k - before)];
+            if (k0 + lane < all && j >= 1 && j <= S.N && j != A.i) {
+                const int bits = coli_bits(wm, S, A, j) & (SDMD_BOND_CONNECT | SDMD_CONSTRAINT_CONNECT), tj = G(S.type)[j];
+                Kin kin;
+                bool late, reached;
+                kin_local(F, A, j, kin, &late);
+                if (!(bits & SDMD_BOND_CONNECT) && A.hbbond != j && !fin_nb_list(wm, A, j) && kin.rr <= calib64) {
+                    const int rp = (bits & SDMD_CONSTRAINT_CONNECT) ? -1 : T.pr[A.type * NT + tj].rp;
+                    double pot;
+                    int sub;
+                    my_causal += late ? 1 : 0;
+                    const double t = coli64(F, A, j, bits, rp, calib64, pot, sub, reached, late, err);
+                    if (t < full.t) { full.t = t; full.pot = pot; full.sub = sub; full.partner = j; fullk = k; }
+                }
+            }
         }
     }
     FPROF(prof, FPH_CONFIRM, pt);
