@@ -107,6 +107,7 @@ struct FSys {
     double *crow;               // [constraint entry][2 + 2 * FCONSTEP]
     int ncell, nblk;
     float L32[3];
+    float eb0, band0;           // the records' rounding in the screen's bands (see ScrBand)
     double Te, rebase_dt;
     double t_stop;              // events later than this stay pending (run_until)
     const void *scrtab;         // ScrTab (FP32 collision table), copied into LDS per launch
@@ -430,11 +431,22 @@ struct Shell {
 __device__ __forceinline__ float fsqrt(float x) { return __builtin_amdgcn_sqrtf(x); }
 __device__ __forceinline__ float frcp(float x) { return __builtin_amdgcn_rcpf(x); }
 
+// How far rounding can move a pair's distance vector: each component is a sum
+// of five values of a cell's size at most, each rounded once in FP32, so the
+// vector is off by D = sqrt(3) 5 2^-24 cells at most (6e-7 with some room).
+// b is then off by D |v|, and r^2 by 2 r D <= 2e-5 r^2 + D^2 / 2e-5.  In cells
+// of up to 6.6 and 23 A the bands hold that beside their floors.
+struct ScrBand { float eb0, band0; };
+static ScrBand screen_band(double cell) {
+    const double D = 6e-7 * cell;
+    return {(float)fmax(4e-6, D), (float)fmax(1e-5, D * D / 2e-5)};
+}
+
 template <class R>
-__device__ __forceinline__ Scr screen_shell(const Shell &c, const R &rad, bool con, float rr, float b, float v2) {
+__device__ __forceinline__ Scr screen_shell(const Shell &c, const R &rad, bool con, float rr, float b, float v2, ScrBand sb) {
     Scr o;
     o.t = FINF; o.e = 0; o.flag = false; o.ks = 0;
-    const float band = 2e-5f * rr + 1e-5f;
+    const float band = 2e-5f * rr + sb.band0;
     if (rr < c.dmin + band) { o.flag = true; return o; }   // core boundary or inside the core
     // count the radii passed (no early exit; four radii read at a time with
     // unconditional loads clamped to the last step, so a group costs one
@@ -464,7 +476,7 @@ __device__ __forceinline__ Scr screen_shell(const Shell &c, const R &rad, bool c
     const bool lopot0 = ks ? ((c.ezero >> (ks - 1)) & 1) : true;
     bool hipot0;
     int cs;
-    const float eb = 1e-5f * fsqrt(rr * v2) + 4e-6f * fsqrt(v2) + 1e-20f;
+    const float eb = 1e-5f * fsqrt(rr * v2) + sb.eb0 * fsqrt(v2) + 1e-20f;
     if (fabsf(b) <= eb) { o.flag = true; return o; }
     if (ks < c.nstep) {
         hipot0 = (c.ezero >> ks) & 1;
@@ -502,7 +514,7 @@ __device__ __forceinline__ Scr screen_shell(const Shell &c, const R &rad, bool c
             o.e = 4.f * (band + o.t * (eb + (v2 * band + 2.f * b * eb) * frcp(2.f * fsqrt(disc2)))) * frcp(D) + 1e-4f * o.t;
         } else {
             o.t = (-b + fsqrt(disc2)) * frcp(v2);
-            o.e = 1e-4f * o.t + 4.f * (eb + band) * frcp(fsqrt(v2 + 1e-30f));
+            o.e = 1e-4f * o.t + 4.f * (eb + band + sb.eb0) * frcp(fsqrt(v2 + 1e-30f));
         }
     }
     if (!(o.t > o.e)) o.flag = true;                         // sign of t uncertain
@@ -689,9 +701,10 @@ __device__ __forceinline__ void fstage(FV &F, const ScrTab &T, FW &wm, FAtom &A,
     if (lane >= 27) cnt = 0;
     if (lane < FMARK) wm.mark[lane] = 0;
     // a cell farther from the atom than the scan radius holds no candidate:
-    // an atom lies inside its cell until its cell-crossing event (FP32
-    // rounding and the crossing's 1e-8 A are far below the margin).  The scan
-    // radius is 0.9 cells or less, which leaves 17 cells of 27.
+    // an atom lies inside its cell until its cell-crossing event.  The margin
+    // of 0.02 A holds that event's 1e-8 A, the record's rounding (6e-8 cells,
+    // so cells of up to 100 000 A) and the rounding of the sum of squares.
+    // The scan radius is 0.9 cells or less, which leaves 17 cells of 27.
     bool reach;
     {
         const float lx = own.x, ly = own.y, lz = own.z;
@@ -700,7 +713,7 @@ __device__ __forceinline__ void fstage(FV &F, const ScrTab &T, FW &wm, FAtom &A,
         const float dy = oy == 0 ? 0.f : fmaxf((oy < 0 ? ly : F.L32[1] - ly) - m, 0.f);
         const float dz = oz == 0 ? 0.f : fmaxf((oz < 0 ? lz : F.L32[2] - lz) - m, 0.f);
         const float c2 = (float)((S.cutoffr * SDMD_EXTEND_RATIO) * (S.cutoffr * SDMD_EXTEND_RATIO));
-        reach = dx * dx + dy * dy + dz * dz <= c2 + (2e-5f * c2 + 1e-5f);
+        reach = dx * dx + dy * dy + dz * dz <= c2 + (2e-5f * c2 + F.band0);
     }
     // PBCandCrossCellTime, TimePrediction.c:598-632, one axis per lane
     {
@@ -897,14 +910,14 @@ __device__ __forceinline__ void screen_near(FV &F, const ScrTab &T, const FW &wm
         c.dmin = sp.dmin; c.dmax = sp.dmax; c.nstep = sp.nstep; c.ezero = sp.ezero;
         rad = T.rad + sp.off;
     }
-    const Scr sc = screen_shell(c, [&](int k) { return rad[k]; }, con, rr, b, v2);
+    const Scr sc = screen_shell(c, [&](int k) { return rad[k]; }, con, rr, b, v2, ScrBand{F.eb0, F.band0});
     o.t = sc.t; o.e = sc.e; o.ks = sc.ks; o.flag = sc.flag || (rr > rsafe);
 }
 
 // One screened candidate in FP64 (TimePrediction.c:79-179) in the shell the
 // screen found: no radius lies inside the screen's band around the pair's
-// distance, so the FP64 search would end in the same shell, and the shell's
-// limits and energies load together with j's state (one round trip).
+// distance (nor the scan radius), so the FP64 search would end in the same
+// shell, and the shell's limits and energies load together with j's state (one round trip).
 // Returns +inf when it does not reach JobAssign.
 template <class FW>
 __device__ __forceinline__ double coli64_shell(FV &F, const ScrTab &T, const FW &wm, const FAtom &A, int id, int ks,
@@ -971,7 +984,7 @@ __device__ __forceinline__ void collision_fast(FSys &M, FV &F, unsigned long lon
     const int n = uni(wm.coff[27]);
     const double calib64 = (S.cutoffr * SDMD_EXTEND_RATIO) * (S.cutoffr * SDMD_EXTEND_RATIO);
     const float calib = (float)calib64;
-    const float cband = 2e-5f * calib + 1e-5f, rscan = calib + cband, rsafe = calib - cband;
+    const float cband = 2e-5f * calib + F.band0, rscan = calib + cband, rsafe = calib - cband;
     int screened = 0, confirmed = 0;                       // wave-uniform
     int my_causal = 0;
     Best mine;
@@ -2771,6 +2784,9 @@ int sdmd_fast_open(sdmd_gpu_ctx *c, const sdmd_gpu_opts *o) {
         if (F.nblk > FMAXBLK || N >= (1 << 23)) return SDMD_EUNSUPPORTED;
         if (d->cellnum[0] >= 1024 || d->cellnum[1] >= 1024 || d->cellnum[2] >= 1024) return SDMD_EUNSUPPORTED;
         for (int k = 0; k < 3; k++) F.L32[k] = (float)d->cellsize[k];
+        const ScrBand sb = screen_band(fmax(d->cellsize[0], fmax(d->cellsize[1], d->cellsize[2])));
+        F.eb0 = sb.eb0;
+        F.band0 = sb.band0;
         F.Te = d->currenttime;
         F.tlast = d->currenttime;
         F.rebase_dt = 0.5;
