@@ -80,8 +80,9 @@ typedef struct {
     int32_t helpers;       /* fast: helper workgroups per system that take re-predictions on other
                               CUs (0 = as many as the GPU holds beside the owners, -1 = none;
                               with a number, `block` is taken as it is) */
-    int32_t window;        /* plain: neighbour candidates scanned per pass of a prediction (0 = 1728,
-                              the staging area; 1..1728: more passes, the same result) */
+    int32_t window;        /* plain: neighbour candidates scanned per pass of a prediction (0 = as
+                              many as the staging area holds, 768; 1..1728, above 768 like 768:
+                              a smaller window takes more passes and gives the same result) */
 } sdmd_gpu_opts;
 
 /* one popped event (same layout as the reference trace dump) */

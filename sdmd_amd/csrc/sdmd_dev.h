@@ -664,16 +664,9 @@ static __device__ void list_refresh(int *l, int target) {   // ListRefresh(targe
 
 // ---------------------------------------------------------------- events (lane 0), Events.c
 // Positions and cell membership come from a view: V.pos(j, p) stores atom
-// j's position at the event time (the stored position for the swept engine,
-// x0 + v (t - t0) for the local-time engine); V.first(cell) / V.next(cell, j)
+// j's position at the event time (the stored position with the steps it lacks
+// for the swept engine, x0 + v (t - t0) for the local-time engine); V.first(cell) / V.next(cell, j)
 // walk the atoms of a cell (linked list or cell array).
-struct PosStored {
-    const Sys &S;
-    __device__ void pos(int j, double *p) const { p[0] = G(S.x)[j]; p[1] = G(S.y)[j]; p[2] = G(S.z)[j]; }
-    __device__ int first(int cell) const { return G(S.celllist)[S.N + cell]; }
-    __device__ int next(int, int j) const { return G(S.celllist)[j]; }
-};
-
 template <class P>
 static __device__ __forceinline__ void image_near(const Sys &S, const P &V, int i, int j, double *p) {
     const int ci[3] = {G(S.cx)[i], G(S.cy)[i], G(S.cz)[i]}, cj[3] = {G(S.cx)[j], G(S.cy)[j], G(S.cz)[j]};
@@ -837,9 +830,12 @@ static __device__ void hb_event(Sys &S, int i, int j, int nbi, int nbj, int *err
 // Energy sums: workgroup (x, y) of EWAVES wavefronts leaves the sums of its
 // threads' a and b and the OR of their error flags for system x in
 // part[ENERGY_PART * (x * gridDim.y + y) ..]; k_energy_reduce adds a system's
-// workgroups.  Every addition keeps its rounding error (Knuth's TwoSum), so
-// the result is the exact sum of the terms rounded once whatever the split,
-// and the energies of a state are the same on every call.
+// workgroups.  Every addition keeps its rounding error (Knuth's TwoSum), the
+// errors are summed beside the sum and added at the end: the result is off by
+// one rounding and n^2 u^2 times the sum of the terms' absolute values (u =
+// 2^-53) at most, so the split shows only where terms cancel by twelve digits
+// or a sum lies halfway between two numbers.  A state's energies are the same
+// on every call (fixed order).
 constexpr int EWAVES = 4;
 constexpr int ENERGY_PART = 5;            // two sums with their errors, the flag
 struct Sum2 {

@@ -9,8 +9,8 @@
 //                times are absolute, so popping an event touches only the
 //                atoms it involves (UpdateData/TimeForward of
 //                ToolFunctions.c:23-36 disappear)
-//   cells        fixed-capacity cell arrays (count + 64 slots per cell) with
-//                an FP32 mirror record per slot: offset from the cell's
+//   cells        cell arrays (a count and 64 to 1 024 slots per cell, twice the
+//                start's fullest cell) with an FP32 mirror record per slot: offset from the cell's
 //                lower corner, time offset from a system epoch, velocity,
 //                atom id and type
 //   screen       pair times are screened in FP32 on the mirror (cell-relative
@@ -21,9 +21,10 @@
 //                bound are re-solved in FP64 with the reference formulas;
 //                the FP64 minimum is the prediction
 //   batches      each round takes every pending event earlier than the
-//                smallest third-earliest time of any 64-atom block
-//                (second-earliest when that set is too large), so the set
-//                is exactly a prefix of the event order, and executes
+//                smallest third-earliest time of any 64-atom block (when that
+//                set is too large, second-earliest, or in a run of a large
+//                system up to a time those of a window of time), so the set is
+//                exactly a prefix of the event order, and executes
 //                concurrently every event whose atoms are at least
 //                2 cells (3 when a cell crossing or an H-bond event is
 //                involved) and two cell widths from the atoms of every
@@ -66,7 +67,7 @@ constexpr float FINF = 3.0e38f;
 // not a snapshot at one time
 // FERR_JOBS: a round's re-predictions were not all completed within
 // FJOB_WAIT ticks (the wait is bounded so the launch always ends)
-enum { FERR_SELECT = 20, FERR_SLOT = 21, FERR_ROW = 22, FERR_CAND = 23, FERR_NBLK = 24, FERR_CAUSAL = 25,
+enum { FERR_SELECT = 20, FERR_SLOT = 21, FERR_CAUSAL = 25,
        FERR_DRAIN = 26, FERR_JOBS = 27 };
 
 // phases timed (by wavefront 0) when profiling is on
@@ -609,12 +610,6 @@ struct BondPre {
     long long cj;
 };
 
-// 64-bit lane broadcast (the value of lane L to every lane)
-__device__ __forceinline__ long long rl64(long long v, int L) {
-    const int lo = __builtin_amdgcn_readlane((int)v, L);
-    const int hi = __builtin_amdgcn_readlane((int)(v >> 32), L);
-    return (long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo);
-}
 __device__ __forceinline__ int rl32(int v, int L) { return __builtin_amdgcn_readlane(v, L); }
 
 // c_OX, c_OY, c_OZ with two bits per cell (offset + 1)
@@ -1879,12 +1874,6 @@ __device__ __forceinline__ int int_load(int *p) { return __hip_atomic_load(p, __
 // drops it (the s_waitcnt builtin was found removed from the event loop by
 // the wait-count pass, and it does not order memory operations)
 __device__ __forceinline__ void wait_stores() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
-// agent-scope release (L2 write-back), waited for before the caller's next
-// store, which publishes what came before
-__device__ __forceinline__ void release_agent() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-    wait_stores();
-}
 __device__ __forceinline__ void acquire_agent() { __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent"); }
 // the XCD this wavefront runs on (hwreg XCC_ID, bits 3:0)
 __device__ __forceinline__ int xcc_id() { return __builtin_amdgcn_s_getreg((3 << 11) | (0 << 6) | 20) & 15; }
@@ -2940,7 +2929,6 @@ int sdmd_fast_open(sdmd_gpu_ctx *c, const sdmd_gpu_opts *o) {
                                   Sh.nbnum};
             for (int L = 0; L < 10; L++) setg(8 + L, d4[L], 1, 0, 0);
             for (int k = 0; k < SDMD_NBSLOTS; k++) setg(18 + k, Sh.nbp, SDMD_NBSLOTS, k, 0);
-            setg(24, Sh.cmap_off, 1, 0, 0); setg(25, Sh.cmap_off, 1, 1, 0);
             setg(26, Sh.bond_off, 1, 0, 0); setg(27, Sh.bond_off, 1, 1, 0);
             setg(28, Sh.con_off, 1, 0, 0); setg(29, Sh.con_off, 1, 1, 0);
             setg(30, Sh.hbitype, 1, 0, 0); setg(31, F.rowlo, 1, 0, 0);

@@ -141,7 +141,7 @@ __device__ __forceinline__ void pos_now(SYS &S, const Smem &sm, int j, double *p
     p[0] = x; p[1] = y; p[2] = z;
 }
 
-struct PosLazy {      // PosStored with the steps an atom has not taken yet
+struct PosLazy {      // the stored positions with the steps an atom has not taken yet
     const Sys &S;
     const Smem &sm;
     __device__ void pos(int j, double *p) const { pos_now(S, sm, j, p); }

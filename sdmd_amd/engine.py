@@ -108,14 +108,14 @@ class GpuEngine:
 
     mode "plain": the reference's swept FP64 state, bit-exact event sequence.
     mode "fast":  local-time state, FP32 screen + FP64 confirm, concurrent
-                  independent events (one per wavefront); `validate` re-solves
-                  every collision candidate in FP64 and counts agreement;
+                  independent events (one per wavefront); `validate` compares
+                  every prediction with a full FP64 scan and counts agreement;
                   `helpers` workgroups per system take re-predictions on
                   other CUs (0: as many as fit, in workgroups of at most 256
                   threads; -1: none; a number: that many, of `block` threads).
     `window` (plain): neighbour candidates per pass of a prediction's
-    windowed scan (0: 1728); a smaller window takes more passes and gives
-    the same result."""
+    windowed scan (0: 768, also the most); a smaller window takes more passes
+    and gives the same result."""
 
     PHASES = ["pop", "sweep", "event", "stage", "gather", "bondsel", "eval", "select", "hb", "tail", "tree"]
     FAST_PHASES = ["select", "exec", "stage", "screen", "confirm", "other", "tree", "event", "bond", "scan", "collect"]
