@@ -970,8 +970,9 @@ struct HBPre { int role, aanum, protein, hbbond; };
 // A lone wavefront issues a dependent instruction every 8 cycles and an
 // independent one every 5 (measured), so what counts is how often the long
 // screen runs: once per 64 listed candidates instead of once per 64 scanned.
-// VAL: validation mode (the winner of a full FP64 scan compared), a separate
-// instantiation so that the screened path carries none of its state
+// VAL: validation mode (the winner of a full FP64 scan compared), kernels of
+// their own: as a second form inside the same kernels its registers slowed the
+// screened path of the 8-wavefront shape by 14 %
 template <int FQ, bool VAL, class FW>
 __device__ __forceinline__ void collision_fast(FSys &M, FV &F, unsigned long long *prof, const ScrTab &T, FW &wm, const FAtom &A, const Own &own,
                                                Group<FQ> &g, int first, HBPre &hp, Best &best, long long &nscreen,
@@ -1227,7 +1228,7 @@ __device__ __forceinline__ double hbfree64(FV &F, const FAtom &A, int j, double 
 }
 
 // Predict for atom i at time t (its state is at t); writes the event record
-template <int FQ, class FW>
+template <int FQ, bool VAL, class FW>
 __device__ __forceinline__ void predict_fast(FSys &M, FV &F0, unsigned long long *prof, const ScrTab &T, FW &wm, int i,
                                              double t, WStats &ws, int *err) {
     const int lane = threadIdx.x & 63;
@@ -1275,8 +1276,9 @@ __device__ __forceinline__ void predict_fast(FSys &M, FV &F0, unsigned long long
     Best cw = init;
     cw.t = __builtin_inf();
     HBPre hp;
-    if (F.validate) collision_fast<FQ, true>(M, F, prof, T, wm, A, own, g, first, hp, cw, nscreen, nconf, err);
-    else collision_fast<FQ, false>(M, F, prof, T, wm, A, own, g, first, hp, cw, nscreen, nconf, err);
+    // (its own view: the constants read before would be held over it, 407
+    // vector registers spilled against 228 in the 8-wavefront shape)
+    collision_fast<FQ, VAL>(M, view_anew(F0), prof, T, wm, A, own, g, first, hp, cw, nscreen, nconf, err);
     if (prof) pt = wall_clock64();
     // JobAssign order: bonds first, then the collision winner if strictly earlier
     if (cw.partner > 0 && cw.t > 0 && best.t > cw.t) best = cw;
@@ -2059,7 +2061,7 @@ __global__ __launch_bounds__(256) void k_fast_records(FSys *systems) {
 // workgroups per system (one wavefront per atom at a time).  Bound by the
 // instruction count of a prediction (about 9 us on one wavefront); with
 // one workgroup per system a 26 080-atom system took 58 ms on one CU.
-template <int W>
+template <int W, bool VAL>
 __global__ __launch_bounds__(64 * W) void k_fast_predict(FSys *systems) {
     __shared__ FSys Fl;
     __shared__ FWave<flist(W)> w[W];
@@ -2081,7 +2083,7 @@ __global__ __launch_bounds__(64 * W) void k_fast_predict(FSys *systems) {
     wave_sync();
     int err = 0;
     for (int i = 1 + blockIdx.y * W + wave; i <= S.N; i += W * gridDim.y) {
-        predict_fast<4>(F, C, nullptr, tab, w[wave], i, G(F.t0)[i], ws, &err);
+        predict_fast<4, VAL>(F, C, nullptr, tab, w[wave], i, G(F.t0)[i], ws, &err);
         if (__ballot(err != 0)) break;              // uniform across the wave
     }
     if (err) atomicCAS(&Fg.s.error, 0, err);
@@ -2168,7 +2170,7 @@ __global__ __launch_bounds__(64 * EWAVES) void k_fast_energy(FSys *systems, doub
 
 // A helper workgroup: its wavefronts claim the owner's published jobs
 // (re-predictions) until the owner stops, then add their statistics to hp.
-template <int W, int FQ>
+template <int W, int FQ, bool VAL>
 __device__ __forceinline__ void helper_loop(FSys &F, FV &C, const ScrTab &tab, FShared<W> &sh, FJobs *J, FHelp *hp, int xcc) {
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     WStats &ws = sh.w[wave].st;             // in LDS: no registers held across the loop
@@ -2201,7 +2203,7 @@ __device__ __forceinline__ void helper_loop(FSys &F, FV &C, const ScrTab &tab, F
         const double t = J->job[q].t, Te = J->job[q].Te;
         if (lane == 0) F.Te = Te;                // every wave of the round writes the same epoch
         int err = 0;
-        predict_fast<FQ>(F, C, nullptr, tab, sh.w[wave], a, t, ws, &err);
+        predict_fast<FQ, VAL>(F, C, nullptr, tab, sh.w[wave], a, t, ws, &err);
         const bool failed = __ballot(err != 0) != 0;
         if (err) atomicCAS(&J->err, 0, err);
         wait_stores();                           // the event record is in the L2 before the count
@@ -2228,7 +2230,7 @@ __device__ __forceinline__ void helper_loop(FSys &F, FV &C, const ScrTab &tab, F
 // Workgroup b serves system (b % 8) + 8 * ((b / 8) / (1 + H)) as owner
 // (role 0) or helper (roles 1..H), so with round-robin dispatch over the 8
 // XCDs all workgroups of a system share one XCD's L2.
-template <int W, int FQ>
+template <int W, int FQ, bool VAL>
 __global__ __launch_bounds__(64 * W) void k_fast_run(FSys *systems, FJobs *jobs, FHelp *help, int nsys, int H,
                                                      long long npops, long long budget, double t_end) {
     __shared__ FSys Fl;
@@ -2254,7 +2256,7 @@ __global__ __launch_bounds__(64 * W) void k_fast_run(FSys *systems, FJobs *jobs,
             F.max_screen_err = F.max_time_err = 0;
         }
         __syncthreads();
-        helper_loop<W, FQ>(F, C, tab, sh, J, help + sys, xcc);
+        helper_loop<W, FQ, VAL>(F, C, tab, sh, J, help + sys, xcc);
         return;
     }
     if (H > 0 && tid == 0) {                     // helpers on this XCD may join
@@ -2576,7 +2578,7 @@ __global__ __launch_bounds__(64 * W) void k_fast_run(FSys *systems, FJobs *jobs,
         // takes the next one from the LDS counter or from the job word
         for (int r = wave < nren ? wave : -1; r >= 0;) {
             const int q = ren_at(r);
-            predict_fast<FQ>(F, C, prof, tab, sh.w[wave], sh.ren_a[q], sh.ren_t[q], ws, &err);
+            predict_fast<FQ, VAL>(F, C, prof, tab, sh.w[wave], sh.ren_a[q], sh.ren_t[q], ws, &err);
             if (shared && r >= W && lane == 0) job_done(J, false);
             if (__ballot(err != 0)) break;          // uniform across the wave
             r = -1;
@@ -2664,10 +2666,10 @@ __global__ __launch_bounds__(64 * W) void k_fast_run(FSys *systems, FJobs *jobs,
     fsys_store<W>(&systems[sys], Fl);
 }
 
-// The event loop for workgroups of W wavefronts.  This file is compiled once
-// per W with SDMD_FAST_WAVES = W (the units build in parallel; each holds the
-// event loop of its W) and once without it for the host side and the bulk
-// prediction.
+// The event loop for workgroups of W wavefronts.  This file is compiled for
+// each W with SDMD_FAST_WAVES = W, once with and once without SDMD_FAST_VALIDATE
+// (the units build in parallel; each holds the event loop of its W), and once
+// without either for the host side and the bulk prediction.
 struct FastRun {
     hipStream_t stream;
     FSys *sys;
@@ -2677,21 +2679,25 @@ struct FastRun {
     long long npops, budget;
     double t_end;
 };
-template <int W> void fast_launch_run(const FastRun &r);
+template <int W, bool VAL> void fast_launch_run(const FastRun &r);
 
 #ifdef SDMD_FAST_WAVES
-// one workgroup per system and role, 8 * ceil(nsys / 8) * (1 + helpers) in all
-template <int W>
+#ifdef SDMD_FAST_VALIDATE
+constexpr bool FVALIDATE = true;
+#else
+constexpr bool FVALIDATE = false;
+#endif
+// one workgroup per system and role, 8 * ceil(nsys / 8) * (1 + helpers) in
+// all; validation has one staging depth (which does not change results)
+template <int W, bool VAL>
 void fast_launch_run(const FastRun &r) {
     const dim3 g(8 * ((r.nsys + 7) / 8) * (1 + r.helpers)), b(64 * W);
-    if (r.depth == 2)
-        hipLaunchKernelGGL((k_fast_run<W, 2>), g, b, 0, r.stream, r.sys, r.jobs, r.help, r.nsys, r.helpers, r.npops,
-                           r.budget, r.t_end);
-    else
-        hipLaunchKernelGGL((k_fast_run<W, 4>), g, b, 0, r.stream, r.sys, r.jobs, r.help, r.nsys, r.helpers, r.npops,
-                           r.budget, r.t_end);
+    auto *run = &k_fast_run<W, 4, VAL>;
+    if constexpr (!VAL)
+        if (r.depth == 2) run = &k_fast_run<W, 2, VAL>;
+    hipLaunchKernelGGL(run, g, b, 0, r.stream, r.sys, r.jobs, r.help, r.nsys, r.helpers, r.npops, r.budget, r.t_end);
 }
-template void fast_launch_run<SDMD_FAST_WAVES>(const FastRun &);
+template void fast_launch_run<SDMD_FAST_WAVES, FVALIDATE>(const FastRun &);
 #endif
 
 }  // namespace sdmd
@@ -2988,12 +2994,16 @@ static int run_waves(const FastState *fs) {
     return (!fs->tuned && fs->autoshape && fs->helpers > 0 && fs->waves > 4) ? 4 : fs->waves;
 }
 
-#define FDISPATCH(fn, ...) do { switch (run_waves(fs)) { \
-    case 4: fn<4>(__VA_ARGS__); break; \
-    case 8: fn<8>(__VA_ARGS__); break; \
-    case 12: fn<12>(__VA_ARGS__); break; \
-    case 16: fn<16>(__VA_ARGS__); break; \
-    default: fn<1>(__VA_ARGS__); break; } } while (0)
+template <bool VAL>
+static void launch_shape(int waves, const FastRun &r) {
+    switch (waves) {
+    case 4: fast_launch_run<4, VAL>(r); break;
+    case 8: fast_launch_run<8, VAL>(r); break;
+    case 12: fast_launch_run<12, VAL>(r); break;
+    case 16: fast_launch_run<16, VAL>(r); break;
+    default: fast_launch_run<1, VAL>(r); break;
+    }
+}
 
 // the event loop for the context's shape (wavefronts x staging depth x
 // helper workgroups), after a reset of the job words
@@ -3001,7 +3011,8 @@ static void launch_run(sdmd_gpu_ctx *c, long long pops, long long budget, double
     FastState *fs = c->fast;
     hipLaunchKernelGGL(k_fast_jobs_reset, dim3((c->nsys + 255) / 256), dim3(256), 0, c->stream, fs->jobs, c->nsys);
     const FastRun r = {c->stream, fs->dev, fs->jobs, fs->help, c->nsys, fs->helpers, fs->depth, pops, budget, t_end};
-    FDISPATCH(fast_launch_run, r);
+    if (fs->validate) launch_shape<true>(run_waves(fs), r);
+    else launch_shape<false>(run_waves(fs), r);
 }
 
 static int budget_ticks(double max_ms, long long *out) {
@@ -3044,7 +3055,8 @@ int sdmd_fast_prepare(sdmd_gpu_ctx *c) {
     const int want = (maxn + 7) / 8, fit = (1024 + c->nsys - 1) / c->nsys;
     const dim3 gp(c->nsys, want < fit ? want : fit), ga(c->nsys, gp.y < 64 ? gp.y : 64);
     hipLaunchKernelGGL(k_fast_records, ga, dim3(256), 0, c->stream, fs->dev);
-    hipLaunchKernelGGL((k_fast_predict<8>), gp, dim3(512), 0, c->stream, fs->dev);
+    if (fs->validate) hipLaunchKernelGGL((k_fast_predict<8, true>), gp, dim3(512), 0, c->stream, fs->dev);
+    else hipLaunchKernelGGL((k_fast_predict<8, false>), gp, dim3(512), 0, c->stream, fs->dev);
     hipLaunchKernelGGL(k_fast_blocks, ga, dim3(256), 0, c->stream, fs->dev);
     if (hipGetLastError() != hipSuccess) return SDMD_EDEVICE;   // launch rejected (shape, resources)
     HIPV(hipEventRecord(c->ev1, c->stream));
