@@ -20,11 +20,12 @@ LIB = os.path.join(PKG, "libsdmd.so")
 ARCH = os.environ.get("SDMD_OFFLOAD_ARCH", "gfx950")
 
 HOST_SOURCES = ["host/sdmd_host.c", "host/sdmd_remd.c", "host/sdmd_io.c"]
-# (source, extra flags, object): the fast engine's kernels are one unit per
-# workgroup size (SDMD_FAST_WAVES wavefronts), without and with validation,
-# compiled side by side
+# (source, extra flags, object), compiled side by side: the fast engine's
+# kernels are one unit per workgroup size (SDMD_FAST_WAVES wavefronts), without
+# and with validation; the plain event loop is one without and one with phase times
 FAST_WAVES = (8, 4, 16, 12, 1)
 HIP_UNITS = [("sdmd_fast.hip", ["-DSDMD_FAST_WAVES=%d" % w], "sdmd_fast_w%d.o" % w) for w in FAST_WAVES]
+HIP_UNITS += [("sdmd_gpu.hip", ["-DSDMD_PLAIN_RUN=%d" % p], "sdmd_plain%d.o" % p) for p in (0, 1)]
 HIP_UNITS += [("sdmd_gpu.hip", [], "sdmd_gpu.hip.o"), ("sdmd_fast.hip", [], "sdmd_fast.hip.o")]
 HIP_UNITS += [("sdmd_fast.hip", ["-DSDMD_FAST_WAVES=%d" % w, "-DSDMD_FAST_VALIDATE"], "sdmd_fast_w%dv.o" % w)
               for w in FAST_WAVES]

@@ -1379,6 +1379,7 @@ __device__ __forceinline__ void tab_load(PairTab &T, const Sys &S) {
     __syncthreads();
 }
 
+#ifndef SDMD_PLAIN_RUN
 // ---------------------------------------------------------------- bulk Predict(1..N)
 // Prepare predicts the atoms in order (SGThread.c:47-62), and atom i's
 // CheckDuplication may take over the record of an earlier atom j whose event
@@ -1534,9 +1535,25 @@ __global__ __launch_bounds__(B) void k_bulk_finish(Sys *systems) {
     sys_store<B>(&systems[blockIdx.x], Sl);
 }
 
+#endif  // SDMD_PLAIN_RUN
+
+// ---------------------------------------------------------------- event loop
+// Compiled apart (this file with SDMD_PLAIN_RUN = 0 and = 1, beside the unit
+// without it): phase times have kernels of their own, because their marks cost
+// a run that takes none 2 %.
+struct PlainRun {
+    hipStream_t stream;
+    Sys *sys;
+    int nsys;
+    long long npops, budget;
+    double t_end, t_out;
+};
+template <int B, bool PROF> void plain_launch_run(const PlainRun &r);
+
+#ifdef SDMD_PLAIN_RUN
 // t_out: stop after the first executed event that leaves the clock at or
 // past t_out -- where SingleThreadRun writes its output (SGThread.c:130-139)
-template <int B>
+template <int B, bool PROF>
 __global__ __launch_bounds__(B) void k_run(Sys *systems, long long npops, long long budget, double t_end,
                                            double t_out) {
     __shared__ Smem sm;
@@ -1546,7 +1563,7 @@ __global__ __launch_bounds__(B) void k_run(Sys *systems, long long npops, long l
     sys_load<B>(Sl, &systems[blockIdx.x]);
     Sys &S = Sl;                           // counters and clock
     SV &V = fixed_view(systems + blockIdx.x);
-    unsigned long long *const prof = V.prof;
+    unsigned long long *const prof = PROF ? V.prof : nullptr;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const unsigned long long t_start = wall_clock64();
     // npops < 0 asks for -npops executed events instead of pops
@@ -1615,6 +1632,18 @@ __global__ __launch_bounds__(B) void k_run(Sys *systems, long long npops, long l
     sys_store<B>(&systems[blockIdx.x], Sl);
 }
 
+template <int B, bool PROF>
+void plain_launch_run(const PlainRun &r) {
+    hipLaunchKernelGGL((k_run<B, PROF>), dim3(r.nsys), dim3(B), 0, r.stream, r.sys, r.npops, r.budget, r.t_end, r.t_out);
+}
+template void plain_launch_run<64, SDMD_PLAIN_RUN>(const PlainRun &);
+template void plain_launch_run<128, SDMD_PLAIN_RUN>(const PlainRun &);
+template void plain_launch_run<256, SDMD_PLAIN_RUN>(const PlainRun &);
+template void plain_launch_run<512, SDMD_PLAIN_RUN>(const PlainRun &);
+template void plain_launch_run<1024, SDMD_PLAIN_RUN>(const PlainRun &);
+
+}  // namespace sdmd
+#else
 // cell arrays from the lists, for every cell of every system
 __global__ __launch_bounds__(256) void k_cells(const Sys *systems) {
     const Sys &S = systems[blockIdx.x];
@@ -2067,7 +2096,9 @@ static void launch_prepare(sdmd_gpu_ctx *c) {
 }
 template <int B>
 static void launch_run(sdmd_gpu_ctx *c, long long n, long long budget, double t_end, double t_out) {
-    hipLaunchKernelGGL((k_run<B>), dim3(c->nsys), dim3(B), 0, c->stream, c->dev_sys, n, budget, t_end, t_out);
+    const PlainRun r = {c->stream, c->dev_sys, c->nsys, n, budget, t_end, t_out};
+    if (c->host_sys[0].prof) plain_launch_run<B, true>(r);
+    else plain_launch_run<B, false>(r);
 }
 template <int B>
 static void launch_op(sdmd_gpu_ctx *c, int s, int op, Renew renew, int a, int b) {
@@ -2544,3 +2575,4 @@ extern "C" int sdmd_gpu_run_graph(sdmd_gpu_ctx *c, int32_t launches, double max_
     if (c->mode != SDMD_MODE_FAST) return SDMD_EUNSUPPORTED;
     return sdmd_fast_run_graph(c, launches, max_ms);
 }
+#endif  // SDMD_PLAIN_RUN
