@@ -65,7 +65,9 @@ typedef struct {
     int32_t mode;          /* SDMD_MODE_PLAIN or SDMD_MODE_FAST */
     int32_t block;         /* threads per system workgroup: plain 64..1024 (power of two),
                               fast 64, 256, 512 or 1024 (one re-prediction per wavefront
-                              at a time; the autotuner may also pick 768); 0 = 256.  Fast: 512
+                              at a time; the autotuner may also pick 768); 0 = 256.  Plain: 64
+                              and 128 run as 256 where there are more systems than CUs (a
+                              workgroup takes a CU to itself; same results).  Fast: 512
                               and more run as 256 where the number of helpers is left to the
                               engine too and helpers share the predictions (the faster shape;
                               same results), unless the autotuner measured otherwise */

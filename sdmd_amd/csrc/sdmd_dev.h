@@ -916,6 +916,7 @@ struct sdmd_dyn_block { char *dev; size_t bytes; };
 struct sdmd_gpu_ctx {
     int nsys;
     int block;
+    int run_block;             // plain event loop: see sdmd_gpu_open
     int mode;
     hipStream_t stream;
     hipEvent_t ev0, ev1;

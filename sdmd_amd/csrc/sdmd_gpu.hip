@@ -1999,6 +1999,14 @@ extern "C" int sdmd_gpu_open(const sdmd_system_desc *const *systems, int32_t nsy
     c->nsys = nsys;
     c->block = block;
     c->mode = mode;
+    // an event loop's workgroup fills a CU's LDS (130 KB of tables and
+    // candidates): with more systems than CUs a small one leaves the other
+    // SIMDs idle while systems wait (400 pops of 512 systems of 59 atoms: 64
+    // threads 15.3 ms, 256 threads 10.4 ms)
+    int cus = 0, at = 0;
+    if (hipGetDevice(&at) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, at) != hipSuccess)
+        cus = 0;
+    c->run_block = (cus > 0 && nsys > cus && block < 256) ? 256 : block;
     if (hipStreamCreate(&c->stream) != hipSuccess) { free(c); return SDMD_EDEVICE; }
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || resolve_scratch(dev, &c->scratch) != SDMD_OK) {
@@ -2105,7 +2113,7 @@ static void launch_op(sdmd_gpu_ctx *c, int s, int op, Renew renew, int a, int b)
     hipLaunchKernelGGL((k_op<B>), dim3(1), dim3(B), 0, c->stream, c->dev_sys, s, op, renew, a, b, c->status);
 }
 
-#define DISPATCH(fn, ...) do { switch (c->block) { \
+#define DISPATCH(block, fn, ...) do { switch (block) { \
     case 64: fn<64>(__VA_ARGS__); break; case 128: fn<128>(__VA_ARGS__); break; \
     case 256: fn<256>(__VA_ARGS__); break; case 512: fn<512>(__VA_ARGS__); break; \
     default: fn<1024>(__VA_ARGS__); break; } } while (0)
@@ -2170,7 +2178,7 @@ static int run_bounded(sdmd_gpu_ctx *c, int64_t pops, double max_ms, double t_en
         budget = (long long)(max_ms * khz);
     }
     HIPV(hipEventRecord(c->ev0, c->stream));
-    DISPATCH(launch_run, c, (long long)pops, budget, t_end, t_out);
+    DISPATCH(c->run_block, launch_run, c, (long long)pops, budget, t_end, t_out);
     HIPV(hipEventRecord(c->ev1, c->stream));
     if (hipGetLastError() != hipSuccess) return SDMD_EDEVICE;
     if (hipStreamSynchronize(c->stream) != hipSuccess) return SDMD_EDEVICE;
@@ -2203,7 +2211,7 @@ static int run_op(sdmd_gpu_ctx *c, int s, int op, const int32_t *renew, int a, i
         for (int k = 1; k <= n; k++)
             if (list.a[k] < 1 || list.a[k] > c->host_sys[s].N) return SDMD_EINVAL;
     }
-    DISPATCH(launch_op, c, s, op, list, a, b);
+    DISPATCH(c->block, launch_op, c, s, op, list, a, b);
     return op_result(c, s);
 }
 
@@ -2482,7 +2490,7 @@ extern "C" int sdmd_remd_run(sdmd_gpu_ctx *c, sdmd_remd_temp *temps, sdmd_rand_s
     for (int cy = 0; cy < cycles && !rc; cy++) {
         if (c->mode == SDMD_MODE_FAST) rc = sdmd_fast_launch_events(c, interval);
         else {
-            DISPATCH(launch_run, c, (long long)-interval, 1LL << 62, INFINIT, INFINITY);
+            DISPATCH(c->run_block, launch_run, c, (long long)-interval, 1LL << 62, INFINIT, INFINITY);
             rc = hip_ok(hipGetLastError());
         }
         if (!rc) rc = energy_launch(c, c->dev_energy);
